@@ -115,24 +115,34 @@ struct JobDev {
 
 // One Widom binning job: insertion points of (seed, stream) sorted into a
 // regular grid of fractional bins.  Plain-old-data; kernels take an array.
+// A job of many bins is sorted in two steps: into `ngroups` groups of `group`
+// consecutive bins, then each group into its bins (group = 1: one step).
 struct BinJob {
     uint64_t seed;
     uint64_t n;            // insertions
     uint32_t stream;
     int nb[3];             // bins per fractional axis
-    uint32_t *count;       // nbins + 1 counts (zeroed by k_bin_zero)
+    int group;             // bins per group
+    int ngroups;           // ceil(bins / group)
+    uint32_t *count;       // group counts (zeroed by k_bin_zero)
     uint32_t *start;       // nbins + 1 exclusive prefix sums
-    uint32_t *cursor;      // nbins fill cursors
+    uint32_t *cursor;      // ngroups + 1 fill cursors; a group's end after the scatter
     uint32_t *sorted;      // n insertion indices, grouped by bin
+    uint2 *tmp;            // two steps: n (bin in its group, insertion) pairs, grouped
     long long block0;      // first binning block of this job in a launch
+    long long gblock0;     // first second-step block (one per group) of this job
 };
 
 // Kernel launch geometry.
 constexpr int kWG = 256;      // threads per workgroup (4 wave64)
 constexpr int kMaxSeg = 64;   // list segments per fill pass
 constexpr int kMaxTypes = 64; // pair types a region sub-list can index
-constexpr int kLdsBinsMax = 32768; // Widom bins a binning block histograms in LDS (128 KiB)
-constexpr int kBinChunk = 16384;  // insertions per binning block
+constexpr int kBinWG = 1024;      // threads of a binning scatter block
+constexpr int kBinChunkMax = 16384;  // insertions per binning block, at most
+constexpr int kBinGroups = 1024;  // groups of a Widom job that is binned in two steps
+constexpr int kBinDirectMax = 4096;  // bins up to which a job is binned in one step
+constexpr int kBinGroupMax = 15360;  // bins a group may hold (the second step's LDS counts)
+constexpr int kBinLdsKeys = 7168;    // keys a binning block histograms in LDS (28 KiB)
 constexpr int kRegionRecords = 8192;  // entries of one workgroup's region sub-list (near-list
                                       // indices, 32 KiB)
 constexpr long long kMinGridItems = 2048;  // regions per grid before regions shrink

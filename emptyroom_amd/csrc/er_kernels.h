@@ -48,11 +48,17 @@ hipError_t launch_fill_u64(unsigned long long *p, unsigned long long v, long lon
 
 // --- Widom binning (batched) --------------------------------------------------
 // jobs: device array of njobs BinJob whose block0 fields number the blocks of
-// `chunk` insertions each; total_blocks = sum over jobs of ceil(n / chunk).
-// Order: zero, count, scan, scatter (all on one stream).
+// `chunk` insertions each (total_blocks = sum over jobs of ceil(n / chunk)) and
+// whose gblock0 fields number the groups of the grouped jobs (total_groups).
+// max_keys: largest ngroups; max_group: largest group.
+// Order: zero, count, scan, scatter, sort of the groups (all on one stream).
 hipError_t launch_bin_all(const BinJob *jobs, int njobs, long long total_blocks, int chunk,
-                          long long max_bins, hipStream_t s);
+                          long long max_keys, int max_group, long long total_groups,
+                          hipStream_t s);
 int bin_blocks(uint64_t n, int chunk);
+int bin_chunk(uint64_t total_insertions, long long max_keys);
+// Group size and count for a job of nbins bins (group 1: binned in one step).
+void bin_groups(long long nbins, int *group, int *ngroups);
 
 // --- tiled energy kernel ------------------------------------------------------
 // Runs the work items [0, total_items) of the jobs (device array) with a

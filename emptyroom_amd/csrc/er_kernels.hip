@@ -182,15 +182,26 @@ __device__ __forceinline__ uint32_t widom_bin(const double f[3], const int nb[3]
     return (uint32_t)((b[0] * nb[1] + b[1]) * nb[2] + b[2]);
 }
 
-// Batched binning.  Each block takes `chunk` consecutive insertion indices of
-// one job, histograms their bins in LDS and touches global memory once per
-// bin it saw: the count pass adds its counts, the scatter pass reserves a
-// range of the bin's slots and hands them out through LDS atomics.  The order
-// inside a bin is therefore arbitrary; no result depends on it (every
-// insertion of a bin sees the same candidate list, and sums run over
-// insertion indices).  The histogram lives in dynamic LDS sized per launch
-// for the largest job's bins (lds_bins, at most kLdsBinsMax); jobs with more
-// bins than that use one global atomic per insertion.
+// Batched binning.  A job's keys are its bins, or, when it has many, groups of
+// consecutive bins.  Each block takes `chunk` consecutive insertion indices of
+// one job, histograms their keys in LDS and touches global memory once per key
+// it saw: the count pass adds its counts, the scatter pass reserves a range of
+// the key's slots and hands them out through LDS atomics.  A grouped job's
+// scatter writes (bin in the group, insertion) pairs, which a last pass, one
+// block per group, sorts into bins.  The order inside a bin is therefore
+// arbitrary; no result depends on it (every insertion of a bin sees the same
+// candidate list, and sums run over insertion indices).
+//
+// A Philox point costs ~20 quarter-rate multiplies, so only the count pass
+// makes the points; it leaves each insertion's bin for the scatter pass in the
+// one of `sorted` and `tmp` that the scatter does not write.
+//
+// The groups keep the histogram at a few KiB and the scattered runs long:
+// 1.73e7 insertions of 36036 bins took 711 us to count and 1364 us to scatter
+// with one global atomic per insertion; now 64 us to count (the points), 67 us
+// to scatter and 80 us to sort the groups.  The scatter is bound by its stores:
+// written straight from the lanes they took 241 us.  16 jobs of 1e6 insertions
+// and ~2080 bins each (one step): 48 + 159 us before, 51 + 69 us now.
 __device__ __forceinline__ int bin_job_of(const BinJob *__restrict__ jobs, int njobs,
                                           long long blk) {
     int lo = 0, hi = njobs - 1;
@@ -204,80 +215,181 @@ __device__ __forceinline__ int bin_job_of(const BinJob *__restrict__ jobs, int n
 
 __global__ __launch_bounds__(kWG) void k_bin_zero(const BinJob *__restrict__ jobs) {
     const BinJob &J = jobs[blockIdx.x];
-    const long long nbt = (long long)J.nb[0] * J.nb[1] * J.nb[2];
-    for (long long b = threadIdx.x; b <= nbt; b += kWG) J.count[b] = 0u;
+    for (int b = threadIdx.x; b < J.ngroups; b += kWG) J.count[b] = 0u;
 }
 
 __global__ __launch_bounds__(kWG) void k_bin_count(const BinJob *__restrict__ jobs, int njobs,
-                                                   int chunk, int lds_bins) {
+                                                   int chunk, int lds_keys) {
     extern __shared__ uint32_t s_hist[];
     const int j = bin_job_of(jobs, njobs, blockIdx.x);
     const BinJob &J = jobs[j];
     const uint64_t i0 = (uint64_t)(blockIdx.x - J.block0) * (uint64_t)chunk;
     const uint64_t i1 = i0 + (uint64_t)chunk < J.n ? i0 + (uint64_t)chunk : J.n;
-    const int nbt = J.nb[0] * J.nb[1] * J.nb[2];
-    if (nbt > lds_bins) {
-        for (uint64_t i = i0 + threadIdx.x; i < i1; i += kWG) {
-            double f[3];
-            widom_point(J.seed, J.stream, i, f);
-            atomicAdd(&J.count[widom_bin(f, J.nb)], 1u);
-        }
-        return;
+    const uint32_t group = (uint32_t)J.group;
+    const bool lds = J.ngroups <= lds_keys;
+    uint32_t *__restrict__ keys = group > 1 ? J.sorted : reinterpret_cast<uint32_t *>(J.tmp);
+    if (lds) {
+        for (int b = threadIdx.x; b < J.ngroups; b += kWG) s_hist[b] = 0u;
+        __syncthreads();
     }
-    for (int b = threadIdx.x; b < nbt; b += kWG) s_hist[b] = 0u;
-    __syncthreads();
     for (uint64_t i = i0 + threadIdx.x; i < i1; i += kWG) {
         double f[3];
         widom_point(J.seed, J.stream, i, f);
-        atomicAdd(&s_hist[widom_bin(f, J.nb)], 1u);
+        const uint32_t bin = widom_bin(f, J.nb);
+        const uint32_t key = group > 1 ? bin / group : bin;
+        keys[i] = bin;
+        atomicAdd(lds ? &s_hist[key] : &J.count[key], 1u);
     }
+    if (!lds) return;
     __syncthreads();
-    for (int b = threadIdx.x; b < nbt; b += kWG)
+    for (int b = threadIdx.x; b < J.ngroups; b += kWG)
         if (s_hist[b]) atomicAdd(&J.count[b], s_hist[b]);
 }
 
 __global__ __launch_bounds__(kWG) void k_bin_scan(const BinJob *__restrict__ jobs) {
     const BinJob &J = jobs[blockIdx.x];
-    const long long nbt = (long long)J.nb[0] * J.nb[1] * J.nb[2];
-    block_exclusive_scan(J.count, nbt, J.start, J.cursor);
+    block_exclusive_scan(J.count, J.ngroups, J.cursor, J.group > 1 ? nullptr : J.start);
 }
 
-__global__ __launch_bounds__(kWG) void k_bin_scatter(const BinJob *__restrict__ jobs, int njobs,
-                                                     int chunk, int lds_bins) {
+// A thread holds the keys of its PER insertions: they are read once, with PER
+// loads in flight.  The block sorts its insertions by key in LDS before it
+// writes them, so that a wave's store covers a few runs of consecutive slots
+// instead of 64 separate lines.
+template <int PER>
+__global__ __launch_bounds__(kBinWG) void k_bin_scatter(const BinJob *__restrict__ jobs,
+                                                        int njobs, int lds_keys) {
     extern __shared__ uint32_t s_hist[];
+    __shared__ uint32_t s_part[kBinWG / 64];
+    constexpr int chunk = PER * kBinWG;
+    const int tid = threadIdx.x;
     const int j = bin_job_of(jobs, njobs, blockIdx.x);
     const BinJob &J = jobs[j];
     const uint64_t i0 = (uint64_t)(blockIdx.x - J.block0) * (uint64_t)chunk;
-    const uint64_t i1 = i0 + (uint64_t)chunk < J.n ? i0 + (uint64_t)chunk : J.n;
-    const int nbt = J.nb[0] * J.nb[1] * J.nb[2];
-    if (nbt > lds_bins) {
-        for (uint64_t i = i0 + threadIdx.x; i < i1; i += kWG) {
-            double f[3];
-            widom_point(J.seed, J.stream, i, f);
-            const uint32_t pos = atomicAdd(&J.cursor[widom_bin(f, J.nb)], 1u);
-            J.sorted[pos] = (uint32_t)i;
+    const int cnt = (int)(J.n - i0 < (uint64_t)chunk ? J.n - i0 : (uint64_t)chunk);
+    const uint32_t group = (uint32_t)J.group;
+    const int nk = J.ngroups;
+    const uint32_t *__restrict__ keys =
+        (group > 1 ? J.sorted : reinterpret_cast<const uint32_t *>(J.tmp)) + i0;
+    uint32_t bin[PER];
+#pragma unroll
+    for (int q = 0; q < PER; ++q) {
+        const int l = q * kBinWG + tid;
+        bin[q] = keys[l < cnt ? l : 0];
+    }
+    if (nk > lds_keys) {
+#pragma unroll
+        for (int q = 0; q < PER; ++q) {
+            const int l = q * kBinWG + tid;
+            if (l >= cnt) continue;
+            const uint32_t key = group > 1 ? bin[q] / group : bin[q];
+            const uint32_t pos = atomicAdd(&J.cursor[key], 1u);
+            if (group > 1) J.tmp[pos] = make_uint2(bin[q] - key * group, (uint32_t)(i0 + l));
+            else J.sorted[pos] = (uint32_t)(i0 + l);
         }
         return;
     }
-    for (int b = threadIdx.x; b < nbt; b += kWG) s_hist[b] = 0u;
+    // s_hist[nk]: counts, then first slots in the block's order; s_dst[nk]:
+    // first slot in the job's order; s_key, s_loc[chunk]: the sorted insertions
+    uint32_t *s_dst = s_hist + nk;
+    uint32_t *s_loc = s_dst + nk;
+    uint16_t *s_key = reinterpret_cast<uint16_t *>(s_loc + chunk);
+    for (int b = tid; b < nk; b += kBinWG) s_hist[b] = 0u;
     __syncthreads();
-    for (uint64_t i = i0 + threadIdx.x; i < i1; i += kWG) {
-        double f[3];
-        widom_point(J.seed, J.stream, i, f);
-        atomicAdd(&s_hist[widom_bin(f, J.nb)], 1u);
+#pragma unroll
+    for (int q = 0; q < PER; ++q)
+        if (q * kBinWG + tid < cnt)
+            atomicAdd(&s_hist[group > 1 ? bin[q] / group : bin[q]], 1u);
+    __syncthreads();
+    // exclusive scan of the counts (consecutive keys per thread), each key's
+    // share of the job's slots reserved on the way
+    const int per = (nk + kBinWG - 1) / kBinWG;
+    const int p0 = tid * per < nk ? tid * per : nk, p1 = p0 + per < nk ? p0 + per : nk;
+    uint32_t sum = 0;
+    for (int b = p0; b < p1; ++b) sum += s_hist[b];
+    uint32_t inc = sum;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+        const uint32_t v = __shfl_up(inc, d, 64);
+        if ((tid & 63) >= d) inc += v;
+    }
+    if ((tid & 63) == 63) s_part[tid >> 6] = inc;
+    __syncthreads();
+    uint32_t run = inc - sum;
+    for (int w = 0; w < (tid >> 6); ++w) run += s_part[w];
+    for (int b = p0; b < p1; ++b) {
+        const uint32_t c = s_hist[b];
+        s_hist[b] = run;
+        // dst - first: what a slot in the block's order is moved by
+        if (c) s_dst[b] = atomicAdd(&J.cursor[b], c) - run;
+        run += c;
     }
     __syncthreads();
-    // reserve each bin's share of slots; s_hist then holds this block's next slot
-    for (int b = threadIdx.x; b < nbt; b += kWG) {
-        const uint32_t h = s_hist[b];
-        if (h) s_hist[b] = atomicAdd(&J.cursor[b], h);
+#pragma unroll
+    for (int q = 0; q < PER; ++q) {
+        const int l = q * kBinWG + tid;
+        if (l >= cnt) continue;
+        const uint32_t key = group > 1 ? bin[q] / group : bin[q];
+        const uint32_t slot = atomicAdd(&s_hist[key], 1u);
+        s_key[slot] = (uint16_t)key;
+        // bin in the group (< kBinGroupMax < 2^14) and insertion in the chunk (< 2^14)
+        s_loc[slot] = (uint32_t)l | ((bin[q] - key * group) << 14);
     }
     __syncthreads();
-    for (uint64_t i = i0 + threadIdx.x; i < i1; i += kWG) {
-        double f[3];
-        widom_point(J.seed, J.stream, i, f);
-        const uint32_t pos = atomicAdd(&s_hist[widom_bin(f, J.nb)], 1u);
-        J.sorted[pos] = (uint32_t)i;
+    for (int l = tid; l < cnt; l += kBinWG) {
+        const uint32_t v = s_loc[l], pos = s_dst[s_key[l]] + (uint32_t)l;
+        const uint32_t ins = (uint32_t)i0 + (v & 0x3fffu);
+        if (group > 1) J.tmp[pos] = make_uint2(v >> 14, ins);
+        else J.sorted[pos] = ins;
+    }
+}
+
+// Second step of grouped jobs: block = one group, whose pairs lie between the
+// cursors its neighbour and itself ended at.
+__global__ __launch_bounds__(kWG) void k_bin_fine(const BinJob *__restrict__ jobs, int njobs) {
+    extern __shared__ uint32_t s_cnt[];
+    __shared__ uint32_t s_part[kWG];
+    int lo = 0, hi = njobs - 1;
+    while (lo < hi) {
+        const int mid = (lo + hi + 1) >> 1;
+        if (jobs[mid].gblock0 <= blockIdx.x) lo = mid;
+        else hi = mid - 1;
+    }
+    const BinJob &J = jobs[lo];
+    const int g = (int)(blockIdx.x - J.gblock0);
+    if (J.group <= 1 || g >= J.ngroups) return;
+    const int tid = threadIdx.x;
+    const int nbt = J.nb[0] * J.nb[1] * J.nb[2], b0 = g * J.group;
+    const int nb = b0 + J.group < nbt ? J.group : nbt - b0;
+    const uint32_t e0 = g > 0 ? J.cursor[g - 1] : 0u, e1 = J.cursor[g];
+    for (int b = tid; b < nb; b += kWG) s_cnt[b] = 0u;
+    __syncthreads();
+    for (uint32_t e = e0 + tid; e < e1; e += kWG) atomicAdd(&s_cnt[J.tmp[e].x], 1u);
+    __syncthreads();
+    // exclusive scan of the group's bins: per consecutive counts per thread
+    const int per = (nb + kWG - 1) / kWG;
+    const int p0 = tid * per < nb ? tid * per : nb, p1 = p0 + per < nb ? p0 + per : nb;
+    uint32_t sum = 0;
+    for (int b = p0; b < p1; ++b) sum += s_cnt[b];
+    s_part[tid] = sum;
+    __syncthreads();
+    for (int d = 1; d < kWG; d <<= 1) {
+        const uint32_t add = tid >= d ? s_part[tid - d] : 0u;
+        __syncthreads();
+        s_part[tid] += add;
+        __syncthreads();
+    }
+    uint32_t run = e0 + s_part[tid] - sum;
+    for (int b = p0; b < p1; ++b) {
+        const uint32_t c = s_cnt[b];
+        s_cnt[b] = run;
+        J.start[b0 + b] = run;
+        run += c;
+    }
+    if (g == J.ngroups - 1 && tid == 0) J.start[nbt] = (uint32_t)J.n;
+    __syncthreads();
+    for (uint32_t e = e0 + tid; e < e1; e += kWG) {
+        const uint2 v = J.tmp[e];
+        J.sorted[atomicAdd(&s_cnt[v.x], 1u)] = v.y;
     }
 }
 
@@ -1495,33 +1607,55 @@ hipError_t launch_fill_u64(unsigned long long *p, unsigned long long v, long lon
 
 int bin_blocks(uint64_t n, int chunk) { return (int)((n + (uint64_t)chunk - 1) / (uint64_t)chunk); }
 
+// Insertions per binning block: long chunks give long runs per key and few
+// global atomics, but a launch needs ~1000 blocks, and a block zeroes and
+// flushes its whole histogram, which a chunk of 2 insertions per key pays for.
+int bin_chunk(uint64_t total_insertions, long long max_keys) {
+    int chunk = kBinWG;
+    while (chunk < kBinChunkMax && ((uint64_t)chunk * 1024 < total_insertions || chunk < 2 * max_keys))
+        chunk <<= 1;
+    return chunk;
+}
+
+void bin_groups(long long nbins, int *group, int *ngroups) {
+    long long g = 1;
+    if (nbins > kBinDirectMax) g = (nbins + kBinGroups - 1) / kBinGroups;
+    if (g > kBinGroupMax) g = kBinGroupMax;
+    *group = (int)g;
+    *ngroups = (int)((nbins + g - 1) / g);
+}
+
 hipError_t launch_bin_all(const BinJob *jobs, int njobs, long long total_blocks, int chunk,
-                          long long max_bins, hipStream_t s) {
+                          long long max_keys, int max_group, long long total_groups,
+                          hipStream_t s) {
     if (njobs <= 0 || total_blocks <= 0) return hipSuccess;
-    if (chunk < kWG || total_blocks > (1LL << 31) - 1 || max_bins <= 0) return hipErrorInvalidValue;
-    // histogram in LDS for every job when the largest fits, sized for it
-    int lds_bins = max_bins <= kLdsBinsMax ? (int)max_bins : 0;
-    if (lds_bins > 16384) {
-        // more than 64 KiB of dynamic LDS must be allowed per kernel
-        static const bool big_lds_ok =
-            hipFuncSetAttribute((const void *)k_bin_count,
-                                hipFuncAttributeMaxDynamicSharedMemorySize,
-                                kLdsBinsMax * (int)sizeof(uint32_t)) == hipSuccess &&
-            hipFuncSetAttribute((const void *)k_bin_scatter,
-                                hipFuncAttributeMaxDynamicSharedMemorySize,
-                                kLdsBinsMax * (int)sizeof(uint32_t)) == hipSuccess;
-        if (!big_lds_ok) {
-            (void)hipGetLastError();
-            lds_bins = 0;
-        }
-    }
-    const size_t lds_bytes = sizeof(uint32_t) * (size_t)(lds_bins > 0 ? lds_bins : 1);
+    if (chunk < kBinWG || chunk > kBinChunkMax || (chunk & (chunk - 1)) ||
+        total_blocks > (1LL << 31) - 1 || max_keys <= 0 || max_group < 1 ||
+        max_group > kBinGroupMax || total_groups < 0 || total_groups > (1LL << 31) - 1)
+        return hipErrorInvalidValue;
+    // a job whose keys do not fit the histogram uses one global atomic per insertion
+    const int lds_keys = (int)(max_keys < kBinLdsKeys ? max_keys : kBinLdsKeys);
+    const size_t lds_bytes = sizeof(uint32_t) * (size_t)lds_keys;
     hipLaunchKernelGGL(k_bin_zero, dim3(njobs), dim3(kWG), 0, s, jobs);
     hipLaunchKernelGGL(k_bin_count, dim3((unsigned)total_blocks), dim3(kWG), lds_bytes, s, jobs,
-                       njobs, chunk, lds_bins);
+                       njobs, chunk, lds_keys);
     hipLaunchKernelGGL(k_bin_scan, dim3(njobs), dim3(kWG), 0, s, jobs);
-    hipLaunchKernelGGL(k_bin_scatter, dim3((unsigned)total_blocks), dim3(kWG), lds_bytes, s, jobs,
-                       njobs, chunk, lds_bins);
+    const size_t scatter_lds = 2 * lds_bytes + 6 * (size_t)chunk;
+#define ER_SCATTER(P)                                                                          \
+    if (chunk == P * kBinWG) {                                                                 \
+        static const bool lds_ok =                                                             \
+            hipFuncSetAttribute((const void *)k_bin_scatter<P>,                                \
+                                hipFuncAttributeMaxDynamicSharedMemorySize,                    \
+                                8 * kBinLdsKeys + 6 * P * kBinWG) == hipSuccess;               \
+        if (!lds_ok) return hipErrorInvalidValue;                                              \
+        hipLaunchKernelGGL(k_bin_scatter<P>, dim3((unsigned)total_blocks), dim3(kBinWG),       \
+                           scatter_lds, s, jobs, njobs, lds_keys);                             \
+    }
+    ER_SCATTER(1) ER_SCATTER(2) ER_SCATTER(4) ER_SCATTER(8) ER_SCATTER(16)
+#undef ER_SCATTER
+    if (total_groups > 0)
+        hipLaunchKernelGGL(k_bin_fine, dim3((unsigned)total_groups), dim3(kWG),
+                           sizeof(uint32_t) * (size_t)max_group, s, jobs, njobs);
     return hipGetLastError();
 }
 

@@ -711,17 +711,21 @@ BinJob make_bin_job(const WidomBuffers &wb, uint64_t n_ins, uint64_t seed, uint3
     j.start = wb.start;
     j.cursor = wb.cursor;
     j.sorted = wb.sorted;
-    j.block0 = 0;
+    // the energies are written after the binning: their n doubles hold its n pairs
+    static_assert(sizeof(uint2) == sizeof(double), "binning pairs share the energy buffer");
+    j.tmp = reinterpret_cast<uint2 *>(wb.e);
+    bin_groups((long long)wb.nbins[0] * wb.nbins[1] * wb.nbins[2], &j.group, &j.ngroups);
     return j;
 }
 
 int widom_enqueue_binning(Context *ctx, WidomBuffers &wb, uint64_t n_ins, uint64_t seed,
                           uint32_t stream_id, hipStream_t s) {
     (void)ctx;
-    const long long nb = (long long)wb.nbins[0] * wb.nbins[1] * wb.nbins[2];
     wb.job = make_bin_job(wb, n_ins, seed, stream_id);
     HIP_TRY(hipMemcpyAsync(wb.d_job, &wb.job, sizeof(BinJob), hipMemcpyHostToDevice, s));
-    HIP_TRY(launch_bin_all(wb.d_job, 1, bin_blocks(n_ins, kBinChunk), kBinChunk, nb, s));
+    const int chunk = bin_chunk(n_ins, wb.job.ngroups);
+    HIP_TRY(launch_bin_all(wb.d_job, 1, bin_blocks(n_ins, chunk), chunk, wb.job.ngroups,
+                           wb.job.group, wb.job.group > 1 ? wb.job.ngroups : 0, s));
     return ST_OK;
 }
 
@@ -960,8 +964,8 @@ double job_cost_per_item(const FrameworkDev *fw, const JobDev &j, const Tuning &
 
 int Batch::record(hipStream_t s) {
     // every Widom task's binning in one launch per phase
-    HIP_TRY(launch_bin_all(d_bin_jobs, (int)bin_jobs.size(), bin_blocks_total, kBinChunk,
-                           std::max<long long>(bin_max, 1), s));
+    HIP_TRY(launch_bin_all(d_bin_jobs, (int)bin_jobs.size(), bin_blocks_total, bin_chunk_len,
+                           bin_max_keys, bin_max_group, bin_groups_total, s));
     // jobs are partitioned: [0, n_mixed) mixed math, [n_mixed, njobs) FP64 grids
     int n_mixed = 0;
     long long items_mixed = 0, items_fp64 = 0;
@@ -1015,6 +1019,7 @@ int batch_create(Context *ctx, const Task *tasks, int n, bool use_graph, Batch *
         return st;
     };
     std::vector<std::pair<double, JobDev>> mixed, fp64;
+    uint64_t ins_total = 0;
     for (int t = 0; t < n; t++) {
         const Task &tk = tasks[t];
         if (!tk.fw) {
@@ -1053,10 +1058,11 @@ int batch_create(Context *ctx, const Task *tasks, int n, bool use_graph, Batch *
             int st = widom_prepare(ctx, tk.fw, tk.n_ins, &b->wbufs[t], &b->owned);
             if (st) return fail(st);
             BinJob bj = make_bin_job(b->wbufs[t], tk.n_ins, tk.seed, 0u);
-            bj.block0 = b->bin_blocks_total;
-            b->bin_blocks_total += bin_blocks(tk.n_ins, kBinChunk);
-            b->bin_max = std::max<long long>(
-                b->bin_max, (long long)bj.nb[0] * bj.nb[1] * bj.nb[2]);
+            bj.gblock0 = b->bin_groups_total;
+            if (bj.group > 1) b->bin_groups_total += bj.ngroups;
+            b->bin_max_keys = std::max<long long>(b->bin_max_keys, bj.ngroups);
+            b->bin_max_group = std::max(b->bin_max_group, bj.group);
+            ins_total += tk.n_ins;
             b->bin_jobs.push_back(bj);
             // many jobs share the launch: a Widom job needs only its share of
             // the device's work items
@@ -1065,6 +1071,11 @@ int batch_create(Context *ctx, const Task *tasks, int n, bool use_graph, Batch *
                                       tk.temperature);
             mixed.push_back({job_cost_per_item(tk.fw, j, ctx->tuning), j});
         }
+    }
+    b->bin_chunk_len = bin_chunk(ins_total, b->bin_max_keys);
+    for (BinJob &bj : b->bin_jobs) {
+        bj.block0 = b->bin_blocks_total;
+        b->bin_blocks_total += bin_blocks(bj.n, b->bin_chunk_len);
     }
     // Longest-processing-time order: the most expensive items are handed out first.
     auto by_cost = [](const std::pair<double, JobDev> &a, const std::pair<double, JobDev> &c) {

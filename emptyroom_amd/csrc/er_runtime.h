@@ -262,7 +262,8 @@ class Batch {
     JobDev *d_jobs = nullptr;
     std::vector<BinJob> bin_jobs;      // Widom binning of every task with insertions
     BinJob *d_bin_jobs = nullptr;
-    long long bin_blocks_total = 0, bin_max = 0;
+    long long bin_blocks_total = 0, bin_groups_total = 0, bin_max_keys = 0;
+    int bin_chunk_len = 0, bin_max_group = 1;
     long long total_items = 0;
     int math = MATH_MIXED;
     double2 *d_partials = nullptr;     // kReduceBlocks per task
