@@ -82,7 +82,7 @@ struct JobDev {
     int ntypes;
     int kind;           // JobKind
     int mode;           // OutMode
-    int pad0;
+    int interp;         // grid: the far field of 2 x 2 x 2 tiles from nodes (see grid_block)
     // grid
     int n[3];           // grid points per axis, endpoints included
     int tile[3];        // tile extent in points
@@ -145,6 +145,12 @@ constexpr int kBinGroupMax = 15360;  // bins a group may hold (the second step's
 constexpr int kBinLdsKeys = 7168;    // keys a binning block histograms in LDS (28 KiB)
 constexpr int kRegionRecords = 8192;  // entries of one workgroup's region sub-list (near-list
                                       // indices, 32 KiB)
+constexpr int kNodes = 8;        // Chebyshev nodes per axis of a block of 2 x 2 x 2 grid tiles
+constexpr double kNodeReach = 8.0;  // far atoms of a block lie at least this many times its
+                                    // half-extent away from every point
+constexpr int kNodeRecords = kNodes * kNodes * kNodes * 8 / 32;  // LDS records the values take
+constexpr long long kNodeMinBlocks = 1024;  // see use_nodes
+constexpr double kNodeMinFar = 140.0;
 constexpr long long kMinGridItems = 2048;  // regions per grid before regions shrink
 
 }  // namespace er

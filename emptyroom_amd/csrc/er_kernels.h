@@ -11,7 +11,15 @@
 namespace er {
 
 // Pair-math variants of the tiled energy kernel.
-enum Math : int { MATH_MIXED = 0, MATH_FP64 = 1, MATH_COUNT = 2, MATH_OVERLAP = 3 };
+// (MATH_NODES: FP32 grids whose blocks of tiles take their far field from nodes)
+enum Math : int { MATH_MIXED = 0, MATH_FP64 = 1, MATH_COUNT = 2, MATH_OVERLAP = 3,
+                  MATH_NODES = 4 };
+
+// The variant that computes a grid or Widom job.
+inline int job_math(const JobDev &j) {
+    if (j.kind != JOB_GRID) return MATH_MIXED;
+    return j.mode == OUT_F64 ? MATH_FP64 : j.interp ? MATH_NODES : MATH_MIXED;
+}
 
 // Framework atom in fractional coordinates with its type index (atoms are
 // grouped by type before upload).

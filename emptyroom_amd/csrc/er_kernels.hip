@@ -41,6 +41,14 @@ namespace {
 
 __device__ __forceinline__ int uniform(int v) { return __builtin_amdgcn_readfirstlane(v); }
 
+// The same pointer, unknown to the compiler: what is read through it is read
+// again instead of being held in registers around a loop.
+template <class T>
+__device__ __forceinline__ T *reread(T *p) {
+    asm volatile("" : "+s"(p));
+    return p;
+}
+
 __device__ __forceinline__ int lanes_below(uint64_t mask) {
     return __builtin_amdgcn_mbcnt_hi((uint32_t)(mask >> 32),
                                      __builtin_amdgcn_mbcnt_lo((uint32_t)mask, 0u));
@@ -701,7 +709,7 @@ __device__ __forceinline__ void wave_shell_lists(const JobDev *__restrict__ J,
 //   of the tile): r^2 = |a|^2 + |p|^2 - 2 p.a in FP64 (three FMAs and an add;
 //   |a| <= r_c + R keeps the cancellation below 13x), then in FP32
 //   u = 1/r^2, and per point the sums S3 = sum u^3 and S6 = sum u^6 over at
-//   most kFlushPairs pairs of one type, flushed into the FP64 energy as
+//   most FLUSH pairs of one type, flushed into the FP64 energy as
 //   4 eps (sigma^12 S6 - sigma^6 S3).  sigma and eps stay FP64, so their
 //   rounding adds no error common to every pair of a type.
 //   Shell pairs: the same, behind the strict FP64 test r^2 < r_c^2.
@@ -716,7 +724,7 @@ __device__ __forceinline__ void wave_shell_lists(const JobDev *__restrict__ J,
 // into the wave's own lists of LDS byte offsets wl (wave_shell_lists).
 // phase (wave-uniform): 0 every record, per segment far, shell, near; 1 only
 // the near records; 2 only the far and shell records.
-template <int PPL, int MATH, bool XL>
+template <int PPL, int MATH, bool XL, int FLUSH = kFlushPairs>
 __device__ __forceinline__ void eval_list(const JobDev *__restrict__ J,
                                           const double4 *__restrict__ L, int cap,
                                           const int *__restrict__ seg, int nseg,
@@ -795,14 +803,14 @@ __device__ __forceinline__ void eval_list(const JobDev *__restrict__ J,
                 }
             };
             // far records [fb, fe), then shell records [sb, se): FP32 sums of
-            // kFlushPairs pairs per point (blocks of 8 unrolled records),
+            // FLUSH pairs per point (blocks of 8 unrolled records),
             // then flushed into the FP64 energy
             auto blocks = [&](int b, int e, auto &&pair_at) {
-                for (int r = b; r < e; r += kFlushPairs) {
+                for (int r = b; r < e; r += FLUSH) {
                     float a3[PPL], a6[PPL];
 #pragma unroll
                     for (int q = 0; q < PPL; ++q) a3[q] = a6[q] = 0.0f;
-                    const int re = r + kFlushPairs < e ? r + kFlushPairs : e;
+                    const int re = r + FLUSH < e ? r + FLUSH : e;
 #pragma unroll 1
                     for (int h = r; h < re; h += 8) {
                         if (h + 8 <= re) {
@@ -957,6 +965,95 @@ __device__ __forceinline__ void eval_list(const JobDev *__restrict__ J,
     }
 }
 
+// ---- far field of a block of tiles from nodes -------------------------------
+//
+// Lagrange weights of the kNodes Chebyshev nodes x_a = cos((2 a + 1) pi / 16) at
+// the m equally spaced points of an axis whose first and last lie at -1 and 1
+// (m = 1: at 0): w[m][i][a].
+struct NodeWeights {
+    double x[kNodes];
+    double w[17][16][kNodes];
+};
+
+constexpr NodeWeights make_node_weights() {
+    NodeWeights t{};
+    const double c[4] = {0.98078528040323044912618, 0.83146961230254523707878,
+                         0.55557023301960222474283, 0.19509032201612826784829};
+    for (int a = 0; a < 4; ++a) {
+        t.x[a] = c[a];
+        t.x[kNodes - 1 - a] = -c[a];
+    }
+    for (int m = 1; m <= 16; ++m)
+        for (int i = 0; i < m; ++i) {
+            const double z = m > 1 ? (2.0 * i - (m - 1)) / (m - 1) : 0.0;
+            for (int a = 0; a < kNodes; ++a) {
+                double p = 1.0, q = 1.0;
+                for (int b = 0; b < kNodes; ++b)
+                    if (b != a) {
+                        p *= z - t.x[b];
+                        q *= t.x[a] - t.x[b];
+                    }
+                t.w[m][i][a] = p / q;
+            }
+        }
+    return t;
+}
+
+static __device__ const NodeWeights kNodeWeights = make_node_weights();
+
+// A block's node values (LDS, [a][b][c]) and where a tile lies in it.
+struct BlockNodes {
+    const double *value = nullptr;  // nullptr: no nodes
+    int points[3] = {1, 1, 1};      // grid points of the block per axis (at most 16)
+    int first[3] = {0, 0, 0};       // the tile's first point in the block
+};
+
+// This lane's two points (il + 4 q, jl, kl) of an 8 x 8 x 8 tile: the block's
+// interpolated far field, one axis after the other; g and h: 512 doubles each.
+__device__ __forceinline__ void node_energies(const BlockNodes &bn, int il, int jl, int kl,
+                                              double *__restrict__ g, double *__restrict__ h,
+                                              double (&e)[2]) {
+    auto row = [&](int d, int l) {
+        const int i = bn.first[d] + l;
+        return kNodeWeights.w[bn.points[d]][i < bn.points[d] ? i : bn.points[d] - 1];
+    };
+    double w[kNodes];
+    const double *r = row(2, kl);
+#pragma unroll
+    for (int c = 0; c < kNodes; ++c) w[c] = r[c];
+#pragma unroll
+    for (int q = 0; q < 2; ++q) {
+        const double *v = bn.value + ((il + 4 * q) * kNodes + jl) * kNodes;
+        double s = 0.0;
+#pragma unroll
+        for (int c = 0; c < kNodes; ++c) s = fma(w[c], v[c], s);
+        g[((il + 4 * q) * kNodes + jl) * 8 + kl] = s;
+    }
+    __syncthreads();
+    r = row(1, jl);
+#pragma unroll
+    for (int b = 0; b < kNodes; ++b) w[b] = r[b];
+#pragma unroll
+    for (int q = 0; q < 2; ++q) {
+        const double *v = g + (il + 4 * q) * kNodes * 8 + kl;
+        double s = 0.0;
+#pragma unroll
+        for (int b = 0; b < kNodes; ++b) s = fma(w[b], v[b * 8], s);
+        h[((il + 4 * q) * 8 + jl) * 8 + kl] = s;
+    }
+    __syncthreads();
+    double v[kNodes];
+#pragma unroll
+    for (int a = 0; a < kNodes; ++a) v[a] = h[(a * 8 + jl) * 8 + kl];
+#pragma unroll
+    for (int q = 0; q < 2; ++q) {
+        r = row(0, il + 4 * q);
+        e[q] = 0.0;
+#pragma unroll
+        for (int a = 0; a < kNodes; ++a) e[q] = fma(r[a], v[a], e[q]);
+    }
+}
+
 // Energies of one grid tile (tile coordinates tc), candidates streamed from
 // src / tbeg (the framework's near list, or a region's sub-list of it).
 template <int PPL, int MATH>
@@ -964,7 +1061,8 @@ __device__ void grid_tile(const JobDev *__restrict__ J, const int tc[3],
                           const double4 *__restrict__ src, const uint32_t *__restrict__ sidx,
                           const int *__restrict__ tbeg, int cap,
                           double4 *__restrict__ s_list, int *__restrict__ s_seg,
-                          int *__restrict__ s_cnt, uint16_t *__restrict__ s_wl) {
+                          int *__restrict__ s_cnt, uint16_t *__restrict__ s_wl,
+                          const BlockNodes nodes = BlockNodes()) {
     const int tid = threadIdx.x;
     int i0[3], i1[3];
     double lo[3], hi[3];
@@ -1056,6 +1154,15 @@ __device__ void grid_tile(const JobDev *__restrict__ J, const int tc[3],
         }
         __syncthreads();
     } while (cur_t < J->ntypes);
+    if constexpr (MATH == MATH_MIXED && PPL == 2) {
+        if (nodes.value) {  // quadrant layout (8 x 8 x 8 tile)
+            double far[2], *g = reinterpret_cast<double *>(s_list);
+            node_energies(nodes, lane >> 4, (wave & 1) * 4 + ((lane >> 2) & 3),
+                          (wave >> 1) * 4 + (lane & 3), g, g + 512, far);
+            acc[0] += far[0];
+            acc[1] += far[1];
+        }
+    }
 #pragma unroll
     for (int q = 0; q < PPL; ++q) {
         if (!ok[q]) continue;
@@ -1115,14 +1222,169 @@ __device__ bool build_region_list(const JobDev *__restrict__ J, double cx, doubl
         }
     }
     if (tid == 0) rbeg[J->ntypes] = n;
-    // the sub-list is read back by every wave of the workgroup
-    __threadfence();
+    // the sub-list is read back by the waves of this workgroup only
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
     __syncthreads();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
     return true;
 }
 
+// A block of up to 2 x 2 x 2 tiles of 8 x 8 x 8 points (first tile b0, bn tiles
+// per axis) of a fine FP32 grid.  An atom inside r_c of every point of the
+// block and at least kNodeReach half-extents away from it gives a smooth field
+// there: its pairs are evaluated at 8 x 8 x 8 Chebyshev nodes of the block's
+// box, and the sum is interpolated to the block's 4096 points (node_energies) -- an
+// eighth of the pairs.  Every other atom of the source goes into a list of the
+// block (blist, in the source's order), from which the tiles are computed
+// directly, as without nodes.  Direct tiles are bound by VALU issue (98% of the
+// cycles), and at 0.1 A half of what they issue is for such pairs: a grid of
+// 1.48e7 points and 3000 atoms (0.21 atoms/A^3) issued 5.0e9 wave instructions
+// in 10.3 ms and now issues 3.5e9 in 7.2 ms; one of 4.9e7 points and 2400 atoms
+// (0.05 atoms/A^3) took 10.6 and takes 7.8 ms.
+//
+// Accuracy: an atom at D from the middle of a segment of half-length h through
+// the box has a Chebyshev interpolation error on it of at most
+// 2 C(13, 5) (h / 2 D)^8 of its own r^-6 (the Gegenbauer coefficients of
+// |D - x|^-6; C(19, 11) for r^-12); with D >= 8 h that is 6e-7 for an atom on the
+// segment's own axis and 10 to 100 times less elsewhere.  Against direct FP64
+// sums over the far atoms of blocks at 0.1 A (0.12 atoms/A^3, cells of 65 to 112
+// degrees, far fields of 300 to 2000 K): 4e-7 to 3e-6 K rms, 2e-5 K at most,
+// less than the FP32 arithmetic of the same pairs rounds off; the errors of
+// whole grids against the direct method are the same with and without nodes.
+// The node sums are flushed twice as often as the points' (at an eighth of the
+// pairs that is free).
+//
+// Returns no nodes if the block's list does not fit blist_cap.
+__device__ BlockNodes grid_block(const JobDev *__restrict__ J, const int b0[3], const int bn[3],
+                           const double4 *__restrict__ src, const uint32_t *__restrict__ sidx,
+                           const int *__restrict__ tbeg, uint32_t *__restrict__ blist,
+                           int blist_cap, int *__restrict__ bbeg, int cap,
+                           double4 *__restrict__ s_list, int *__restrict__ s_seg,
+                           int *__restrict__ s_cnt) {
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const double *t = J->t;
+    BlockNodes nodes;
+    double lo[3], hi[3], half[3], h = 0.0;
+#pragma unroll
+    for (int d = 0; d < 3; ++d) {
+        const int i0 = b0[d] * J->tile[d], e = i0 + bn[d] * J->tile[d];
+        const int i1 = (e < J->n[d] ? e : J->n[d]) - 1;
+        nodes.points[d] = i1 - i0 + 1;
+        lo[d] = 1.0 * i0 / (J->n[d] - 1);
+        hi[d] = 1.0 * i1 / (J->n[d] - 1);
+        half[d] = 0.5 * (hi[d] - lo[d]);
+        const double hd = half[d] * sqrt(t[d] * t[d] + t[3 + d] * t[3 + d] + t[6 + d] * t[6 + d]);
+        h = hd > h ? hd : h;
+    }
+    const Tile bs = tile_sphere(t, lo, hi);
+    const double in2 = (J->rc + bs.R + kMargin) * (J->rc + bs.R + kMargin);
+    const double far_r = J->rc - bs.R - kMargin;
+    const double far2 = far_r > 0.0 ? far_r * far_r : -1.0;
+    // this lane's nodes (a = wave + 4 q, b, c), relative to the block's centre
+    double px[2], py[2], pz[2], acc[2];
+#pragma unroll
+    for (int q = 0; q < 2; ++q) {
+        frac_to_cart(t, half[0] * kNodeWeights.x[wave + 4 * q],
+                     half[1] * kNodeWeights.x[lane >> 3], half[2] * kNodeWeights.x[lane & 7],
+                     px[q], py[q], pz[q]);
+        acc[q] = 0.0;
+    }
+    const bool xl = t[3] == 0.0 && t[6] == 0.0;
+    int nf = 0, nseg = 0, nb = 0;
+    auto evaluate = [&]() {
+        __syncthreads();
+        if (xl)
+            eval_list<2, MATH_MIXED, true, kFlushPairs / 2>(
+                J, s_list, cap, s_seg, nseg, px, py, pz, acc, bs.R, false,
+                make_double4(0.0, 0.0, 0.0, 0.0), nullptr, 2);
+        else
+            eval_list<2, MATH_MIXED, false, kFlushPairs / 2>(
+                J, s_list, cap, s_seg, nseg, px, py, pz, acc, bs.R, false,
+                make_double4(0.0, 0.0, 0.0, 0.0), nullptr, 2);
+        __syncthreads();
+        nf = 0;
+        nseg = 0;
+    };
+    auto segment = [&](int ty, int f0) {
+        if (nf <= f0) return;
+        if (tid == 0) {
+            int *g = s_seg + kSegInts * nseg;
+            g[0] = ty;
+            g[1] = f0;
+            g[2] = nf;
+            g[3] = g[4] = g[5] = g[6] = 0;
+        }
+        ++nseg;
+    };
+    for (int ty = 0; ty < J->ntypes; ++ty) {
+        if (tid == 0) bbeg[ty] = nb;
+        double rn = J->types[ty].rclose;
+        rn = (rn > kNodeReach * h ? rn : kNodeReach * h) + bs.R + kMargin;
+        const double near2 = rn * rn;
+        const int pe = uniform(tbeg[ty + 1]);
+        int f0 = nf;
+        for (int pos = uniform(tbeg[ty]); pos < pe; pos += kWG) {
+            if (nf + kWG > cap) {
+                segment(ty, f0);
+                evaluate();
+                f0 = 0;
+            }
+            const int idx = pos + tid;
+            int at = 0;
+            bool far = false, keep = false;
+            double4 A = make_double4(0.0, 0.0, 0.0, 0.0);
+            if (idx < pe) {
+                at = sidx ? (int)sidx[idx] : idx;
+                const double4 S = src[at];
+                const double dx = S.x - bs.cx, dy = S.y - bs.cy, dz = S.z - bs.cz;
+                const double d2 = dx * dx + dy * dy + dz * dz;
+                A = make_double4(dx, dy, dz, d2);
+                far = d2 < far2 && d2 > near2;
+                keep = d2 < in2 && !far;
+            }
+            const uint64_t bf = __ballot(far), bk = __ballot(keep);
+            if (lane == 0) {
+                s_cnt[2 * wave] = __popcll(bf);
+                s_cnt[2 * wave + 1] = __popcll(bk);
+            }
+            __syncthreads();
+            int of = nf, ok = nb, tf = 0, tk = 0;
+#pragma unroll
+            for (int w = 0; w < kWG / 64; ++w) {
+                const int cf = s_cnt[2 * w], ck = s_cnt[2 * w + 1];
+                if (w < wave) {
+                    of += cf;
+                    ok += ck;
+                }
+                tf += cf;
+                tk += ck;
+            }
+            __syncthreads();
+            if (nb + tk > blist_cap) return BlockNodes();  // uniform
+            if (far) s_list[of + lanes_below(bf)] = A;
+            if (keep) blist[ok + lanes_below(bk)] = (uint32_t)at;
+            nf = uniform(nf + tf);
+            nb = uniform(nb + tk);
+        }
+        segment(ty, f0);
+        if (nseg == kMaxSeg) evaluate();
+    }
+    if (tid == 0) bbeg[J->ntypes] = nb;
+    evaluate();
+    // the list's last kNodeRecords records hold the values while the block's
+    // tiles are computed (with a list shorter by as much)
+    double *value = reinterpret_cast<double *>(s_list + cap - kNodeRecords);
+#pragma unroll
+    for (int q = 0; q < 2; ++q) value[(wave + 4 * q) * 64 + lane] = acc[q];
+    nodes.value = value;
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+    __syncthreads();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+    return nodes;
+}
+
 template <int PPL, int MATH>
-__global__ __launch_bounds__(kWG) void k_tiles(const JobDev *__restrict__ jobs, int njobs,
+__global__ __launch_bounds__(kWG, MATH == MATH_NODES ? 4 : 1) void k_tiles(const JobDev *__restrict__ jobs, int njobs,
                                                long long total_items,
                                                unsigned long long *__restrict__ counter,
                                                int cap, uint32_t *__restrict__ scratch,
@@ -1130,14 +1392,14 @@ __global__ __launch_bounds__(kWG) void k_tiles(const JobDev *__restrict__ jobs, 
     extern __shared__ double4 s_list[];
     __shared__ int s_seg[kSegInts * kMaxSeg];
     __shared__ int s_cnt[7 * (kWG / 64)];  // fill: 3 counts + 4 stop fields per wave
-    __shared__ int s_rbeg[kMaxTypes + 1];
+    __shared__ int s_rbeg[kMaxTypes + 1], s_bbeg[MATH == MATH_NODES ? kMaxTypes + 1 : 1];
     __shared__ double s_red[kWG / 64];
     __shared__ long long s_item;
     const int tid = threadIdx.x;
     uint32_t *__restrict__ slice =
         scratch ? scratch + (size_t)blockIdx.x * (size_t)scratch_cap : nullptr;
     // per-wave shell offset lists after the LDS list (FP32 and FP64 grids)
-    uint16_t *__restrict__ s_wl = (MATH == MATH_MIXED || MATH == MATH_FP64)
+    uint16_t *__restrict__ s_wl = (MATH == MATH_MIXED || MATH == MATH_FP64 || MATH == MATH_NODES)
         ? reinterpret_cast<uint16_t *>(s_list + cap) + (tid >> 6) * mixed_far_shell_cap(cap)
         : nullptr;
 
@@ -1198,7 +1460,9 @@ __global__ __launch_bounds__(kWG) void k_tiles(const JobDev *__restrict__ jobs, 
         const double4 *src = J->near;
         const uint32_t *sidx = nullptr;
         const int *tbeg = J->type_begin;
-        if (nt > 1 && slice && J->ntypes <= kMaxTypes) {
+        // (a lone block of 2 x 2 x 2 tiles streams the near list itself)
+        const bool lone = MATH == MATH_NODES && tn[0] <= 2 && tn[1] <= 2 && tn[2] <= 2;
+        if (nt > 1 && !lone && slice && J->ntypes <= kMaxTypes) {
             // region centre: middle of the region's box
             double lo[3], hi[3], clo[3], chi[3];
             int tc[3];
@@ -1238,6 +1502,33 @@ __global__ __launch_bounds__(kWG) void k_tiles(const JobDev *__restrict__ jobs, 
                 tbeg = s_rbeg;
             }
         }
+        if constexpr (MATH == MATH_NODES) {
+            // regions of a grid with nodes hold whole blocks of 2 x 2 x 2 tiles
+            const int used = sidx ? uniform(tbeg[J->ntypes]) : 0;
+            for (int bi = 0; bi < tn[0]; bi += 2)
+                for (int bj = 0; bj < tn[1]; bj += 2)
+                    for (int bk = 0; bk < tn[2]; bk += 2) {
+                        const int b0[3] = {t0[0] + bi, t0[1] + bj, t0[2] + bk};
+                        const int bn[3] = {bi + 1 < tn[0] ? 2 : 1, bj + 1 < tn[1] ? 2 : 1,
+                                           bk + 1 < tn[2] ? 2 : 1};
+                        BlockNodes nodes = grid_block(reread(J), b0, bn, src, sidx, tbeg, slice + used,
+                                                      scratch_cap - used, s_bbeg, cap, s_list,
+                                                      s_seg, s_cnt);
+                        const uint32_t *bidx = nodes.value ? slice + used : sidx;
+                        const int *bbeg = nodes.value ? s_bbeg : tbeg;
+                        for (int ti = 0; ti < bn[0] * bn[1] * bn[2]; ++ti) {
+                            const int o0 = ti / (bn[1] * bn[2]), o1 = (ti / bn[2]) % bn[1],
+                                      o2 = ti % bn[2];
+                            const int tc[3] = {b0[0] + o0, b0[1] + o1, b0[2] + o2};
+                            nodes.first[0] = 8 * o0;
+                            nodes.first[1] = 8 * o1;
+                            nodes.first[2] = 8 * o2;
+                            grid_tile<PPL, MATH_MIXED>(reread(J), tc, src, bidx, bbeg,
+                                                       cap - kNodeRecords, s_list, s_seg, s_cnt, s_wl, nodes);
+                        }
+                    }
+            continue;
+        } else {
         for (int ti = 0; ti < nt; ++ti) {
             int tc[3];
             cell_of(ti, tc);
@@ -1438,6 +1729,7 @@ __global__ __launch_bounds__(kWG) void k_tiles(const JobDev *__restrict__ jobs, 
 #pragma unroll
             for (int q = 0; q < PW; ++q)
                 if (q < mode && rok[q]) J->e_out[rins[q]] = rt[q];
+        }
         }
     }
 }
@@ -1661,7 +1953,7 @@ hipError_t launch_bin_all(const BinJob *jobs, int njobs, long long total_blocks,
 
 size_t tiles_lds_bytes(int cap, int math) {
     size_t b = (size_t)cap * sizeof(double4);
-    if (math == MATH_MIXED || math == MATH_FP64)
+    if (math == MATH_MIXED || math == MATH_FP64 || math == MATH_NODES)
         b += (size_t)(kWG / 64) * mixed_far_shell_cap(cap) * sizeof(uint16_t);
     return (b + 15) & ~(size_t)15;
 }
@@ -1672,6 +1964,8 @@ hipError_t launch_tiles(int math, int ppl, const JobDev *jobs, int njobs, long l
     if (total <= 0) return hipSuccess;
     if (cap < 2 * kWG || wgs <= 0) return hipErrorInvalidValue;
     if (scratch && scratch_cap < kWG) return hipErrorInvalidValue;
+    if (math == MATH_NODES && (!scratch || cap < 2 * kWG + kNodeRecords))
+        return hipErrorInvalidValue;
 #define ER_TILES(P, M)                                                                     \
     if (ppl == P && math == M)                                                             \
         return launch_tiles_t<P, M>(jobs, njobs, total, ctr, wgs, cap, scratch, scratch_cap, s);
@@ -1679,6 +1973,7 @@ hipError_t launch_tiles(int math, int ppl, const JobDev *jobs, int njobs, long l
     ER_TILES(1, MATH_FP64) ER_TILES(2, MATH_FP64) ER_TILES(4, MATH_FP64)
     ER_TILES(1, MATH_COUNT) ER_TILES(2, MATH_COUNT) ER_TILES(4, MATH_COUNT)
     ER_TILES(1, MATH_OVERLAP) ER_TILES(2, MATH_OVERLAP) ER_TILES(4, MATH_OVERLAP)
+    ER_TILES(2, MATH_NODES)
 #undef ER_TILES
     return hipErrorInvalidValue;
 }
@@ -1690,6 +1985,7 @@ int tiles_occupancy(int math, int ppl, int cap) {
     ER_OCC(1, MATH_FP64) ER_OCC(2, MATH_FP64) ER_OCC(4, MATH_FP64)
     ER_OCC(1, MATH_COUNT) ER_OCC(2, MATH_COUNT) ER_OCC(4, MATH_COUNT)
     ER_OCC(1, MATH_OVERLAP) ER_OCC(2, MATH_OVERLAP) ER_OCC(4, MATH_OVERLAP)
+    ER_OCC(2, MATH_NODES)
 #undef ER_OCC
     return 1;
 }

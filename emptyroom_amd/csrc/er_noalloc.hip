@@ -100,10 +100,11 @@ int grid_compute_noalloc(Context *ctx, FrameworkDev *fw, const int n[3], int pre
     JobDev *d_job = reinterpret_cast<JobDev *>(base + kNoAllocJobOffset);
     uint32_t *slices = reinterpret_cast<uint32_t *>(base + kNoAllocListOffset);
 
-    const int math = precision == 1 ? MATH_FP64 : MATH_MIXED;
     // regions sized for this array's slices; a tile's list, and so every
     // value, does not depend on the region it is in
-    const JobDev job = make_grid_job(fw, n, precision, d_out, ctx->tuning, math, kNoAllocRecords);
+    const JobDev job = make_grid_job(fw, n, precision, d_out, ctx->tuning,
+                                     precision == 1 ? MATH_FP64 : MATH_MIXED, kNoAllocRecords);
+    const int math = job_math(job);
     hipStream_t s = ctx->stream;
     if ((e = hipMemcpyAsync(d_job, &job, sizeof(job), hipMemcpyHostToDevice, s)) != hipSuccess)
         return hip_fail("job copy", e);

@@ -230,7 +230,8 @@ int tiles_workgroups(const Context *ctx, int math, long long items, int scratch_
 
 int scratch_ensure(Context *ctx, hipStream_t s, uint32_t **buf, int *wgs) {
     int occ = 1;
-    for (int m : {(int)MATH_MIXED, (int)MATH_FP64, (int)MATH_COUNT, (int)MATH_OVERLAP})
+    for (int m : {(int)MATH_MIXED, (int)MATH_FP64, (int)MATH_COUNT, (int)MATH_OVERLAP,
+                  (int)MATH_NODES})
         occ = std::max(occ, tiles_occupancy(m, ctx->tuning.ppl, ctx->tuning.cap));
     int need = ctx->n_cu * occ;
     if (*buf && *wgs >= need) return ST_OK;
@@ -522,6 +523,52 @@ void choose_grid_region(const FrameworkDev *fw, const int n[3], const int tile[3
     choose_region(fw, frac, nt, tu, kMinGridItems, region, slice_records);
 }
 
+namespace {
+
+// Whether a grid takes the far field of each block of 2 x 2 x 2 tiles from
+// nodes (see grid_block): FP32 grids in the default tile, ...
+bool use_nodes(const FrameworkDev *fw, const int n[3], const int tile[3], const Tuning &tu,
+               int math) {
+    if (math != MATH_MIXED || tu.ppl != 2 || tu.cap < 2 * kWG + kNodeRecords ||
+        fw->ntypes > kMaxTypes)
+        return false;
+    long long blocks = 1;
+    double h = 0.0, r2 = 0.0, half[3];
+    for (int d = 0; d < 3; d++) {
+        if (tile[d] != 8) return false;
+        blocks *= (n[d] + 15) / 16;
+        half[d] = 0.5 * std::min(15, n[d] - 1) / (n[d] - 1);
+        h = std::max(h, half[d] * std::sqrt(fw->t[d] * fw->t[d] + fw->t[3 + d] * fw->t[3 + d] +
+                                            fw->t[6 + d] * fw->t[6 + d]));
+    }
+    for (int c = 0; c < 4; c++) {
+        const double f[3] = {half[0], c & 1 ? half[1] : -half[1], c & 2 ? half[2] : -half[2]};
+        double s = 0.0;
+        for (int k = 0; k < 3; k++) {
+            const double x = fw->t[3 * k] * f[0] + fw->t[3 * k + 1] * f[1] + fw->t[3 * k + 2] * f[2];
+            s += x * x;
+        }
+        r2 = std::max(r2, s);
+    }
+    // ... with enough blocks to fill the device when the grid runs alone, and
+    // enough far atoms per block to pay for its interpolation.  Cubic-ish cells at
+    // 0.1 A, us without / with nodes: 0.1 atoms/A^3 (430 expected far atoms)
+    // 1728 blocks 2098 / 1686, 1000 blocks 1106 / 1071, 512 blocks 579 / 717;
+    // 4096 blocks at 0.1 atoms/A^3 5965 / 4190, 0.03 (128 far atoms) 2086 / 2050,
+    // 0.012 (51) 1267 / 1493.
+    double lo = kNodeReach * h;
+    for (const TypeParams &tp : fw->types) lo = std::max(lo, tp.rclose);
+    lo += std::sqrt(r2);
+    const double hi = fw->rc - std::sqrt(r2);
+    const double pi = 3.14159265358979323846;
+    const double far = hi > lo ? 4.0 / 3.0 * pi * (hi * hi * hi - lo * lo * lo) * fw->n_atoms /
+                                     std::max(fw->volume, 1e-9)
+                               : 0.0;
+    return blocks >= kNodeMinBlocks && far >= kNodeMinFar;
+}
+
+}  // namespace
+
 JobDev make_grid_job(const FrameworkDev *fw, const int n[3], int precision, void *d_out,
                      const Tuning &tu, int math, int slice_records) {
     JobDev j;
@@ -538,13 +585,25 @@ JobDev make_grid_job(const FrameworkDev *fw, const int n[3], int precision, void
     j.mode = math == MATH_COUNT ? OUT_COUNT : (precision == 1 ? OUT_F64 : OUT_F32);
     int tile[3], region[3];
     choose_grid_tile(fw, n, tu, tile);
-    choose_grid_region(fw, n, tile, tu, region, slice_records);
+    j.interp = use_nodes(fw, n, tile, tu, math);
+    if (j.interp) {
+        // regions of whole blocks; a slice also holds a block's list, about a
+        // third of its region's
+        const int block[3] = {2 * tile[0], 2 * tile[1], 2 * tile[2]};
+        Tuning shorter = tu;  // a block's own list makes long regions pay less
+        shorter.region_len *= 0.75;
+        choose_grid_region(fw, n, block, shorter, region, slice_records * 3 / 4);
+        for (int d = 0; d < 3; d++) region[d] *= 2;
+    } else {
+        choose_grid_region(fw, n, tile, tu, region, slice_records);
+    }
     long long items = 1;
     for (int d = 0; d < 3; d++) {
         j.n[d] = n[d];
         j.tile[d] = tile[d];
         j.ntiles[d] = (n[d] + tile[d] - 1) / tile[d];
-        j.region[d] = std::min(region[d], j.ntiles[d]);
+        // (an odd tile count ends in a block of one tile)
+        j.region[d] = std::min(region[d], j.interp ? j.ntiles[d] + j.ntiles[d] % 2 : j.ntiles[d]);
         j.nregions[d] = (j.ntiles[d] + j.region[d] - 1) / j.region[d];
         items *= j.nregions[d];
         // point boxes; the quadrant of a tile holds its i range and half its
@@ -795,7 +854,8 @@ int grid_compute(Context *ctx, FrameworkDev *fw, const int n[3], int precision, 
     };
     if (hipMemcpyAsync(d_job, &job, sizeof(job), hipMemcpyHostToDevice, s) != hipSuccess)
         return fail(ST_HIP);
-    if ((st = run_jobs(ctx, math, d_job, 1, job.n_items, ctx->d_counter))) return fail(st);
+    if ((st = run_jobs(ctx, job_math(job), d_job, 1, job.n_items, ctx->d_counter)))
+        return fail(st);
     if (host_out &&
         hipMemcpyAsync(host_out, g->d_data, g->bytes(), hipMemcpyDeviceToHost, s) != hipSuccess) {
         set_error("grid_compute: device-to-host copy failed");
@@ -949,6 +1009,9 @@ Batch::~Batch() {
 
 namespace {
 
+// Launches of a batch, in this order.
+constexpr int kBatchMath[kBatchLaunches] = {MATH_NODES, MATH_MIXED, MATH_FP64};
+
 // Expected in-cutoff pairs per point: the ordering key of the LPT schedule.
 double job_cost_per_item(const FrameworkDev *fw, const JobDev &j, const Tuning &tu) {
     const double pi = 3.14159265358979323846;
@@ -966,35 +1029,25 @@ int Batch::record(hipStream_t s) {
     // every Widom task's binning in one launch per phase
     HIP_TRY(launch_bin_all(d_bin_jobs, (int)bin_jobs.size(), bin_blocks_total, bin_chunk_len,
                            bin_max_keys, bin_max_group, bin_groups_total, s));
-    // jobs are partitioned: [0, n_mixed) mixed math, [n_mixed, njobs) FP64 grids
-    int n_mixed = 0;
-    long long items_mixed = 0, items_fp64 = 0;
-    for (const JobDev &j : jobs) {
-        if (j.kind == JOB_GRID && j.mode == OUT_F64) items_fp64 += j.n_items;
-        else {
-            n_mixed++;
-            items_mixed += j.n_items;
-        }
-    }
+    // jobs are grouped by variant, each group one launch with its own counter
     const bool ev_on = timing && !use_graph;
     timed_launches = 0;
-    HIP_TRY(launch_fill_u64(d_counter, 0ull, 2, s));
-    if (items_mixed > 0) {
-        if (ev_on) HIP_TRY(hipEventRecord(ev[0], s));
-        HIP_TRY(launch_tiles(MATH_MIXED, ctx->tuning.ppl, d_jobs, n_mixed, items_mixed, d_counter,
-                             persistent_wgs(ctx, MATH_MIXED, items_mixed), ctx->tuning.cap,
-                             ctx->d_scratch, kRegionRecords, s));
-        if (ev_on) HIP_TRY(hipEventRecord(ev[1], s));
-        timed_launches |= 1;
-    }
-    if (items_fp64 > 0) {
-        if (ev_on) HIP_TRY(hipEventRecord(ev[2], s));
-        HIP_TRY(launch_tiles(MATH_FP64, ctx->tuning.ppl, d_jobs + n_mixed,
-                             (int)jobs.size() - n_mixed, items_fp64, d_counter + 1,
-                             persistent_wgs(ctx, MATH_FP64, items_fp64), ctx->tuning.cap,
-                             ctx->d_scratch, kRegionRecords, s));
-        if (ev_on) HIP_TRY(hipEventRecord(ev[3], s));
-        timed_launches |= 2;
+    HIP_TRY(launch_fill_u64(d_counter, 0ull, kBatchLaunches, s));
+    size_t j0 = 0;
+    for (int k = 0; k < kBatchLaunches; k++) {
+        const int math = kBatchMath[k];
+        size_t j1 = j0;
+        long long items = 0;
+        while (j1 < jobs.size() && job_math(jobs[j1]) == math) items += jobs[j1++].n_items;
+        if (items > 0) {
+            if (ev_on) HIP_TRY(hipEventRecord(ev[2 * k], s));
+            HIP_TRY(launch_tiles(math, ctx->tuning.ppl, d_jobs + j0, (int)(j1 - j0), items,
+                                 d_counter + k, persistent_wgs(ctx, math, items),
+                                 ctx->tuning.cap, ctx->d_scratch, kRegionRecords, s));
+            if (ev_on) HIP_TRY(hipEventRecord(ev[2 * k + 1], s));
+            timed_launches |= 1 << k;
+        }
+        j0 = j1;
     }
     // every Widom run's sums in two launches (same per-run order as one run alone)
     HIP_TRY(launch_widom_reduce_many(d_reduce, (int)reduce.size(), s));
@@ -1018,7 +1071,7 @@ int batch_create(Context *ctx, const Task *tasks, int n, bool use_graph, Batch *
         delete b;
         return st;
     };
-    std::vector<std::pair<double, JobDev>> mixed, fp64;
+    std::vector<std::pair<double, JobDev>> found;
     uint64_t ins_total = 0;
     for (int t = 0; t < n; t++) {
         const Task &tk = tasks[t];
@@ -1047,8 +1100,7 @@ int batch_create(Context *ctx, const Task *tasks, int n, bool use_graph, Batch *
             b->grids[t] = g;
             const int math = tk.precision == 1 ? MATH_FP64 : MATH_MIXED;
             JobDev j = make_grid_job(tk.fw, tk.grid_n, tk.precision, g->d_data, ctx->tuning, math);
-            (math == MATH_FP64 ? fp64 : mixed)
-                .push_back({job_cost_per_item(tk.fw, j, ctx->tuning), j});
+            found.push_back({job_cost_per_item(tk.fw, j, ctx->tuning), j});
         }
         if (tk.n_ins > 0) {
             if (!(tk.temperature > 0.0)) {
@@ -1069,7 +1121,7 @@ int batch_create(Context *ctx, const Task *tasks, int n, bool use_graph, Batch *
             JobDev j = make_widom_job(tk.fw, tk.n_ins, tk.seed, b->wbufs[t], ctx->tuning,
                                       std::max<long long>(1, kMinGridItems / std::max(n, 1)),
                                       tk.temperature);
-            mixed.push_back({job_cost_per_item(tk.fw, j, ctx->tuning), j});
+            found.push_back({job_cost_per_item(tk.fw, j, ctx->tuning), j});
         }
     }
     b->bin_chunk_len = bin_chunk(ins_total, b->bin_max_keys);
@@ -1081,25 +1133,21 @@ int batch_create(Context *ctx, const Task *tasks, int n, bool use_graph, Batch *
     auto by_cost = [](const std::pair<double, JobDev> &a, const std::pair<double, JobDev> &c) {
         return a.first > c.first;
     };
-    std::stable_sort(mixed.begin(), mixed.end(), by_cost);
-    std::stable_sort(fp64.begin(), fp64.end(), by_cost);
-    long long begin = 0;
-    for (auto &pj : mixed) {
-        pj.second.item_begin = begin;
-        begin += pj.second.n_items;
-        b->jobs.push_back(pj.second);
-    }
-    begin = 0;
-    for (auto &pj : fp64) {
-        pj.second.item_begin = begin;
-        begin += pj.second.n_items;
-        b->jobs.push_back(pj.second);
+    std::stable_sort(found.begin(), found.end(), by_cost);
+    for (const int math : kBatchMath) {
+        long long begin = 0;
+        for (auto &pj : found) {
+            if (job_math(pj.second) != math) continue;
+            pj.second.item_begin = begin;
+            begin += pj.second.n_items;
+            b->jobs.push_back(pj.second);
+        }
     }
     int st = ST_OK;
     if ((st = pool_alloc(ctx, std::max<size_t>(b->jobs.size(), 1), &b->d_jobs, &b->owned)) ||
         (st = pool_alloc(ctx, (size_t)std::max(n, 1) * kReduceBlocks, &b->d_partials, &b->owned)) ||
         (st = pool_alloc(ctx, (size_t)std::max(n, 1) * 2, &b->d_sums, &b->owned)) ||
-        (st = pool_alloc(ctx, 2, &b->d_counter, &b->owned)) ||
+        (st = pool_alloc(ctx, kBatchLaunches, &b->d_counter, &b->owned)) ||
         (st = pool_alloc(ctx, std::max<size_t>(b->bin_jobs.size(), 1), &b->d_bin_jobs,
                          &b->owned)) ||
         (st = pool_alloc(ctx, (size_t)std::max(n, 1), &b->d_reduce, &b->owned)))
@@ -1191,7 +1239,7 @@ int batch_kernel_ms(Batch *b, double *ms, int *launches) {
     *ms = 0.0;
     int n = 0;
     if (b->timing && !b->use_graph) {
-        for (int k = 0; k < 2; k++)
+        for (int k = 0; k < kBatchLaunches; k++)
             if (b->timed_launches & (1 << k)) {
                 float t = 0.0f;
                 HIP_TRY(hipEventElapsedTime(&t, b->ev[2 * k], b->ev[2 * k + 1]));

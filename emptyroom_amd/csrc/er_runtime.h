@@ -252,6 +252,8 @@ struct Task {
     uint64_t seed = 0;
 };
 
+constexpr int kBatchLaunches = 3;  // tiled-kernel variants of a batch, one launch each
+
 class Batch {
   public:
     Context *ctx = nullptr;
@@ -277,7 +279,7 @@ class Batch {
     bool use_graph = true;
     // eager runs only: events around each tiled-kernel launch of the last run
     bool timing = false;
-    hipEvent_t ev[4] = {nullptr, nullptr, nullptr, nullptr};
+    hipEvent_t ev[2 * kBatchLaunches] = {};
     int timed_launches = 0;
     std::vector<void *> owned;
     ~Batch();

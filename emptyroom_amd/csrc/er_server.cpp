@@ -64,8 +64,6 @@ size_t work_estimate(const RequestSpec &s) {
     return b;
 }
 
-bool is_fp64_grid(const JobDev &j) { return j.kind == JOB_GRID && j.mode == OUT_F64; }
-
 }  // namespace
 
 struct Server::FwEntry {
@@ -503,11 +501,10 @@ void Server::run() {
                     ready.push_back(r);
             if (ready.empty()) break;
             // the pair-math variant of this launch: that of the oldest ready
-            // request's pending work (FP64 grid first)
+            // request's pending work (its grid first)
             const Req *o = ready.front();
-            const bool fp64 = is_fp64_grid(o->grid_job) && o->grid_next < o->grid_job.n_items;
-            const int math = fp64 ? MATH_FP64 : MATH_MIXED;
-            auto job_math = [](const JobDev &j) { return is_fp64_grid(j) ? MATH_FP64 : MATH_MIXED; };
+            const int math = o->grid_next < o->grid_job.n_items ? job_math(o->grid_job)
+                                                                : MATH_MIXED;
             long long nkind = 0;
             for (Req *r : ready)
                 for (int kind = 0; kind < 2; kind++) {
