@@ -56,10 +56,12 @@ __host__ __device__ inline void widom_point(uint64_t seed, uint32_t stream, uint
 // Pair parameters of one (guest, framework-atom-type) combination after
 // Lorentz-Berthelot mixing: sig2 = sigma_ij^2, eps4 = 4 eps_ij.  rclose is the
 // distance below which a pair is evaluated on the FP64 path.
+// c3 = -eps4 sigma^6 and c6 = eps4 sigma^12 scale the sums of r^-6 and r^-12.
 struct alignas(16) TypeParams {
     double sig2;
     double eps4;
     double rclose;
+    double c3, c6;
     double pad;
 };
 
@@ -76,7 +78,7 @@ struct JobDev {
     double rc2;         // r_c^2
     double rc;          // r_c
     double min_r2;      // r^2 clamp: 1e-24 grid, 1e-32 Widom
-    const double4 *near;      // image atoms near the cell, grouped by type (x, y, z, 0)
+    const double4 *near;      // image atoms near the cell, grouped by type (x, y, z, r_FP64)
     const int *type_begin;    // ntypes + 1 offsets into near
     const TypeParams *types;  // ntypes
     int ntypes;
@@ -107,6 +109,10 @@ struct JobDev {
     // the full one centred on it
     double cell_box[3];
     double wave_box[3];
+    // radii of the spheres around them, with the classification margin; inv[d]
+    // is the fractional step of a grid point (1 / (n - 1)) or a bin (1 / nbins)
+    double cell_R, wave_R;
+    double inv[3];
     // scheduling
     long long item_begin;  // first global work item of this job
     long long n_items;     // grid tiles or Widom bins of this job in this launch
@@ -145,6 +151,9 @@ constexpr int kBinGroupMax = 15360;  // bins a group may hold (the second step's
 constexpr int kBinLdsKeys = 7168;    // keys a binning block histograms in LDS (28 KiB)
 constexpr int kRegionRecords = 8192;  // entries of one workgroup's region sub-list (near-list
                                       // indices, 32 KiB)
+// Margin (Angstrom) applied to every list classification so that FP64 rounding
+// of radii and distances can never misclassify a pair.
+constexpr double kMargin = 1e-6;
 constexpr int kNodes = 8;        // Chebyshev nodes per axis of a block of 2 x 2 x 2 grid tiles
 constexpr double kNodeReach = 8.0;  // far atoms of a block lie at least this many times its
                                     // half-extent away from every point

@@ -40,6 +40,7 @@ struct NearPlan {
     const AtomDev *atoms;     // n atoms, grouped by type
     const int *type_atom0;    // ntypes + 1 atom offsets
     const int *type_block0;   // ntypes + 1 block offsets of the padded enumeration
+    const TypeParams *types;  // ntypes
     int nblocks;
     int n_images;
 };

@@ -67,6 +67,7 @@ __device__ __forceinline__ void frac_to_cart(const double *t, double fx, double 
 
 struct NearItem {
     bool valid;
+    int type;
     double gx, gy, gz;  // fractional position of the image atom
 };
 
@@ -75,6 +76,7 @@ __device__ __forceinline__ NearItem near_item(const NearPlan &p, int blk, int ti
     it.valid = false;
     int t = 0;
     while (t + 1 < p.ntypes && p.type_block0[t + 1] <= blk) ++t;
+    it.type = t;
     const int a0 = p.type_atom0[t];
     const int cnt = p.type_atom0[t + 1] - a0;
     const long long q = (long long)(blk - p.type_block0[t]) * kWG + tid;
@@ -118,7 +120,7 @@ __global__ __launch_bounds__(kWG) void k_near_write(NearPlan p, const uint32_t *
         for (int w = 0; w < wave; ++w) off += s_w[w];
         double x, y, z;
         frac_to_cart(p.t, it.gx, it.gy, it.gz, x, y, z);
-        near[off] = make_double4(x, y, z, 0.0);
+        near[off] = make_double4(x, y, z, p.types[it.type].rclose);
     }
 }
 
@@ -411,14 +413,12 @@ __global__ void k_fill_u64(unsigned long long *p, unsigned long long v, long lon
 // Tiled energy kernel
 // ---------------------------------------------------------------------------
 
-// Margin (Angstrom) applied to every list classification so that FP64
-// rounding of the tile radius and distances can never misclassify a pair.
-constexpr double kMargin = 1e-6;
-
 enum : int { CAT_NONE = 0, CAT_FAR = 1, CAT_SHELL = 2, CAT_NEAR = 3 };
 
-// Ints per list segment: type, far begin/end, shell begin/end, near begin/end.
-constexpr int kSegInts = 7;
+// Ints per list segment: type, far begin, shell begin, near begin.  The types of
+// a pass are consecutive, so a segment ends where the next begins; the entry
+// after the last holds the pass's counts.
+constexpr int kSegInts = 4;
 
 // Pairs per point summed in FP32 (far and shell pairs of one type) before the
 // sum is scaled and added to the FP64 energy.
@@ -430,19 +430,45 @@ struct Tile {
 
 __device__ __forceinline__ Tile tile_sphere(const double *t, const double lo[3],
                                             const double hi[3]) {
-    double mid[3] = {0.5 * (lo[0] + hi[0]), 0.5 * (lo[1] + hi[1]), 0.5 * (lo[2] + hi[2])};
     Tile s;
-    frac_to_cart(t, mid[0], mid[1], mid[2], s.cx, s.cy, s.cz);
+    frac_to_cart(t, 0.5 * (lo[0] + hi[0]), 0.5 * (lo[1] + hi[1]), 0.5 * (lo[2] + hi[2]), s.cx,
+                 s.cy, s.cz);
+    const double h[3] = {0.5 * (hi[0] - lo[0]), 0.5 * (hi[1] - lo[1]), 0.5 * (hi[2] - lo[2])};
     double r2 = 0.0;
-    for (int c = 0; c < 8; ++c) {
-        double d[3] = {((c & 4) ? hi[0] : lo[0]) - mid[0], ((c & 2) ? hi[1] : lo[1]) - mid[1],
-                       ((c & 1) ? hi[2] : lo[2]) - mid[2]};
+    for (int c = 0; c < 4; ++c) {  // opposite corners are equally far
         double x, y, z;
-        frac_to_cart(t, d[0], d[1], d[2], x, y, z);
-        double q = x * x + y * y + z * z;
+        frac_to_cart(t, h[0], c & 2 ? h[1] : -h[1], c & 1 ? h[2] : -h[2], x, y, z);
+        const double q = x * x + y * y + z * z;
         r2 = q > r2 ? q : r2;
     }
     s.R = sqrt(r2) * (1.0 + 1e-12) + kMargin;
+    return s;
+}
+
+// i / (n - 1), correctly rounded (src/writegrid.cu:122-127 divides): the quotient
+// from the rounded reciprocal, corrected by its exact remainder.  Equal to the
+// division for every 0 <= i < n <= 65536, in 3 instead of ~12 instructions.
+__device__ __forceinline__ double grid_frac(const JobDev *__restrict__ J, int d, int i) {
+    const double q = (double)i * J->inv[d];
+    return fma(fma(-q, (double)(J->n[d] - 1), (double)i), J->inv[d], q);
+}
+
+// Sphere of cell tc (a tile's points or a bin): the middle of its own box, the
+// radius of a full cell's, which covers a partial edge tile's as well.
+__device__ __forceinline__ Tile cell_sphere(const JobDev *__restrict__ J, const int tc[3]) {
+    double f[3];
+#pragma unroll
+    for (int d = 0; d < 3; ++d) {
+        double i = tc[d] + 0.5;
+        if (J->kind == JOB_GRID) {
+            const int a = tc[d] * J->tile[d], e = a + J->tile[d];
+            i = 0.5 * (a + (e < J->n[d] ? e : J->n[d]) - 1);
+        }
+        f[d] = i * J->inv[d];
+    }
+    Tile s;
+    frac_to_cart(J->t, f[0], f[1], f[2], s.cx, s.cy, s.cz);
+    s.R = J->cell_R;
     return s;
 }
 
@@ -464,8 +490,15 @@ __device__ __forceinline__ int near_region_start(int cap) {
 // (a - c, |a - c|^2), and keep the source order, so the list (and every sum
 // over it) depends only on the tile and the source.  The source is the near
 // list src, position p holding src[p], or, with sidx, a sub-list of it,
-// position p holding src[sidx[p]].  Returns the number of segments written
-// to seg.
+// position p holding src[sidx[p]].  Returns the number of segments (one per
+// type, in the source's order) written to seg.
+//
+// Chunks of 256 records run across type boundaries (a record carries its type's
+// switch radius): six types of 50 records take two rounds of loads, ballots and
+// barriers instead of six.  With the cells' radii made on the host and the
+// quotients of grid_frac this took a Henry run of 1.73e7 insertions in a 424-atom
+// cell (36036 bins) from 2.52 to 2.27 ms and a 4.9e7-point grid of 2400 atoms from
+// 7.77 to 6.71 ms, where the setup of a tile cost a third of its instructions.
 template <int MATH>
 __device__ int fill_list(const JobDev *__restrict__ J, const double4 *__restrict__ src,
                          const uint32_t *__restrict__ sidx, const int *__restrict__ tbeg,
@@ -480,7 +513,7 @@ __device__ int fill_list(const JobDev *__restrict__ J, const double4 *__restrict
     // Squared-distance forms of the tests on d = |image atom - tile centre|:
     //   some point may be inside r_c:     d - R <  r_c             (in2)
     //   every point is inside r_c:        d + R <  r_c             (far2)
-    //   some point may be inside r_FP64:  d - R <= r_FP64          (near2, per type)
+    //   some point may be inside r_FP64:  d - R <= r_FP64          (near, per type)
     // each widened by kMargin so FP64 rounding cannot misclassify.
     const double in2 = (rc + tl.R + kMargin) * (rc + tl.R + kMargin);
     const double far_r = rc - tl.R - kMargin;
@@ -500,43 +533,29 @@ __device__ int fill_list(const JobDev *__restrict__ J, const double4 *__restrict
     const double *hb = J->cell_box;
     const double rout = rc + kMargin, rout2 = rout * rout;
     const double *tm = J->t;
-    double near2 = -1.0;
-    int near_t = -1;
-    int nf = 0, ns = 0, nn = 0, nseg = 0, f0 = 0, s0 = 0, n0 = 0;
-    while (cur_t < ntypes) {
-        if (MATH == MATH_MIXED && near_t != cur_t) {
-            const double rn = J->types[cur_t].rclose + tl.R + kMargin;
-            near2 = rn * rn;
-            near_t = cur_t;
-        }
-        const int tend = uniform(tbeg[cur_t + 1]);
-        if (cur_pos >= tend) {
-            if (nf > f0 || ns > s0 || nn > n0) {
-                if (tid == 0) {
-                    int *g = seg + kSegInts * nseg;
-                    g[0] = cur_t; g[1] = f0; g[2] = nf; g[3] = s0; g[4] = ns; g[5] = n0; g[6] = nn;
-                }
-                ++nseg;
-            }
-            f0 = nf;
-            s0 = ns;
-            n0 = nn;
-            ++cur_t;
-            if (cur_t < ntypes) cur_pos = uniform(tbeg[cur_t]);
-            continue;
-        }
-        if (nseg >= kMaxSeg) break;
+    while (cur_t + 1 < ntypes && uniform(tbeg[cur_t + 1]) <= cur_pos) ++cur_t;
+    const int first_t = cur_t;
+    // a pass takes at most kMaxSeg types
+    const int last_t = first_t + kMaxSeg < ntypes ? first_t + kMaxSeg : ntypes;
+    const int end = uniform(tbeg[last_t]);
+    int nf = 0, ns = 0, nn = 0, nseg = 1;
+    if (tid == 0) {
+        seg[0] = first_t;
+        seg[1] = seg[2] = seg[3] = 0;
+    }
+    while (cur_pos < end) {
         const int idx = cur_pos + tid;
         int cat = CAT_NONE;
         double4 A = make_double4(0.0, 0.0, 0.0, 0.0);
-        if (idx < tend) {
+        if (idx < end) {
             const double4 S = src[sidx ? (int)sidx[idx] : idx];
             const double dx = S.x - tl.cx, dy = S.y - tl.cy, dz = S.z - tl.cz;
             const double d2 = dx * dx + dy * dy + dz * dz;
             A = make_double4(dx, dy, dz, d2);
             if (d2 < in2) {
+                const double rn = S.w + tl.R + kMargin;
                 if (MATH == MATH_FP64 && d2 <= clamp2) cat = CAT_NEAR;
-                else if (MATH == MATH_MIXED && d2 <= near2) cat = CAT_NEAR;
+                else if (MATH == MATH_MIXED && d2 <= rn * rn) cat = CAT_NEAR;
                 else cat = (MATH != MATH_OVERLAP && d2 < far2) ? CAT_FAR : CAT_SHELL;
                 if (cat == CAT_SHELL && !wave_lists) {
                     const double h = hb[0] * fabs(tm[0] * dx + tm[3] * dy + tm[6] * dz) +
@@ -568,6 +587,20 @@ __device__ int fill_list(const JobDev *__restrict__ J, const double4 *__restrict
             tf += cf;
             ts += cs;
             tn += cn;
+        }
+        // types that begin in this chunk: the counts before their first record
+        while (first_t + nseg < last_t) {
+            const int p = uniform(tbeg[first_t + nseg]) - cur_pos;
+            if (p >= kWG) break;
+            if (wave == p >> 6 && lane == 0) {
+                const uint64_t below = (1ull << (p & 63)) - 1ull;
+                int *g = seg + kSegInts * nseg;
+                g[0] = first_t + nseg;
+                g[1] = of + __popcll(bf & below);
+                g[2] = os + __popcll(bs & below);
+                g[3] = on + __popcll(bn & below);
+            }
+            ++nseg;
         }
         // A pass takes the kept records in source order up to the first one
         // that does not fit (far + shell share [0, capA), near [capA, cap)),
@@ -609,7 +642,8 @@ __device__ int fill_list(const JobDev *__restrict__ J, const double4 *__restrict
             ns = uniform(x[2]);
             nn = uniform(x[3]);
             cur_pos += 64 * stop + uniform(x[0]);
-            __syncthreads();  // x is read by every thread before it is reused
+            // types that begin at or after the stop belong to the next pass
+            while (nseg > 1 && uniform(tbeg[first_t + nseg - 1]) >= cur_pos) --nseg;
             break;
         }
         nf = uniform(nf + tf);
@@ -617,12 +651,19 @@ __device__ int fill_list(const JobDev *__restrict__ J, const double4 *__restrict
         nn = uniform(nn + tn);
         cur_pos += kWG;
     }
-    if (nf > f0 || ns > s0 || nn > n0) {
-        if (tid == 0) {
-            int *g = seg + kSegInts * nseg;
-            g[0] = cur_t; g[1] = f0; g[2] = nf; g[3] = s0; g[4] = ns; g[5] = n0; g[6] = nn;
-        }
-        ++nseg;
+    if (cur_pos >= end) {
+        cur_pos = end;
+        cur_t = last_t;
+        // (types whose records all lie before the end have begun; empty ones at
+        // the very end may not have)
+    } else {
+        cur_t = first_t + nseg - 1;
+    }
+    if (tid == 0) {
+        int *g = seg + kSegInts * nseg;
+        g[1] = nf;
+        g[2] = ns;
+        g[3] = nn;
     }
     return nseg;
 }
@@ -747,10 +788,12 @@ __device__ __forceinline__ void eval_list(const JobDev *__restrict__ J,
         p2[q] = px[q] * px[q] + py[q] * py[q] + pz[q] * pz[q];
     }
     for (int s = 0; s < nseg; ++s) {
-        const int t = uniform(seg[kSegInts * s]);
-        const int fb = uniform(seg[kSegInts * s + 1]), fe = uniform(seg[kSegInts * s + 2]);
-        const int sb = uniform(seg[kSegInts * s + 3]), se = uniform(seg[kSegInts * s + 4]);
-        const int nb = uniform(seg[kSegInts * s + 5]), ne = uniform(seg[kSegInts * s + 6]);
+        const int *g = seg + kSegInts * s;
+        const int t = uniform(g[0]);
+        const int fb = uniform(g[1]), fe = uniform(g[kSegInts + 1]);
+        const int sb = uniform(g[2]), se = uniform(g[kSegInts + 2]);
+        const int nb = uniform(g[3]), ne = uniform(g[kSegInts + 3]);
+        if (fe - fb + se - sb + ne - nb == 0) continue;
         const TypeParams P = J->types[t];
         if (MATH == MATH_OVERLAP) {
             // src/computegridsheet.h:154: overlap iff r^2 < sigma_ij^2 (every
@@ -777,8 +820,7 @@ __device__ __forceinline__ void eval_list(const JobDev *__restrict__ J,
             continue;
         }
         if (MATH == MATH_MIXED) {
-            const double sig6 = P.sig2 * P.sig2 * P.sig2;
-            const double c6 = P.eps4 * sig6 * sig6, c3 = -P.eps4 * sig6;
+            const double c6 = P.c6, c3 = P.c3;
             auto far_pair = [&](const double4 &A, float (&s3)[PPL], float (&s6)[PPL]) {
                 double r2[PPL];
                 pair_r2<PPL, XL>(A, mx, my, mz, p2, r2);
@@ -899,8 +941,7 @@ __device__ __forceinline__ void eval_list(const JobDev *__restrict__ J,
         // sigma^12 u^6| + |4 eps sigma^6 u^3| -- the size of the rounding the
         // expanded r^2 already leaves (|a|^2 + |p|^2 - 2 p.a cancels ~13 FP64
         // ulps of |a|^2).  Near records take two steps.
-        const double sig6 = P.sig2 * P.sig2 * P.sig2;
-        const double c6 = P.eps4 * sig6 * sig6, c3 = -P.eps4 * sig6;
+        const double c6 = P.c6, c3 = P.c3;
         double b3[PPL], b6[PPL];
 #pragma unroll
         for (int q = 0; q < PPL; ++q) b3[q] = b6[q] = 0.0;
@@ -1065,17 +1106,13 @@ __device__ void grid_tile(const JobDev *__restrict__ J, const int tc[3],
                           const BlockNodes nodes = BlockNodes()) {
     const int tid = threadIdx.x;
     int i0[3], i1[3];
-    double lo[3], hi[3];
 #pragma unroll
     for (int d = 0; d < 3; ++d) {
         i0[d] = tc[d] * J->tile[d];
         const int e = i0[d] + J->tile[d];
         i1[d] = (e < J->n[d] ? e : J->n[d]) - 1;
-        // src/writegrid.cu:122-127
-        lo[d] = 1.0 * i0[d] / (J->n[d] - 1);
-        hi[d] = 1.0 * i1[d] / (J->n[d] - 1);
     }
-    const Tile tl = tile_sphere(J->t, lo, hi);
+    const Tile tl = cell_sphere(J, tc);
     double px[PPL], py[PPL], pz[PPL], acc[PPL];
     long long oidx[PPL];
     bool ok[PPL];
@@ -1109,8 +1146,8 @@ __device__ void grid_tile(const JobDev *__restrict__ J, const int tc[3],
             gj = i0[1];
             gk = i0[2];
         }
-        frac_to_cart(J->t, 1.0 * gi / (J->n[0] - 1), 1.0 * gj / (J->n[1] - 1),
-                     1.0 * gk / (J->n[2] - 1), px[q], py[q], pz[q]);
+        frac_to_cart(J->t, grid_frac(J, 0, gi), grid_frac(J, 1, gj), grid_frac(J, 2, gk), px[q],
+                     py[q], pz[q]);
         px[q] -= tl.cx;
         py[q] -= tl.cy;
         pz[q] -= tl.cz;
@@ -1123,7 +1160,8 @@ __device__ void grid_tile(const JobDev *__restrict__ J, const int tc[3],
     const bool xl = PPL > 1 && (quad || kWG % (t1 * t2) == 0) && J->t[3] == 0.0 &&
                     J->t[6] == 0.0;
     // The sphere around this wave's valid points (quadrant layout): its
-    // index box is the tile's i range times the quadrant's j and k ranges.
+    // index box is the tile's i range times the quadrant's j and k ranges; a
+    // full quadrant's radius covers a partial one's.
     bool ws = false, idle = false;
     double4 wsph = make_double4(0.0, 0.0, 0.0, 0.0);
     if (quad) {
@@ -1132,10 +1170,10 @@ __device__ void grid_tile(const JobDev *__restrict__ J, const int tc[3],
         const int ke = kb + h2 - 1 < i1[2] ? kb + h2 - 1 : i1[2];
         idle = jb > i1[1] || kb > i1[2];  // no point of this wave is on the grid
         if (!idle) {
-            const double wlo[3] = {lo[0], 1.0 * jb / (J->n[1] - 1), 1.0 * kb / (J->n[2] - 1)};
-            const double whi[3] = {hi[0], 1.0 * je / (J->n[1] - 1), 1.0 * ke / (J->n[2] - 1)};
-            const Tile w = tile_sphere(J->t, wlo, whi);
-            wsph = make_double4(w.cx - tl.cx, w.cy - tl.cy, w.cz - tl.cz, w.R);
+            double wx, wy, wz;
+            frac_to_cart(J->t, 0.5 * (i0[0] + i1[0]) * J->inv[0], 0.5 * (jb + je) * J->inv[1],
+                         0.5 * (kb + ke) * J->inv[2], wx, wy, wz);
+            wsph = make_double4(wx - tl.cx, wy - tl.cy, wz - tl.cz, J->wave_R);
             ws = true;
         }
     }
@@ -1193,35 +1231,39 @@ __device__ bool build_region_list(const JobDev *__restrict__ J, double cx, doubl
                                   double in2, uint32_t *__restrict__ out, int cap_s,
                                   int *__restrict__ rbeg, int *__restrict__ s_cnt) {
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    int n = 0;
-    for (int t = 0; t < J->ntypes; ++t) {
-        if (tid == 0) rbeg[t] = n;
-        const int b = uniform(J->type_begin[t]), e = uniform(J->type_begin[t + 1]);
-        for (int pos = b; pos < e; pos += kWG) {
-            const int idx = pos + tid;
-            bool keep = false;
-            double4 A = make_double4(0.0, 0.0, 0.0, 0.0);
-            if (idx < e) {
-                A = J->near[idx];
-                const double dx = A.x - cx, dy = A.y - cy, dz = A.z - cz;
-                keep = dx * dx + dy * dy + dz * dz < in2;
-            }
-            const uint64_t bk = __ballot(keep);
-            if (lane == 0) s_cnt[wave] = __popcll(bk);
-            __syncthreads();
-            int off = n, tot = 0;
-#pragma unroll
-            for (int w = 0; w < kWG / 64; ++w) {
-                if (w < wave) off += s_cnt[w];
-                tot += s_cnt[w];
-            }
-            __syncthreads();
-            if (n + tot > cap_s) return false;  // uniform
-            if (keep) out[off + lanes_below(bk)] = (uint32_t)idx;
-            n = uniform(n + tot);
+    const int ntypes = J->ntypes, end = uniform(J->type_begin[ntypes]);
+    int n = 0, t = 0;
+    for (int pos = 0; pos < end; pos += kWG) {
+        const int idx = pos + tid;
+        bool keep = false;
+        if (idx < end) {
+            const double4 A = J->near[idx];
+            const double dx = A.x - cx, dy = A.y - cy, dz = A.z - cz;
+            keep = dx * dx + dy * dy + dz * dz < in2;
         }
+        const uint64_t bk = __ballot(keep);
+        if (lane == 0) s_cnt[wave] = __popcll(bk);
+        __syncthreads();
+        int off = n, tot = 0;
+#pragma unroll
+        for (int w = 0; w < kWG / 64; ++w) {
+            if (w < wave) off += s_cnt[w];
+            tot += s_cnt[w];
+        }
+        __syncthreads();
+        if (n + tot > cap_s) return false;  // uniform
+        if (keep) out[off + lanes_below(bk)] = (uint32_t)idx;
+        // types that begin in this chunk
+        for (; t < ntypes; ++t) {
+            const int p = uniform(J->type_begin[t]) - pos;
+            if (p >= kWG) break;
+            if (wave == p >> 6 && lane == 0)
+                rbeg[t] = off + __popcll(bk & ((1ull << (p & 63)) - 1ull));
+        }
+        n = uniform(n + tot);
     }
-    if (tid == 0) rbeg[J->ntypes] = n;
+    for (; t <= ntypes; ++t)
+        if (tid == 0) rbeg[t] = n;
     // the sub-list is read back by the waves of this workgroup only
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
     __syncthreads();
@@ -1290,8 +1332,12 @@ __device__ BlockNodes grid_block(const JobDev *__restrict__ J, const int b0[3], 
         acc[q] = 0.0;
     }
     const bool xl = t[3] == 0.0 && t[6] == 0.0;
-    int nf = 0, nseg = 0, nb = 0;
+    const int ntypes = J->ntypes, end = uniform(tbeg[ntypes]);
+    const double reach = (kNodeReach * h) + bs.R + kMargin, reach2 = reach * reach;
+    int nf = 0, nb = 0, first_t = 0, nseg = 0, nt = 0;  // nt: types begun
+    // the far records so far, types first_t .. first_t + nseg - 1, at the nodes
     auto evaluate = [&]() {
+        if (tid == 0) s_seg[kSegInts * nseg + 1] = nf;
         __syncthreads();
         if (xl)
             eval_list<2, MATH_MIXED, true, kFlushPairs / 2>(
@@ -1302,74 +1348,73 @@ __device__ BlockNodes grid_block(const JobDev *__restrict__ J, const int b0[3], 
                 J, s_list, cap, s_seg, nseg, px, py, pz, acc, bs.R, false,
                 make_double4(0.0, 0.0, 0.0, 0.0), nullptr, 2);
         __syncthreads();
-        nf = 0;
-        nseg = 0;
     };
-    auto segment = [&](int ty, int f0) {
-        if (nf <= f0) return;
-        if (tid == 0) {
-            int *g = s_seg + kSegInts * nseg;
-            g[0] = ty;
-            g[1] = f0;
-            g[2] = nf;
-            g[3] = g[4] = g[5] = g[6] = 0;
+    for (int i = tid; i <= kMaxSeg; i += kWG)
+        s_seg[kSegInts * i + 2] = s_seg[kSegInts * i + 3] = 0;  // no shell, no near records
+    for (int pos = 0; pos < end; pos += kWG) {
+        if (nf + kWG > cap) {
+            evaluate();
+            // the pass that follows begins inside the last type begun
+            nf = 0;
+            first_t = nt - 1;
+            nseg = 1;
+            if (tid == 0) {
+                s_seg[0] = first_t;
+                s_seg[1] = 0;
+            }
         }
-        ++nseg;
-    };
-    for (int ty = 0; ty < J->ntypes; ++ty) {
-        if (tid == 0) bbeg[ty] = nb;
-        double rn = J->types[ty].rclose;
-        rn = (rn > kNodeReach * h ? rn : kNodeReach * h) + bs.R + kMargin;
-        const double near2 = rn * rn;
-        const int pe = uniform(tbeg[ty + 1]);
-        int f0 = nf;
-        for (int pos = uniform(tbeg[ty]); pos < pe; pos += kWG) {
-            if (nf + kWG > cap) {
-                segment(ty, f0);
-                evaluate();
-                f0 = 0;
-            }
-            const int idx = pos + tid;
-            int at = 0;
-            bool far = false, keep = false;
-            double4 A = make_double4(0.0, 0.0, 0.0, 0.0);
-            if (idx < pe) {
-                at = sidx ? (int)sidx[idx] : idx;
-                const double4 S = src[at];
-                const double dx = S.x - bs.cx, dy = S.y - bs.cy, dz = S.z - bs.cz;
-                const double d2 = dx * dx + dy * dy + dz * dz;
-                A = make_double4(dx, dy, dz, d2);
-                far = d2 < far2 && d2 > near2;
-                keep = d2 < in2 && !far;
-            }
-            const uint64_t bf = __ballot(far), bk = __ballot(keep);
-            if (lane == 0) {
-                s_cnt[2 * wave] = __popcll(bf);
-                s_cnt[2 * wave + 1] = __popcll(bk);
-            }
-            __syncthreads();
-            int of = nf, ok = nb, tf = 0, tk = 0;
+        const int idx = pos + tid;
+        int at = 0;
+        bool far = false, keep = false;
+        double4 A = make_double4(0.0, 0.0, 0.0, 0.0);
+        if (idx < end) {
+            at = sidx ? (int)sidx[idx] : idx;
+            const double4 S = src[at];
+            const double dx = S.x - bs.cx, dy = S.y - bs.cy, dz = S.z - bs.cz;
+            const double d2 = dx * dx + dy * dy + dz * dz;
+            const double rn = S.w + bs.R + kMargin;
+            A = make_double4(dx, dy, dz, d2);
+            far = d2 < far2 && d2 > reach2 && d2 > rn * rn;
+            keep = d2 < in2 && !far;
+        }
+        const uint64_t bf = __ballot(far), bk = __ballot(keep);
+        if (lane == 0) {
+            s_cnt[2 * wave] = __popcll(bf);
+            s_cnt[2 * wave + 1] = __popcll(bk);
+        }
+        __syncthreads();
+        int of = nf, ok = nb, tf = 0, tk = 0;
 #pragma unroll
-            for (int w = 0; w < kWG / 64; ++w) {
-                const int cf = s_cnt[2 * w], ck = s_cnt[2 * w + 1];
-                if (w < wave) {
-                    of += cf;
-                    ok += ck;
-                }
-                tf += cf;
-                tk += ck;
+        for (int w = 0; w < kWG / 64; ++w) {
+            const int cf = s_cnt[2 * w], ck = s_cnt[2 * w + 1];
+            if (w < wave) {
+                of += cf;
+                ok += ck;
             }
-            __syncthreads();
-            if (nb + tk > blist_cap) return BlockNodes();  // uniform
-            if (far) s_list[of + lanes_below(bf)] = A;
-            if (keep) blist[ok + lanes_below(bk)] = (uint32_t)at;
-            nf = uniform(nf + tf);
-            nb = uniform(nb + tk);
+            tf += cf;
+            tk += ck;
         }
-        segment(ty, f0);
-        if (nseg == kMaxSeg) evaluate();
+        __syncthreads();
+        if (nb + tk > blist_cap) return BlockNodes();  // uniform
+        if (far) s_list[of + lanes_below(bf)] = A;
+        if (keep) blist[ok + lanes_below(bk)] = (uint32_t)at;
+        // types that begin in this chunk
+        for (; nt < ntypes; ++nt) {
+            const int p = uniform(tbeg[nt]) - pos;
+            if (p >= kWG) break;
+            if (wave == p >> 6 && lane == 0) {
+                const uint64_t below = (1ull << (p & 63)) - 1ull;
+                bbeg[nt] = ok + __popcll(bk & below);
+                s_seg[kSegInts * nseg] = nt;
+                s_seg[kSegInts * nseg + 1] = of + __popcll(bf & below);
+            }
+            ++nseg;
+        }
+        nf = uniform(nf + tf);
+        nb = uniform(nb + tk);
     }
-    if (tid == 0) bbeg[J->ntypes] = nb;
+    for (; nt <= ntypes; ++nt)
+        if (tid == 0) bbeg[nt] = nb;
     evaluate();
     // the list's last kNodeRecords records hold the values while the block's
     // tiles are computed (with a list shorter by as much)
@@ -1390,10 +1435,9 @@ __global__ __launch_bounds__(kWG, MATH == MATH_NODES ? 4 : 1) void k_tiles(const
                                                int cap, uint32_t *__restrict__ scratch,
                                                int scratch_cap) {
     extern __shared__ double4 s_list[];
-    __shared__ int s_seg[kSegInts * kMaxSeg];
+    __shared__ int s_seg[kSegInts * (kMaxSeg + 1)];
     __shared__ int s_cnt[7 * (kWG / 64)];  // fill: 3 counts + 4 stop fields per wave
     __shared__ int s_rbeg[kMaxTypes + 1], s_bbeg[MATH == MATH_NODES ? kMaxTypes + 1 : 1];
-    __shared__ double s_red[kWG / 64];
     __shared__ long long s_item;
     const int tid = threadIdx.x;
     uint32_t *__restrict__ slice =
@@ -1437,21 +1481,6 @@ __global__ __launch_bounds__(kWG, MATH == MATH_NODES ? 4 : 1) void k_tiles(const
             tn[d] = (e < ncell[d] ? e : ncell[d]) - t0[d];
         }
         const int nt = tn[0] * tn[1] * tn[2];
-        // fractional box of cell tc: a tile's grid points, or a bin
-        auto cell_box = [&](const int tc[3], double lo[3], double hi[3]) {
-#pragma unroll
-            for (int d = 0; d < 3; ++d) {
-                if (grid) {
-                    const int a = tc[d] * J->tile[d];  // src/writegrid.cu:122-127
-                    const int b = a + J->tile[d];
-                    lo[d] = 1.0 * a / (J->n[d] - 1);
-                    hi[d] = 1.0 * ((b < J->n[d] ? b : J->n[d]) - 1) / (J->n[d] - 1);
-                } else {
-                    lo[d] = (double)tc[d] / J->nbins[d];
-                    hi[d] = (double)(tc[d] + 1) / J->nbins[d];
-                }
-            }
-        };
         auto cell_of = [&](int ti, int tc[3]) {
             tc[0] = t0[0] + ti / (tn[1] * tn[2]);
             tc[1] = t0[1] + (ti / tn[2]) % tn[1];
@@ -1463,39 +1492,29 @@ __global__ __launch_bounds__(kWG, MATH == MATH_NODES ? 4 : 1) void k_tiles(const
         // (a lone block of 2 x 2 x 2 tiles streams the near list itself)
         const bool lone = MATH == MATH_NODES && tn[0] <= 2 && tn[1] <= 2 && tn[2] <= 2;
         if (nt > 1 && !lone && slice && J->ntypes <= kMaxTypes) {
-            // region centre: middle of the region's box
-            double lo[3], hi[3], clo[3], chi[3];
+            // region centre: middle of its first and last cell's centres, which
+            // all others lie between; R: to the corner of that box, and a cell's
+            // radius
             int tc[3];
             cell_of(0, tc);
-            cell_box(tc, lo, clo);
+            const Tile ca = cell_sphere(J, tc);
             cell_of(nt - 1, tc);
-            cell_box(tc, chi, hi);
-            double cx, cy, cz;
-            frac_to_cart(J->t, 0.5 * (lo[0] + hi[0]), 0.5 * (lo[1] + hi[1]),
-                         0.5 * (lo[2] + hi[2]), cx, cy, cz);
-            // R = max over cells of |c_t - c| + R_t (one cell per thread)
-            double r = 0.0;
-            for (int ti = tid; ti < nt; ti += kWG) {
-                cell_of(ti, tc);
-                double tlo[3], thi[3];
-                cell_box(tc, tlo, thi);
-                const Tile ts = tile_sphere(J->t, tlo, thi);
-                const double dx = ts.cx - cx, dy = ts.cy - cy, dz = ts.cz - cz;
-                const double rt = sqrt(dx * dx + dy * dy + dz * dz) + ts.R;
-                r = rt > r ? rt : r;
-            }
+            const Tile cb = cell_sphere(J, tc);
+            const double cx = 0.5 * (ca.cx + cb.cx), cy = 0.5 * (ca.cy + cb.cy),
+                         cz = 0.5 * (ca.cz + cb.cz);
+            double r2 = 0.0;
+            for (int c = 0; c < 4; ++c) {
+                double h[3], x, y, z;
 #pragma unroll
-            for (int o = 32; o >= 1; o >>= 1) {
-                const double v = __shfl_xor(r, o, 64);
-                r = v > r ? v : r;
+                for (int d = 0; d < 3; ++d) {
+                    const double w = (tn[d] - 1) * (grid ? J->tile[d] : 1) * J->inv[d];
+                    h[d] = (d == 1 && (c & 2)) || (d == 2 && (c & 1)) ? -0.5 * w : 0.5 * w;
+                }
+                frac_to_cart(J->t, h[0], h[1], h[2], x, y, z);
+                const double q = x * x + y * y + z * z;
+                r2 = q > r2 ? q : r2;
             }
-            if ((tid & 63) == 0) s_red[tid >> 6] = r;
-            __syncthreads();
-            double R = s_red[0];
-#pragma unroll
-            for (int w = 1; w < kWG / 64; ++w) R = s_red[w] > R ? s_red[w] : R;
-            R = R * (1.0 + 1e-12) + kMargin;
-            __syncthreads();
+            const double R = (sqrt(r2) + J->cell_R) * (1.0 + 1e-12) + kMargin;
             const double rr = J->rc + R + kMargin;
             if (build_region_list(J, cx, cy, cz, rr * rr, slice, scratch_cap, s_rbeg, s_cnt)) {
                 sidx = slice;
@@ -1646,9 +1665,7 @@ __global__ __launch_bounds__(kWG, MATH == MATH_NODES ? 4 : 1) void k_tiles(const
             const int b = (tc[0] * J->nbins[1] + tc[1]) * J->nbins[2] + tc[2];
             const uint32_t s0 = J->bin_start[b], s1 = J->bin_start[b + 1];
             if (s0 == s1) continue;
-            double lo[3], hi[3];
-            cell_box(tc, lo, hi);
-            const Tile tl = tile_sphere(J->t, lo, hi);
+            const Tile tl = cell_sphere(J, tc);
             // one chunk: this wave's points per lane (wave-uniform; 0 for a
             // wave with no slot); several chunks: -1.  Only the FP32-grid /
             // Widom pair math keeps bins resident: Widom jobs never run with
@@ -1690,12 +1707,12 @@ __global__ __launch_bounds__(kWG, MATH == MATH_NODES ? 4 : 1) void k_tiles(const
                 double lb_near = 0.0, lb_fs = 0.0, lb_later = 0.0;
                 if (J->sat_e > 0.0) {
                     for (int sg = 0; sg < nseg; ++sg) {
-                        const int *g = s_seg + kSegInts * sg;
+                        const int *g = s_seg + kSegInts * sg, *e = g + kSegInts;
                         const double eps = 0.25 * J->types[uniform(g[0])].eps4;
                         lb_fs -= eps * J->fs_floor *
-                                 (double)(uniform(g[2]) - uniform(g[1]) + uniform(g[4]) -
-                                                uniform(g[3]));
-                        lb_near -= eps * (double)(uniform(g[6]) - uniform(g[5]));
+                                 (double)(uniform(e[1]) - uniform(g[1]) + uniform(e[2]) -
+                                          uniform(g[2]));
+                        lb_near -= eps * (double)(uniform(e[3]) - uniform(g[3]));
                     }
                     // source records after this pass, each at -eps of its type:
                     // the rest of the current type, then every later type

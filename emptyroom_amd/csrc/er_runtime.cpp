@@ -322,6 +322,10 @@ int framework_upload(Context *ctx, const Particle *atoms, int n, const double t[
             tp.sig2 = atoms[i].sig2;
             tp.eps4 = 4.0 * atoms[i].eps;
             tp.rclose = std::sqrt(std::max(atoms[i].sig2, 0.0) / ctx->tuning.s2_switch);
+            const double sig6 = tp.sig2 * tp.sig2 * tp.sig2;
+            tp.c3 = -tp.eps4 * sig6;
+            tp.c6 = tp.eps4 * sig6 * sig6;
+            tp.pad = 0.0;
             fw->types.push_back(tp);
             type_of[i] = id;
         } else {
@@ -396,6 +400,7 @@ int framework_upload(Context *ctx, const Particle *atoms, int n, const double t[
     plan.atoms = fw->d_atoms;
     plan.type_atom0 = fw->d_type_atom0;
     plan.type_block0 = fw->d_type_block0;
+    plan.types = fw->d_types;
     HIP_TRY(launch_near_count(plan, fw->d_block_count, s));
     HIP_TRY(launch_near_offsets(plan, fw->d_block_count, fw->d_block_off, fw->d_type_begin, s));
     HIP_TRY(launch_near_write(plan, fw->d_block_off, fw->d_near, s));
@@ -525,6 +530,26 @@ void choose_grid_region(const FrameworkDev *fw, const int n[3], const int tile[3
 
 namespace {
 
+// Radius of the sphere around a parallelepiped of fractional half-extents half[],
+// with the margin every list classification allows for FP64 rounding.
+double box_radius(const double t[9], const double half[3]) {
+    double r2 = 0.0;
+    for (int c = 0; c < 4; c++) {
+        const double f[3] = {half[0], c & 1 ? half[1] : -half[1], c & 2 ? half[2] : -half[2]};
+        double q = 0.0;
+        for (int k = 0; k < 3; k++) {
+            const double x = t[3 * k] * f[0] + t[3 * k + 1] * f[1] + t[3 * k + 2] * f[2];
+            q += x * x;
+        }
+        r2 = std::max(r2, q);
+    }
+    return std::sqrt(r2) * (1.0 + 1e-12) + kMargin;
+}
+
+}  // namespace
+
+namespace {
+
 // Whether a grid takes the far field of each block of 2 x 2 x 2 tiles from
 // nodes (see grid_block): FP32 grids in the default tile, ...
 bool use_nodes(const FrameworkDev *fw, const int n[3], const int tile[3], const Tuning &tu,
@@ -533,22 +558,13 @@ bool use_nodes(const FrameworkDev *fw, const int n[3], const int tile[3], const 
         fw->ntypes > kMaxTypes)
         return false;
     long long blocks = 1;
-    double h = 0.0, r2 = 0.0, half[3];
+    double h = 0.0, half[3];
     for (int d = 0; d < 3; d++) {
         if (tile[d] != 8) return false;
         blocks *= (n[d] + 15) / 16;
         half[d] = 0.5 * std::min(15, n[d] - 1) / (n[d] - 1);
         h = std::max(h, half[d] * std::sqrt(fw->t[d] * fw->t[d] + fw->t[3 + d] * fw->t[3 + d] +
                                             fw->t[6 + d] * fw->t[6 + d]));
-    }
-    for (int c = 0; c < 4; c++) {
-        const double f[3] = {half[0], c & 1 ? half[1] : -half[1], c & 2 ? half[2] : -half[2]};
-        double s = 0.0;
-        for (int k = 0; k < 3; k++) {
-            const double x = fw->t[3 * k] * f[0] + fw->t[3 * k + 1] * f[1] + fw->t[3 * k + 2] * f[2];
-            s += x * x;
-        }
-        r2 = std::max(r2, s);
     }
     // ... with enough blocks to fill the device when the grid runs alone, and
     // enough far atoms per block to pay for its interpolation.  Cubic-ish cells at
@@ -558,8 +574,9 @@ bool use_nodes(const FrameworkDev *fw, const int n[3], const int tile[3], const 
     // 0.012 (51) 1267 / 1493.
     double lo = kNodeReach * h;
     for (const TypeParams &tp : fw->types) lo = std::max(lo, tp.rclose);
-    lo += std::sqrt(r2);
-    const double hi = fw->rc - std::sqrt(r2);
+    const double R = box_radius(fw->t, half);
+    lo += R;
+    const double hi = fw->rc - R;
     const double pi = 3.14159265358979323846;
     const double far = hi > lo ? 4.0 / 3.0 * pi * (hi * hi * hi - lo * lo * lo) * fw->n_atoms /
                                      std::max(fw->volume, 1e-9)
@@ -608,10 +625,14 @@ JobDev make_grid_job(const FrameworkDev *fw, const int n[3], int precision, void
         items *= j.nregions[d];
         // point boxes; the quadrant of a tile holds its i range and half its
         // j and k ranges (used only where the kernel takes that layout)
-        const int wave_pts = d == 0 ? tile[d] : std::max(tile[d] / 2, 1);
-        j.cell_box[d] = 0.5 * (double)(tile[d] - 1) / (double)(n[d] - 1);
+        const int pts = std::min(tile[d], n[d]);
+        const int wave_pts = d == 0 ? pts : std::min(std::max(tile[d] / 2, 1), n[d]);
+        j.cell_box[d] = 0.5 * (double)(pts - 1) / (double)(n[d] - 1);
         j.wave_box[d] = 0.5 * (double)(wave_pts - 1) / (double)(n[d] - 1);
+        j.inv[d] = 1.0 / (double)(n[d] - 1);
     }
+    j.cell_R = box_radius(fw->t, j.cell_box);
+    j.wave_R = box_radius(fw->t, j.wave_box);
     j.out = d_out;
     j.n_items = items;
     return j;
@@ -635,7 +656,9 @@ JobDev make_widom_job(const FrameworkDev *fw, uint64_t n_ins, uint64_t seed,
     for (int d = 0; d < 3; d++) {
         j.nbins[d] = wb.nbins[d];
         j.cell_box[d] = 0.5 / (double)wb.nbins[d];
+        j.inv[d] = 1.0 / (double)wb.nbins[d];
     }
+    j.cell_R = box_radius(fw->t, j.cell_box);
     j.sorted = wb.sorted;
     j.bin_start = wb.start;
     j.seed = seed;
