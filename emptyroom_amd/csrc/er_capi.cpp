@@ -200,15 +200,15 @@ int er_grid_compute(er_context *ctx, er_framework *fw, const int n[3], int preci
 
 int er_grid_download(er_grid *grid, void *host_out) {
     if (!grid || !host_out) return arg_error("er_grid_download: null argument");
-    er::GridDev *g = G(grid);
-    if (hipSetDevice(g->ctx->device) != hipSuccess ||
-        hipMemcpyAsync(host_out, g->d_data, g->bytes(), hipMemcpyDeviceToHost, g->ctx->stream) !=
-            hipSuccess ||
-        hipStreamSynchronize(g->ctx->stream) != hipSuccess) {
-        er::set_error("er_grid_download: copy failed");
-        return er::ST_HIP;
-    }
-    return ST_OK;
+    return guarded([&]() -> int {
+        er::GridDev *g = G(grid);
+        if (hipSetDevice(g->ctx->device) != hipSuccess ||
+            g->ctx->transfer->out(host_out, g->d_data, g->bytes(), g->ctx->stream) != hipSuccess) {
+            er::set_error("er_grid_download: copy failed");
+            return er::ST_HIP;
+        }
+        return ST_OK;
+    });
 }
 
 int er_grid_info(const er_grid *grid, int n[3], int *precision) {

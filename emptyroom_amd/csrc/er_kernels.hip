@@ -453,8 +453,28 @@ __device__ __forceinline__ double grid_frac(const JobDev *__restrict__ J, int d,
     return fma(fma(-q, (double)(J->n[d] - 1), (double)i), J->inv[d], q);
 }
 
-// Sphere of cell tc (a tile's points or a bin): the middle of its own box, the
-// radius of a full cell's, which covers a partial edge tile's as well.
+// Sphere around the grid points i0 .. i1 of a tile (or of a wave's part of one);
+// R: the radius if they are a full one's (J->cell_R, J->wave_R).
+__device__ __forceinline__ Tile points_sphere(const JobDev *__restrict__ J, const int i0[3],
+                                              const int i1[3], bool full, double R) {
+    if (!full) {  // at the far faces of the grid only
+        double lo[3], hi[3];
+#pragma unroll
+        for (int d = 0; d < 3; ++d) {
+            lo[d] = grid_frac(J, d, i0[d]);
+            hi[d] = grid_frac(J, d, i1[d]);
+        }
+        return tile_sphere(J->t, lo, hi);
+    }
+    Tile s;
+    frac_to_cart(J->t, 0.5 * (i0[0] + i1[0]) * J->inv[0], 0.5 * (i0[1] + i1[1]) * J->inv[1],
+                 0.5 * (i0[2] + i1[2]) * J->inv[2], s.cx, s.cy, s.cz);
+    s.R = R;
+    return s;
+}
+
+// Sphere around cell tc (a full tile's points, or less at the far faces, with the
+// full tile's radius; or a bin).
 __device__ __forceinline__ Tile cell_sphere(const JobDev *__restrict__ J, const int tc[3]) {
     double f[3];
 #pragma unroll
@@ -1112,11 +1132,14 @@ __device__ void grid_tile(const JobDev *__restrict__ J, const int tc[3],
         const int e = i0[d] + J->tile[d];
         i1[d] = (e < J->n[d] ? e : J->n[d]) - 1;
     }
-    const Tile tl = cell_sphere(J, tc);
+    const int t0 = J->tile[0], t1 = J->tile[1], t2 = J->tile[2];
+    const Tile tl = points_sphere(J, i0, i1,
+                                  i1[0] - i0[0] == t0 - 1 && i1[1] - i0[1] == t1 - 1 &&
+                                      i1[2] - i0[2] == t2 - 1,
+                                  J->cell_R);
     double px[PPL], py[PPL], pz[PPL], acc[PPL];
     long long oidx[PPL];
     bool ok[PPL];
-    const int t0 = J->tile[0], t1 = J->tile[1], t2 = J->tile[2];
     // Quadrant layout (FP32 and FP64 grids, even t1 and t2, t0 divisible by PPL): wave w
     // owns the (j, k) quadrant (w & 1, w >> 1) of the tile and all of its i;
     // lane l holds points i = il + q * t0 / PPL.  Otherwise point p = tid +
@@ -1160,8 +1183,7 @@ __device__ void grid_tile(const JobDev *__restrict__ J, const int tc[3],
     const bool xl = PPL > 1 && (quad || kWG % (t1 * t2) == 0) && J->t[3] == 0.0 &&
                     J->t[6] == 0.0;
     // The sphere around this wave's valid points (quadrant layout): its
-    // index box is the tile's i range times the quadrant's j and k ranges; a
-    // full quadrant's radius covers a partial one's.
+    // index box is the tile's i range times the quadrant's j and k ranges.
     bool ws = false, idle = false;
     double4 wsph = make_double4(0.0, 0.0, 0.0, 0.0);
     if (quad) {
@@ -1170,10 +1192,12 @@ __device__ void grid_tile(const JobDev *__restrict__ J, const int tc[3],
         const int ke = kb + h2 - 1 < i1[2] ? kb + h2 - 1 : i1[2];
         idle = jb > i1[1] || kb > i1[2];  // no point of this wave is on the grid
         if (!idle) {
-            double wx, wy, wz;
-            frac_to_cart(J->t, 0.5 * (i0[0] + i1[0]) * J->inv[0], 0.5 * (jb + je) * J->inv[1],
-                         0.5 * (kb + ke) * J->inv[2], wx, wy, wz);
-            wsph = make_double4(wx - tl.cx, wy - tl.cy, wz - tl.cz, J->wave_R);
+            const int w0[3] = {i0[0], jb, kb}, w1[3] = {i1[0], je, ke};
+            const Tile w = points_sphere(J, w0, w1,
+                                         i1[0] - i0[0] == t0 - 1 && je - jb == h1 - 1 &&
+                                             ke - kb == h2 - 1,
+                                         J->wave_R);
+            wsph = make_double4(w.cx - tl.cx, w.cy - tl.cy, w.cz - tl.cz, w.R);
             ws = true;
         }
     }

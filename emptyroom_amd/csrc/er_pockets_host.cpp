@@ -148,8 +148,7 @@ int grid_upload(Context *ctx, const float *host, const int n[3], GridDev **out) 
         delete g;
         return ST_NOMEM;
     }
-    if (hipMemcpyAsync(g->d_data, host, g->bytes(), hipMemcpyHostToDevice, ctx->stream) !=
-            hipSuccess ||
+    if (ctx->transfer->in(g->d_data, host, g->bytes(), ctx->stream) != hipSuccess ||
         hipStreamSynchronize(ctx->stream) != hipSuccess) {
         delete g;
         set_error("grid_upload: copy failed");
@@ -292,8 +291,8 @@ int label_chunk(Context *ctx, GridDev *const *grids, int ng, double temperature,
         HIP_TRY(launch_cc_segments(d_tab, ng, blocks, seg, s));
         for (int g = 0; g < ng; g++)
             if (seg_host[g])
-                HIP_TRY(hipMemcpyAsync(seg_host[g], seg + tab[g].seg0, sizeof(int) * tab[g].nv,
-                                       hipMemcpyDeviceToHost, s));
+                HIP_TRY(ctx->transfer->out(seg_host[g], seg + tab[g].seg0,
+                                          sizeof(int) * tab[g].nv, s));
     }
     HIP_TRY(hipStreamSynchronize(s));
     for (int g = 0; g < ng; g++) n_pockets[g] = np[g];
@@ -381,8 +380,7 @@ int widom_grid_run(Context *ctx, GridDev *g, uint64_t n_ins, double temperature,
     double sums[2];
     HIP_TRY(hipMemcpyAsync(sums, ctx->d_sums, sizeof(sums), hipMemcpyDeviceToHost, s));
     if (energies_host)
-        HIP_TRY(hipMemcpyAsync(energies_host, e, sizeof(double) * n_ins, hipMemcpyDeviceToHost,
-                               s));
+        HIP_TRY(ctx->transfer->out(energies_host, e, sizeof(double) * n_ins, s));
     HIP_TRY(hipStreamSynchronize(s));
     out->sum_b = sums[0];
     out->sum_eb = sums[1];
@@ -406,10 +404,9 @@ int grid_energies(Context *ctx, GridDev *g, const double *frac_host, uint64_t n,
     double *f = sc.get<double>(3 * n), *e = sc.get<double>(n);
     if (!f || !e) return ST_NOMEM;
     hipStream_t s = ctx->stream;
-    HIP_TRY(hipMemcpyAsync(f, frac_host, sizeof(double) * 3 * n, hipMemcpyHostToDevice, s));
+    HIP_TRY(ctx->transfer->in(f, frac_host, sizeof(double) * 3 * n, s));
     HIP_TRY(launch_grid_energies(g->d_data, g->precision, g->n, f, (long long)n, e, s));
-    HIP_TRY(hipMemcpyAsync(out_host, e, sizeof(double) * n, hipMemcpyDeviceToHost, s));
-    HIP_TRY(hipStreamSynchronize(s));
+    HIP_TRY(ctx->transfer->out(out_host, e, sizeof(double) * n, s));
     return ST_OK;
 }
 

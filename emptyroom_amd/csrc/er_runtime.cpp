@@ -204,6 +204,7 @@ int context_create(int device, size_t hbm_cap, Context **out) {
     c->device = device;
     c->hbm_cap = hbm_cap;
     c->n_cu = prop.multiProcessorCount;
+    c->transfer = Transfer::of_device(device);
     if (hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking) != hipSuccess) {
         delete c;
         set_error("hipStreamCreateWithFlags failed");
@@ -879,8 +880,7 @@ int grid_compute(Context *ctx, FrameworkDev *fw, const int n[3], int precision, 
         return fail(ST_HIP);
     if ((st = run_jobs(ctx, job_math(job), d_job, 1, job.n_items, ctx->d_counter)))
         return fail(st);
-    if (host_out &&
-        hipMemcpyAsync(host_out, g->d_data, g->bytes(), hipMemcpyDeviceToHost, s) != hipSuccess) {
+    if (host_out && ctx->transfer->out(host_out, g->d_data, g->bytes(), s) != hipSuccess) {
         set_error("grid_compute: device-to-host copy failed");
         return fail(ST_HIP);
     }
@@ -923,8 +923,7 @@ int widom_run(Context *ctx, FrameworkDev *fw, uint64_t n_ins, double temperature
     double sums[2];
     HIP_TRY(hipMemcpyAsync(sums, ctx->d_sums, sizeof(sums), hipMemcpyDeviceToHost, s));
     if (energies_host)
-        HIP_TRY(hipMemcpyAsync(energies_host, wb.e, sizeof(double) * n_ins, hipMemcpyDeviceToHost,
-                               s));
+        HIP_TRY(ctx->transfer->out(energies_host, wb.e, sizeof(double) * n_ins, s));
     HIP_TRY(hipStreamSynchronize(s));
     out->sum_b = sums[0];
     out->sum_eb = sums[1];
@@ -953,8 +952,7 @@ int count_incut_grid(Context *ctx, FrameworkDev *fw, const int n[3], unsigned lo
     HIP_TRY(launch_sum_u32(d_cnt, p, d_sum, s));
     HIP_TRY(hipMemcpyAsync(out, d_sum, sizeof(*out), hipMemcpyDeviceToHost, s));
     if (per_point_host)
-        HIP_TRY(hipMemcpyAsync(per_point_host, d_cnt, sizeof(uint32_t) * p,
-                               hipMemcpyDeviceToHost, s));
+        HIP_TRY(ctx->transfer->out(per_point_host, d_cnt, sizeof(uint32_t) * p, s));
     HIP_TRY(hipStreamSynchronize(s));
     return ST_OK;
 }
@@ -987,7 +985,7 @@ int accessibility_grid(Context *ctx, const Particle *atoms, int n_atoms, const d
     hipStream_t s = ctx->stream;
     HIP_TRY(hipMemcpyAsync(d_job, &job, sizeof(job), hipMemcpyHostToDevice, s));
     ST_TRY(run_jobs(ctx, MATH_OVERLAP, d_job, 1, job.n_items, ctx->d_counter));
-    HIP_TRY(hipMemcpyAsync(host_out, d_out, sizeof(double) * p, hipMemcpyDeviceToHost, s));
+    HIP_TRY(ctx->transfer->out(host_out, d_out, sizeof(double) * p, s));
     HIP_TRY(hipStreamSynchronize(s));
     return ST_OK;
 }

@@ -14,6 +14,7 @@
 
 #include "er_common.h"
 #include "er_kernels.h"
+#include "er_transfer.h"
 
 namespace er {
 
@@ -100,6 +101,7 @@ class Context {
     int scratch_wgs = 0;
     void *h_stage = nullptr;       // pinned host staging of pocket labelling results
     size_t h_stage_bytes = 0;
+    std::shared_ptr<Transfer> transfer;  // copies from and to the caller's arrays
     ~Context();
     // Pinned host buffer of at least `bytes` (kept, grown on demand); nullptr
     // with the error set if the allocation fails.

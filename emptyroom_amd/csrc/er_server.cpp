@@ -137,6 +137,10 @@ Server::Server(Context *ctx, const ServerConfig &cfg) : ctx_(ctx), cfg_(cfg) {
             status_ = ST_NOMEM;
         launches_.push_back(std::move(L));
     }
+    if (hipStreamCreateWithFlags(&fetch_stream_, hipStreamNonBlocking) != hipSuccess) {
+        fetch_stream_ = nullptr;
+        status_ = ST_HIP;
+    }
     (void)hipGetLastError();
     // The admission budget: the context's cap, or else what the device holds
     // now (free memory plus the pool's reserve) less a margin, so that an
@@ -170,6 +174,10 @@ Server::~Server() {
         ctx_->pool.free(L->d_jobs);
         ctx_->pool.free(L->d_counter);
         ctx_->pool.free(L->d_scratch);
+    }
+    if (fetch_stream_) {
+        (void)hipStreamSynchronize(fetch_stream_);
+        (void)hipStreamDestroy(fetch_stream_);
     }
     for (auto &kv : all_) {
         Req *r = kv.second.get();
@@ -612,7 +620,7 @@ int Server::fetch_grid(uint64_t ticket, void *host) {
     GridDev *g = r->grid;
     r->fetching++;  // release() waits until this copy is over
     lk.unlock();
-    const hipError_t e = hipMemcpy(host, g->d_data, g->bytes(), hipMemcpyDeviceToHost);
+    const hipError_t e = ctx_->transfer->out(host, g->d_data, g->bytes(), fetch_stream_);
     lk.lock();
     r->fetching--;
     done_cv_.notify_all();

@@ -120,6 +120,7 @@ class Server {
     void trim_idle();
 
     Context *ctx_;
+    hipStream_t fetch_stream_ = nullptr;  // grids to their clients
     ServerConfig cfg_;
     size_t cap_ = 0;
     std::mutex mu_;
