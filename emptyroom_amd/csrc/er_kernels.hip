@@ -519,7 +519,7 @@ __device__ __forceinline__ int near_region_start(int cap) {
 // quotients of grid_frac this took a Henry run of 1.73e7 insertions in a 424-atom
 // cell (36036 bins) from 2.52 to 2.27 ms and a 4.9e7-point grid of 2400 atoms from
 // 7.77 to 6.71 ms, where the setup of a tile cost a third of its instructions.
-template <int MATH>
+template <int MATH, int WG>
 __device__ int fill_list(const JobDev *__restrict__ J, const double4 *__restrict__ src,
                          const uint32_t *__restrict__ sidx, const int *__restrict__ tbeg,
                          const Tile &tl, int &cur_t, int &cur_pos,
@@ -597,7 +597,7 @@ __device__ int fill_list(const JobDev *__restrict__ J, const double4 *__restrict
         __syncthreads();
         int of = nf, os = ns, on = nn, tf = 0, ts = 0, tn = 0;
 #pragma unroll
-        for (int w = 0; w < kWG / 64; ++w) {
+        for (int w = 0; w < WG / 64; ++w) {
             const int cf = s_cnt[3 * w], cs = s_cnt[3 * w + 1], cn = s_cnt[3 * w + 2];
             if (w < wave) {
                 of += cf;
@@ -611,7 +611,7 @@ __device__ int fill_list(const JobDev *__restrict__ J, const double4 *__restrict
         // types that begin in this chunk: the counts before their first record
         while (first_t + nseg < last_t) {
             const int p = uniform(tbeg[first_t + nseg]) - cur_pos;
-            if (p >= kWG) break;
+            if (p >= WG) break;
             if (wave == p >> 6 && lane == 0) {
                 const uint64_t below = (1ull << (p & 63)) - 1ull;
                 int *g = seg + kSegInts * nseg;
@@ -639,7 +639,7 @@ __device__ int fill_list(const JobDev *__restrict__ J, const double4 *__restrict
         const uint64_t bx = __ballot(!fits);
         if (lane == 0) {
             // this wave's first record that does not fit, and the counts before it
-            int *x = s_cnt + 3 * (kWG / 64) + 4 * wave;
+            int *x = s_cnt + 3 * (WG / 64) + 4 * wave;
             if (bx) {
                 const int l = __builtin_ctzll(bx);
                 const uint64_t below = (1ull << l) - 1ull;
@@ -654,10 +654,10 @@ __device__ int fill_list(const JobDev *__restrict__ J, const double4 *__restrict
         __syncthreads();
         int stop = -1;
 #pragma unroll
-        for (int w = kWG / 64 - 1; w >= 0; --w)
-            if (s_cnt[3 * (kWG / 64) + 4 * w] < 64) stop = w;
+        for (int w = WG / 64 - 1; w >= 0; --w)
+            if (s_cnt[3 * (WG / 64) + 4 * w] < 64) stop = w;
         if (stop >= 0) {
-            const int *x = s_cnt + 3 * (kWG / 64) + 4 * stop;
+            const int *x = s_cnt + 3 * (WG / 64) + 4 * stop;
             nf = uniform(x[1]);
             ns = uniform(x[2]);
             nn = uniform(x[3]);
@@ -669,7 +669,7 @@ __device__ int fill_list(const JobDev *__restrict__ J, const double4 *__restrict
         nf = uniform(nf + tf);
         ns = uniform(ns + ts);
         nn = uniform(nn + tn);
-        cur_pos += kWG;
+        cur_pos += WG;
     }
     if (cur_pos >= end) {
         cur_pos = end;
@@ -1204,7 +1204,7 @@ __device__ void grid_tile(const JobDev *__restrict__ J, const int tc[3],
     int cur_t = 0, cur_pos = uniform(tbeg[0]);
     do {
         const int nseg =
-            fill_list<MATH>(J, src, sidx, tbeg, tl, cur_t, cur_pos, cap, s_list, s_seg, s_cnt);
+            fill_list<MATH, kWG>(J, src, sidx, tbeg, tl, cur_t, cur_pos, cap, s_list, s_seg, s_cnt);
         __syncthreads();
         if (!idle) {
             if (xl)
@@ -1723,7 +1723,7 @@ __global__ __launch_bounds__(kWG, MATH == MATH_NODES ? 4 : 1) void k_tiles(const
             int cur_t = 0, cur_pos = uniform(tbeg[0]);
             bool first = true;
             do {
-                const int nseg = fill_list<MATH>(J, src, sidx, tbeg, tl, cur_t, cur_pos, cap, s_list,
+                const int nseg = fill_list<MATH, kWG>(J, src, sidx, tbeg, tl, cur_t, cur_pos, cap, s_list,
                                                  s_seg, s_cnt);
                 __syncthreads();
                 // -eps_ij for every record of this pass (near; far and shell)
@@ -1772,6 +1772,332 @@ __global__ __launch_bounds__(kWG, MATH == MATH_NODES ? 4 : 1) void k_tiles(const
                 if (q < mode && rok[q]) J->e_out[rins[q]] = rt[q];
         }
         }
+    }
+}
+
+// ---- small jobs -----------------------------------------------------------
+//
+// A grid or Widom run of a few dozen cells leaves most of the device idle: the
+// launch takes as long as one workgroup's chain of fills and pairs, with one
+// wave on a SIMD to wait for every LDS read and every FP64 result.  Such jobs
+// (JobDev::parts) give each cell four workgroups of eight waves, or of four when
+// the device would not hold them all at once.  A workgroup has the 128 points of
+// one wave of grid_tile or of a bin (two per lane), makes the same lists, and its
+// waves share the records out: group g of 16 far or shell records (the FP32 sums'
+// groups, so every FP32 sum is the same) or of 8 near records goes to wave g mod
+// WAVES, and the waves' FP64 energies are added in order at the end.
+//
+// us a call, one workgroup per cell / eight waves / four waves: FP32 grid of 8
+// cells, 400 atoms 114 / 54 / 65, 64 cells 85 / 46 / 56, 216 cells 80 / 77 / 65,
+// 343 cells 87 / - / 88; Henry run of 1e3 insertions (2 bins), 1500 atoms 716 /
+// 235 / 304, 2e4 (42) 320 / 147 / 184, 1e5 (209) 260 / 231 / 212, 1.5e5 (313) 285 /
+// - / 275, 2e5 (417) 343 / - / 373.
+constexpr int kNearGroup = 8;
+
+// This wave's groups of the LDS list, for the points of all of the workgroup.
+// wn: wave-far and wave-shell counts per segment of the shared lists wl (grid
+// tiles; segment's entries at its shell offset), or nullptr.
+template <int MATH, bool XL, int WAVES>
+__device__ __forceinline__ void eval_groups(const JobDev *__restrict__ J,
+                                            const double4 *__restrict__ L, int cap,
+                                            const int *__restrict__ seg, int nseg,
+                                            const double (&px)[2], const double (&py)[2],
+                                            const double (&pz)[2], double (&acc)[2], double R,
+                                            const int *__restrict__ wn,
+                                            const uint16_t *__restrict__ wl) {
+    const int wave = uniform(threadIdx.x >> 6);
+    const double rc2 = J->rc2, min_r2 = J->min_r2;
+    const int capA = near_region_start<MATH>(cap);
+    const double4 *__restrict__ Ls = L + capA - 1, *__restrict__ Ln = L + capA;
+    const char *__restrict__ Lb = reinterpret_cast<const char *>(L);
+    double mx[2], my[2], mz[2], p2[2];
+#pragma unroll
+    for (int q = 0; q < 2; ++q) {
+        mx[q] = -2.0 * px[q];
+        my[q] = -2.0 * py[q];
+        mz[q] = -2.0 * pz[q];
+        p2[q] = px[q] * px[q] + py[q] * py[q] + pz[q] * pz[q];
+    }
+    int u = 0;  // groups before this one
+    for (int s = 0; s < nseg; ++s) {
+        const int *g = seg + kSegInts * s;
+        const int fb = uniform(g[1]), fe = uniform(g[kSegInts + 1]);
+        const int sb = uniform(g[2]), se = uniform(g[kSegInts + 2]);
+        const int nb = uniform(g[3]), ne = uniform(g[kSegInts + 3]);
+        if (fe - fb + se - sb + ne - nb == 0) continue;
+        const TypeParams P = J->types[uniform(g[0])];
+        // groups of `size` records of [0, n) that are this wave's
+        auto mine = [&](int n, auto size, auto &&group) {
+            constexpr int S = decltype(size)::value;
+            for (int r = S * ((wave - u) & (WAVES - 1)); r < n; r += S * WAVES)
+                group(r, r + S < n ? r + S : n);
+            u += (n + S - 1) / S;
+        };
+        using sixteen = std::integral_constant<int, kFlushPairs>;
+        using eight = std::integral_constant<int, kNearGroup>;
+        auto fp32 = [&](auto &&rec, auto test) {
+            return [&, rec](int b, int e) {
+                float a3[2] = {0.0f, 0.0f}, a6[2] = {0.0f, 0.0f};
+                auto pair = [&](int k) {
+                    double r2[2];
+                    pair_r2<2, XL>(rec(k), mx, my, mz, p2, r2);
+#pragma unroll
+                    for (int q = 0; q < 2; ++q) {
+                        const float w = __builtin_amdgcn_rcpf((float)r2[q]);
+                        if (decltype(test)::value) {
+                            float w3 = w * w * w;
+                            w3 = r2[q] < rc2 ? w3 : 0.0f;  // src/computegridsheet.h:79
+                            a3[q] += w3;
+                            a6[q] = __builtin_fmaf(w3, w3, a6[q]);
+                        } else {
+                            const float w2 = w * w, w3 = w2 * w;
+                            a3[q] = __builtin_fmaf(w2, w, a3[q]);
+                            a6[q] = __builtin_fmaf(w3, w3, a6[q]);
+                        }
+                    }
+                };
+                int k = b;
+                for (; k + 4 <= e; k += 4) {
+#pragma unroll
+                    for (int v = 0; v < 4; ++v) pair(k + v);
+                }
+                for (; k < e; ++k) pair(k);
+#pragma unroll
+                for (int q = 0; q < 2; ++q)
+                    acc[q] = fma(P.c6, (double)a6[q], fma(P.c3, (double)a3[q], acc[q]));
+            };
+        };
+        // FP64 pairs: NEWTON steps, the reference's clamp and cutoff test
+        auto fp64 = [&](auto &&r2_of, auto newton, auto clamp, auto test) {
+            return [&, r2_of](int b, int e) {
+                double b3[2] = {0.0, 0.0}, b6[2] = {0.0, 0.0};
+                auto pair = [&](int k) {
+                    double r2[2];
+                    r2_of(k, r2);
+#pragma unroll
+                    for (int q = 0; q < 2; ++q) {
+                        const double rr = decltype(clamp)::value ? fmax(r2[q], min_r2) : r2[q];
+                        double y = (double)__builtin_amdgcn_rcpf((float)rr);
+#pragma unroll
+                        for (int i = 0; i < decltype(newton)::value; ++i)
+                            y = fma(fma(-rr, y, 1.0), y, y);
+                        double y3 = y * y * y;
+                        if (decltype(test)::value) y3 = rr < rc2 ? y3 : 0.0;
+                        b3[q] += y3;
+                        b6[q] = fma(y3, y3, b6[q]);
+                    }
+                };
+                int k = b;
+                for (; k + 4 <= e; k += 4) {
+#pragma unroll
+                    for (int v = 0; v < 4; ++v) pair(k + v);
+                }
+                for (; k < e; ++k) pair(k);
+#pragma unroll
+                for (int q = 0; q < 2; ++q)
+                    acc[q] = fma(P.c6, b6[q], fma(P.c3, b3[q], acc[q]));
+            };
+        };
+        using no = std::integral_constant<bool, false>;
+        using yes = std::integral_constant<bool, true>;
+        using one = std::integral_constant<int, 1>;
+        using two = std::integral_constant<int, 2>;
+        auto far_rec = [&](int k) { return L[fb + k]; };
+        auto shell_rec = [&](int k) { return Ls[-(sb + k)]; };
+        auto wfar_rec = [&](int k) {
+            return *reinterpret_cast<const double4 *>(Lb + wl[sb + k]);
+        };
+        auto wshell_rec = [&](int k) {
+            return *reinterpret_cast<const double4 *>(Lb + wl[se - 1 - k]);
+        };
+        auto near_rec = [&](int k) { return Ln[nb + k]; };
+        const int nwf = wn ? uniform(wn[2 * s]) : 0;
+        const int nws = wn ? uniform(wn[2 * s + 1]) : se - sb;
+        if (MATH == MATH_MIXED) {
+            mine(fe - fb, sixteen(), fp32(far_rec, no()));
+            if (wn) {
+                mine(nwf, sixteen(), fp32(wfar_rec, no()));
+                mine(nws, sixteen(), fp32(wshell_rec, yes()));
+            } else {
+                mine(nws, sixteen(), fp32(shell_rec, yes()));
+            }
+            auto r2_of = [&](int k, double (&r2)[2]) {
+                pair_r2<2, XL>(near_rec(k), mx, my, mz, p2, r2);
+            };
+            if (P.rclose + 2.0 * R + 3.0 * kMargin < J->rc)  // see eval_list
+                mine(ne - nb, eight(), fp64(r2_of, one(), yes(), no()));
+            else
+                mine(ne - nb, eight(), fp64(r2_of, one(), yes(), yes()));
+        } else {
+            auto expanded = [&](auto &&rec) {
+                return [&, rec](int k, double (&r2)[2]) {
+                    pair_r2<2, XL>(rec(k), mx, my, mz, p2, r2);
+                };
+            };
+            mine(fe - fb, eight(), fp64(expanded(far_rec), one(), no(), no()));
+            if (wn) {
+                mine(nwf, eight(), fp64(expanded(wfar_rec), one(), no(), no()));
+                mine(nws, eight(), fp64(expanded(wshell_rec), one(), no(), yes()));
+            } else {
+                mine(nws, eight(), fp64(expanded(shell_rec), one(), no(), yes()));
+            }
+            auto differences = [&](int k, double (&r2)[2]) {
+                const double4 A = near_rec(k);
+#pragma unroll
+                for (int q = 0; q < 2; ++q) {
+                    const double dx = px[q] - A.x, dy = py[q] - A.y, dz = pz[q] - A.z;
+                    r2[q] = dx * dx + dy * dy + dz * dz;
+                }
+            };
+            mine(ne - nb, eight(), fp64(differences, two(), yes(), yes()));
+        }
+    }
+}
+
+template <int MATH, int WAVES>
+__global__ __launch_bounds__(64 * WAVES, 4) void k_parts(const JobDev *__restrict__ jobs,
+                                                         int njobs, int cap) {
+    extern __shared__ double4 s_list[];
+    __shared__ int s_seg[kSegInts * (kMaxSeg + 1)];
+    __shared__ int s_wn[2 * kMaxSeg];
+    __shared__ int s_cnt[7 * WAVES];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const long long item = blockIdx.x;
+    int jl = 0, jh = njobs - 1;
+    while (jl < jh) {
+        const int mid = (jl + jh + 1) >> 1;
+        if (jobs[mid].item_begin <= item) jl = mid;
+        else jh = mid - 1;
+    }
+    const JobDev *__restrict__ J = jobs + jl;
+    const long long local = item - J->item_begin + J->local0;
+    const int part = (int)(local & 3);
+    const bool grid = MATH == MATH_FP64 || J->kind == JOB_GRID;
+    const int *nc = grid ? J->ntiles : J->nbins;
+    int tc[3];
+    const long long cell = local >> 2;
+    tc[2] = (int)(cell % nc[2]);
+    tc[1] = (int)((cell / nc[2]) % nc[1]);
+    tc[0] = (int)(cell / ((long long)nc[1] * nc[2]));
+    uint16_t *__restrict__ s_wl = reinterpret_cast<uint16_t *>(s_list + cap);
+
+    // a tile: the part's quadrant, as a wave of grid_tile has it; a bin: the
+    // insertions a wave of k_tiles has of each 512
+    int i0[3] = {0, 0, 0}, i1[3] = {0, 0, 0};
+    const int h1 = J->tile[1] / 2, h2 = J->tile[2] / 2;
+    uint32_t s0 = 0, s1 = 0;
+    Tile tl;
+    double4 wsph = make_double4(0.0, 0.0, 0.0, 0.0);
+    if (grid) {
+#pragma unroll
+        for (int d = 0; d < 3; ++d) {
+            i0[d] = tc[d] * J->tile[d];
+            const int e = i0[d] + J->tile[d];
+            i1[d] = (e < J->n[d] ? e : J->n[d]) - 1;
+        }
+        const int jb = i0[1] + (part & 1) * h1, kb = i0[2] + (part >> 1) * h2;
+        const int je = jb + h1 - 1 < i1[1] ? jb + h1 - 1 : i1[1];
+        const int ke = kb + h2 - 1 < i1[2] ? kb + h2 - 1 : i1[2];
+        if (jb > i1[1] || kb > i1[2]) return;  // no point of the part is on the grid
+        tl = points_sphere(J, i0, i1,
+                           i1[0] - i0[0] == J->tile[0] - 1 && i1[1] - i0[1] == J->tile[1] - 1 &&
+                               i1[2] - i0[2] == J->tile[2] - 1,
+                           J->cell_R);
+        const int w0[3] = {i0[0], jb, kb}, w1[3] = {i1[0], je, ke};
+        const Tile w = points_sphere(J, w0, w1,
+                                     i1[0] - i0[0] == J->tile[0] - 1 && je - jb == h1 - 1 &&
+                                         ke - kb == h2 - 1,
+                                     J->wave_R);
+        wsph = make_double4(w.cx - tl.cx, w.cy - tl.cy, w.cz - tl.cz, w.R);
+    } else {
+        const int b = (tc[0] * nc[1] + tc[1]) * nc[2] + tc[2];
+        s0 = J->bin_start[b];
+        s1 = J->bin_start[b + 1];
+        tl = cell_sphere(J, tc);
+    }
+    const bool xl = grid && J->t[3] == 0.0 && J->t[6] == 0.0;
+    // (a grid's part is one round; a bin has one for every 512 insertions)
+    for (uint32_t c = s0 + 64u * part; grid || c < s1; c += 512u) {
+        double px[2], py[2], pz[2], acc[2];
+        long long at[2];
+        bool ok[2];
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {
+            acc[q] = 0.0;
+            if (grid) {
+                int gi = i0[0] + lane / (h1 * h2) + q * (J->tile[0] / 2);
+                int gj = i0[1] + (part & 1) * h1 + (lane / h2) % h1;
+                int gk = i0[2] + (part >> 1) * h2 + lane % h2;
+                ok[q] = gi <= i1[0] && gj <= i1[1] && gk <= i1[2];
+                if (!ok[q]) {
+                    gi = i0[0];
+                    gj = i0[1];
+                    gk = i0[2];
+                }
+                frac_to_cart(J->t, grid_frac(J, 0, gi), grid_frac(J, 1, gj), grid_frac(J, 2, gk),
+                             px[q], py[q], pz[q]);
+                at[q] = (long long)gk + (long long)gj * J->n[2] +
+                        (long long)gi * J->n[1] * J->n[2];
+            } else {
+                const uint64_t slot = (uint64_t)c + lane + 256u * q;
+                ok[q] = slot < s1;
+                at[q] = J->sorted[ok[q] ? slot : c];
+                double f[3];
+                widom_point(J->seed, J->stream, (uint64_t)at[q], f);
+                frac_to_cart(J->t, f[0], f[1], f[2], px[q], py[q], pz[q]);
+            }
+            px[q] -= tl.cx;
+            py[q] -= tl.cy;
+            pz[q] -= tl.cz;
+        }
+        int cur_t = 0, cur_pos = uniform(J->type_begin[0]);
+        do {
+            const int nseg = fill_list<MATH, 64 * WAVES>(J, J->near, nullptr, J->type_begin, tl,
+                                                      cur_t, cur_pos, cap, s_list, s_seg, s_cnt);
+            __syncthreads();
+            if (grid) {
+                // each segment's shell records against the part's points, a wave
+                // per segment
+                const int capA = near_region_start<MATH>(cap);
+                for (int s = wave; s < nseg; s += WAVES) {
+                    const int sb = uniform(s_seg[kSegInts * s + 2]),
+                              se = uniform(s_seg[kSegInts * (s + 1) + 2]);
+                    int nwf = 0, nws = 0;
+                    if (se > sb)
+                        wave_shell_lists(J, s_list + capA - 1, capA, se - sb, sb, se, wsph,
+                                         s_wl + sb, nwf, nws);
+                    if (lane == 0) {
+                        s_wn[2 * s] = nwf;
+                        s_wn[2 * s + 1] = nws;
+                    }
+                }
+                __syncthreads();
+            }
+            if (xl)
+                eval_groups<MATH, true, WAVES>(J, s_list, cap, s_seg, nseg, px, py, pz, acc, tl.R, s_wn,
+                                        s_wl);
+            else
+                eval_groups<MATH, false, WAVES>(J, s_list, cap, s_seg, nseg, px, py, pz, acc, tl.R,
+                                         grid ? s_wn : nullptr, s_wl);
+            __syncthreads();
+        } while (cur_t < J->ntypes);
+        // the waves' energies, added in order
+        double *red = reinterpret_cast<double *>(s_list);
+#pragma unroll
+        for (int q = 0; q < 2; ++q) red[(2 * wave + q) * 64 + lane] = acc[q];
+        __syncthreads();
+        if (wave < 2) {
+            double e = 0.0;
+            for (int w = 0; w < WAVES; ++w) e += red[(2 * w + wave) * 64 + lane];
+            const long long o = wave == 0 ? at[0] : at[1];
+            if (wave == 0 ? ok[0] : ok[1]) {
+                if (!grid) J->e_out[o] = e;
+                else if (J->mode == OUT_F64) ((double *)J->out)[o] = e;
+                else ((float *)J->out)[o] = (float)(e < (double)FLT_MAX ? e : (double)FLT_MAX);
+            }
+        }
+        if (grid) return;
+        __syncthreads();
     }
 }
 
@@ -1891,8 +2217,9 @@ int grid_blocks(long long n, int per_block, int cap_blocks) {
 template <int PPL, int MATH>
 hipError_t launch_tiles_t(const JobDev *jobs, int njobs, long long total, unsigned long long *ctr,
                           int wgs, int cap, uint32_t *scratch, int scratch_cap, hipStream_t s) {
-    hipLaunchKernelGGL((k_tiles<PPL, MATH>), dim3(wgs), dim3(kWG), tiles_lds_bytes(cap, MATH), s, jobs,
-                       njobs, total, ctr, cap, scratch, scratch_cap);
+    hipLaunchKernelGGL((k_tiles<PPL, MATH>), dim3(wgs), dim3(kWG),
+                       tiles_lds_bytes(cap, MATH), s, jobs, njobs, total, ctr, cap, scratch,
+                       scratch_cap);
     return hipGetLastError();
 }
 
@@ -1900,7 +2227,8 @@ template <int PPL, int MATH>
 int occupancy_t(int cap) {
     int n = 0;
     if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, k_tiles<PPL, MATH>, kWG,
-                                                     tiles_lds_bytes(cap, MATH)) != hipSuccess)
+                                                     tiles_lds_bytes(cap, MATH)) !=
+        hipSuccess)
         return 1;
     return n > 0 ? n : 1;
 }
@@ -1999,10 +2327,30 @@ size_t tiles_lds_bytes(int cap, int math) {
     return (b + 15) & ~(size_t)15;
 }
 
+static hipError_t launch_parts(int math, const JobDev *jobs, int njobs, long long total,
+                               int cap, hipStream_t s) {
+    if (total <= 0) return hipSuccess;
+    if (cap < 2 * kWG || total > (1LL << 31) - 1) return hipErrorInvalidValue;
+    // one list of shell offsets for the workgroup
+    const size_t lds = ((size_t)cap * (sizeof(double4) + sizeof(uint16_t)) + 15) & ~(size_t)15;
+#define ER_PARTS(V, M, W)                                                                     \
+    if (math == V)                                                                            \
+        hipLaunchKernelGGL((k_parts<M, W>), dim3((unsigned)total), dim3(64 * W), lds, s, jobs, \
+                           njobs, cap);
+    ER_PARTS(MATH_PARTS8, MATH_MIXED, 8)
+    ER_PARTS(MATH_PARTS8_FP64, MATH_FP64, 8)
+    ER_PARTS(MATH_PARTS4, MATH_MIXED, 4)
+    ER_PARTS(MATH_PARTS4_FP64, MATH_FP64, 4)
+#undef ER_PARTS
+    return hipGetLastError();
+}
+
 hipError_t launch_tiles(int math, int ppl, const JobDev *jobs, int njobs, long long total,
                         unsigned long long *ctr, int wgs, int cap, uint32_t *scratch,
                         int scratch_cap, hipStream_t s) {
     if (total <= 0) return hipSuccess;
+    if (math >= MATH_PARTS8 && math <= MATH_PARTS4_FP64)
+        return launch_parts(math, jobs, njobs, total, cap, s);
     if (cap < 2 * kWG || wgs <= 0) return hipErrorInvalidValue;
     if (scratch && scratch_cap < kWG) return hipErrorInvalidValue;
     if (math == MATH_NODES && (!scratch || cap < 2 * kWG + kNodeRecords))

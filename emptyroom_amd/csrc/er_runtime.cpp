@@ -636,7 +636,25 @@ JobDev make_grid_job(const FrameworkDev *fw, const int n[3], int precision, void
     j.wave_R = box_radius(fw->t, j.wave_box);
     j.out = d_out;
     j.n_items = items;
+    if (math == MATH_MIXED || math == MATH_FP64) use_parts(&j, tu);
     return j;
+}
+
+void use_parts(JobDev *j, const Tuning &tu) {
+    const bool grid = j->kind == JOB_GRID;
+    const int *nc = grid ? j->ntiles : j->nbins;
+    const long long cells = (long long)nc[0] * nc[1] * nc[2];
+    // (16-bit offsets into the list, and two workgroups' LDS per CU)
+    if (j->interp || cells > kPartCells4 || tu.cap > 2048) return;
+    // the quadrant layout of grid_tile with two points per lane; insertions have
+    // the same energies whatever the points per lane
+    if (grid && (tu.ppl != 2 || j->tile[0] % 2 || j->tile[1] % 2 || j->tile[2] % 2)) return;
+    j->parts = cells <= kPartCells8 ? 8 : 4;
+    for (int d = 0; d < 3; d++) {
+        j->region[d] = 1;
+        j->nregions[d] = nc[d];
+    }
+    j->n_items = 4 * cells;
 }
 
 JobDev make_widom_job(const FrameworkDev *fw, uint64_t n_ins, uint64_t seed,
@@ -912,12 +930,13 @@ int widom_run(Context *ctx, FrameworkDev *fw, uint64_t n_ins, double temperature
     // sums are, and saturated insertions may stop early
     JobDev job = make_widom_job(fw, n_ins, seed, wb, ctx->tuning, kMinGridItems,
                                 energies_host ? 0.0 : temperature);
+    use_parts(&job, ctx->tuning);
     JobDev *d_job = nullptr;
     ST_TRY(pool_alloc(ctx, 1, &d_job, &tmp.ptrs));
     hipStream_t s = ctx->stream;
     HIP_TRY(hipMemcpyAsync(d_job, &job, sizeof(job), hipMemcpyHostToDevice, s));
     ST_TRY(widom_enqueue_binning(ctx, wb, n_ins, seed, 0u, s));
-    ST_TRY(run_jobs(ctx, MATH_MIXED, d_job, 1, job.n_items, ctx->d_counter));
+    ST_TRY(run_jobs(ctx, job_math(job), d_job, 1, job.n_items, ctx->d_counter));
     HIP_TRY(launch_widom_partials(wb.e, (long long)n_ins, temperature, ctx->d_partials, s));
     HIP_TRY(launch_widom_final(ctx->d_partials, ctx->d_sums, s));
     double sums[2];
@@ -1031,7 +1050,9 @@ Batch::~Batch() {
 namespace {
 
 // Launches of a batch, in this order.
-constexpr int kBatchMath[kBatchLaunches] = {MATH_NODES, MATH_MIXED, MATH_FP64};
+constexpr int kBatchMath[kBatchLaunches] = {MATH_NODES,  MATH_MIXED,       MATH_FP64,
+                                              MATH_PARTS4, MATH_PARTS4_FP64, MATH_PARTS8,
+                                              MATH_PARTS8_FP64};
 
 // Expected in-cutoff pairs per point: the ordering key of the LPT schedule.
 double job_cost_per_item(const FrameworkDev *fw, const JobDev &j, const Tuning &tu) {
@@ -1142,6 +1163,7 @@ int batch_create(Context *ctx, const Task *tasks, int n, bool use_graph, Batch *
             JobDev j = make_widom_job(tk.fw, tk.n_ins, tk.seed, b->wbufs[t], ctx->tuning,
                                       std::max<long long>(1, kMinGridItems / std::max(n, 1)),
                                       tk.temperature);
+            use_parts(&j, ctx->tuning);
             found.push_back({job_cost_per_item(tk.fw, j, ctx->tuning), j});
         }
     }

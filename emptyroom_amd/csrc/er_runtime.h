@@ -216,6 +216,9 @@ void choose_region(const FrameworkDev *fw, const double cell_frac[3], const int 
 JobDev make_widom_job(const FrameworkDev *fw, uint64_t n_ins, uint64_t seed,
                       const WidomBuffers &wb, const Tuning &tu, long long min_items,
                       double temperature = 0.0);
+// Makes a grid or Widom job of few cells a job of parts (see k_parts): the
+// choice depends on the cells and the knobs alone, so a job is the same on every path.
+void use_parts(JobDev *j, const Tuning &tu);
 // Allocates the Widom buffers of a job (owned pointers appended to `owned`).
 int widom_prepare(Context *ctx, FrameworkDev *fw, uint64_t n_ins, WidomBuffers *wb,
                   std::vector<void *> *owned);
@@ -254,7 +257,7 @@ struct Task {
     uint64_t seed = 0;
 };
 
-constexpr int kBatchLaunches = 3;  // tiled-kernel variants of a batch, one launch each
+constexpr int kBatchLaunches = 7;  // tiled-kernel variants of a batch, one launch each
 
 class Batch {
   public:

@@ -340,6 +340,7 @@ bool Server::admit_one(Req *r, FwEntry *hit) {
         if (st == ST_OK) {
             r->widom_job = make_widom_job(r->fw, s.n_ins, s.seed, r->wb, ctx_->tuning,
                                           kMinGridItems, s.temperature);
+            use_parts(&r->widom_job, ctx_->tuning);
             r->items_total += r->widom_job.n_items;
             st = widom_enqueue_binning(ctx_, r->wb, s.n_ins, s.seed, 0u, ctx_->stream);
         }
@@ -511,8 +512,8 @@ void Server::run() {
             // the pair-math variant of this launch: that of the oldest ready
             // request's pending work (its grid first)
             const Req *o = ready.front();
-            const int math = o->grid_next < o->grid_job.n_items ? job_math(o->grid_job)
-                                                                : MATH_MIXED;
+            const int math = job_math(o->grid_next < o->grid_job.n_items ? o->grid_job
+                                                                         : o->widom_job);
             long long nkind = 0;
             for (Req *r : ready)
                 for (int kind = 0; kind < 2; kind++) {
