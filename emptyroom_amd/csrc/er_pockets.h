@@ -52,8 +52,11 @@ constexpr int kTriBlocks = 4096;
 // interpolated on an FP32 (precision 0) or FP64 (precision 1) grid.
 hipError_t launch_grid_energies(const void *g, int precision, const int n[3], const double *f,
                                 long long npos, double *out, hipStream_t s);
-hipError_t launch_widom_grid(const float *g, const int n[3], uint64_t seed, uint32_t stream,
-                             uint64_t nins, double temperature, double *e_out, double2 *partials,
-                             hipStream_t s);
+// faces (nullable): room for tri_faces_bytes, the corners of every cell side by side.
+hipError_t launch_widom_grid(const float *g, float4 *faces, const int n[3], uint64_t seed,
+                             uint32_t stream, uint64_t nins, double temperature, double *e_out,
+                             double2 *partials, hipStream_t s);
+// Bytes of the face records a run should use, 0 if it is better without.
+size_t tri_faces_bytes(const int n[3], uint64_t nins);
 
 }  // namespace er

@@ -460,33 +460,79 @@ __global__ __launch_bounds__(kWG) void k_cc_block(const CCGrid *__restrict__ gri
 
 // Trilinear energy of src/gcmc.cc:145-177 after the wrap of src/gcmc.cc:74-77,
 // with the lower index clamped to N-2 (f = 1 reads node N-1).
-template <class T>
-__device__ __forceinline__ double trilinear(const T *__restrict__ g, int nx, int ny, int nz,
-                                            double xf, double yf, double zf) {
+struct TriCell {
+    int ix, iy, iz;
+    double xd, yd, zd;
+};
+
+__device__ __forceinline__ TriCell tri_cell(int nx, int ny, int nz, double xf, double yf,
+                                            double zf) {
     // Separate multiplies and adds, as the reference's host code computes
     // them: next to blocked (1e13 K) nodes a fused multiply-add changes the
     // interpolated energy far beyond rounding of the result.
 #pragma clang fp contract(off)
+    TriCell c;
     const double dx = 1.0 / (nx - 1), dy = 1.0 / (ny - 1), dz = 1.0 / (nz - 1);
     int ix = (int)floor(xf / dx), iy = (int)floor(yf / dy), iz = (int)floor(zf / dz);
-    ix = ix > nx - 2 ? nx - 2 : (ix < 0 ? 0 : ix);
-    iy = iy > ny - 2 ? ny - 2 : (iy < 0 ? 0 : iy);
-    iz = iz > nz - 2 ? nz - 2 : (iz < 0 ? 0 : iz);
-    const double xd = (xf - ix * dx) / dx;
-    const double yd = (yf - iy * dy) / dy;
-    const double zd = (zf - iz * dz) / dz;
+    c.ix = ix > nx - 2 ? nx - 2 : (ix < 0 ? 0 : ix);
+    c.iy = iy > ny - 2 ? ny - 2 : (iy < 0 ? 0 : iy);
+    c.iz = iz > nz - 2 ? nz - 2 : (iz < 0 ? 0 : iz);
+    c.xd = (xf - c.ix * dx) / dx;
+    c.yd = (yf - c.iy * dy) / dy;
+    c.zd = (zf - c.iz * dz) / dz;
+    return c;
+}
+
+__device__ __forceinline__ double tri_blend(const TriCell &c, double g000, double g100,
+                                            double g010, double g110, double g001, double g101,
+                                            double g011, double g111) {
+#pragma clang fp contract(off)
+    const double c00 = g000 * (1.0 - c.xd) + c.xd * g100;
+    const double c10 = g010 * (1.0 - c.xd) + c.xd * g110;
+    const double c01 = g001 * (1.0 - c.xd) + c.xd * g101;
+    const double c11 = g011 * (1.0 - c.xd) + c.xd * g111;
+    const double c0 = c00 * (1.0 - c.yd) + c10 * c.yd;
+    const double c1 = c01 * (1.0 - c.yd) + c11 * c.yd;
+    return c0 * (1 - c.zd) + c1 * c.zd;
+}
+
+template <class T>
+__device__ __forceinline__ double trilinear(const T *__restrict__ g, int nx, int ny, int nz,
+                                            double xf, double yf, double zf) {
+    const TriCell c = tri_cell(nx, ny, nz, xf, yf, zf);
     const long long syz = (long long)ny * nz;
-    const long long b = (long long)iz + (long long)iy * nz + (long long)ix * syz;
-    const double g000 = g[b], g100 = g[b + syz], g010 = g[b + nz], g110 = g[b + syz + nz];
-    const double g001 = g[b + 1], g101 = g[b + syz + 1], g011 = g[b + nz + 1],
-                 g111 = g[b + syz + nz + 1];
-    const double c00 = g000 * (1.0 - xd) + xd * g100;
-    const double c10 = g010 * (1.0 - xd) + xd * g110;
-    const double c01 = g001 * (1.0 - xd) + xd * g101;
-    const double c11 = g011 * (1.0 - xd) + xd * g111;
-    const double c0 = c00 * (1.0 - yd) + c10 * yd;
-    const double c1 = c01 * (1.0 - yd) + c11 * yd;
-    return c0 * (1 - zd) + c1 * zd;
+    const long long b = (long long)c.iz + (long long)c.iy * nz + (long long)c.ix * syz;
+    return tri_blend(c, g[b], g[b + syz], g[b + nz], g[b + syz + nz], g[b + 1], g[b + syz + 1],
+                     g[b + nz + 1], g[b + syz + nz + 1]);
+}
+
+// faces[(j (nz - 1) + k) nx + i] = the grid's values at (i, j..j+1, k..k+1): the
+// eight corners of cell (i, j, k) are two consecutive records.  A block takes
+// 64 k by 16 i of one j through LDS, so that both sides move whole lines.
+constexpr int kFaceK = 64, kFaceI = 16;
+
+__global__ __launch_bounds__(kWG) void k_tri_faces(const float *__restrict__ g, int nx, int ny,
+                                                   int nz, float4 *__restrict__ faces) {
+    __shared__ float s[2][kFaceI][kFaceK + 2];
+    const int nkb = (nz - 1 + kFaceK - 1) / kFaceK, nib = (nx + kFaceI - 1) / kFaceI;
+    int b = blockIdx.x;
+    const int k0 = (b % nkb) * kFaceK;
+    b /= nkb;
+    const int i0 = (b % nib) * kFaceI, j = b / nib;
+    for (int t = threadIdx.x; t < 2 * kFaceI * (kFaceK + 1); t += kWG) {
+        const int k = t % (kFaceK + 1), i = (t / (kFaceK + 1)) % kFaceI,
+                  d = t / ((kFaceK + 1) * kFaceI);
+        if (k0 + k < nz && i0 + i < nx)
+            s[d][i][k] = g[(long long)(k0 + k) + (long long)(j + d) * nz +
+                           (long long)(i0 + i) * ny * nz];
+    }
+    __syncthreads();
+    for (int t = threadIdx.x; t < kFaceI * kFaceK; t += kWG) {
+        const int i = t % kFaceI, k = t / kFaceI;
+        if (k0 + k < nz - 1 && i0 + i < nx)
+            faces[((long long)j * (nz - 1) + k0 + k) * nx + i0 + i] =
+                make_float4(s[0][i][k], s[0][i][k + 1], s[1][i][k], s[1][i][k + 1]);
+    }
 }
 
 // Guest-framework energy at caller-given fractional positions: the wrap of
@@ -508,8 +554,14 @@ __global__ __launch_bounds__(kWG) void k_grid_energies(const T *__restrict__ g, 
 // its threads stride through it, and the block writes one (sum b, sum E b)
 // partial in a fixed order, so the result does not depend on scheduling.
 // e_out (nullable) receives the energy of every insertion.
-__global__ __launch_bounds__(kWG) void k_widom_grid(const float *__restrict__ g, int nx, int ny,
-                                                    int nz, uint64_t seed, uint32_t stream,
+//
+// The kernel is bound by the lines its gathers bring into L1 (4.1 of 128 bytes
+// an insertion from the grid, 15.8 TB/s) and, beyond the 4 MiB of an XCD's L2,
+// into L2.  With FACES the corners are two neighbouring records, 1.1 lines.
+template <bool FACES>
+__global__ __launch_bounds__(kWG) void k_widom_grid(const float *__restrict__ g,
+                                                    const float4 *__restrict__ faces, int nx,
+                                                    int ny, int nz, uint64_t seed, uint32_t stream,
                                                     uint64_t n, double temperature,
                                                     double *__restrict__ e_out,
                                                     double2 *__restrict__ partials) {
@@ -520,8 +572,17 @@ __global__ __launch_bounds__(kWG) void k_widom_grid(const float *__restrict__ g,
     for (uint64_t i = lo + threadIdx.x; i < hi; i += kWG) {
         double f[3];
         widom_point(seed, stream, i, f);
-        const double E = trilinear(g, nx, ny, nz, f[0] - floor(f[0]), f[1] - floor(f[1]),
-                                   f[2] - floor(f[2]));
+        double E;
+        if (FACES) {
+            const TriCell c = tri_cell(nx, ny, nz, f[0] - floor(f[0]), f[1] - floor(f[1]),
+                                       f[2] - floor(f[2]));
+            const float4 *r = faces + ((long long)c.iy * (nz - 1) + c.iz) * nx + c.ix;
+            const float4 u = r[0], v = r[1];
+            E = tri_blend(c, u.x, v.x, u.z, v.z, u.y, v.y, u.w, v.w);
+        } else {
+            E = trilinear(g, nx, ny, nz, f[0] - floor(f[0]), f[1] - floor(f[1]),
+                          f[2] - floor(f[2]));
+        }
         if (e_out) e_out[i] = E;
         const double bz = exp(-E / temperature);
         sb += bz;
@@ -602,12 +663,34 @@ hipError_t launch_cc_block(const CCGrid *grids, int ng, long long total_blocks, 
     return hipGetLastError();
 }
 
-hipError_t launch_widom_grid(const float *g, const int n[3], uint64_t seed, uint32_t stream,
-                             uint64_t nins, double temperature, double *e_out, double2 *partials,
-                             hipStream_t s) {
+// Records pay for their pass when insertions outnumber the voxels, and not where
+// the grid fits the L2 of an XCD but its records (four times as large) do not.
+// us without / with records (their pass included), 1e7 insertions: 0.8 MB grid
+// 166 / 95, 4.0 MB 165 / 160, 7.9 MB 324 / 188, 16 MB 502 / 222, 42 MB 660 / 258;
+// 1e6 insertions: 0.8 MB 23 / 22, 7.9 MB 37 / 35, 16 MB 55 / 47, 42 MB 71 / 69.
+size_t tri_faces_bytes(const int n[3], uint64_t nins) {
+    const uint64_t nv = (uint64_t)n[0] * n[1] * n[2];
+    const bool fits = nv <= (1u << 18), large = nv >= 1300000 && nv <= (1u << 27);
+    if (!(fits || large) || nins < 1000000 || nins < nv / 2) return 0;
+    return sizeof(float4) * (size_t)(n[1] - 1) * (n[2] - 1) * n[0];
+}
+
+hipError_t launch_widom_grid(const float *g, float4 *faces, const int n[3], uint64_t seed,
+                             uint32_t stream, uint64_t nins, double temperature, double *e_out,
+                             double2 *partials, hipStream_t s) {
     if (nins == 0) return hipSuccess;
-    hipLaunchKernelGGL(k_widom_grid, dim3(kTriBlocks), dim3(kWG), 0, s, g, n[0], n[1], n[2], seed,
-                       stream, nins, temperature, e_out, partials);
+    if (!faces) {
+        hipLaunchKernelGGL(k_widom_grid<false>, dim3(kTriBlocks), dim3(kWG), 0, s, g, faces, n[0],
+                           n[1], n[2], seed, stream, nins, temperature, e_out, partials);
+        return hipGetLastError();
+    }
+    const long long blocks = (long long)(n[1] - 1) * ((n[0] + kFaceI - 1) / kFaceI) *
+                             ((n[2] - 1 + kFaceK - 1) / kFaceK);
+    if (blocks > (1LL << 31) - 1) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(k_tri_faces, dim3((unsigned)blocks), dim3(kWG), 0, s, g, n[0], n[1], n[2],
+                       faces);
+    hipLaunchKernelGGL(k_widom_grid<true>, dim3(kTriBlocks), dim3(kWG), 0, s, g, faces, n[0], n[1],
+                       n[2], seed, stream, nins, temperature, e_out, partials);
     return hipGetLastError();
 }
 

@@ -374,8 +374,11 @@ int widom_grid_run(Context *ctx, GridDev *g, uint64_t n_ins, double temperature,
     double2 *partials = sc.get<double2>(kTriBlocks);
     if ((energies_host && !e) || !partials) return ST_NOMEM;
     hipStream_t s = ctx->stream;
-    HIP_TRY(launch_widom_grid((const float *)g->d_data, g->n, seed, 1u, n_ins, temperature, e,
-                              partials, s));
+    // (without the memory for them the run does without face records)
+    const size_t fb = tri_faces_bytes(g->n, n_ins);
+    float4 *faces = fb ? (float4 *)sc.get<char>(fb) : nullptr;
+    HIP_TRY(launch_widom_grid((const float *)g->d_data, faces, g->n, seed, 1u, n_ins, temperature,
+                              e, partials, s));
     HIP_TRY(launch_widom_final_n(partials, kTriBlocks, ctx->d_sums, s));
     double sums[2];
     HIP_TRY(hipMemcpyAsync(sums, ctx->d_sums, sizeof(sums), hipMemcpyDeviceToHost, s));
