@@ -257,14 +257,12 @@ int direct_widom(Context *ctx, const Particle *atoms, int n_atoms, const double 
                        dim3(kDirectWG), 0, s, J, seed, (long long)n_ins, e);
     HIP_TRY(hipGetLastError());
     HIP_TRY(launch_widom_partials(e, (long long)n_ins, temperature, ctx->d_partials, s));
-    HIP_TRY(launch_widom_final(ctx->d_partials, ctx->d_sums, s));
-    double sums[2];
-    HIP_TRY(hipMemcpyAsync(sums, ctx->d_sums, sizeof(sums), hipMemcpyDeviceToHost, s));
+    HIP_TRY(launch_widom_final(ctx->d_partials, ctx->h_sums, s));
     if (energies_host)
         HIP_TRY(hipMemcpyAsync(energies_host, e, sizeof(double) * n_ins, hipMemcpyDeviceToHost, s));
     HIP_TRY(hipStreamSynchronize(s));
-    out->sum_b = sums[0];
-    out->sum_eb = sums[1];
+    out->sum_b = ctx->h_sums[0];
+    out->sum_eb = ctx->h_sums[1];
     out->n = n_ins;
     return ST_OK;
 }

@@ -55,6 +55,11 @@ hipError_t launch_near_offsets(const NearPlan &p, const uint32_t *block_count,
 hipError_t launch_near_write(const NearPlan &p, const uint32_t *block_off, double4 *near,
                              hipStream_t s);
 
+// --- one job's descriptors -----------------------------------------------------
+// Writes *d_job (and, with bin, *d_bin, whose counts it clears) and zeroes *counter.
+hipError_t launch_setup(const JobDev &job, JobDev *d_job, unsigned long long *counter,
+                        const BinJob *bin, BinJob *d_bin, hipStream_t s);
+
 // --- fills ------------------------------------------------------------------
 hipError_t launch_fill_u64(unsigned long long *p, unsigned long long v, long long n,
                            hipStream_t s);
@@ -64,10 +69,11 @@ hipError_t launch_fill_u64(unsigned long long *p, unsigned long long v, long lon
 // `chunk` insertions each (total_blocks = sum over jobs of ceil(n / chunk)) and
 // whose gblock0 fields number the groups of the grouped jobs (total_groups).
 // max_keys: largest ngroups; max_group: largest group.
-// Order: zero, count, scan, scatter, sort of the groups (all on one stream).
+// Order: zero (unless cleared), count, scan, scatter, sort of the groups (all on
+// one stream).
 hipError_t launch_bin_all(const BinJob *jobs, int njobs, long long total_blocks, int chunk,
                           long long max_keys, int max_group, long long total_groups,
-                          hipStream_t s);
+                          bool cleared, hipStream_t s);
 int bin_blocks(uint64_t n, int chunk);
 int bin_chunk(uint64_t total_insertions, long long max_keys);
 // Group size and count for a job of nbins bins (group 1: binned in one step).

@@ -5,8 +5,8 @@
 // The device memory the tiled kernel needs beyond its input (the resident
 // framework) and its output (the caller's grid) is a fixed array of this
 // library, `scratch`, one copy per device:
-//   [0, 256)          work counter of the persistent launch (cleared by a
-//                     fill kernel before every launch)
+//   [0, 256)          work counter of the persistent launch (cleared before
+//                     every launch)
 //   [256, 4096)       the job descriptor
 //   [4096, ...)       region sub-lists: kNoAllocSlices slices of
 //                     kNoAllocRecords near-list indices (4 B), one per
@@ -106,16 +106,13 @@ int grid_compute_noalloc(Context *ctx, FrameworkDev *fw, const int n[3], int pre
                                      precision == 1 ? MATH_FP64 : MATH_MIXED, kNoAllocRecords);
     const int math = job_math(job);
     hipStream_t s = ctx->stream;
-    if ((e = hipMemcpyAsync(d_job, &job, sizeof(job), hipMemcpyHostToDevice, s)) != hipSuccess)
-        return hip_fail("job copy", e);
-    if ((e = launch_fill_u64(counter, 0ull, 1, s)) != hipSuccess)
-        return hip_fail("counter clear", e);
+    if ((e = launch_setup(job, d_job, counter, nullptr, nullptr, s)) != hipSuccess)
+        return hip_fail("job setup", e);
     const int wgs = tiles_workgroups(ctx, math, job.n_items, kNoAllocSlices);
     if ((e = launch_tiles(math, ctx->tuning.ppl, d_job, 1, job.n_items, counter, wgs,
                           ctx->tuning.cap, slices, kNoAllocRecords, s)) != hipSuccess)
         return hip_fail("tile kernel launch", e);
-    // the job descriptor was copied from this frame's stack: wait for the
-    // whole call before returning
+    // the call returns when the grid is written
     if ((e = hipStreamSynchronize(s)) != hipSuccess) return hip_fail("synchronize", e);
     return ST_OK;
 }

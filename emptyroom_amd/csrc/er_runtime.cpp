@@ -163,7 +163,7 @@ Context::~Context() {
     }
     pool.free(d_counter);
     pool.free(d_partials);
-    pool.free(d_sums);
+    if (h_sums) (void)hipHostFree(h_sums);
     pool.free(d_scratch);
     if (h_stage) (void)hipHostFree(h_stage);
 }
@@ -212,7 +212,7 @@ int context_create(int device, size_t hbm_cap, Context **out) {
     }
     if (pool_alloc(c, 1, &c->d_counter, nullptr) != ST_OK ||
         pool_alloc(c, kReduceBlocks, &c->d_partials, nullptr) != ST_OK ||
-        pool_alloc(c, 2, &c->d_sums, nullptr) != ST_OK ||
+        hipHostMalloc((void **)&c->h_sums, 2 * sizeof(double)) != hipSuccess ||
         scratch_ensure(c, c->stream, &c->d_scratch, &c->scratch_wgs) != ST_OK) {
         delete c;
         return ST_NOMEM;
@@ -376,28 +376,35 @@ int framework_upload(Context *ctx, const Particle *atoms, int n, const double t[
     plan.nblocks = type_block0[nt];
     plan.n_images = (int)fw->n_images;
     fw->near_capacity = std::max<size_t>(1, (size_t)n * cap_atoms);
+    // atoms, pair parameters and the type tables as one block: one copy
+    auto pad = [](size_t b) { return (b + 255) & ~(size_t)255; };
+    const size_t o_types = pad(sizeof(AtomDev) * std::max(n, 1));
+    const size_t o_atom0 = o_types + pad(sizeof(TypeParams) * std::max(nt, 1));
+    const size_t o_block0 = o_atom0 + pad(sizeof(int) * (nt + 1));
+    const size_t total = o_block0 + pad(sizeof(int) * (nt + 1));
+    std::vector<char> block(total, 0);
+    std::memcpy(block.data(), grouped.data(), sizeof(AtomDev) * (size_t)n);
+    if (nt > 0)
+        std::memcpy(block.data() + o_types, fw->types.data(), sizeof(TypeParams) * (size_t)nt);
+    std::memcpy(block.data() + o_atom0, type_atom0.data(), sizeof(int) * (nt + 1));
+    std::memcpy(block.data() + o_block0, type_block0.data(), sizeof(int) * (nt + 1));
     int st = ST_OK;
-    if ((st = pool_alloc(ctx, n > 0 ? n : 1, &fw->d_atoms, &fw->owned)) ||
-        (st = pool_alloc(ctx, nt + 1, &fw->d_type_atom0, &fw->owned)) ||
-        (st = pool_alloc(ctx, nt + 1, &fw->d_type_block0, &fw->owned)) ||
+    char *d_block = nullptr;
+    if ((st = pool_alloc(ctx, total, &d_block, &fw->owned)) ||
         (st = pool_alloc(ctx, nt + 1, &fw->d_type_begin, &fw->owned)) ||
-        (st = pool_alloc(ctx, nt > 0 ? nt : 1, &fw->d_types, &fw->owned)) ||
         (st = pool_alloc(ctx, fw->near_capacity, &fw->d_near, &fw->owned)) ||
         (st = pool_alloc(ctx, plan.nblocks + 1, &fw->d_block_count, &fw->owned)) ||
         (st = pool_alloc(ctx, plan.nblocks + 1, &fw->d_block_off, &fw->owned))) {
         delete fw;
         return st;
     }
+    fw->d_atoms = (AtomDev *)d_block;
+    fw->d_types = (TypeParams *)(d_block + o_types);
+    fw->d_type_atom0 = (int *)(d_block + o_atom0);
+    fw->d_type_block0 = (int *)(d_block + o_block0);
     hipStream_t s = ctx->stream;
-    HIP_TRY(hipMemcpyAsync(fw->d_atoms, grouped.data(), sizeof(AtomDev) * std::max(n, 1),
-                           hipMemcpyHostToDevice, s));
-    HIP_TRY(hipMemcpyAsync(fw->d_type_atom0, type_atom0.data(), sizeof(int) * (nt + 1),
-                           hipMemcpyHostToDevice, s));
-    HIP_TRY(hipMemcpyAsync(fw->d_type_block0, type_block0.data(), sizeof(int) * (nt + 1),
-                           hipMemcpyHostToDevice, s));
-    if (nt > 0)
-        HIP_TRY(hipMemcpyAsync(fw->d_types, fw->types.data(), sizeof(TypeParams) * nt,
-                               hipMemcpyHostToDevice, s));
+    std::unique_ptr<FrameworkDev> owner(fw);
+    HIP_TRY(ctx->transfer->in(d_block, block.data(), total, s));
     plan.atoms = fw->d_atoms;
     plan.type_atom0 = fw->d_type_atom0;
     plan.type_block0 = fw->d_type_block0;
@@ -406,7 +413,7 @@ int framework_upload(Context *ctx, const Particle *atoms, int n, const double t[
     HIP_TRY(launch_near_offsets(plan, fw->d_block_count, fw->d_block_off, fw->d_type_begin, s));
     HIP_TRY(launch_near_write(plan, fw->d_block_off, fw->d_near, s));
     HIP_TRY(hipStreamSynchronize(s));
-    *out = fw;
+    *out = owner.release();
     return ST_OK;
 }
 
@@ -733,16 +740,17 @@ int persistent_wgs(Context *ctx, int math, long long items) {
     return tiles_workgroups(ctx, math, items, ctx->scratch_wgs);
 }
 
-// Launch one job array on the context stream with the context's counter.
-int run_jobs(Context *ctx, int math, JobDev *d_jobs, int njobs, long long total,
-             unsigned long long *d_counter) {
-    hipStream_t s = ctx->stream;
-    HIP_TRY(launch_fill_u64(d_counter, 0ull, 1, s));
-    HIP_TRY(launch_tiles(math, ctx->tuning.ppl, d_jobs, njobs, total, d_counter,
+// Launch one job, whose descriptor is written and whose counter is clear.
+int run_job(Context *ctx, int math, const JobDev *d_job, long long total) {
+    HIP_TRY(launch_tiles(math, ctx->tuning.ppl, d_job, 1, total, ctx->d_counter,
                          persistent_wgs(ctx, math, total), ctx->tuning.cap, ctx->d_scratch,
-                         kRegionRecords, s));
+                         kRegionRecords, ctx->stream));
     return ST_OK;
 }
+
+// Grids of so many bytes reach the host over the link as they are computed (us a
+// call, copied / written by the kernel: 55 KB 63 / 57, 131 KB 62 / 59, 256 KB 75 / 78).
+constexpr size_t kPinnedGrid = 128 << 10;
 
 struct Scoped {
     Context *ctx;
@@ -798,6 +806,7 @@ int widom_prepare(Context *ctx, FrameworkDev *fw, uint64_t n_ins, WidomBuffers *
     ST_TRY(pool_alloc(ctx, n_ins, &wb->sorted, owned));
     ST_TRY(pool_alloc(ctx, n_ins, &wb->e, owned));
     ST_TRY(pool_alloc(ctx, 1, &wb->d_job, owned));
+    ST_TRY(pool_alloc(ctx, 1, &wb->d_bin, owned));
     return ST_OK;
 }
 
@@ -819,17 +828,15 @@ BinJob make_bin_job(const WidomBuffers &wb, uint64_t n_ins, uint64_t seed, uint3
     return j;
 }
 
-int widom_enqueue_binning(Context *ctx, WidomBuffers &wb, uint64_t n_ins, uint64_t seed,
-                          uint32_t stream_id, hipStream_t s) {
-    (void)ctx;
-    wb.job = make_bin_job(wb, n_ins, seed, stream_id);
-    HIP_TRY(hipMemcpyAsync(wb.d_job, &wb.job, sizeof(BinJob), hipMemcpyHostToDevice, s));
-    const int chunk = bin_chunk(n_ins, wb.job.ngroups);
-    HIP_TRY(launch_bin_all(wb.d_job, 1, bin_blocks(n_ins, chunk), chunk, wb.job.ngroups,
-                           wb.job.group, wb.job.group > 1 ? wb.job.ngroups : 0, s));
+int widom_enqueue_binning(const JobDev &job, WidomBuffers &wb, uint64_t n_ins, uint64_t seed,
+                          uint32_t stream_id, unsigned long long *counter, hipStream_t s) {
+    const BinJob bin = make_bin_job(wb, n_ins, seed, stream_id);
+    HIP_TRY(launch_setup(job, wb.d_job, counter, &bin, wb.d_bin, s));
+    const int chunk = bin_chunk(n_ins, bin.ngroups);
+    HIP_TRY(launch_bin_all(wb.d_bin, 1, bin_blocks(n_ins, chunk), chunk, bin.ngroups, bin.group,
+                           bin.group > 1 ? bin.ngroups : 0, true, s));
     return ST_OK;
 }
-
 
 size_t framework_near_capacity(int n_atoms, const double t[9], const int rep[3], double rc2) {
     double inv[9];
@@ -875,14 +882,19 @@ int grid_compute(Context *ctx, FrameworkDev *fw, const int n[3], int precision, 
     g->fw = fw;
     std::memcpy(g->n, n, sizeof(g->n));
     g->precision = precision;
-    g->d_data = ctx->pool.alloc(g->bytes());
-    if (!g->d_data) {
+    // a small grid that only the host wants is written to pinned memory by the kernel
+    char *pinned = nullptr;
+    std::unique_lock<std::mutex> held;
+    if (host_out && !resident && g->bytes() <= kPinnedGrid)
+        held = ctx->transfer->small(&pinned);
+    if (!pinned) g->d_data = ctx->pool.alloc(g->bytes());
+    if (!pinned && !g->d_data) {
         delete g;
         return ST_NOMEM;
     }
     Scoped tmp{ctx, {}};
     const int math = precision == 1 ? MATH_FP64 : MATH_MIXED;
-    JobDev job = make_grid_job(fw, n, precision, g->d_data, ctx->tuning, math);
+    JobDev job = make_grid_job(fw, n, precision, pinned ? pinned : g->d_data, ctx->tuning, math);
     JobDev *d_job = nullptr;
     int st = pool_alloc(ctx, 1, &d_job, &tmp.ptrs);
     if (st) {
@@ -894,11 +906,13 @@ int grid_compute(Context *ctx, FrameworkDev *fw, const int n[3], int precision, 
         delete g;
         return code;
     };
-    if (hipMemcpyAsync(d_job, &job, sizeof(job), hipMemcpyHostToDevice, s) != hipSuccess)
+    if (launch_setup(job, d_job, ctx->d_counter, nullptr, nullptr, s) != hipSuccess) {
+        set_error("grid_compute: launch failed");
         return fail(ST_HIP);
-    if ((st = run_jobs(ctx, job_math(job), d_job, 1, job.n_items, ctx->d_counter)))
-        return fail(st);
-    if (host_out && ctx->transfer->out(host_out, g->d_data, g->bytes(), s) != hipSuccess) {
+    }
+    if ((st = run_job(ctx, job_math(job), d_job, job.n_items))) return fail(st);
+    if (host_out && !pinned &&
+        ctx->transfer->out(host_out, g->d_data, g->bytes(), s) != hipSuccess) {
         set_error("grid_compute: device-to-host copy failed");
         return fail(ST_HIP);
     }
@@ -906,6 +920,7 @@ int grid_compute(Context *ctx, FrameworkDev *fw, const int n[3], int precision, 
         set_error(std::string("grid_compute: ") + hipGetErrorString(hipGetLastError()));
         return fail(ST_HIP);
     }
+    if (pinned) std::memcpy(host_out, pinned, g->bytes());
     if (resident) *resident = g;
     else delete g;
     return ST_OK;
@@ -931,21 +946,16 @@ int widom_run(Context *ctx, FrameworkDev *fw, uint64_t n_ins, double temperature
     JobDev job = make_widom_job(fw, n_ins, seed, wb, ctx->tuning, kMinGridItems,
                                 energies_host ? 0.0 : temperature);
     use_parts(&job, ctx->tuning);
-    JobDev *d_job = nullptr;
-    ST_TRY(pool_alloc(ctx, 1, &d_job, &tmp.ptrs));
     hipStream_t s = ctx->stream;
-    HIP_TRY(hipMemcpyAsync(d_job, &job, sizeof(job), hipMemcpyHostToDevice, s));
-    ST_TRY(widom_enqueue_binning(ctx, wb, n_ins, seed, 0u, s));
-    ST_TRY(run_jobs(ctx, job_math(job), d_job, 1, job.n_items, ctx->d_counter));
+    ST_TRY(widom_enqueue_binning(job, wb, n_ins, seed, 0u, ctx->d_counter, s));
+    ST_TRY(run_job(ctx, job_math(job), wb.d_job, job.n_items));
     HIP_TRY(launch_widom_partials(wb.e, (long long)n_ins, temperature, ctx->d_partials, s));
-    HIP_TRY(launch_widom_final(ctx->d_partials, ctx->d_sums, s));
-    double sums[2];
-    HIP_TRY(hipMemcpyAsync(sums, ctx->d_sums, sizeof(sums), hipMemcpyDeviceToHost, s));
+    HIP_TRY(launch_widom_final(ctx->d_partials, ctx->h_sums, s));
     if (energies_host)
         HIP_TRY(ctx->transfer->out(energies_host, wb.e, sizeof(double) * n_ins, s));
     HIP_TRY(hipStreamSynchronize(s));
-    out->sum_b = sums[0];
-    out->sum_eb = sums[1];
+    out->sum_b = ctx->h_sums[0];
+    out->sum_eb = ctx->h_sums[1];
     out->n = n_ins;
     return ST_OK;
 }
@@ -965,8 +975,8 @@ int count_incut_grid(Context *ctx, FrameworkDev *fw, const int n[3], unsigned lo
     ST_TRY(pool_alloc(ctx, 1, &d_job, &tmp.ptrs));
     JobDev job = make_grid_job(fw, n, 0, d_cnt, ctx->tuning, MATH_COUNT);
     hipStream_t s = ctx->stream;
-    HIP_TRY(hipMemcpyAsync(d_job, &job, sizeof(job), hipMemcpyHostToDevice, s));
-    ST_TRY(run_jobs(ctx, MATH_COUNT, d_job, 1, job.n_items, ctx->d_counter));
+    HIP_TRY(launch_setup(job, d_job, ctx->d_counter, nullptr, nullptr, s));
+    ST_TRY(run_job(ctx, MATH_COUNT, d_job, job.n_items));
     HIP_TRY(launch_fill_u64(d_sum, 0ull, 1, s));
     HIP_TRY(launch_sum_u32(d_cnt, p, d_sum, s));
     HIP_TRY(hipMemcpyAsync(out, d_sum, sizeof(*out), hipMemcpyDeviceToHost, s));
@@ -1002,8 +1012,8 @@ int accessibility_grid(Context *ctx, const Particle *atoms, int n_atoms, const d
     ST_TRY(pool_alloc(ctx, 1, &d_job, &tmp.ptrs));
     JobDev job = make_grid_job(fw, n, 1, d_out, ctx->tuning, MATH_OVERLAP);
     hipStream_t s = ctx->stream;
-    HIP_TRY(hipMemcpyAsync(d_job, &job, sizeof(job), hipMemcpyHostToDevice, s));
-    ST_TRY(run_jobs(ctx, MATH_OVERLAP, d_job, 1, job.n_items, ctx->d_counter));
+    HIP_TRY(launch_setup(job, d_job, ctx->d_counter, nullptr, nullptr, s));
+    ST_TRY(run_job(ctx, MATH_OVERLAP, d_job, job.n_items));
     HIP_TRY(ctx->transfer->out(host_out, d_out, sizeof(double) * p, s));
     HIP_TRY(hipStreamSynchronize(s));
     return ST_OK;
@@ -1017,14 +1027,11 @@ int count_incut_widom(Context *ctx, FrameworkDev *fw, uint64_t n_ins, uint64_t s
     WidomBuffers wb;
     ST_TRY(widom_prepare(ctx, fw, n_ins, &wb, &tmp.ptrs));
     unsigned long long *d_sum = nullptr;
-    JobDev *d_job = nullptr;
     ST_TRY(pool_alloc(ctx, 1, &d_sum, &tmp.ptrs));
-    ST_TRY(pool_alloc(ctx, 1, &d_job, &tmp.ptrs));
     JobDev job = make_widom_job(fw, n_ins, seed, wb, ctx->tuning, kMinGridItems);
     hipStream_t s = ctx->stream;
-    HIP_TRY(hipMemcpyAsync(d_job, &job, sizeof(job), hipMemcpyHostToDevice, s));
-    ST_TRY(widom_enqueue_binning(ctx, wb, n_ins, seed, 0u, s));
-    ST_TRY(run_jobs(ctx, MATH_COUNT, d_job, 1, job.n_items, ctx->d_counter));
+    ST_TRY(widom_enqueue_binning(job, wb, n_ins, seed, 0u, ctx->d_counter, s));
+    ST_TRY(run_job(ctx, MATH_COUNT, wb.d_job, job.n_items));
     HIP_TRY(launch_fill_u64(d_sum, 0ull, 1, s));
     HIP_TRY(launch_sum_f64_counts(wb.e, (long long)n_ins, d_sum, s));
     HIP_TRY(hipMemcpyAsync(out, d_sum, sizeof(*out), hipMemcpyDeviceToHost, s));
@@ -1070,7 +1077,7 @@ double job_cost_per_item(const FrameworkDev *fw, const JobDev &j, const Tuning &
 int Batch::record(hipStream_t s) {
     // every Widom task's binning in one launch per phase
     HIP_TRY(launch_bin_all(d_bin_jobs, (int)bin_jobs.size(), bin_blocks_total, bin_chunk_len,
-                           bin_max_keys, bin_max_group, bin_groups_total, s));
+                           bin_max_keys, bin_max_group, bin_groups_total, false, s));
     // jobs are grouped by variant, each group one launch with its own counter
     const bool ev_on = timing && !use_graph;
     timed_launches = 0;
@@ -1189,21 +1196,22 @@ int batch_create(Context *ctx, const Task *tasks, int n, bool use_graph, Batch *
     int st = ST_OK;
     if ((st = pool_alloc(ctx, std::max<size_t>(b->jobs.size(), 1), &b->d_jobs, &b->owned)) ||
         (st = pool_alloc(ctx, (size_t)std::max(n, 1) * kReduceBlocks, &b->d_partials, &b->owned)) ||
-        (st = pool_alloc(ctx, (size_t)std::max(n, 1) * 2, &b->d_sums, &b->owned)) ||
         (st = pool_alloc(ctx, kBatchLaunches, &b->d_counter, &b->owned)) ||
         (st = pool_alloc(ctx, std::max<size_t>(b->bin_jobs.size(), 1), &b->d_bin_jobs,
                          &b->owned)) ||
         (st = pool_alloc(ctx, (size_t)std::max(n, 1), &b->d_reduce, &b->owned)))
         return fail(st);
-    for (int t = 0; t < n; t++)
-        if (b->tasks[t].n_ins > 0)
-            b->reduce.push_back({b->wbufs[t].e, (long long)b->tasks[t].n_ins,
-                                 b->tasks[t].temperature, b->d_partials + (size_t)t * kReduceBlocks,
-                                 b->d_sums + 2 * (size_t)t});
     if (hipHostMalloc((void **)&b->h_sums, sizeof(double) * 2 * std::max(n, 1)) != hipSuccess) {
         set_error("batch_create: pinned host allocation failed");
         return fail(ST_NOMEM);
     }
+    std::memset(b->h_sums, 0, sizeof(double) * 2 * std::max(n, 1));
+    b->sums.assign(2 * (size_t)std::max(n, 1), 0.0);
+    for (int t = 0; t < n; t++)
+        if (b->tasks[t].n_ins > 0)
+            b->reduce.push_back({b->wbufs[t].e, (long long)b->tasks[t].n_ins,
+                                 b->tasks[t].temperature, b->d_partials + (size_t)t * kReduceBlocks,
+                                 b->h_sums + 2 * (size_t)t});
     if ((!b->jobs.empty() &&
          hipMemcpyAsync(b->d_jobs, b->jobs.data(), sizeof(JobDev) * b->jobs.size(),
                         hipMemcpyHostToDevice, ctx->stream) != hipSuccess) ||
@@ -1255,11 +1263,8 @@ int batch_wait(Batch *b) {
         return ST_ARG;
     }
     Context *ctx = b->ctx;
-    const size_t n = b->tasks.size();
-    if (n > 0)
-        HIP_TRY(hipMemcpyAsync(b->h_sums, b->d_sums, sizeof(double) * 2 * n,
-                               hipMemcpyDeviceToHost, ctx->stream));
     HIP_TRY(hipStreamSynchronize(ctx->stream));
+    std::copy_n(b->h_sums, b->sums.size(), b->sums.begin());
     return ST_OK;
 }
 
@@ -1300,8 +1305,8 @@ int batch_result(Batch *b, int i, WidomResult *out, GridDev **grid) {
         return ST_ARG;
     }
     if (out) {
-        out->sum_b = b->h_sums[2 * i];
-        out->sum_eb = b->h_sums[2 * i + 1];
+        out->sum_b = b->sums[2 * i];
+        out->sum_eb = b->sums[2 * i + 1];
         out->n = b->tasks[i].n_ins;
     }
     if (grid) *grid = b->grids[i];

@@ -96,7 +96,7 @@ class Context {
     DevicePool pool{this};
     unsigned long long *d_counter = nullptr;  // work counter of plain launches
     double2 *d_partials = nullptr;
-    double *d_sums = nullptr;
+    double *h_sums = nullptr;                 // pinned; the reductions write it
     uint32_t *d_scratch = nullptr;  // region sub-lists, scratch_wgs * kRegionRecords indices
     int scratch_wgs = 0;
     void *h_stage = nullptr;       // pinned host staging of pocket labelling results
@@ -193,8 +193,8 @@ struct WidomBuffers {
     int nbins[3] = {1, 1, 1};
     uint32_t *count = nullptr, *start = nullptr, *cursor = nullptr, *sorted = nullptr;
     double *e = nullptr;
-    BinJob job{};               // host copy of the binning job (source of the upload)
-    BinJob *d_job = nullptr;    // device copy
+    JobDev *d_job = nullptr;    // descriptors, written by launch_setup
+    BinJob *d_bin = nullptr;
 };
 BinJob make_bin_job(const WidomBuffers &wb, uint64_t n_ins, uint64_t seed, uint32_t stream_id);
 void choose_widom_bins(const FrameworkDev *fw, uint64_t n_ins, const Tuning &tu, int nb[3]);
@@ -222,9 +222,10 @@ void use_parts(JobDev *j, const Tuning &tu);
 // Allocates the Widom buffers of a job (owned pointers appended to `owned`).
 int widom_prepare(Context *ctx, FrameworkDev *fw, uint64_t n_ins, WidomBuffers *wb,
                   std::vector<void *> *owned);
-// Enqueues point generation, binning and the bin-sorted index list on s.
-int widom_enqueue_binning(Context *ctx, WidomBuffers &wb, uint64_t n_ins, uint64_t seed,
-                          uint32_t stream_id, hipStream_t s);
+// Enqueues on s: the job's descriptors, *counter cleared, point generation,
+// binning and the bin-sorted index list.
+int widom_enqueue_binning(const JobDev &job, WidomBuffers &wb, uint64_t n_ins, uint64_t seed,
+                          uint32_t stream_id, unsigned long long *counter, hipStream_t s);
 // Upper bound on the near-list records framework_upload allocates.
 size_t framework_near_capacity(int n_atoms, const double t[9], const int rep[3], double rc2);
 
@@ -274,11 +275,11 @@ class Batch {
     long long total_items = 0;
     int math = MATH_MIXED;
     double2 *d_partials = nullptr;     // kReduceBlocks per task
-    double *d_sums = nullptr;          // 2 per task
     std::vector<WidomReduce> reduce;   // reduction of every task with insertions
     WidomReduce *d_reduce = nullptr;
     unsigned long long *d_counter = nullptr;
-    double *h_sums = nullptr;          // pinned
+    double *h_sums = nullptr;          // pinned, 2 per task; the reductions write it
+    std::vector<double> sums;          // of the last run waited for
     hipGraph_t graph = nullptr;
     hipGraphExec_t exec = nullptr;
     bool use_graph = true;

@@ -342,7 +342,8 @@ bool Server::admit_one(Req *r, FwEntry *hit) {
                                           kMinGridItems, s.temperature);
             use_parts(&r->widom_job, ctx_->tuning);
             r->items_total += r->widom_job.n_items;
-            st = widom_enqueue_binning(ctx_, r->wb, s.n_ins, s.seed, 0u, ctx_->stream);
+            st = widom_enqueue_binning(r->widom_job, r->wb, s.n_ins, s.seed, 0u,
+                                       ctx_->d_counter, ctx_->stream);
         }
         if (st == ST_OK && hipHostMalloc((void **)&r->h_sums, 2 * sizeof(double)) != hipSuccess)
             st = ST_NOMEM;
@@ -448,20 +449,14 @@ void Server::run() {
             } else if (r->items_done == r->items_total) {
                 if (r->spec.n_ins && !r->reducing) {
                     hipStream_t s = launches_[0]->stream;
-                    double2 *part = nullptr;
-                    double *sums = nullptr;
-                    part = (double2 *)ctx_->pool.alloc(sizeof(double2) * kReduceBlocks);
-                    sums = (double *)ctx_->pool.alloc(2 * sizeof(double));
+                    double2 *part =
+                        (double2 *)ctx_->pool.alloc(sizeof(double2) * kReduceBlocks);
                     if (part) r->owned.push_back(part);
-                    if (sums) r->owned.push_back(sums);
                     hipError_t e = hipErrorOutOfMemory;
-                    if (part && sums) {
+                    if (part) {
                         e = launch_widom_partials(r->wb.e, (long long)r->spec.n_ins,
                                                   r->spec.temperature, part, s);
-                        if (e == hipSuccess) e = launch_widom_final(part, sums, s);
-                        if (e == hipSuccess)
-                            e = hipMemcpyAsync(r->h_sums, sums, 2 * sizeof(double),
-                                               hipMemcpyDeviceToHost, s);
+                        if (e == hipSuccess) e = launch_widom_final(part, r->h_sums, s);
                         if (e == hipSuccess) e = hipEventRecord(r->reduced, s);
                     }
                     if (e != hipSuccess) {

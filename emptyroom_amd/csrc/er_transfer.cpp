@@ -13,7 +13,6 @@ namespace er {
 
 namespace {
 
-constexpr size_t kSmall = 1 << 20;    // bytes up to which one small buffer is used
 constexpr size_t kSlot = 2 << 20;     // bytes of a slot (37 us of the link)
 constexpr int kSlots = 8;
 constexpr size_t kPiece = 256 << 10;  // bytes copied at a time
@@ -110,6 +109,11 @@ Transfer::~Transfer() {
         (void)hipHostFree(slot_[i]);
     }
     if (small_) (void)hipHostFree(small_);
+    if (in_done_) {
+        (void)hipEventSynchronize(in_done_);
+        (void)hipEventDestroy(in_done_);
+    }
+    if (in_) (void)hipHostFree(in_);
 }
 
 std::shared_ptr<Transfer> Transfer::of_device(int device) {
@@ -237,13 +241,35 @@ hipError_t Transfer::out(void *host, const void *dev, size_t bytes, hipStream_t 
 }
 
 hipError_t Transfer::in(void *dev, const void *host, size_t bytes, hipStream_t s) {
-    std::unique_lock<std::mutex> lk(busy_, std::defer_lock);
-    if (bytes <= kSmall && lk.try_lock() && ensure(0, false)) {
-        std::memcpy(small_, host, bytes);
-        const hipError_t e = hipMemcpyAsync(dev, small_, bytes, hipMemcpyHostToDevice, s);
-        return e == hipSuccess ? hipStreamSynchronize(s) : e;  // the buffer is free again
+    std::unique_lock<std::mutex> lk(in_mu_);
+    if (bytes <= kSmall && !in_) {
+        if (hipEventCreateWithFlags(&in_done_, hipEventDisableTiming) != hipSuccess ||
+            hipHostMalloc((void **)&in_, kSmall) != hipSuccess) {
+            (void)hipGetLastError();
+            if (in_done_) (void)hipEventDestroy(in_done_);
+            in_done_ = nullptr;
+            in_ = nullptr;
+        }
     }
-    return hipMemcpyAsync(dev, host, bytes, hipMemcpyHostToDevice, s);
+    if (bytes > kSmall || !in_) {
+        lk.unlock();
+        return hipMemcpyAsync(dev, host, bytes, hipMemcpyHostToDevice, s);
+    }
+    hipError_t e = hipEventSynchronize(in_done_);  // the copy before this one
+    if (e != hipSuccess) return e;
+    std::memcpy(in_, host, bytes);
+    e = hipMemcpyAsync(dev, in_, bytes, hipMemcpyHostToDevice, s);
+    if (e == hipSuccess) e = hipEventRecord(in_done_, s);
+    if (e != hipSuccess) (void)hipStreamSynchronize(s);
+    return e;
+}
+
+std::unique_lock<std::mutex> Transfer::small(char **p) {
+    *p = nullptr;
+    std::unique_lock<std::mutex> lk(busy_, std::defer_lock);
+    if (lk.try_lock() && ensure(0, false)) *p = small_;
+    else if (lk.owns_lock()) lk.unlock();
+    return lk;
 }
 
 }  // namespace er

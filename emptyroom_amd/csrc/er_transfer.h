@@ -10,7 +10,7 @@
 // 156, 16 MiB 970 / 630, 64 MiB 6640 / 2240, 256 MiB 25700 / 7260.  Uploads above
 // 1 MiB reach 30 GB/s by the runtime's own path, which they keep.
 //
-// The contexts of a device share one Transfer (the pinned memory, 17 MiB at
+// The contexts of a device share one Transfer (the pinned memory, 18 MiB at
 // most, and the threads are made by the first copy that uses them and given back
 // with the last context).  One copy at a time uses it; a copy that finds it in
 // use takes the runtime's path.
@@ -37,6 +37,10 @@ class Transfer {
     hipError_t out(void *host, const void *dev, size_t bytes, hipStream_t s);
     // host -> dev on stream s; host memory must stay until s has passed the copy.
     hipError_t in(void *dev, const void *host, size_t bytes, hipStream_t s);
+    // The small buffer (kSmall bytes, device-accessible) for as long as the lock
+    // is held; *p = nullptr if it is in use or cannot be had.
+    std::unique_lock<std::mutex> small(char **p);
+    static constexpr size_t kSmall = 1 << 20;
 
   private:
     struct Job;
@@ -44,6 +48,9 @@ class Transfer {
     void start(Job *job);
     void finish();
     void work();
+    std::mutex in_mu_;              // guards the upload buffer and its last copy's event
+    char *in_ = nullptr;
+    hipEvent_t in_done_ = nullptr;
     std::mutex busy_;               // held by the copy that uses what follows
     char *small_ = nullptr;
     std::vector<char *> slot_;      // pinned, one size
