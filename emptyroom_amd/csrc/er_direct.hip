@@ -257,7 +257,7 @@ int direct_widom(Context *ctx, const Particle *atoms, int n_atoms, const double 
                        dim3(kDirectWG), 0, s, J, seed, (long long)n_ins, e);
     HIP_TRY(hipGetLastError());
     HIP_TRY(launch_widom_partials(e, (long long)n_ins, temperature, ctx->d_partials, s));
-    HIP_TRY(launch_widom_final(ctx->d_partials, ctx->h_sums, s));
+    HIP_TRY(launch_widom_final(ctx->d_partials, reduce_blocks((long long)n_ins), ctx->h_sums, s));
     if (energies_host)
         HIP_TRY(hipMemcpyAsync(energies_host, e, sizeof(double) * n_ins, hipMemcpyDeviceToHost, s));
     HIP_TRY(hipStreamSynchronize(s));

@@ -101,15 +101,20 @@ __host__ __device__ inline int mixed_far_shell_cap(int cap) {
 int tiles_occupancy(int math, int ppl, int cap);
 
 // --- reductions ---------------------------------------------------------------
-// Boltzmann sums of one job: partial[g] for g < nblk over fixed index ranges.
-constexpr int kReduceBlocks = 240;
+// Boltzmann sums of one job: partial[g] for g < reduce_blocks(n) over fixed index
+// ranges.
+constexpr int kReduceBlocks = 1024;  // partials of a run, at most
+// Blocks a run of n energies is summed in: eight energies a thread until the device
+// is full.
+__host__ __device__ inline int reduce_blocks(long long n) {
+    const long long b = (n + 2047) / 2048;
+    return b < 1 ? 1 : b > kReduceBlocks ? kReduceBlocks : (int)b;
+}
 hipError_t launch_widom_partials(const double *e, long long n, double temperature,
                                  double2 *partials, hipStream_t s);
 // Fixed-order sum of nblk partials (out[0] = sum_b, out[1] = sum_Eb).
-hipError_t launch_widom_final_n(const double2 *partials, int nblk, double *out, hipStream_t s);
-// out[0] = sum_b, out[1] = sum_Eb: fixed-order sum of the kReduceBlocks partials.
-hipError_t launch_widom_final(const double2 *partials, double *out, hipStream_t s);
-// One Widom run's reduction: energies e[0, n), kReduceBlocks partials, two sums.
+hipError_t launch_widom_final(const double2 *partials, int nblk, double *out, hipStream_t s);
+// One Widom run's reduction: energies e[0, n), reduce_blocks(n) partials, two sums.
 struct WidomReduce {
     const double *e;
     long long n;

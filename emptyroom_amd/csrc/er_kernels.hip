@@ -209,7 +209,7 @@ __device__ __forceinline__ uint32_t widom_bin(const double f[3], const int nb[3]
 // The groups keep the histogram at a few KiB and the scattered runs long:
 // 1.73e7 insertions of 36036 bins took 711 us to count and 1364 us to scatter
 // with one global atomic per insertion; now 64 us to count (the points), 67 us
-// to scatter and 80 us to sort the groups.  The scatter is bound by its stores:
+// to scatter and 67 us to sort the groups.  The scatter is bound by its stores:
 // written straight from the lanes they took 241 us.  16 jobs of 1e6 insertions
 // and ~2080 bins each (one step): 48 + 159 us before, 51 + 69 us now.
 __device__ __forceinline__ int bin_job_of(const BinJob *__restrict__ jobs, int njobs,
@@ -354,10 +354,14 @@ __global__ __launch_bounds__(kBinWG) void k_bin_scatter(const BinJob *__restrict
 }
 
 // Second step of grouped jobs: block = one group, whose pairs lie between the
-// cursors its neighbour and itself ended at.
-__global__ __launch_bounds__(kWG) void k_bin_fine(const BinJob *__restrict__ jobs, int njobs) {
+// cursors its neighbour and itself ended at.  A thread keeps its first kFinePer pairs
+// (all of them in a group of up to 20480, as 1024 groups of 2e7 insertions have) for
+// the second pass, which then reads nothing: 1.73e7 insertions took 80 us with both
+// passes reading, 67 us now (138 MB read, 69 MB written).
+constexpr int kFinePer = 20;
+__global__ __launch_bounds__(kBinWG) void k_bin_fine(const BinJob *__restrict__ jobs, int njobs) {
     extern __shared__ uint32_t s_cnt[];
-    __shared__ uint32_t s_part[kWG];
+    __shared__ uint32_t s_part[kBinWG / 64];
     int lo = 0, hi = njobs - 1;
     while (lo < hi) {
         const int mid = (lo + hi + 1) >> 1;
@@ -371,24 +375,35 @@ __global__ __launch_bounds__(kWG) void k_bin_fine(const BinJob *__restrict__ job
     const int nbt = J.nb[0] * J.nb[1] * J.nb[2], b0 = g * J.group;
     const int nb = b0 + J.group < nbt ? J.group : nbt - b0;
     const uint32_t e0 = g > 0 ? J.cursor[g - 1] : 0u, e1 = J.cursor[g];
-    for (int b = tid; b < nb; b += kWG) s_cnt[b] = 0u;
+    uint2 v[kFinePer];
+#pragma unroll
+    for (int q = 0; q < kFinePer; ++q) {
+        const uint32_t e = e0 + (uint32_t)(q * kBinWG + tid);
+        v[q] = J.tmp[e < e1 ? e : 0u];
+    }
+    for (int b = tid; b < nb; b += kBinWG) s_cnt[b] = 0u;
     __syncthreads();
-    for (uint32_t e = e0 + tid; e < e1; e += kWG) atomicAdd(&s_cnt[J.tmp[e].x], 1u);
+#pragma unroll
+    for (int q = 0; q < kFinePer; ++q)
+        if (e0 + (uint32_t)(q * kBinWG + tid) < e1) atomicAdd(&s_cnt[v[q].x], 1u);
+    for (uint32_t e = e0 + kFinePer * kBinWG + tid; e < e1; e += kBinWG)
+        atomicAdd(&s_cnt[J.tmp[e].x], 1u);
     __syncthreads();
     // exclusive scan of the group's bins: per consecutive counts per thread
-    const int per = (nb + kWG - 1) / kWG;
+    const int per = (nb + kBinWG - 1) / kBinWG;
     const int p0 = tid * per < nb ? tid * per : nb, p1 = p0 + per < nb ? p0 + per : nb;
     uint32_t sum = 0;
     for (int b = p0; b < p1; ++b) sum += s_cnt[b];
-    s_part[tid] = sum;
-    __syncthreads();
-    for (int d = 1; d < kWG; d <<= 1) {
-        const uint32_t add = tid >= d ? s_part[tid - d] : 0u;
-        __syncthreads();
-        s_part[tid] += add;
-        __syncthreads();
+    uint32_t inc = sum;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+        const uint32_t u = __shfl_up(inc, d, 64);
+        if ((tid & 63) >= d) inc += u;
     }
-    uint32_t run = e0 + s_part[tid] - sum;
+    if ((tid & 63) == 63) s_part[tid >> 6] = inc;
+    __syncthreads();
+    uint32_t run = e0 + inc - sum;
+    for (int w = 0; w < (tid >> 6); ++w) run += s_part[w];
     for (int b = p0; b < p1; ++b) {
         const uint32_t c = s_cnt[b];
         s_cnt[b] = run;
@@ -397,9 +412,13 @@ __global__ __launch_bounds__(kWG) void k_bin_fine(const BinJob *__restrict__ job
     }
     if (g == J.ngroups - 1 && tid == 0) J.start[nbt] = (uint32_t)J.n;
     __syncthreads();
-    for (uint32_t e = e0 + tid; e < e1; e += kWG) {
-        const uint2 v = J.tmp[e];
-        J.sorted[atomicAdd(&s_cnt[v.x], 1u)] = v.y;
+#pragma unroll
+    for (int q = 0; q < kFinePer; ++q)
+        if (e0 + (uint32_t)(q * kBinWG + tid) < e1)
+            J.sorted[atomicAdd(&s_cnt[v[q].x], 1u)] = v[q].y;
+    for (uint32_t e = e0 + kFinePer * kBinWG + tid; e < e1; e += kBinWG) {
+        const uint2 u = J.tmp[e];
+        J.sorted[atomicAdd(&s_cnt[u.x], 1u)] = u.y;
     }
 }
 
@@ -2141,7 +2160,9 @@ __device__ __forceinline__ double wave_sum(double v) {
 
 // Block g of G sums exp(-E/T) (src/doHenry.h:107) and E exp(-E/T) over the
 // contiguous insertion range [g n / G, (g+1) n / G) in a fixed order (thread
-// stride, then a fixed shuffle tree and the four wave sums in order).
+// stride, then a fixed shuffle tree and the four wave sums in order).  About 70
+// VALU instructions a value, most of them the division and the exponential: as 240
+// blocks, one wave per SIMD, 1.73e7 energies took 110 us; 39 us now (3.5 TB/s).
 __device__ __forceinline__ void widom_partial_block(const double *e, long long n,
                                                    double temperature, long long g, long long G,
                                                    double2 *partials, double *s_b,
@@ -2206,14 +2227,15 @@ __global__ __launch_bounds__(kWG) void k_widom_final(const double2 *partials, in
 __global__ __launch_bounds__(kWG) void k_widom_partials_many(const WidomReduce *runs) {
     __shared__ double s_b[kWG / 64], s_eb[kWG / 64];
     const WidomReduce &R = runs[blockIdx.x / kReduceBlocks];
-    widom_partial_block(R.e, R.n, R.temperature, blockIdx.x % kReduceBlocks, kReduceBlocks,
-                        R.partials, s_b, s_eb);
+    const int g = blockIdx.x % kReduceBlocks, G = reduce_blocks(R.n);
+    if (g >= G) return;
+    widom_partial_block(R.e, R.n, R.temperature, g, G, R.partials, s_b, s_eb);
 }
 
 __global__ __launch_bounds__(kWG) void k_widom_final_many(const WidomReduce *runs) {
     __shared__ double s_b[kWG / 64], s_eb[kWG / 64];
     const WidomReduce &R = runs[blockIdx.x];
-    widom_final_block(R.partials, kReduceBlocks, R.out, s_b, s_eb);
+    widom_final_block(R.partials, reduce_blocks(R.n), R.out, s_b, s_eb);
 }
 
 __global__ __launch_bounds__(kWG) void k_sum_u32(const uint32_t *v, long long n,
@@ -2356,7 +2378,7 @@ hipError_t launch_bin_all(const BinJob *jobs, int njobs, long long total_blocks,
     ER_SCATTER(1) ER_SCATTER(2) ER_SCATTER(4) ER_SCATTER(8) ER_SCATTER(16)
 #undef ER_SCATTER
     if (total_groups > 0)
-        hipLaunchKernelGGL(k_bin_fine, dim3((unsigned)total_groups), dim3(kWG),
+        hipLaunchKernelGGL(k_bin_fine, dim3((unsigned)total_groups), dim3(kBinWG),
                            sizeof(uint32_t) * (size_t)max_group, s, jobs, njobs);
     return hipGetLastError();
 }
@@ -2422,7 +2444,7 @@ int tiles_occupancy(int math, int ppl, int cap) {
 
 hipError_t launch_widom_partials(const double *e, long long n, double temperature,
                                  double2 *partials, hipStream_t s) {
-    hipLaunchKernelGGL(k_widom_partials, dim3(kReduceBlocks), dim3(kWG), 0, s, e, n, temperature,
+    hipLaunchKernelGGL(k_widom_partials, dim3(reduce_blocks(n)), dim3(kWG), 0, s, e, n, temperature,
                        partials);
     return hipGetLastError();
 }
@@ -2435,12 +2457,7 @@ hipError_t launch_widom_reduce_many(const WidomReduce *runs, int nruns, hipStrea
     return hipGetLastError();
 }
 
-hipError_t launch_widom_final(const double2 *partials, double *out, hipStream_t s) {
-    hipLaunchKernelGGL(k_widom_final, dim3(1), dim3(kWG), 0, s, partials, kReduceBlocks, out);
-    return hipGetLastError();
-}
-
-hipError_t launch_widom_final_n(const double2 *partials, int nblk, double *out, hipStream_t s) {
+hipError_t launch_widom_final(const double2 *partials, int nblk, double *out, hipStream_t s) {
     hipLaunchKernelGGL(k_widom_final, dim3(1), dim3(kWG), 0, s, partials, nblk, out);
     return hipGetLastError();
 }

@@ -379,7 +379,7 @@ int widom_grid_run(Context *ctx, GridDev *g, uint64_t n_ins, double temperature,
     float4 *faces = fb ? (float4 *)sc.get<char>(fb) : nullptr;
     HIP_TRY(launch_widom_grid((const float *)g->d_data, faces, g->n, seed, 1u, n_ins, temperature,
                               e, partials, s));
-    HIP_TRY(launch_widom_final_n(partials, kTriBlocks, ctx->h_sums, s));
+    HIP_TRY(launch_widom_final(partials, kTriBlocks, ctx->h_sums, s));
     if (energies_host)
         HIP_TRY(ctx->transfer->out(energies_host, e, sizeof(double) * n_ins, s));
     HIP_TRY(hipStreamSynchronize(s));

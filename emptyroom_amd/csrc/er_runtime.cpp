@@ -950,7 +950,7 @@ int widom_run(Context *ctx, FrameworkDev *fw, uint64_t n_ins, double temperature
     ST_TRY(widom_enqueue_binning(job, wb, n_ins, seed, 0u, ctx->d_counter, s));
     ST_TRY(run_job(ctx, job_math(job), wb.d_job, job.n_items));
     HIP_TRY(launch_widom_partials(wb.e, (long long)n_ins, temperature, ctx->d_partials, s));
-    HIP_TRY(launch_widom_final(ctx->d_partials, ctx->h_sums, s));
+    HIP_TRY(launch_widom_final(ctx->d_partials, reduce_blocks((long long)n_ins), ctx->h_sums, s));
     if (energies_host)
         HIP_TRY(ctx->transfer->out(energies_host, wb.e, sizeof(double) * n_ins, s));
     HIP_TRY(hipStreamSynchronize(s));
