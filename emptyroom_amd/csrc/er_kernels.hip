@@ -464,8 +464,10 @@ enum : int { CAT_NONE = 0, CAT_FAR = 1, CAT_SHELL = 2, CAT_NEAR = 3 };
 
 // Ints per list segment: type, far begin, shell begin, near begin.  The types of
 // a pass are consecutive, so a segment ends where the next begins; the entry
-// after the last holds the pass's counts.
+// after the last holds the pass's counts, and in place of the type whether a near
+// pair may need the clamp of r^2.
 constexpr int kSegInts = 4;
+constexpr int kClampBit = 1 << 16;
 
 // Pairs per point summed in FP32 (far and shell pairs of one type) before the
 // sum is scaled and added to the FP64 energy.
@@ -585,8 +587,9 @@ __device__ int fill_list(const JobDev *__restrict__ J, const double4 *__restrict
     const double in2 = (rc + tl.R + kMargin) * (rc + tl.R + kMargin);
     const double far_r = rc - tl.R - kMargin;
     const double far2 = far_r > 0.0 ? far_r * far_r : -1.0;
-    // FP64 grids: near (clamp possible) only if some point may lie within
-    // kMargin of the atom, d <= R + kMargin
+    // the clamp of r^2 (at most 1e-24 A^2) can matter only if some point may lie
+    // within kMargin of the atom, d <= R + kMargin.  FP64 grids: those are the near
+    // records; the others: a pass that keeps none of them is evaluated without it
     const double clamp2 = (tl.R + kMargin) * (tl.R + kMargin);
     // The cell's points lie in a parallelepiped around the centre:
     // J->cell_box[d] times cell vector t_d on either side (a bin's box; a
@@ -605,7 +608,7 @@ __device__ int fill_list(const JobDev *__restrict__ J, const double4 *__restrict
     // a pass takes at most kMaxSeg types
     const int last_t = first_t + kMaxSeg < ntypes ? first_t + kMaxSeg : ntypes;
     const int end = uniform(tbeg[last_t]);
-    int nf = 0, ns = 0, nn = 0, nseg = 1;
+    int nf = 0, ns = 0, nn = 0, nseg = 1, clamp = 0;
     if (tid == 0) {
         seg[0] = first_t;
         seg[1] = seg[2] = seg[3] = 0;
@@ -636,16 +639,19 @@ __device__ int fill_list(const JobDev *__restrict__ J, const double4 *__restrict
         const uint64_t bf = __ballot(cat == CAT_FAR);
         const uint64_t bs = __ballot(cat == CAT_SHELL);
         const uint64_t bn = __ballot(cat == CAT_NEAR);
+        const bool at = MATH == MATH_MIXED && __ballot(cat == CAT_NEAR && A.w <= clamp2);
         if (lane == 0) {
             s_cnt[3 * wave] = __popcll(bf);
             s_cnt[3 * wave + 1] = __popcll(bs);
-            s_cnt[3 * wave + 2] = __popcll(bn);
+            s_cnt[3 * wave + 2] = __popcll(bn) | (at ? kClampBit : 0);
         }
         __syncthreads();
         int of = nf, os = ns, on = nn, tf = 0, ts = 0, tn = 0;
 #pragma unroll
         for (int w = 0; w < WG / 64; ++w) {
-            const int cf = s_cnt[3 * w], cs = s_cnt[3 * w + 1], cn = s_cnt[3 * w + 2];
+            const int cf = s_cnt[3 * w], cs = s_cnt[3 * w + 1];
+            const int cn = s_cnt[3 * w + 2] & ~kClampBit;
+            clamp |= s_cnt[3 * w + 2] & kClampBit;
             if (w < wave) {
                 of += cf;
                 os += cs;
@@ -728,6 +734,7 @@ __device__ int fill_list(const JobDev *__restrict__ J, const double4 *__restrict
     }
     if (tid == 0) {
         int *g = seg + kSegInts * nseg;
+        g[0] = clamp;
         g[1] = nf;
         g[2] = ns;
         g[3] = nn;
@@ -842,6 +849,7 @@ __device__ __forceinline__ void eval_list(const JobDev *__restrict__ J,
                                           double4 wsph = make_double4(0.0, 0.0, 0.0, 0.0),
                                           uint16_t *__restrict__ wl = nullptr, int phase = 0) {
     const bool do_fs = phase != 1, do_near = phase != 2;
+    const bool clamp = MATH == MATH_MIXED && do_near && uniform(seg[kSegInts * nseg]) != 0;
     const double rc2 = J->rc2, min_r2 = J->min_r2;
     const int capA = near_region_start<MATH>(cap);
     const double4 *__restrict__ Ls = L + capA - 1;  // shell k at Ls[-k]
@@ -971,14 +979,16 @@ __device__ __forceinline__ void eval_list(const JobDev *__restrict__ J,
             // strict cutoff test (src/computegridsheet.h:79) passes for every
             // pair and is skipped.
             const bool all_in = P.rclose + 2.0 * R + 3.0 * kMargin < J->rc;
-            auto near_pairs = [&](auto test) {
+            // Most passes hold no record that a point may sit on (kClampBit): without
+            // the clamp two points take 27 instead of 30 VALU instructions a record.
+            auto near_pairs = [&](auto clamp, auto test) {
                 for (int k = nb; k < ne; ++k) {
                     double r2[PPL];
                     pair_r2<PPL, XL>(Ln[k], mx, my, mz, p2, r2);
 #pragma unroll
                     for (int q = 0; q < PPL; ++q) {
                         // src/computegridsheet.h:77 (r^2 is never NaN, so fmax is the clamp)
-                        const double rr = fmax(r2[q], min_r2);
+                        const double rr = decltype(clamp)::value ? fmax(r2[q], min_r2) : r2[q];
                         double y = (double)__builtin_amdgcn_rcpf((float)rr);
                         y = fma(fma(-rr, y, 1.0), y, y);
                         double y3 = y * y * y;
@@ -988,8 +998,11 @@ __device__ __forceinline__ void eval_list(const JobDev *__restrict__ J,
                     }
                 }
             };
-            if (all_in) near_pairs(std::integral_constant<bool, false>());
-            else near_pairs(std::integral_constant<bool, true>());
+            using no = std::integral_constant<bool, false>;
+            using yes = std::integral_constant<bool, true>;
+            if (!all_in) near_pairs(yes(), yes());
+            else if (clamp) near_pairs(yes(), no());
+            else near_pairs(no(), no());
 #pragma unroll
             for (int q = 0; q < PPL; ++q) acc[q] = fma(c6, b6[q], fma(c3, b3[q], acc[q]));
             continue;
@@ -1865,6 +1878,7 @@ __device__ __forceinline__ void eval_groups(const JobDev *__restrict__ J,
         mz[q] = -2.0 * pz[q];
         p2[q] = px[q] * px[q] + py[q] * py[q] + pz[q] * pz[q];
     }
+    const bool clamp = MATH == MATH_MIXED && uniform(seg[kSegInts * nseg]) != 0;
     int u = 0;  // groups before this one
     for (int s = 0; s < nseg; ++s) {
         const int *g = seg + kSegInts * s;
@@ -1971,10 +1985,12 @@ __device__ __forceinline__ void eval_groups(const JobDev *__restrict__ J,
             auto r2_of = [&](int k, double (&r2)[2]) {
                 pair_r2<2, XL>(near_rec(k), mx, my, mz, p2, r2);
             };
-            if (P.rclose + 2.0 * R + 3.0 * kMargin < J->rc)  // see eval_list
+            if (P.rclose + 2.0 * R + 3.0 * kMargin >= J->rc)  // see eval_list
+                mine(ne - nb, eight(), fp64(r2_of, one(), yes(), yes()));
+            else if (clamp)
                 mine(ne - nb, eight(), fp64(r2_of, one(), yes(), no()));
             else
-                mine(ne - nb, eight(), fp64(r2_of, one(), yes(), yes()));
+                mine(ne - nb, eight(), fp64(r2_of, one(), no(), no()));
         } else {
             auto expanded = [&](auto &&rec) {
                 return [&, rec](int k, double (&r2)[2]) {
