@@ -94,7 +94,8 @@ struct JobDev {
     void *out;          // float*, double* or uint32_t* by mode; index k + j*nz + i*ny*nz
     // Widom
     int nbins[3];       // insertion bins per fractional axis
-    int parts;          // > 0: an item is a quarter of a cell, for so many waves (see k_parts)
+    int parts;          // > 0: waves that share the points of one (see k_parts); an item is a
+                        // quarter of a cell, or with 2 a cell
     const uint32_t *sorted;     // insertion indices ordered by bin
     const uint32_t *bin_start;  // nbins_total + 1 offsets into sorted
     uint64_t seed;
@@ -160,8 +161,8 @@ constexpr double kNodeReach = 8.0;  // far atoms of a block lie at least this ma
 constexpr int kNodeRecords = kNodes * kNodes * kNodes * 8 / 32;  // LDS records the values take
 constexpr long long kNodeMinBlocks = 1024;  // see use_nodes
 constexpr double kNodeMinFar = 140.0;
-// cells up to which a job's cells are shared out to workgroups of eight / four waves
-constexpr long long kPartCells8 = 128, kPartCells4 = 320;
+// cells up to which the points of a wave are shared by eight / four / two waves
+constexpr long long kPartCells8 = 128, kPartCells4 = 320, kPartCells2 = 512;
 constexpr long long kMinGridItems = 2048;  // regions per grid before regions shrink
 
 }  // namespace er

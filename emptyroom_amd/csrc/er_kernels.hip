@@ -544,7 +544,7 @@ __device__ __forceinline__ Tile cell_sphere(const JobDev *__restrict__ J, const 
 // Split of the LDS list: [0, capA) holds far records (from 0 upwards) and
 // shell records (from capA-1 downwards); [capA, cap) holds near records.
 template <int MATH>
-__device__ __forceinline__ int near_region_start(int cap) {
+__host__ __device__ __forceinline__ int near_region_start(int cap) {
     if (MATH == MATH_FP64) return cap - kWG;  // near: atoms within R of the tile centre
     if (MATH == MATH_COUNT || MATH == MATH_OVERLAP) return cap - kWG;  // no near records
     return mixed_far_shell_cap(cap);
@@ -1845,19 +1845,24 @@ __global__ __launch_bounds__(kWG, MATH == MATH_NODES ? 4 : 1) void k_tiles(const
 // one wave of grid_tile or of a bin (two per lane), makes the same lists, and its
 // waves share the records out: group g of 16 far or shell records (the FP32 sums'
 // groups, so every FP32 sum is the same) or of 8 near records goes to wave g mod
-// WAVES, and the waves' FP64 energies are added in order at the end.
+// WAVES, and the waves' FP64 energies are added in order at the end.  For grids up
+// to twice as many cells as CUs a workgroup of eight waves has a whole cell, two
+// waves for each of its four parts, which share the list: up to four waves on a
+// SIMD instead of two, in one round.
 //
 // us a call, one workgroup per cell / eight waves / four waves: FP32 grid of 8
 // cells, 400 atoms 114 / 54 / 65, 64 cells 85 / 46 / 56, 216 cells 80 / 77 / 65,
 // 343 cells 87 / - / 88; Henry run of 1e3 insertions (2 bins), 1500 atoms 716 /
 // 235 / 304, 2e4 (42) 320 / 147 / 184, 1e5 (209) 260 / 231 / 212, 1.5e5 (313) 285 /
-// - / 275, 2e5 (417) 343 / - / 373.
+// - / 275, 2e5 (417) 343 / - / 373.  One workgroup per cell / two waves a part: FP32
+// grid of 343 cells, 400 atoms 83 / 74, 512 cells 83 / 77, 729 cells 95 / 101; FP64
+// 95 / 81, 95 / 83, 109 / 109.
 constexpr int kNearGroup = 8;
 
 // This wave's groups of the LDS list, for the points of all of the workgroup.
 // wn: wave-far and wave-shell counts per segment of the shared lists wl (grid
 // tiles; segment's entries at its shell offset), or nullptr.
-template <int MATH, bool XL, int WAVES>
+template <int MATH, bool XL, int WAVES, int PARTS>
 __device__ __forceinline__ void eval_groups(const JobDev *__restrict__ J,
                                             const double4 *__restrict__ L, int cap,
                                             const int *__restrict__ seg, int nseg,
@@ -1865,7 +1870,7 @@ __device__ __forceinline__ void eval_groups(const JobDev *__restrict__ J,
                                             const double (&pz)[2], double (&acc)[2], double R,
                                             const int *__restrict__ wn,
                                             const uint16_t *__restrict__ wl) {
-    const int wave = uniform(threadIdx.x >> 6);
+    const int wave = uniform(threadIdx.x >> 6) & (WAVES - 1);  // of the part's waves
     const double rc2 = J->rc2, min_r2 = J->min_r2;
     const int capA = near_region_start<MATH>(cap);
     const double4 *__restrict__ Ls = L + capA - 1, *__restrict__ Ln = L + capA;
@@ -2017,13 +2022,14 @@ __device__ __forceinline__ void eval_groups(const JobDev *__restrict__ J,
     }
 }
 
-template <int MATH, int WAVES>
-__global__ __launch_bounds__(64 * WAVES, 4) void k_parts(const JobDev *__restrict__ jobs,
-                                                         int njobs, int cap) {
+template <int MATH, int WAVES, int PARTS>
+__global__ __launch_bounds__(64 * WAVES * PARTS, 4) void k_parts(const JobDev *__restrict__ jobs,
+                                                                 int njobs, int cap) {
+    constexpr int WG = 64 * WAVES * PARTS;
     extern __shared__ double4 s_list[];
     __shared__ int s_seg[kSegInts * (kMaxSeg + 1)];
-    __shared__ int s_wn[2 * kMaxSeg];
-    __shared__ int s_cnt[7 * WAVES];
+    __shared__ int s_wn_all[PARTS][2 * kMaxSeg];
+    __shared__ int s_cnt[7 * (WG / 64)];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const long long item = blockIdx.x;
     int jl = 0, jh = njobs - 1;
@@ -2034,21 +2040,26 @@ __global__ __launch_bounds__(64 * WAVES, 4) void k_parts(const JobDev *__restric
     }
     const JobDev *__restrict__ J = jobs + jl;
     const long long local = item - J->item_begin + J->local0;
-    const int part = (int)(local & 3);
-    const bool grid = MATH == MATH_FP64 || J->kind == JOB_GRID;
+    const int part = PARTS == 4 ? uniform(wave / WAVES) : (int)(local & 3);
+    const int pwave = wave & (WAVES - 1);  // of the part's waves
+    const bool grid = MATH == MATH_FP64 || PARTS == 4 || J->kind == JOB_GRID;
     const int *nc = grid ? J->ntiles : J->nbins;
     int tc[3];
-    const long long cell = local >> 2;
+    const long long cell = PARTS == 4 ? local : local >> 2;
     tc[2] = (int)(cell % nc[2]);
     tc[1] = (int)((cell / nc[2]) % nc[1]);
     tc[0] = (int)(cell / ((long long)nc[1] * nc[2]));
-    uint16_t *__restrict__ s_wl = reinterpret_cast<uint16_t *>(s_list + cap);
+    const int capA = near_region_start<MATH>(cap);
+    uint16_t *__restrict__ s_wl =
+        reinterpret_cast<uint16_t *>(s_list + cap) + (PARTS == 4 ? part * capA : 0);
+    int *s_wn = s_wn_all[PARTS == 4 ? part : 0];
 
     // a tile: the part's quadrant, as a wave of grid_tile has it; a bin: the
     // insertions a wave of k_tiles has of each 512
     int i0[3] = {0, 0, 0}, i1[3] = {0, 0, 0};
     const int h1 = J->tile[1] / 2, h2 = J->tile[2] / 2;
     uint32_t s0 = 0, s1 = 0;
+    bool idle = false;
     Tile tl;
     double4 wsph = make_double4(0.0, 0.0, 0.0, 0.0);
     if (grid) {
@@ -2061,12 +2072,14 @@ __global__ __launch_bounds__(64 * WAVES, 4) void k_parts(const JobDev *__restric
         const int jb = i0[1] + (part & 1) * h1, kb = i0[2] + (part >> 1) * h2;
         const int je = jb + h1 - 1 < i1[1] ? jb + h1 - 1 : i1[1];
         const int ke = kb + h2 - 1 < i1[2] ? kb + h2 - 1 : i1[2];
-        if (jb > i1[1] || kb > i1[2]) return;  // no point of the part is on the grid
+        idle = jb > i1[1] || kb > i1[2];  // no point of the part is on the grid
+        if (PARTS == 1 && idle) return;
         tl = points_sphere(J, i0, i1,
                            i1[0] - i0[0] == J->tile[0] - 1 && i1[1] - i0[1] == J->tile[1] - 1 &&
                                i1[2] - i0[2] == J->tile[2] - 1,
                            J->cell_R);
-        const int w0[3] = {i0[0], jb, kb}, w1[3] = {i1[0], je, ke};
+        const int w0[3] = {i0[0], idle ? i0[1] : jb, idle ? i0[2] : kb};
+        const int w1[3] = {i1[0], idle ? i0[1] : je, idle ? i0[2] : ke};
         const Tile w = points_sphere(J, w0, w1,
                                      i1[0] - i0[0] == J->tile[0] - 1 && je - jb == h1 - 1 &&
                                          ke - kb == h2 - 1,
@@ -2115,18 +2128,17 @@ __global__ __launch_bounds__(64 * WAVES, 4) void k_parts(const JobDev *__restric
         }
         int cur_t = 0, cur_pos = uniform(J->type_begin[0]);
         do {
-            const int nseg = fill_list<MATH, 64 * WAVES>(J, J->near, nullptr, J->type_begin, tl,
+            const int nseg = fill_list<MATH, WG>(J, J->near, nullptr, J->type_begin, tl,
                                                       cur_t, cur_pos, cap, s_list, s_seg, s_cnt);
             __syncthreads();
             if (grid) {
                 // each segment's shell records against the part's points, a wave
                 // per segment
-                const int capA = near_region_start<MATH>(cap);
-                for (int s = wave; s < nseg; s += WAVES) {
+                for (int s = pwave; s < nseg; s += WAVES) {
                     const int sb = uniform(s_seg[kSegInts * s + 2]),
                               se = uniform(s_seg[kSegInts * (s + 1) + 2]);
                     int nwf = 0, nws = 0;
-                    if (se > sb)
+                    if (se > sb && !idle)
                         wave_shell_lists(J, s_list + capA - 1, capA, se - sb, sb, se, wsph,
                                          s_wl + sb, nwf, nws);
                     if (lane == 0) {
@@ -2136,12 +2148,14 @@ __global__ __launch_bounds__(64 * WAVES, 4) void k_parts(const JobDev *__restric
                 }
                 __syncthreads();
             }
-            if (xl)
-                eval_groups<MATH, true, WAVES>(J, s_list, cap, s_seg, nseg, px, py, pz, acc, tl.R, s_wn,
-                                        s_wl);
-            else
-                eval_groups<MATH, false, WAVES>(J, s_list, cap, s_seg, nseg, px, py, pz, acc, tl.R,
-                                         grid ? s_wn : nullptr, s_wl);
+            if (idle) {
+            } else if (xl) {
+                eval_groups<MATH, true, WAVES, PARTS>(J, s_list, cap, s_seg, nseg, px, py, pz, acc,
+                                                      tl.R, s_wn, s_wl);
+            } else {
+                eval_groups<MATH, false, WAVES, PARTS>(J, s_list, cap, s_seg, nseg, px, py, pz,
+                                                       acc, tl.R, grid ? s_wn : nullptr, s_wl);
+            }
             __syncthreads();
         } while (cur_t < J->ntypes);
         // the waves' energies, added in order
@@ -2149,11 +2163,12 @@ __global__ __launch_bounds__(64 * WAVES, 4) void k_parts(const JobDev *__restric
 #pragma unroll
         for (int q = 0; q < 2; ++q) red[(2 * wave + q) * 64 + lane] = acc[q];
         __syncthreads();
-        if (wave < 2) {
+        if (pwave < 2) {
             double e = 0.0;
-            for (int w = 0; w < WAVES; ++w) e += red[(2 * w + wave) * 64 + lane];
-            const long long o = wave == 0 ? at[0] : at[1];
-            if (wave == 0 ? ok[0] : ok[1]) {
+            const int w0 = PARTS == 4 ? part * WAVES : 0;
+            for (int w = w0; w < w0 + WAVES; ++w) e += red[(2 * w + pwave) * 64 + lane];
+            const long long o = pwave == 0 ? at[0] : at[1];
+            if (pwave == 0 ? ok[0] : ok[1]) {
                 if (!grid) J->e_out[o] = e;
                 else if (J->mode == OUT_F64) ((double *)J->out)[o] = e;
                 else ((float *)J->out)[o] = (float)(e < (double)FLT_MAX ? e : (double)FLT_MAX);
@@ -2410,16 +2425,20 @@ static hipError_t launch_parts(int math, const JobDev *jobs, int njobs, long lon
                                int cap, hipStream_t s) {
     if (total <= 0) return hipSuccess;
     if (cap < 2 * kWG || total > (1LL << 31) - 1) return hipErrorInvalidValue;
-    // one list of shell offsets for the workgroup
-    const size_t lds = ((size_t)cap * (sizeof(double4) + sizeof(uint16_t)) + 15) & ~(size_t)15;
-#define ER_PARTS(V, M, W)                                                                     \
-    if (math == V)                                                                            \
-        hipLaunchKernelGGL((k_parts<M, W>), dim3((unsigned)total), dim3(64 * W), lds, s, jobs, \
-                           njobs, cap);
-    ER_PARTS(MATH_PARTS8, MATH_MIXED, 8)
-    ER_PARTS(MATH_PARTS8_FP64, MATH_FP64, 8)
-    ER_PARTS(MATH_PARTS4, MATH_MIXED, 4)
-    ER_PARTS(MATH_PARTS4_FP64, MATH_FP64, 4)
+    // a list of shell offsets for each part of the workgroup
+#define ER_PARTS(V, M, W, P)                                                                  \
+    if (math == V) {                                                                          \
+        const size_t lds = (size_t)cap * sizeof(double4) +                                    \
+                           (size_t)P * near_region_start<M>(cap) * sizeof(uint16_t);          \
+        hipLaunchKernelGGL((k_parts<M, W, P>), dim3((unsigned)total), dim3(64 * W * P),       \
+                           (lds + 15) & ~(size_t)15, s, jobs, njobs, cap);                    \
+    }
+    ER_PARTS(MATH_PARTS8, MATH_MIXED, 8, 1)
+    ER_PARTS(MATH_PARTS8_FP64, MATH_FP64, 8, 1)
+    ER_PARTS(MATH_PARTS4, MATH_MIXED, 4, 1)
+    ER_PARTS(MATH_PARTS4_FP64, MATH_FP64, 4, 1)
+    ER_PARTS(MATH_PARTS2, MATH_MIXED, 2, 4)
+    ER_PARTS(MATH_PARTS2_FP64, MATH_FP64, 2, 4)
 #undef ER_PARTS
     return hipGetLastError();
 }
@@ -2428,7 +2447,7 @@ hipError_t launch_tiles(int math, int ppl, const JobDev *jobs, int njobs, long l
                         unsigned long long *ctr, int wgs, int cap, uint32_t *scratch,
                         int scratch_cap, hipStream_t s) {
     if (total <= 0) return hipSuccess;
-    if (math >= MATH_PARTS8 && math <= MATH_PARTS4_FP64)
+    if (math >= MATH_PARTS8 && math <= MATH_PARTS2_FP64)
         return launch_parts(math, jobs, njobs, total, cap, s);
     if (cap < 2 * kWG || wgs <= 0) return hipErrorInvalidValue;
     if (scratch && scratch_cap < kWG) return hipErrorInvalidValue;

@@ -652,16 +652,21 @@ void use_parts(JobDev *j, const Tuning &tu) {
     const int *nc = grid ? j->ntiles : j->nbins;
     const long long cells = (long long)nc[0] * nc[1] * nc[2];
     // (16-bit offsets into the list, and two workgroups' LDS per CU)
-    if (j->interp || cells > kPartCells4 || tu.cap > 2048) return;
+    if (j->interp || cells > kPartCells2 || tu.cap > 2048) return;
+    // the part kernel does not stop at saturation, which in dense frameworks saves
+    // more than two waves a part gain (Henry runs of 320 to 512 bins, us without / with:
+    // 400 atoms 145 / 137, 3000 atoms 387 / 426); runs that return the energies gain 6%,
+    // but their sums are to be those of the runs that stop, to the bit
+    if (cells > kPartCells4 && !grid) return;
     // the quadrant layout of grid_tile with two points per lane; insertions have
     // the same energies whatever the points per lane
     if (grid && (tu.ppl != 2 || j->tile[0] % 2 || j->tile[1] % 2 || j->tile[2] % 2)) return;
-    j->parts = cells <= kPartCells8 ? 8 : 4;
+    j->parts = cells <= kPartCells8 ? 8 : cells <= kPartCells4 ? 4 : 2;
     for (int d = 0; d < 3; d++) {
         j->region[d] = 1;
         j->nregions[d] = nc[d];
     }
-    j->n_items = 4 * cells;
+    j->n_items = j->parts == 2 ? cells : 4 * cells;
 }
 
 JobDev make_widom_job(const FrameworkDev *fw, uint64_t n_ins, uint64_t seed,
@@ -1058,8 +1063,8 @@ namespace {
 
 // Launches of a batch, in this order.
 constexpr int kBatchMath[kBatchLaunches] = {MATH_NODES,  MATH_MIXED,       MATH_FP64,
-                                              MATH_PARTS4, MATH_PARTS4_FP64, MATH_PARTS8,
-                                              MATH_PARTS8_FP64};
+                                              MATH_PARTS2, MATH_PARTS2_FP64, MATH_PARTS4,
+                                              MATH_PARTS4_FP64, MATH_PARTS8, MATH_PARTS8_FP64};
 
 // Expected in-cutoff pairs per point: the ordering key of the LPT schedule.
 double job_cost_per_item(const FrameworkDev *fw, const JobDev &j, const Tuning &tu) {

@@ -258,7 +258,7 @@ struct Task {
     uint64_t seed = 0;
 };
 
-constexpr int kBatchLaunches = 7;  // tiled-kernel variants of a batch, one launch each
+constexpr int kBatchLaunches = 9;  // tiled-kernel variants of a batch, one launch each
 
 class Batch {
   public:
