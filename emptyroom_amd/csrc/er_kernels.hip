@@ -839,7 +839,7 @@ __device__ __forceinline__ void wave_shell_lists(const JobDev *__restrict__ J,
 // into the wave's own lists of LDS byte offsets wl (wave_shell_lists).
 // phase (wave-uniform): 0 every record, per segment far, shell, near; 1 only
 // the near records; 2 only the far and shell records.
-template <int PPL, int MATH, bool XL, int FLUSH = kFlushPairs>
+template <int PPL, int MATH, bool XL, int FLUSH = kFlushPairs, int NEAR = 1>
 __device__ __forceinline__ void eval_list(const JobDev *__restrict__ J,
                                           const double4 *__restrict__ L, int cap,
                                           const int *__restrict__ seg, int nseg,
@@ -981,7 +981,10 @@ __device__ __forceinline__ void eval_list(const JobDev *__restrict__ J,
             const bool all_in = P.rclose + 2.0 * R + 3.0 * kMargin < J->rc;
             // Most passes hold no record that a point may sit on (kClampBit): without
             // the clamp two points take 27 instead of 30 VALU instructions a record.
+            // Grid tiles have NEAR = 2 records in flight (4.9e7 points, 2400 atoms: 6.48 ms
+            // with one, 6.37 with two); bins one (a Henry run of 1.7e7: 2.11, 2.15 ms).
             auto near_pairs = [&](auto clamp, auto test) {
+#pragma unroll NEAR
                 for (int k = nb; k < ne; ++k) {
                     double r2[PPL];
                     pair_r2<PPL, XL>(Ln[k], mx, my, mz, p2, r2);
@@ -1041,6 +1044,9 @@ __device__ __forceinline__ void eval_list(const JobDev *__restrict__ J,
         };
         using no = std::integral_constant<bool, false>;
         using yes = std::integral_constant<bool, true>;
+        // (two records in flight: a 173^3-point grid of 424 atoms takes 745 us with one,
+        // 662 with two, 663 with four)
+#pragma unroll 2
         for (int k = fb; k < fe; ++k) fp64_pair(L[k], no(), no());
         // wave lists of an FP64 tile hold as many entries as an FP32 tile's
         // (the far + shell part of the FP32 list), which keeps four
@@ -1054,8 +1060,10 @@ __device__ __forceinline__ void eval_list(const JobDev *__restrict__ J,
             int nwf, nws;
             wave_shell_lists(J, Ls, capA, wcap, sb, se, wsph, wl, nwf, nws);
             const char *__restrict__ Lb = reinterpret_cast<const char *>(L);
+#pragma unroll 2
             for (int e = 0; e < nwf; ++e)
                 fp64_pair(*reinterpret_cast<const double4 *>(Lb + wl[e]), no(), no());
+#pragma unroll 2
             for (int e = 0; e < nws; ++e)
                 fp64_pair(*reinterpret_cast<const double4 *>(Lb + wl[wcap - 1 - e]), no(), yes());
         } else {
@@ -1268,10 +1276,10 @@ __device__ void grid_tile(const JobDev *__restrict__ J, const int tc[3],
         __syncthreads();
         if (!idle) {
             if (xl)
-                eval_list<PPL, MATH, true>(J, s_list, cap, s_seg, nseg, px, py, pz, acc, tl.R, ws,
+                eval_list<PPL, MATH, true, kFlushPairs, 2>(J, s_list, cap, s_seg, nseg, px, py, pz, acc, tl.R, ws,
                                            wsph, s_wl);
             else
-                eval_list<PPL, MATH, false>(J, s_list, cap, s_seg, nseg, px, py, pz, acc, tl.R,
+                eval_list<PPL, MATH, false, kFlushPairs, 2>(J, s_list, cap, s_seg, nseg, px, py, pz, acc, tl.R,
                                             ws, wsph, s_wl);
         }
         __syncthreads();
