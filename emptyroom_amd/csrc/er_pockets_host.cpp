@@ -391,8 +391,8 @@ int widom_grid_run(Context *ctx, GridDev *g, uint64_t n_ins, double temperature,
 
 // Positions whose coordinates and energies fit the small pinned buffer: the
 // kernel uses it itself.  us a call, copied / direct: 1 position 27 / 18, 1000 31 /
-// 19, 10000 44 / 27, 20000 56 / 39.
-constexpr uint64_t kPinnedPositions = Transfer::kSmall / (4 * sizeof(double));
+// 19, 10000 44 / 27, 20000 56 / 39, 50000 103 / 83, 100000 145 / 142, 130000 166 / 174.
+constexpr uint64_t kPinnedPositions = Transfer::kBuffer / (4 * sizeof(double));
 
 int grid_energies(Context *ctx, GridDev *g, const double *frac_host, uint64_t n,
                   double *out_host) {

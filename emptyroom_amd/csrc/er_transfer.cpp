@@ -128,7 +128,7 @@ std::shared_ptr<Transfer> Transfer::of_device(int device) {
 // The small buffer (chunks = 0), or slots and threads for a copy of so many
 // chunks; what is there stays.
 bool Transfer::ensure(long chunks, bool threads) {
-    if (chunks == 0 && !small_ && hipHostMalloc((void **)&small_, kSmall) != hipSuccess) {
+    if (chunks == 0 && !small_ && hipHostMalloc((void **)&small_, kBuffer) != hipSuccess) {
         (void)hipGetLastError();
         small_ = nullptr;
         return false;

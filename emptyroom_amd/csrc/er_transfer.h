@@ -37,10 +37,11 @@ class Transfer {
     hipError_t out(void *host, const void *dev, size_t bytes, hipStream_t s);
     // host -> dev on stream s; host memory must stay until s has passed the copy.
     hipError_t in(void *dev, const void *host, size_t bytes, hipStream_t s);
-    // The small buffer (kSmall bytes, device-accessible) for as long as the lock
+    // The small buffer (kBuffer bytes, device-accessible) for as long as the lock
     // is held; *p = nullptr if it is in use or cannot be had.
     std::unique_lock<std::mutex> small(char **p);
-    static constexpr size_t kSmall = 1 << 20;
+    static constexpr size_t kSmall = 1 << 20;   // bytes it is used for by copies, at most
+    static constexpr size_t kBuffer = 3 << 20;
 
   private:
     struct Job;
