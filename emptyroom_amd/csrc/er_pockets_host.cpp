@@ -148,7 +148,8 @@ int grid_upload(Context *ctx, const float *host, const int n[3], GridDev **out) 
         delete g;
         return ST_NOMEM;
     }
-    if (ctx->transfer->in(g->d_data, host, g->bytes(), ctx->stream) != hipSuccess ||
+    Transfer::Staged staged;
+    if (ctx->transfer->in(g->d_data, host, g->bytes(), ctx->stream, &staged) != hipSuccess ||
         hipStreamSynchronize(ctx->stream) != hipSuccess) {
         delete g;
         set_error("grid_upload: copy failed");
@@ -423,7 +424,8 @@ int grid_energies(Context *ctx, GridDev *g, const double *frac_host, uint64_t n,
     Scratch sc{ctx, {}};
     double *f = sc.get<double>(3 * n), *e = sc.get<double>(n);
     if (!f || !e) return ST_NOMEM;
-    HIP_TRY(ctx->transfer->in(f, frac_host, sizeof(double) * 3 * n, s));
+    Transfer::Staged staged;
+    HIP_TRY(ctx->transfer->in(f, frac_host, sizeof(double) * 3 * n, s, &staged));
     HIP_TRY(launch_grid_energies(g->d_data, g->precision, g->n, f, (long long)n, e, s));
     HIP_TRY(ctx->transfer->out(out_host, e, sizeof(double) * n, s));
     return ST_OK;

@@ -404,7 +404,8 @@ int framework_upload(Context *ctx, const Particle *atoms, int n, const double t[
     fw->d_type_block0 = (int *)(d_block + o_block0);
     hipStream_t s = ctx->stream;
     std::unique_ptr<FrameworkDev> owner(fw);
-    HIP_TRY(ctx->transfer->in(d_block, block.data(), total, s));
+    Transfer::Staged staged;
+    HIP_TRY(ctx->transfer->in(d_block, block.data(), total, s, &staged));
     plan.atoms = fw->d_atoms;
     plan.type_atom0 = fw->d_type_atom0;
     plan.type_block0 = fw->d_type_block0;

@@ -97,6 +97,24 @@ struct Transfer::Job {
     }
 };
 
+// One event per slot for the length of a copy: the runtime keeps an event's last
+// stream and looks at it again, so an event must not outlive that stream.
+struct Events {
+    hipEvent_t ev[kSlots] = {};
+    bool make(int n) {
+        for (int k = 0; k < n; k++)
+            if (hipEventCreateWithFlags(&ev[k], hipEventDisableTiming) != hipSuccess) {
+                (void)hipGetLastError();
+                return false;
+            }
+        return true;
+    }
+    ~Events() {
+        for (hipEvent_t e : ev)
+            if (e) (void)hipEventDestroy(e);
+    }
+};
+
 Transfer::~Transfer() {
     {
         std::lock_guard<std::mutex> lk(mu_);
@@ -104,15 +122,8 @@ Transfer::~Transfer() {
     }
     cv_.notify_all();
     for (std::thread &t : threads_) t.join();
-    for (size_t i = 0; i < slot_.size(); i++) {
-        (void)hipEventDestroy(ev_[i]);
-        (void)hipHostFree(slot_[i]);
-    }
+    for (char *p : slot_) (void)hipHostFree(p);
     if (small_) (void)hipHostFree(small_);
-    if (in_done_) {
-        (void)hipEventSynchronize(in_done_);
-        (void)hipEventDestroy(in_done_);
-    }
     if (in_) (void)hipHostFree(in_);
 }
 
@@ -134,18 +145,13 @@ bool Transfer::ensure(long chunks, bool threads) {
         return false;
     }
     slot_.reserve(kSlots);
-    ev_.reserve(kSlots);
     while ((long)slot_.size() < std::min<long>(kSlots, chunks)) {
-        hipEvent_t e = nullptr;
         void *p = nullptr;
-        if (hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess ||
-            hipHostMalloc(&p, kSlot) != hipSuccess) {
+        if (hipHostMalloc(&p, kSlot) != hipSuccess) {
             (void)hipGetLastError();
-            if (e) (void)hipEventDestroy(e);
             return false;
         }
         slot_.push_back((char *)p);
-        ev_.push_back(e);
     }
     const long cores = std::max(1l, (long)std::thread::hardware_concurrency());
     try {
@@ -198,7 +204,9 @@ hipError_t Transfer::out(void *host, const void *dev, size_t bytes, hipStream_t 
         return e;
     }
     Job job(host, bytes);
-    if (bytes <= kSmall || !lk.try_lock() || !ensure(job.chunks, bytes >= kFreshMin)) {
+    Events events;
+    if (bytes <= kSmall || !lk.try_lock() || !ensure(job.chunks, bytes >= kFreshMin) ||
+        !events.make((int)std::min<long>(kSlots, job.chunks))) {
         hipError_t e = hipMemcpyAsync(host, dev, bytes, hipMemcpyDeviceToHost, s);
         return e == hipSuccess ? hipStreamSynchronize(s) : e;
     }
@@ -208,7 +216,7 @@ hipError_t Transfer::out(void *host, const void *dev, size_t bytes, hipStream_t 
         const int k = (int)(c % kSlots);
         e = hipMemcpyAsync(slot_[k], (const char *)dev + job.begin(c), job.chunk_bytes(c),
                            hipMemcpyDeviceToHost, s);
-        if (e == hipSuccess) e = hipEventRecord(ev_[k], s);
+        if (e == hipSuccess) e = hipEventRecord(events.ev[k], s);
     };
     for (long c = 0; c < std::min<long>(kSlots, job.chunks) && e == hipSuccess; c++) issue(c);
     if (bytes >= kFreshMin) start(&job);
@@ -217,7 +225,7 @@ hipError_t Transfer::out(void *host, const void *dev, size_t bytes, hipStream_t 
     while (arrived < job.chunks && e == hipSuccess) {
         bool idle = true;
         if (arrived < issued) {
-            e = hipEventQuery(ev_[arrived % kSlots]);
+            e = hipEventQuery(events.ev[arrived % kSlots]);
             if (e == hipSuccess) {
                 job.ready.store(++arrived, std::memory_order_release);
                 idle = false;
@@ -240,28 +248,23 @@ hipError_t Transfer::out(void *host, const void *dev, size_t bytes, hipStream_t 
     return e;
 }
 
-hipError_t Transfer::in(void *dev, const void *host, size_t bytes, hipStream_t s) {
-    std::unique_lock<std::mutex> lk(in_mu_);
-    if (bytes <= kSmall && !in_) {
-        if (hipEventCreateWithFlags(&in_done_, hipEventDisableTiming) != hipSuccess ||
-            hipHostMalloc((void **)&in_, kSmall) != hipSuccess) {
-            (void)hipGetLastError();
-            if (in_done_) (void)hipEventDestroy(in_done_);
-            in_done_ = nullptr;
-            in_ = nullptr;
-        }
-    }
-    if (bytes > kSmall || !in_) {
-        lk.unlock();
+hipError_t Transfer::in(void *dev, const void *host, size_t bytes, hipStream_t s, Staged *hold) {
+    std::unique_lock<std::mutex> lk(in_mu_, std::defer_lock);
+    if (bytes > kSmall || !lk.try_lock())
+        return hipMemcpyAsync(dev, host, bytes, hipMemcpyHostToDevice, s);
+    if (!in_ && hipHostMalloc((void **)&in_, kSmall) != hipSuccess) {
+        (void)hipGetLastError();
+        in_ = nullptr;
         return hipMemcpyAsync(dev, host, bytes, hipMemcpyHostToDevice, s);
     }
-    hipError_t e = hipEventSynchronize(in_done_);  // the copy before this one
-    if (e != hipSuccess) return e;
     std::memcpy(in_, host, bytes);
-    e = hipMemcpyAsync(dev, in_, bytes, hipMemcpyHostToDevice, s);
-    if (e == hipSuccess) e = hipEventRecord(in_done_, s);
-    if (e != hipSuccess) (void)hipStreamSynchronize(s);
-    return e;
+    hold->lk_ = std::move(lk);
+    hold->s_ = s;
+    return hipMemcpyAsync(dev, in_, bytes, hipMemcpyHostToDevice, s);
+}
+
+Transfer::Staged::~Staged() {
+    if (lk_.owns_lock()) (void)hipStreamSynchronize(s_);
 }
 
 std::unique_lock<std::mutex> Transfer::small(char **p) {

@@ -35,8 +35,20 @@ class Transfer {
     // dev -> host on stream s, after what s holds; returns when the bytes are in
     // host memory.
     hipError_t out(void *host, const void *dev, size_t bytes, hipStream_t s);
-    // host -> dev on stream s; host memory must stay until s has passed the copy.
-    hipError_t in(void *dev, const void *host, size_t bytes, hipStream_t s);
+    // Holds the upload buffer of a copy until its stream has passed it (no event does:
+    // one that outlives the stream it was recorded on cannot be waited for).
+    class Staged {
+      public:
+        ~Staged();
+
+      private:
+        friend class Transfer;
+        std::unique_lock<std::mutex> lk_;
+        hipStream_t s_ = nullptr;
+    };
+    // host -> dev on stream s, through the upload buffer if that is free; host
+    // memory must stay until s has passed the copy, and so must *hold.
+    hipError_t in(void *dev, const void *host, size_t bytes, hipStream_t s, Staged *hold);
     // The small buffer (kBuffer bytes, device-accessible) for as long as the lock
     // is held; *p = nullptr if it is in use or cannot be had.
     std::unique_lock<std::mutex> small(char **p);
@@ -49,13 +61,11 @@ class Transfer {
     void start(Job *job);
     void finish();
     void work();
-    std::mutex in_mu_;              // guards the upload buffer and its last copy's event
+    std::mutex in_mu_;              // held by the copy that uses the upload buffer
     char *in_ = nullptr;
-    hipEvent_t in_done_ = nullptr;
     std::mutex busy_;               // held by the copy that uses what follows
     char *small_ = nullptr;
     std::vector<char *> slot_;      // pinned, one size
-    std::vector<hipEvent_t> ev_;    // per slot: its last device copy
     std::vector<std::thread> threads_;
     std::mutex mu_;                 // guards what follows
     std::condition_variable cv_;
