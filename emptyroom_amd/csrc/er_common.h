@@ -160,7 +160,7 @@ constexpr double kNodeReach = 8.0;  // far atoms of a block lie at least this ma
                                     // half-extent away from every point
 constexpr int kNodeRecords = kNodes * kNodes * kNodes * 8 / 32;  // LDS records the values take
 constexpr long long kNodeMinBlocks = 1024;  // see use_nodes
-constexpr double kNodeMinFar = 140.0;
+constexpr double kNodeMinFar = 120.0;
 // cells up to which the points of a wave are shared by eight / four / two waves
 constexpr long long kPartCells8 = 128, kPartCells4 = 320, kPartCells2 = 512;
 constexpr long long kMinGridItems = 2048;  // regions per grid before regions shrink

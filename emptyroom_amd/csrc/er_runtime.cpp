@@ -577,10 +577,10 @@ bool use_nodes(const FrameworkDev *fw, const int n[3], const int tile[3], const 
     }
     // ... with enough blocks to fill the device when the grid runs alone, and
     // enough far atoms per block to pay for its interpolation.  Cubic-ish cells at
-    // 0.1 A, us without / with nodes: 0.1 atoms/A^3 (430 expected far atoms)
-    // 1728 blocks 2098 / 1686, 1000 blocks 1106 / 1071, 512 blocks 579 / 717;
-    // 4096 blocks at 0.1 atoms/A^3 5965 / 4190, 0.03 (128 far atoms) 2086 / 2050,
-    // 0.012 (51) 1267 / 1493.
+    // 0.1 A, us without / with nodes: 0.1 atoms/A^3 (430 expected far atoms) 512 blocks
+    // 576 / 633, 1000 blocks 1085 / 968, 1728 blocks 2046 / 1511, 4096 blocks 5508 / 3540;
+    // 0.03 atoms/A^3 (128) 1000 blocks 390 / 420, 1331 blocks 559 / 545, 4096 blocks
+    // 1862 / 1644; 0.012 (51) 4096 blocks 973 / 1072.  At 0.14 A (66) 2148 / 2374.
     double lo = kNodeReach * h;
     for (const TypeParams &tp : fw->types) lo = std::max(lo, tp.rclose);
     const double R = box_radius(fw->t, half);
