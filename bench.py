@@ -12,8 +12,9 @@ After the timed steps, the default run also measures:
 - the plain path (one framework per launch, synchronous, grids left
   resident as the batch leaves them) on the same work: batched/plain, against
   the workload's 5x target;
-- the tiled kernel on the step's grids alone (the roofline launch: every
-  in-cutoff grid pair is evaluated, 16 FLOP each, VALU-bound) and on its Widom
+- the tiled kernels on the step's grids alone (the roofline launches: 16 FLOP
+  for every in-cutoff grid pair, VALU-bound; the far pairs of fine grids are
+  evaluated at an eighth of the points and interpolated) and on its Widom
   runs alone (an insertion rate: saturated insertions stop early);
 - the same step with FP64 grids (the drop-in writegrid's default precision)
   and the FP64 grids alone against the FP64 vector peak;
@@ -625,9 +626,10 @@ def main():
         gb.close()
         log(f"graph step {graph_ms:.1f} ms")
 
-    # The roofline kernel: the same tiled kernel on the step's grids alone.
-    # Every in-cutoff pair of a grid is evaluated (no early stop), so 16 FLOP
-    # per in-cutoff pair is work the kernel must do.  The Widom share of the
+    # The roofline launches: the same tiled kernels on the step's grids alone.
+    # Every in-cutoff pair of a grid counts in it (no early stop): 16 FLOP each is
+    # the direct method's work, of which fine grids do less (their far pairs come
+    # from nodes, an eighth of the points).  The Widom share of the
     # step is timed on its own too (its insertions may stop once their energy
     # is certain to reach 800 T, so it gets an insertion rate, not FLOP/s).
     grid_tasks = [dict(t, n_insertions=0) for t in tasks]
@@ -833,15 +835,19 @@ def main():
                      "frac_attainable": achieved / PEAK_FP32_UNPACKED_TFLOPS,
                      "traffic": measured_traffic(tuning, len(fws))
                      if args.workload == "config3" and gprec == api.ER_FP32 else None,
-                     "kernel": f"k_tiles<{tuning['ppl']},MIXED> on the step's {len(fws)} grids "
-                               "alone (one launch)" if gprec == api.ER_FP32 else
-                               f"k_tiles<{tuning['ppl']},FP64> on the step's grids alone",
+                     "kernel": f"k_tiles<{tuning['ppl']},MIXED>, its variant with nodes and "
+                               f"k_parts on the step's {len(fws)} grids alone (a launch each)"
+                               if gprec == api.ER_FP32 else
+                               f"k_tiles<{tuning['ppl']},FP64> and k_parts on the step's grids "
+                               "alone",
                      "kernel_ms": grid_ms,
                      "flop_per_pair": FLOP_PER_PAIR,
                      "incut_pairs": incut_grid,
-                     "note": "16 FLOP x every in-cutoff pair of the step's grids (all of them "
-                             "evaluated) / the grid-only launch; peak 157.3 is the packed-FP32 "
-                             "rate, which this build does not use (attainable_peak 78.6)"},
+                     "note": "16 FLOP x every in-cutoff pair of the step's grids / the grid-only "
+                             "launches: the direct method's work per second (the far pairs of "
+                             "fine grids are evaluated at an eighth of the points and "
+                             "interpolated); peak 157.3 is the packed-FP32 rate, which this "
+                             "build does not use (attainable_peak 78.6)"},
         "widom_alone": {"kernel_ms": widom_ms, "insertions_per_s": n_ins / (widom_ms / 1e3),
                         "incut_pairs": incut_widom,
                         "note": "insertions stop once their energy is certain to reach 800 T "

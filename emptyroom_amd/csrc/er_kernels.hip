@@ -20,7 +20,9 @@
 // in FP32 and FP64 grid tiles each wave first re-sorts the shell records
 // against its own, smaller point box.  A Widom bin of at most one chunk of
 // insertions keeps their points and partial energies in registers across
-// its LDS passes.
+// its LDS passes.  Fine FP32 grids take the far field of blocks of tiles from
+// interpolation nodes (grid_block), and jobs of a few hundred cells share the
+// points of a wave between several (k_parts).
 #include "er_kernels.h"
 
 #include <float.h>
@@ -1373,8 +1375,8 @@ __device__ bool build_region_list(const JobDev *__restrict__ J, double cx, doubl
 // directly, as without nodes.  Direct tiles are bound by VALU issue (98% of the
 // cycles), and at 0.1 A half of what they issue is for such pairs: a grid of
 // 1.48e7 points and 3000 atoms (0.21 atoms/A^3) issued 5.0e9 wave instructions
-// in 10.3 ms and now issues 3.5e9 in 7.2 ms; one of 4.9e7 points and 2400 atoms
-// (0.05 atoms/A^3) took 10.6 and takes 7.8 ms.
+// in 10.3 ms and with nodes 3.5e9 in 7.2 ms (6.8 ms with a cheaper tile setup since);
+// one of 4.9e7 points and 2400 atoms (0.05 atoms/A^3) took 10.6, then 7.8 ms (now 6.4).
 //
 // Accuracy: an atom at D from the middle of a segment of half-length h through
 // the box has a Chebyshev interpolation error on it of at most
