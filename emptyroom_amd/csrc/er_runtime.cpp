@@ -1050,6 +1050,7 @@ int count_incut_widom(Context *ctx, FrameworkDev *fw, uint64_t n_ins, uint64_t s
 // ---------------------------------------------------------------------------
 
 Batch::~Batch() {
+    if (ctx) (void)hipStreamSynchronize(ctx->stream);  // a run writes h_sums
     for (hipEvent_t e : ev)
         if (e) (void)hipEventDestroy(e);
     if (exec) (void)hipGraphExecDestroy(exec);

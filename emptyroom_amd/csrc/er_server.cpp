@@ -164,12 +164,17 @@ Server::~Server() {
     cv_.notify_all();
     if (worker_.joinable()) worker_.join();
     (void)hipStreamSynchronize(ctx_->stream);  // uploads and Widom binning
+    for (auto &L : launches_)
+        if (L->stream) (void)hipStreamSynchronize(L->stream);
+    // (an event must not outlive the stream it was recorded on)
+    for (auto &kv : all_) {
+        Req *r = kv.second.get();
+        if (r->ready) (void)hipEventDestroy(r->ready);
+        if (r->reduced) (void)hipEventDestroy(r->reduced);
+    }
     for (auto &L : launches_) {
-        if (L->stream) {
-            (void)hipStreamSynchronize(L->stream);
-            (void)hipStreamDestroy(L->stream);
-        }
         if (L->done) (void)hipEventDestroy(L->done);
+        if (L->stream) (void)hipStreamDestroy(L->stream);
         if (L->h_jobs) (void)hipHostFree(L->h_jobs);
         ctx_->pool.free(L->d_jobs);
         ctx_->pool.free(L->d_counter);
@@ -183,8 +188,6 @@ Server::~Server() {
         Req *r = kv.second.get();
         delete r->grid;
         for (void *p : r->owned) ctx_->pool.free(p);
-        if (r->ready) (void)hipEventDestroy(r->ready);
-        if (r->reduced) (void)hipEventDestroy(r->reduced);
         if (r->h_sums) (void)hipHostFree(r->h_sums);
     }
     for (auto &kv : cache_) delete kv.second->fw;
