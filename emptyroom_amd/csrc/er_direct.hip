@@ -251,7 +251,8 @@ int direct_widom(Context *ctx, const Particle *atoms, int n_atoms, const double 
     int st = direct_setup(ctx, atoms, n_atoms, t, rep, rc2, min_r * min_r, buf, &J);
     if (st != ST_OK) return st;
     double *e = buf.get<double>(n_ins);
-    if (!e) return ST_NOMEM;
+    const double *sums = ctx->sums();
+    if (!e || !sums) return ST_NOMEM;
     hipStream_t s = ctx->stream;
     hipLaunchKernelGGL(k_direct_widom, dim3((unsigned)((n_ins + kDirectWG - 1) / kDirectWG)),
                        dim3(kDirectWG), 0, s, J, seed, (long long)n_ins, e);
@@ -261,8 +262,8 @@ int direct_widom(Context *ctx, const Particle *atoms, int n_atoms, const double 
     if (energies_host)
         HIP_TRY(hipMemcpyAsync(energies_host, e, sizeof(double) * n_ins, hipMemcpyDeviceToHost, s));
     HIP_TRY(hipStreamSynchronize(s));
-    out->sum_b = ctx->h_sums[0];
-    out->sum_eb = ctx->h_sums[1];
+    out->sum_b = sums[0];
+    out->sum_eb = sums[1];
     out->n = n_ins;
     return ST_OK;
 }

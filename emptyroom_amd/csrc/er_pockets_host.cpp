@@ -373,7 +373,8 @@ int widom_grid_run(Context *ctx, GridDev *g, uint64_t n_ins, double temperature,
     Scratch sc{ctx, {}};
     double *e = energies_host ? sc.get<double>(n_ins) : nullptr;
     double2 *partials = sc.get<double2>(kTriBlocks);
-    if ((energies_host && !e) || !partials) return ST_NOMEM;
+    const double *sums = ctx->sums();
+    if ((energies_host && !e) || !partials || !sums) return ST_NOMEM;
     hipStream_t s = ctx->stream;
     // (without the memory for them the run does without face records)
     const size_t fb = tri_faces_bytes(g->n, n_ins);
@@ -384,8 +385,8 @@ int widom_grid_run(Context *ctx, GridDev *g, uint64_t n_ins, double temperature,
     if (energies_host)
         HIP_TRY(ctx->transfer->out(energies_host, e, sizeof(double) * n_ins, s));
     HIP_TRY(hipStreamSynchronize(s));
-    out->sum_b = ctx->h_sums[0];
-    out->sum_eb = ctx->h_sums[1];
+    out->sum_b = sums[0];
+    out->sum_eb = sums[1];
     out->n = n_ins;
     return ST_OK;
 }
@@ -424,8 +425,7 @@ int grid_energies(Context *ctx, GridDev *g, const double *frac_host, uint64_t n,
     Scratch sc{ctx, {}};
     double *f = sc.get<double>(3 * n), *e = sc.get<double>(n);
     if (!f || !e) return ST_NOMEM;
-    Transfer::Staged staged;
-    HIP_TRY(ctx->transfer->in(f, frac_host, sizeof(double) * 3 * n, s, &staged));
+    HIP_TRY(hipMemcpyAsync(f, frac_host, sizeof(double) * 3 * n, hipMemcpyHostToDevice, s));
     HIP_TRY(launch_grid_energies(g->d_data, g->precision, g->n, f, (long long)n, e, s));
     HIP_TRY(ctx->transfer->out(out_host, e, sizeof(double) * n, s));
     return ST_OK;

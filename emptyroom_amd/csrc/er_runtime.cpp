@@ -186,6 +186,15 @@ void *Context::host_stage(size_t bytes) {
     return h_stage;
 }
 
+double *Context::sums() {
+    if (!h_sums && hipHostMalloc((void **)&h_sums, 2 * sizeof(double)) != hipSuccess) {
+        (void)hipGetLastError();
+        h_sums = nullptr;
+        set_error("pinned host allocation failed");
+    }
+    return h_sums;
+}
+
 int context_create(int device, size_t hbm_cap, Context **out) {
     int ndev = 0;
     if (hipGetDeviceCount(&ndev) != hipSuccess || ndev <= 0) {
@@ -212,7 +221,6 @@ int context_create(int device, size_t hbm_cap, Context **out) {
     }
     if (pool_alloc(c, 1, &c->d_counter, nullptr) != ST_OK ||
         pool_alloc(c, kReduceBlocks, &c->d_partials, nullptr) != ST_OK ||
-        hipHostMalloc((void **)&c->h_sums, 2 * sizeof(double)) != hipSuccess ||
         scratch_ensure(c, c->stream, &c->d_scratch, &c->scratch_wgs) != ST_OK) {
         delete c;
         return ST_NOMEM;
@@ -949,6 +957,8 @@ int widom_run(Context *ctx, FrameworkDev *fw, uint64_t n_ins, double temperature
     ST_TRY(widom_prepare(ctx, fw, n_ins, &wb, &tmp.ptrs));
     // energies returned to the caller are computed in full; otherwise only the
     // sums are, and saturated insertions may stop early
+    const double *sums = ctx->sums();
+    if (!sums) return ST_NOMEM;
     JobDev job = make_widom_job(fw, n_ins, seed, wb, ctx->tuning, kMinGridItems,
                                 energies_host ? 0.0 : temperature);
     use_parts(&job, ctx->tuning);
@@ -960,8 +970,8 @@ int widom_run(Context *ctx, FrameworkDev *fw, uint64_t n_ins, double temperature
     if (energies_host)
         HIP_TRY(ctx->transfer->out(energies_host, wb.e, sizeof(double) * n_ins, s));
     HIP_TRY(hipStreamSynchronize(s));
-    out->sum_b = ctx->h_sums[0];
-    out->sum_eb = ctx->h_sums[1];
+    out->sum_b = sums[0];
+    out->sum_eb = sums[1];
     out->n = n_ins;
     return ST_OK;
 }

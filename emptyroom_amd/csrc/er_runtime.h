@@ -96,7 +96,7 @@ class Context {
     DevicePool pool{this};
     unsigned long long *d_counter = nullptr;  // work counter of plain launches
     double2 *d_partials = nullptr;
-    double *h_sums = nullptr;                 // pinned; the reductions write it
+    double *h_sums = nullptr;                 // see sums()
     uint32_t *d_scratch = nullptr;  // region sub-lists, scratch_wgs * kRegionRecords indices
     int scratch_wgs = 0;
     void *h_stage = nullptr;       // pinned host staging of pocket labelling results
@@ -106,6 +106,9 @@ class Context {
     // Pinned host buffer of at least `bytes` (kept, grown on demand); nullptr
     // with the error set if the allocation fails.
     void *host_stage(size_t bytes);
+    // Two pinned doubles that the reductions write, made when first asked for;
+    // nullptr with the error set if that fails.
+    double *sums();
 };
 
 int context_create(int device, size_t hbm_cap, Context **out);

@@ -124,7 +124,6 @@ Transfer::~Transfer() {
     for (std::thread &t : threads_) t.join();
     for (char *p : slot_) (void)hipHostFree(p);
     if (small_) (void)hipHostFree(small_);
-    if (in_) (void)hipHostFree(in_);
 }
 
 std::shared_ptr<Transfer> Transfer::of_device(int device) {
@@ -249,18 +248,14 @@ hipError_t Transfer::out(void *host, const void *dev, size_t bytes, hipStream_t 
 }
 
 hipError_t Transfer::in(void *dev, const void *host, size_t bytes, hipStream_t s, Staged *hold) {
-    std::unique_lock<std::mutex> lk(in_mu_, std::defer_lock);
-    if (bytes > kSmall || !lk.try_lock())
-        return hipMemcpyAsync(dev, host, bytes, hipMemcpyHostToDevice, s);
-    if (!in_ && hipHostMalloc((void **)&in_, kSmall) != hipSuccess) {
-        (void)hipGetLastError();
-        in_ = nullptr;
-        return hipMemcpyAsync(dev, host, bytes, hipMemcpyHostToDevice, s);
-    }
-    std::memcpy(in_, host, bytes);
+    char *pinned = nullptr;
+    std::unique_lock<std::mutex> lk;
+    if (bytes <= kSmall) lk = small(&pinned);
+    if (!pinned) return hipMemcpyAsync(dev, host, bytes, hipMemcpyHostToDevice, s);
+    std::memcpy(pinned, host, bytes);
     hold->lk_ = std::move(lk);
     hold->s_ = s;
-    return hipMemcpyAsync(dev, in_, bytes, hipMemcpyHostToDevice, s);
+    return hipMemcpyAsync(dev, pinned, bytes, hipMemcpyHostToDevice, s);
 }
 
 Transfer::Staged::~Staged() {

@@ -35,8 +35,9 @@ class Transfer {
     // dev -> host on stream s, after what s holds; returns when the bytes are in
     // host memory.
     hipError_t out(void *host, const void *dev, size_t bytes, hipStream_t s);
-    // Holds the upload buffer of a copy until its stream has passed it (no event does:
-    // one that outlives the stream it was recorded on cannot be waited for).
+    // Holds the small buffer of an upload until its stream has passed it (no event does:
+    // one that outlives the stream it was recorded on cannot be waited for).  The holder
+    // makes no other call of this class.
     class Staged {
       public:
         ~Staged();
@@ -46,7 +47,7 @@ class Transfer {
         std::unique_lock<std::mutex> lk_;
         hipStream_t s_ = nullptr;
     };
-    // host -> dev on stream s, through the upload buffer if that is free; host
+    // host -> dev on stream s, through the small buffer if that is free; host
     // memory must stay until s has passed the copy, and so must *hold.
     hipError_t in(void *dev, const void *host, size_t bytes, hipStream_t s, Staged *hold);
     // The small buffer (kBuffer bytes, device-accessible) for as long as the lock
@@ -61,8 +62,6 @@ class Transfer {
     void start(Job *job);
     void finish();
     void work();
-    std::mutex in_mu_;              // held by the copy that uses the upload buffer
-    char *in_ = nullptr;
     std::mutex busy_;               // held by the copy that uses what follows
     char *small_ = nullptr;
     std::vector<char *> slot_;      // pinned, one size
