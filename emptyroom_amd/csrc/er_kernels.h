@@ -98,6 +98,14 @@ __host__ __device__ inline int mixed_far_shell_cap(int cap) {
     const int near_cap = (cap / 3) & ~63;
     return cap - (near_cap < kWG ? kWG : near_cap);
 }
+// Whether a grid tile of t points in a list whose far + shell part holds fs_cap
+// records gives each wave a quadrant of its (j, k) range and all of its i (FP32
+// and FP64 grids; otherwise a lane has points tid + 256 q in k-fastest order).
+// The waves' own shell lists hold 16-bit LDS byte offsets into that part.
+__host__ __device__ inline bool quadrant_tile(const int t[3], int ppl, int fs_cap) {
+    return t[0] % ppl == 0 && t[1] % 2 == 0 && t[2] % 2 == 0 &&
+           fs_cap * (int)sizeof(double4) <= 65536;
+}
 // Resident workgroups per CU for (math, ppl, cap).
 int tiles_occupancy(int math, int ppl, int cap);
 

@@ -1210,15 +1210,13 @@ __device__ void grid_tile(const JobDev *__restrict__ J, const int tc[3],
     double px[PPL], py[PPL], pz[PPL], acc[PPL];
     long long oidx[PPL];
     bool ok[PPL];
-    // Quadrant layout (FP32 and FP64 grids, even t1 and t2, t0 divisible by PPL): wave w
-    // owns the (j, k) quadrant (w & 1, w >> 1) of the tile and all of its i;
-    // lane l holds points i = il + q * t0 / PPL.  Otherwise point p = tid +
-    // 256 q of the tile in k-fastest order.
+    // Quadrant layout (see quadrant_tile): wave w owns the (j, k) quadrant
+    // (w & 1, w >> 1) of the tile and all of its i; lane l holds points
+    // i = il + q * t0 / PPL.  Otherwise point p = tid + 256 q of the tile in
+    // k-fastest order.
     const int wave = tid >> 6, lane = tid & 63;
-    // (the wave lists hold 16-bit LDS byte offsets into the far/shell part)
-    const bool quad = (MATH == MATH_MIXED || MATH == MATH_FP64) && t1 % 2 == 0 &&
-                      t2 % 2 == 0 && t0 % PPL == 0 &&
-                      near_region_start<MATH>(cap) * (int)sizeof(double4) <= 65536;
+    const bool quad = (MATH == MATH_MIXED || MATH == MATH_FP64) &&
+                      quadrant_tile(J->tile, PPL, near_region_start<MATH>(cap));
     const int h1 = t1 / 2, h2 = t2 / 2;
 #pragma unroll
     for (int q = 0; q < PPL; ++q) {
@@ -1287,7 +1285,7 @@ __device__ void grid_tile(const JobDev *__restrict__ J, const int tc[3],
         __syncthreads();
     } while (cur_t < J->ntypes);
     if constexpr (MATH == MATH_MIXED && PPL == 2) {
-        if (nodes.value) {  // quadrant layout (8 x 8 x 8 tile)
+        if (nodes.value) {  // 8 x 8 x 8 tile in the quadrant layout (see use_nodes)
             double far[2], *g = reinterpret_cast<double *>(s_list);
             node_energies(nodes, lane >> 4, (wave & 1) * 4 + ((lane >> 2) & 3),
                           (wave >> 1) * 4 + (lane & 3), g, g + 512, far);

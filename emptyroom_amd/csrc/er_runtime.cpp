@@ -568,11 +568,13 @@ double box_radius(const double t[9], const double half[3]) {
 namespace {
 
 // Whether a grid takes the far field of each block of 2 x 2 x 2 tiles from
-// nodes (see grid_block): FP32 grids in the default tile, ...
+// nodes (see grid_block): FP32 grids in the default tile and its quadrant layout
+// (node_energies has its points; lists of more than ~3136 records leave it), ...
 bool use_nodes(const FrameworkDev *fw, const int n[3], const int tile[3], const Tuning &tu,
                int math) {
     if (math != MATH_MIXED || tu.ppl != 2 || tu.cap < 2 * kWG + kNodeRecords ||
-        fw->ntypes > kMaxTypes)
+        fw->ntypes > kMaxTypes ||
+        !quadrant_tile(tile, tu.ppl, mixed_far_shell_cap(tu.cap - kNodeRecords)))
         return false;
     long long blocks = 1;
     double h = 0.0, half[3];
