@@ -140,6 +140,10 @@ struct BinJob {
     long long gblock0;     // first second-step block (one per group) of this job
 };
 
+// Slot `at` of a run that begins at `begin`.  In 64 bits: a job may have 2^32 - 1
+// insertions, and the slots a wave looks at past the end of its last run lie beyond.
+__host__ __device__ inline uint64_t run_slot(uint32_t begin, uint64_t at) { return begin + at; }
+
 // Kernel launch geometry.
 constexpr int kWG = 256;      // threads per workgroup (4 wave64)
 constexpr int kMaxSeg = 64;   // list segments per fill pass

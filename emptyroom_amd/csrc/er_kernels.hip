@@ -380,15 +380,15 @@ __global__ __launch_bounds__(kBinWG) void k_bin_fine(const BinJob *__restrict__ 
     uint2 v[kFinePer];
 #pragma unroll
     for (int q = 0; q < kFinePer; ++q) {
-        const uint32_t e = e0 + (uint32_t)(q * kBinWG + tid);
+        const uint64_t e = run_slot(e0, q * kBinWG + tid);
         v[q] = J.tmp[e < e1 ? e : 0u];
     }
     for (int b = tid; b < nb; b += kBinWG) s_cnt[b] = 0u;
     __syncthreads();
 #pragma unroll
     for (int q = 0; q < kFinePer; ++q)
-        if (e0 + (uint32_t)(q * kBinWG + tid) < e1) atomicAdd(&s_cnt[v[q].x], 1u);
-    for (uint32_t e = e0 + kFinePer * kBinWG + tid; e < e1; e += kBinWG)
+        if (run_slot(e0, q * kBinWG + tid) < e1) atomicAdd(&s_cnt[v[q].x], 1u);
+    for (uint64_t e = run_slot(e0, kFinePer * kBinWG + tid); e < e1; e += kBinWG)
         atomicAdd(&s_cnt[J.tmp[e].x], 1u);
     __syncthreads();
     // exclusive scan of the group's bins: per consecutive counts per thread
@@ -416,9 +416,9 @@ __global__ __launch_bounds__(kBinWG) void k_bin_fine(const BinJob *__restrict__ 
     __syncthreads();
 #pragma unroll
     for (int q = 0; q < kFinePer; ++q)
-        if (e0 + (uint32_t)(q * kBinWG + tid) < e1)
+        if (run_slot(e0, q * kBinWG + tid) < e1)
             J.sorted[atomicAdd(&s_cnt[v[q].x], 1u)] = v[q].y;
-    for (uint32_t e = e0 + kFinePer * kBinWG + tid; e < e1; e += kBinWG) {
+    for (uint64_t e = run_slot(e0, kFinePer * kBinWG + tid); e < e1; e += kBinWG) {
         const uint2 u = J.tmp[e];
         J.sorted[atomicAdd(&s_cnt[u.x], 1u)] = u.y;
     }
@@ -2101,7 +2101,7 @@ __global__ __launch_bounds__(64 * WAVES * PARTS, 4) void k_parts(const JobDev *_
     }
     const bool xl = grid && J->t[3] == 0.0 && J->t[6] == 0.0;
     // (a grid's part is one round; a bin has one for every 512 insertions)
-    for (uint32_t c = s0 + 64u * part; grid || c < s1; c += 512u) {
+    for (uint64_t c = run_slot(s0, 64 * part); grid || c < s1; c += 512) {
         double px[2], py[2], pz[2], acc[2];
         long long at[2];
         bool ok[2];
@@ -2123,7 +2123,7 @@ __global__ __launch_bounds__(64 * WAVES * PARTS, 4) void k_parts(const JobDev *_
                 at[q] = (long long)gk + (long long)gj * J->n[2] +
                         (long long)gi * J->n[1] * J->n[2];
             } else {
-                const uint64_t slot = (uint64_t)c + lane + 256u * q;
+                const uint64_t slot = c + lane + 256 * q;
                 ok[q] = slot < s1;
                 at[q] = J->sorted[ok[q] ? slot : c];
                 double f[3];
