@@ -620,7 +620,12 @@ int Server::fetch_grid(uint64_t ticket, void *host) {
     GridDev *g = r->grid;
     r->fetching++;  // release() waits until this copy is over
     lk.unlock();
-    const hipError_t e = ctx_->transfer->out(host, g->d_data, g->bytes(), fetch_stream_);
+    // (the copy's events belong to the calling thread's current device)
+    int device = ctx_->device;
+    hipError_t e = hipGetDevice(&device);
+    if (e == hipSuccess) e = hipSetDevice(ctx_->device);
+    if (e == hipSuccess) e = ctx_->transfer->out(host, g->d_data, g->bytes(), fetch_stream_);
+    if (device != ctx_->device) (void)hipSetDevice(device);
     lk.lock();
     r->fetching--;
     done_cv_.notify_all();
