@@ -624,7 +624,11 @@ int Server::fetch_grid(uint64_t ticket, void *host) {
     int device = ctx_->device;
     hipError_t e = hipGetDevice(&device);
     if (e == hipSuccess) e = hipSetDevice(ctx_->device);
-    if (e == hipSuccess) e = ctx_->transfer->out(host, g->d_data, g->bytes(), fetch_stream_);
+    try {
+        if (e == hipSuccess) e = ctx_->transfer->out(host, g->d_data, g->bytes(), fetch_stream_);
+    } catch (...) {  // no host memory for the copy's buffers
+        e = hipErrorOutOfMemory;
+    }
     if (device != ctx_->device) (void)hipSetDevice(device);
     lk.lock();
     r->fetching--;

@@ -12,6 +12,7 @@
 #include <cstring>
 #include <map>
 #include <mutex>
+#include <new>
 #include <thread>
 
 using Clock = std::chrono::steady_clock;
@@ -28,7 +29,7 @@ struct Event {
 std::mutex mu;
 std::map<void *, size_t> device_memory;
 size_t device_used = 0, device_limit = (size_t)64 << 30;
-std::atomic<int> kernel_ms{0}, frees{0}, mallocs{0};
+std::atomic<int> kernel_ms{0}, frees{0}, mallocs{0}, host_throws{0};
 thread_local int device = 0;
 Stream *S(hipStream_t s) { return reinterpret_cast<Stream *>(s); }
 Event *E(hipEvent_t e) { return reinterpret_cast<Event *>(e); }
@@ -39,6 +40,7 @@ extern "C" {
 // --- what a test sets and reads ------------------------------------------------
 void fake_kernel_ms(int ms) { kernel_ms = ms; }
 void fake_device_limit(size_t bytes) { device_limit = bytes; }
+void fake_host_malloc_throws(int on) { host_throws = on; }
 size_t fake_device_used() { return device_used; }
 int fake_mallocs() { return mallocs; }
 int fake_frees() { return frees; }
@@ -84,6 +86,7 @@ hipError_t hipFree(void *p) {
     return hipSuccess;
 }
 hipError_t hipHostMalloc(void **p, size_t n, unsigned) {
+    if (host_throws) throw std::bad_alloc();  // as the library's own host memory can
     *p = std::calloc(1, n);
     return *p ? hipSuccess : hipErrorOutOfMemory;
 }

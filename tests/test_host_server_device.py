@@ -1,4 +1,5 @@
-"""The server's grids can be fetched from any thread, whatever its current device.
+"""The server's grids can be fetched from any thread, whatever its current device, and
+after a fetch that failed.
 
 The host code runs against a stand-in of the HIP runtime with two devices
 (tests/host/fake_hip.cpp), which refuses, as HIP does, an event that is recorded on
@@ -40,3 +41,25 @@ def test_fetch_from_a_thread_of_another_device(lib, n):
     srv.release(ticket)
     srv.close(); ctx.close()
     """)
+
+
+def test_fetch_that_runs_out_of_host_memory(lib):
+    """The copy may throw (its buffers are made by the first one); the ticket can
+    then be fetched again and released."""
+    fake.run(lib, """
+    n = (100, 90, 80)
+    ctx = api.Context(0)
+    srv = api.Server(ctx)
+    ticket = srv.submit(*ARGS, grid_n=n)[1]
+    assert srv.poll(ticket, -1.0).state == api.RQ_DONE
+    fake.fake_host_malloc_throws(1)
+    try:
+        srv.fetch_grid(ticket, n)
+        raise SystemExit("fetched")
+    except api.EmptyRoomError as e:
+        print(e)
+    fake.fake_host_malloc_throws(0)
+    assert srv.fetch_grid(ticket, n).shape == n
+    srv.release(ticket)      # waits for copies that have not ended
+    srv.close(); ctx.close()
+    """, timeout=30.0)
