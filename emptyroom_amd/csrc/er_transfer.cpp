@@ -204,6 +204,12 @@ hipError_t Transfer::out(void *host, const void *dev, size_t bytes, hipStream_t 
     }
     Job job(host, bytes);
     Events events;
+    // what the stream still computes is waited for first: the slots belong to every
+    // context of the device, and the helping threads poll
+    if (bytes > kSmall) {
+        const hipError_t e = hipStreamSynchronize(s);
+        if (e != hipSuccess) return e;
+    }
     if (bytes <= kSmall || !lk.try_lock() || !ensure(job.chunks, bytes >= kFreshMin) ||
         !events.make((int)std::min<long>(kSlots, job.chunks))) {
         hipError_t e = hipMemcpyAsync(host, dev, bytes, hipMemcpyDeviceToHost, s);

@@ -13,7 +13,8 @@
 // The contexts of a device share one Transfer (the pinned memory, 18 MiB at
 // most, and the threads are made by the first copy that uses them and given back
 // with the last context).  One copy at a time uses it; a copy that finds it in
-// use takes the runtime's path.
+// use takes the runtime's path.  The ring is taken when the stream has ended what is
+// before the copy, so neither it nor a core is held while a kernel runs.
 #pragma once
 
 #include <hip/hip_runtime.h>

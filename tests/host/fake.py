@@ -32,6 +32,7 @@ def build(folder) -> str:
 def run(lib: str, body: str, timeout: float = 60.0) -> str:
     code = PRELUDE.format(root=ROOT, lib=lib) + textwrap.dedent(body)
     p = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True,
-                       timeout=timeout)
+                       timeout=timeout, env=dict(os.environ, OMP_NUM_THREADS="1",
+                                                 OPENBLAS_NUM_THREADS="1"))
     assert p.returncode == 0, p.stdout[-2000:] + p.stderr[-4000:]
     return p.stdout

@@ -13,6 +13,7 @@
 #include <map>
 #include <mutex>
 #include <new>
+#include <set>
 #include <thread>
 
 using Clock = std::chrono::steady_clock;
@@ -28,8 +29,9 @@ struct Event {
 };
 std::mutex mu;
 std::map<void *, size_t> device_memory;
+std::set<char *> pinned;  // slots of 2 MiB and more
 size_t device_used = 0, device_limit = (size_t)64 << 30;
-std::atomic<int> kernel_ms{0}, frees{0}, mallocs{0}, host_throws{0};
+std::atomic<int> kernel_ms{0}, frees{0}, mallocs{0}, host_throws{0}, ring_copies{0};
 thread_local int device = 0;
 Stream *S(hipStream_t s) { return reinterpret_cast<Stream *>(s); }
 Event *E(hipEvent_t e) { return reinterpret_cast<Event *>(e); }
@@ -42,6 +44,7 @@ void fake_kernel_ms(int ms) { kernel_ms = ms; }
 void fake_device_limit(size_t bytes) { device_limit = bytes; }
 void fake_host_malloc_throws(int on) { host_throws = on; }
 size_t fake_device_used() { return device_used; }
+int fake_ring_copies() { return ring_copies; }  // copies into pinned blocks of 2 MiB
 int fake_mallocs() { return mallocs; }
 int fake_frees() { return frees; }
 
@@ -88,9 +91,16 @@ hipError_t hipFree(void *p) {
 hipError_t hipHostMalloc(void **p, size_t n, unsigned) {
     if (host_throws) throw std::bad_alloc();  // as the library's own host memory can
     *p = std::calloc(1, n);
+    std::lock_guard<std::mutex> lk(mu);
+    if (n == (2u << 20)) pinned.insert((char *)*p);
     return *p ? hipSuccess : hipErrorOutOfMemory;
 }
-hipError_t hipHostFree(void *p) { std::free(p); return hipSuccess; }
+hipError_t hipHostFree(void *p) {
+    std::lock_guard<std::mutex> lk(mu);
+    pinned.erase((char *)p);
+    std::free(p);
+    return hipSuccess;
+}
 hipError_t hipGetSymbolAddress(void **p, const void *) {
     static void *m = std::calloc(1, (size_t)64 << 20);
     *p = m;
@@ -124,6 +134,8 @@ hipError_t hipEventQuery(hipEvent_t e) {
 hipError_t hipEventElapsedTime(float *ms, hipEvent_t, hipEvent_t) { *ms = 0.0f; return hipSuccess; }
 hipError_t hipMemcpyAsync(void *to, const void *from, size_t n, hipMemcpyKind, hipStream_t) {
     std::memcpy(to, from, n);
+    std::lock_guard<std::mutex> lk(mu);
+    if (pinned.count((char *)to)) ring_copies++;
     return hipSuccess;
 }
 
