@@ -156,6 +156,7 @@ constexpr int kBinGroupMax = 15360;  // bins a group may hold (the second step's
 constexpr int kBinLdsKeys = 7168;    // keys a binning block histograms in LDS (28 KiB)
 constexpr int kRegionRecords = 8192;  // entries of one workgroup's region sub-list (near-list
                                       // indices, 32 KiB)
+constexpr int kBlockList = 3072;  // of these, entries of a block's list (see grid_block)
 // Margin (Angstrom) applied to every list classification so that FP64 rounding
 // of radii and distances can never misclassify a pair.
 constexpr double kMargin = 1e-6;

@@ -1388,11 +1388,12 @@ __device__ bool build_region_list(const JobDev *__restrict__ J, double cx, doubl
 // The node sums are flushed twice as often as the points' (at an eighth of the
 // pairs that is free).
 //
-// Returns no nodes if the block's list does not fit blist_cap.
+// Returns no nodes if the block's list does not fit kBlockList entries, which
+// depends on the block alone.
 __device__ BlockNodes grid_block(const JobDev *__restrict__ J, const int b0[3], const int bn[3],
                            const double4 *__restrict__ src, const uint32_t *__restrict__ sidx,
                            const int *__restrict__ tbeg, uint32_t *__restrict__ blist,
-                           int blist_cap, int *__restrict__ bbeg, int cap,
+                           int *__restrict__ bbeg, int cap,
                            double4 *__restrict__ s_list, int *__restrict__ s_seg,
                            int *__restrict__ s_cnt) {
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -1426,35 +1427,44 @@ __device__ BlockNodes grid_block(const JobDev *__restrict__ J, const int b0[3], 
     const bool xl = t[3] == 0.0 && t[6] == 0.0;
     const int ntypes = J->ntypes, end = uniform(tbeg[ntypes]);
     const double reach = (kNodeReach * h) + bs.R + kMargin, reach2 = reach * reach;
-    int nf = 0, nb = 0, first_t = 0, nseg = 0, nt = 0;  // nt: types begun
-    // the far records so far, types first_t .. first_t + nseg - 1, at the nodes
-    auto evaluate = [&]() {
-        if (tid == 0) s_seg[kSegInts * nseg + 1] = nf;
+    // far records and types first_t .. first_t + nseg - 1 in the list; kept records;
+    // types begun (first_t + nseg)
+    int nf = 0, nb = 0, first_t = 0, nseg = 0, nt = 0;
+    // The first `take` far records at the nodes; what is left of the list is moved to
+    // its front.  A pass ends at a number of kept records, not where a chunk of the
+    // source does, so the sums depend on the records alone.
+    auto evaluate = [&](int take) {
+        __syncthreads();
+        int ns = nseg;  // types that begin before `take`
+        while (ns > 1 && uniform(s_seg[kSegInts * (ns - 1) + 1]) >= take) --ns;
+        const int left = nf - take, segs = nseg - ns + 1;
+        const double4 rest = s_list[tid < left ? take + tid : 0];
+        const int begin = tid < segs ? s_seg[kSegInts * (ns - 1 + tid) + 1] - take : 0;
+        __syncthreads();
+        if (tid == 0) s_seg[kSegInts * ns + 1] = take;
         __syncthreads();
         if (xl)
             eval_list<2, MATH_MIXED, true, kFlushPairs / 2>(
-                J, s_list, cap, s_seg, nseg, px, py, pz, acc, bs.R, false,
+                J, s_list, cap, s_seg, ns, px, py, pz, acc, bs.R, false,
                 make_double4(0.0, 0.0, 0.0, 0.0), nullptr, 2);
         else
             eval_list<2, MATH_MIXED, false, kFlushPairs / 2>(
-                J, s_list, cap, s_seg, nseg, px, py, pz, acc, bs.R, false,
+                J, s_list, cap, s_seg, ns, px, py, pz, acc, bs.R, false,
                 make_double4(0.0, 0.0, 0.0, 0.0), nullptr, 2);
         __syncthreads();
+        first_t += ns - 1;
+        if (tid < left) s_list[tid] = rest;
+        if (tid < segs) {
+            s_seg[kSegInts * tid] = first_t + tid;
+            s_seg[kSegInts * tid + 1] = begin > 0 ? begin : 0;
+        }
+        nf = left;
+        nseg = segs;
     };
+    const int pass = cap - kWG;  // far records of a pass; one more chunk fits behind them
     for (int i = tid; i <= kMaxSeg; i += kWG)
         s_seg[kSegInts * i + 2] = s_seg[kSegInts * i + 3] = 0;  // no shell, no near records
     for (int pos = 0; pos < end; pos += kWG) {
-        if (nf + kWG > cap) {
-            evaluate();
-            // the pass that follows begins inside the last type begun
-            nf = 0;
-            first_t = nt - 1;
-            nseg = 1;
-            if (tid == 0) {
-                s_seg[0] = first_t;
-                s_seg[1] = 0;
-            }
-        }
         const int idx = pos + tid;
         int at = 0;
         bool far = false, keep = false;
@@ -1487,7 +1497,7 @@ __device__ BlockNodes grid_block(const JobDev *__restrict__ J, const int b0[3], 
             tk += ck;
         }
         __syncthreads();
-        if (nb + tk > blist_cap) return BlockNodes();  // uniform
+        if (nb + tk > kBlockList) return BlockNodes();  // uniform
         if (far) s_list[of + lanes_below(bf)] = A;
         if (keep) blist[ok + lanes_below(bk)] = (uint32_t)at;
         // types that begin in this chunk
@@ -1504,10 +1514,11 @@ __device__ BlockNodes grid_block(const JobDev *__restrict__ J, const int b0[3], 
         }
         nf = uniform(nf + tf);
         nb = uniform(nb + tk);
+        if (nf >= pass) evaluate(pass);
     }
     for (; nt <= ntypes; ++nt)
         if (tid == 0) bbeg[nt] = nb;
-    evaluate();
+    if (nf > 0) evaluate(nf);
     // the list's last kNodeRecords records hold the values while the block's
     // tiles are computed (with a list shorter by as much)
     double *value = reinterpret_cast<double *>(s_list + cap - kNodeRecords);
@@ -1608,24 +1619,25 @@ __global__ __launch_bounds__(kWG, MATH == MATH_NODES ? 4 : 1) void k_tiles(const
             }
             const double R = (sqrt(r2) + J->cell_R) * (1.0 + 1e-12) + kMargin;
             const double rr = J->rc + R + kMargin;
-            if (build_region_list(J, cx, cy, cz, rr * rr, slice, scratch_cap, s_rbeg, s_cnt)) {
+            const int room = MATH == MATH_NODES ? scratch_cap - kBlockList : scratch_cap;
+            if (build_region_list(J, cx, cy, cz, rr * rr, slice, room, s_rbeg, s_cnt)) {
                 sidx = slice;
                 tbeg = s_rbeg;
             }
         }
         if constexpr (MATH == MATH_NODES) {
-            // regions of a grid with nodes hold whole blocks of 2 x 2 x 2 tiles
-            const int used = sidx ? uniform(tbeg[J->ntypes]) : 0;
+            // regions of a grid with nodes hold whole blocks of 2 x 2 x 2 tiles; a
+            // block's list has the end of the slice
+            uint32_t *const blist = slice + (scratch_cap - kBlockList);
             for (int bi = 0; bi < tn[0]; bi += 2)
                 for (int bj = 0; bj < tn[1]; bj += 2)
                     for (int bk = 0; bk < tn[2]; bk += 2) {
                         const int b0[3] = {t0[0] + bi, t0[1] + bj, t0[2] + bk};
                         const int bn[3] = {bi + 1 < tn[0] ? 2 : 1, bj + 1 < tn[1] ? 2 : 1,
                                            bk + 1 < tn[2] ? 2 : 1};
-                        BlockNodes nodes = grid_block(reread(J), b0, bn, src, sidx, tbeg, slice + used,
-                                                      scratch_cap - used, s_bbeg, cap, s_list,
-                                                      s_seg, s_cnt);
-                        const uint32_t *bidx = nodes.value ? slice + used : sidx;
+                        BlockNodes nodes = grid_block(reread(J), b0, bn, src, sidx, tbeg, blist,
+                                                      s_bbeg, cap, s_list, s_seg, s_cnt);
+                        const uint32_t *bidx = nodes.value ? blist : sidx;
                         const int *bbeg = nodes.value ? s_bbeg : tbeg;
                         for (int ti = 0; ti < bn[0] * bn[1] * bn[2]; ++ti) {
                             const int o0 = ti / (bn[1] * bn[2]), o1 = (ti / bn[2]) % bn[1],
@@ -2459,7 +2471,8 @@ hipError_t launch_tiles(int math, int ppl, const JobDev *jobs, int njobs, long l
         return launch_parts(math, jobs, njobs, total, cap, s);
     if (cap < 2 * kWG || wgs <= 0) return hipErrorInvalidValue;
     if (scratch && scratch_cap < kWG) return hipErrorInvalidValue;
-    if (math == MATH_NODES && (!scratch || cap < 2 * kWG + kNodeRecords))
+    if (math == MATH_NODES &&
+        (!scratch || scratch_cap < kBlockList + kWG || cap < 2 * kWG + kNodeRecords))
         return hipErrorInvalidValue;
 #define ER_TILES(P, M)                                                                     \
     if (ppl == P && math == M)                                                             \

@@ -623,12 +623,11 @@ JobDev make_grid_job(const FrameworkDev *fw, const int n[3], int precision, void
     choose_grid_tile(fw, n, tu, tile);
     j.interp = use_nodes(fw, n, tile, tu, math);
     if (j.interp) {
-        // regions of whole blocks; a slice also holds a block's list, about a
-        // third of its region's
+        // regions of whole blocks; a slice also holds a block's list
         const int block[3] = {2 * tile[0], 2 * tile[1], 2 * tile[2]};
         Tuning shorter = tu;  // a block's own list makes long regions pay less
         shorter.region_len *= 0.75;
-        choose_grid_region(fw, n, block, shorter, region, slice_records * 3 / 4);
+        choose_grid_region(fw, n, block, shorter, region, slice_records - kBlockList);
         for (int d = 0; d < 3; d++) region[d] *= 2;
     } else {
         choose_grid_region(fw, n, tile, tu, region, slice_records);
