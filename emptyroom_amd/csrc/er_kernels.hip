@@ -826,7 +826,7 @@ __device__ __forceinline__ void wave_shell_lists(const JobDev *__restrict__ J,
 //   of the tile): r^2 = |a|^2 + |p|^2 - 2 p.a in FP64 (three FMAs and an add;
 //   |a| <= r_c + R keeps the cancellation below 13x), then in FP32
 //   u = 1/r^2, and per point the sums S3 = sum u^3 and S6 = sum u^6 over at
-//   most FLUSH pairs of one type, flushed into the FP64 energy as
+//   most kFlushPairs pairs of one type, flushed into the FP64 energy as
 //   4 eps (sigma^12 S6 - sigma^6 S3).  sigma and eps stay FP64, so their
 //   rounding adds no error common to every pair of a type.
 //   Shell pairs: the same, behind the strict FP64 test r^2 < r_c^2.
@@ -841,7 +841,7 @@ __device__ __forceinline__ void wave_shell_lists(const JobDev *__restrict__ J,
 // into the wave's own lists of LDS byte offsets wl (wave_shell_lists).
 // phase (wave-uniform): 0 every record, per segment far, shell, near; 1 only
 // the near records; 2 only the far and shell records.
-template <int PPL, int MATH, bool XL, int FLUSH = kFlushPairs, int NEAR = 1>
+template <int PPL, int MATH, bool XL, int NEAR = 1>
 __device__ __forceinline__ void eval_list(const JobDev *__restrict__ J,
                                           const double4 *__restrict__ L, int cap,
                                           const int *__restrict__ seg, int nseg,
@@ -922,14 +922,14 @@ __device__ __forceinline__ void eval_list(const JobDev *__restrict__ J,
                 }
             };
             // far records [fb, fe), then shell records [sb, se): FP32 sums of
-            // FLUSH pairs per point (blocks of 8 unrolled records),
+            // kFlushPairs pairs per point (blocks of 8 unrolled records),
             // then flushed into the FP64 energy
             auto blocks = [&](int b, int e, auto &&pair_at) {
-                for (int r = b; r < e; r += FLUSH) {
+                for (int r = b; r < e; r += kFlushPairs) {
                     float a3[PPL], a6[PPL];
 #pragma unroll
                     for (int q = 0; q < PPL; ++q) a3[q] = a6[q] = 0.0f;
-                    const int re = r + FLUSH < e ? r + FLUSH : e;
+                    const int re = r + kFlushPairs < e ? r + kFlushPairs : e;
 #pragma unroll 1
                     for (int h = r; h < re; h += 8) {
                         if (h + 8 <= re) {
@@ -1276,11 +1276,11 @@ __device__ void grid_tile(const JobDev *__restrict__ J, const int tc[3],
         __syncthreads();
         if (!idle) {
             if (xl)
-                eval_list<PPL, MATH, true, kFlushPairs, 2>(J, s_list, cap, s_seg, nseg, px, py, pz, acc, tl.R, ws,
-                                           wsph, s_wl);
+                eval_list<PPL, MATH, true, 2>(J, s_list, cap, s_seg, nseg, px, py, pz, acc, tl.R,
+                                              ws, wsph, s_wl);
             else
-                eval_list<PPL, MATH, false, kFlushPairs, 2>(J, s_list, cap, s_seg, nseg, px, py, pz, acc, tl.R,
-                                            ws, wsph, s_wl);
+                eval_list<PPL, MATH, false, 2>(J, s_list, cap, s_seg, nseg, px, py, pz, acc, tl.R,
+                                               ws, wsph, s_wl);
         }
         __syncthreads();
     } while (cur_t < J->ntypes);
@@ -1373,8 +1373,8 @@ __device__ bool build_region_list(const JobDev *__restrict__ J, double cx, doubl
 // directly, as without nodes.  Direct tiles are bound by VALU issue (98% of the
 // cycles), and at 0.1 A half of what they issue is for such pairs: a grid of
 // 1.48e7 points and 3000 atoms (0.21 atoms/A^3) issued 5.0e9 wave instructions
-// in 10.3 ms and with nodes 3.5e9 in 7.2 ms (6.8 ms with a cheaper tile setup since);
-// one of 4.9e7 points and 2400 atoms (0.05 atoms/A^3) took 10.6, then 7.8 ms (now 6.4).
+// in 10.3 ms and with nodes 3.5e9 in 7.2 ms (6.9 ms now); one of 4.9e7 points and
+// 2400 atoms (0.05 atoms/A^3) took 10.6, then 7.8 ms (6.7 now).
 //
 // Accuracy: an atom at D from the middle of a segment of half-length h through
 // the box has a Chebyshev interpolation error on it of at most
@@ -1383,10 +1383,10 @@ __device__ bool build_region_list(const JobDev *__restrict__ J, double cx, doubl
 // segment's own axis and 10 to 100 times less elsewhere.  Against direct FP64
 // sums over the far atoms of blocks at 0.1 A (0.12 atoms/A^3, cells of 65 to 112
 // degrees, far fields of 300 to 2000 K): 4e-7 to 3e-6 K rms, 2e-5 K at most,
-// less than the FP32 arithmetic of the same pairs rounds off; the errors of
-// whole grids against the direct method are the same with and without nodes.
-// The node sums are flushed twice as often as the points' (at an eighth of the
-// pairs that is free).
+// less than the FP32 arithmetic of the same pairs rounds off.  The nodes' pairs are
+// evaluated in FP64 like those of an FP64 grid: interpolated FP32 sums were up to 8%
+// further off (rms) than direct tiles, FP64 ones are 8 to 40% nearer
+// (|E| < 1000 K, 0.07 to 0.12 A), for 2 to 3% of the grid's time.
 //
 // Returns no nodes if the block's list does not fit kBlockList entries, which
 // depends on the block alone.
@@ -1444,13 +1444,9 @@ __device__ BlockNodes grid_block(const JobDev *__restrict__ J, const int b0[3], 
         if (tid == 0) s_seg[kSegInts * ns + 1] = take;
         __syncthreads();
         if (xl)
-            eval_list<2, MATH_MIXED, true, kFlushPairs / 2>(
-                J, s_list, cap, s_seg, ns, px, py, pz, acc, bs.R, false,
-                make_double4(0.0, 0.0, 0.0, 0.0), nullptr, 2);
+            eval_list<2, MATH_FP64, true>(J, s_list, cap, s_seg, ns, px, py, pz, acc, bs.R);
         else
-            eval_list<2, MATH_MIXED, false, kFlushPairs / 2>(
-                J, s_list, cap, s_seg, ns, px, py, pz, acc, bs.R, false,
-                make_double4(0.0, 0.0, 0.0, 0.0), nullptr, 2);
+            eval_list<2, MATH_FP64, false>(J, s_list, cap, s_seg, ns, px, py, pz, acc, bs.R);
         __syncthreads();
         first_t += ns - 1;
         if (tid < left) s_list[tid] = rest;
