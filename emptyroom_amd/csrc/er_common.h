@@ -94,8 +94,10 @@ struct JobDev {
     void *out;          // float*, double* or uint32_t* by mode; index k + j*nz + i*ny*nz
     // Widom
     int nbins[3];       // insertion bins per fractional axis
-    int parts;          // > 0: waves that share the points of one (see k_parts); an item is a
-                        // quarter of a cell, or with 2 a cell
+    int parts;          // > 0: an energy is summed in so many parts (see eval_range)
+    int shared;         // with parts: they are shared out to waves (see k_parts), and an
+                        // item is a quarter of a cell, or with 2 parts a cell
+    int pad0;
     const uint32_t *sorted;     // insertion indices ordered by bin
     const uint32_t *bin_start;  // nbins_total + 1 offsets into sorted
     uint64_t seed;
@@ -166,8 +168,10 @@ constexpr double kNodeReach = 8.0;  // far atoms of a block lie at least this ma
 constexpr int kNodeRecords = kNodes * kNodes * kNodes * 8 / 32;  // LDS records the values take
 constexpr long long kNodeMinBlocks = 1024;  // see use_nodes
 constexpr double kNodeMinFar = 120.0;
-// cells up to which the points of a wave are shared by eight / four / two waves
+// cells up to which the points of a wave are shared by eight / four / two waves; waves
+// up to which jobs of a batch do so (see batch_create)
 constexpr long long kPartCells8 = 128, kPartCells4 = 320, kPartCells2 = 512;
+constexpr double kPartWaves = 1900.0;
 constexpr long long kMinGridItems = 2048;  // regions per grid before regions shrink
 
 }  // namespace er

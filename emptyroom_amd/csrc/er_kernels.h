@@ -12,14 +12,17 @@ namespace er {
 
 // Pair-math variants of the tiled energy kernel.
 // (MATH_NODES: FP32 grids whose blocks of tiles take their far field from nodes)
-// (MATH_PARTS*: small jobs, the points of a wave shared by eight, four or two waves)
+// (MATH_PARTS*: small jobs, the points of a wave shared by eight, four or two waves;
+// MATH_IN_PARTS*: the same jobs in company, the same sums by one wave)
 enum Math : int { MATH_MIXED = 0, MATH_FP64 = 1, MATH_COUNT = 2, MATH_OVERLAP = 3,
                   MATH_NODES = 4, MATH_PARTS8 = 5, MATH_PARTS8_FP64 = 6, MATH_PARTS4 = 7,
-                  MATH_PARTS4_FP64 = 8, MATH_PARTS2 = 9, MATH_PARTS2_FP64 = 10 };
+                  MATH_PARTS4_FP64 = 8, MATH_PARTS2 = 9, MATH_PARTS2_FP64 = 10, MATH_IN_PARTS = 11,
+                  MATH_IN_PARTS_FP64 = 12 };
 
 // The variant that computes a grid or Widom job.
 inline int job_math(const JobDev &j) {
     const bool fp64 = j.kind == JOB_GRID && j.mode == OUT_F64;
+    if (j.parts && !j.shared) return fp64 ? MATH_IN_PARTS_FP64 : MATH_IN_PARTS;
     if (j.parts == 8) return fp64 ? MATH_PARTS8_FP64 : MATH_PARTS8;
     if (j.parts == 4) return fp64 ? MATH_PARTS4_FP64 : MATH_PARTS4;
     if (j.parts == 2) return fp64 ? MATH_PARTS2_FP64 : MATH_PARTS2;

@@ -26,6 +26,7 @@
 #include "er_kernels.h"
 
 #include <float.h>
+#include <limits.h>
 
 #include <type_traits>
 
@@ -820,6 +821,101 @@ __device__ __forceinline__ void wave_shell_lists(const JobDev *__restrict__ J,
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
+// ---- sums in parts ----------------------------------------------------------
+//
+// Jobs of few cells (JobDev::parts) sum an energy in parts, so that several waves
+// can share a point's records (k_parts) and one wave can make the same sum, to the
+// bit, where the device is full without that (k_tiles).  The records of a pass form
+// groups of one segment and kind: 16 far or shell records (the FP32 sums' groups), 8
+// near ones.  Part v of `parts` has the groups [v G / parts, (v + 1) G / parts) of the
+// pass's G, and a pass adds its parts in order.  A grid's groups are numbered segment
+// by segment.  A Widom pass has its near groups first, in parts of their own, so that
+// saturated insertions can stop before the others.
+constexpr int kNearGroup = 8;
+constexpr int kShellGroup = kFlushPairs;
+
+__device__ __forceinline__ int groups_of(int n, int size) { return (n + size - 1) / size; }
+
+__device__ __forceinline__ int part_begin(int v, int groups, int parts) {
+    return (v * groups) >> (parts == 8 ? 3 : parts == 4 ? 2 : 1);
+}
+
+// Groups of a pass: near ones (x) and others (y).  wn(s): segment s's wave-far and
+// (high half) wave-shell records, or just its shell records.
+template <class WN>
+__device__ __forceinline__ int2 count_groups(const int *__restrict__ seg, int nseg, WN wn) {
+    int2 n = make_int2(0, 0);
+    for (int s = 0; s < nseg; ++s) {
+        const int *g = seg + kSegInts * s;
+        const int w = wn(s);
+        n.x += groups_of(uniform(g[kSegInts + 3]) - uniform(g[3]), kNearGroup);
+        n.y += groups_of(uniform(g[kSegInts + 1]) - uniform(g[1]), kShellGroup) +
+               groups_of(w & 0xffff, kShellGroup) + groups_of(w >> 16, kShellGroup);
+    }
+    return make_int2(uniform(n.x), uniform(n.y));
+}
+
+// What eval_list does about parts: nothing, ...
+struct NoParts {
+    static constexpr bool on = false, one = false;
+};
+
+// ... sums them one after the other: e, the energies of the current part, is added to
+// sum where the next part begins, ...  (u, v and next are wave-uniform, which the
+// compiler does not see by itself: 5% of the kernel's VALU instructions.)
+template <int P>
+struct PartSums {
+    static constexpr bool on = true, one = false;
+    double (&sum)[P];
+    int groups, parts;
+    int u = 0, v = 0, next = 0;  // next group, next part, its first group
+    __device__ __forceinline__ PartSums(double (&s)[P], int g, int p) : sum(s), groups(g), parts(p) {}
+    __device__ __forceinline__ bool ended() const { return uniform(u) == uniform(next); }
+    // up to n groups of one part begin here
+    __device__ __forceinline__ int run(double (&e)[P], int n) {
+        u = uniform(u);
+        next = uniform(next);
+        if (u == next) {
+            flush(e);
+            v = uniform(v);
+            while (next <= u) next = part_begin(++v, groups, parts);
+        }
+        const int r = n < next - u ? n : next - u;
+        u += r;
+        return r;
+    }
+    __device__ __forceinline__ void flush(double (&e)[P]) {
+#pragma unroll
+        for (int q = 0; q < P; ++q) {
+            sum[q] += e[q];
+            e[q] = 0.0;
+        }
+    }
+};
+
+// ... or makes one of them, the groups [lo, hi).
+struct OnePart {
+    static constexpr bool on = true, one = true;
+    int lo, hi;
+    int u = 0;
+    __device__ __forceinline__ OnePart(int v, int groups, int parts)
+        : lo(part_begin(v, groups, parts)), hi(part_begin(v + 1, groups, parts)) {}
+    // whether the next n groups are not the part's
+    __device__ __forceinline__ bool skip(int n) {
+        if (u + n > lo && u < hi) return false;
+        u = uniform(u + n);
+        return true;
+    }
+    // records [b, e) in groups of `size`: those of the part
+    __device__ __forceinline__ void clip(int &b, int &e, int size) {
+        const int count = groups_of(e - b, size);
+        const int first = lo > u ? lo - u : 0, end = hi - u < count ? hi - u : count;
+        u = uniform(u + count);
+        if (end < count) e = b + size * (end > 0 ? end : 0);
+        b += size * first;
+    }
+};
+
 // Energies (or in-cutoff counts) of this lane's PPL points against the LDS
 // list.  Points and records are relative to the tile centre c.
 //   Far pairs (inside r_c and beyond the FP64 switch radius for every point
@@ -841,7 +937,9 @@ __device__ __forceinline__ void wave_shell_lists(const JobDev *__restrict__ J,
 // into the wave's own lists of LDS byte offsets wl (wave_shell_lists).
 // phase (wave-uniform): 0 every record, per segment far, shell, near; 1 only
 // the near records; 2 only the far and shell records.
-template <int PPL, int MATH, bool XL, int NEAR = 1>
+// pb: see "sums in parts".  With parts the wave's shell lists are there already, a
+// segment's at its shell offset, and lane s of `lengths` holds their lengths.
+template <int PPL, int MATH, bool XL, int NEAR = 1, class PB = NoParts>
 __device__ __forceinline__ void eval_list(const JobDev *__restrict__ J,
                                           const double4 *__restrict__ L, int cap,
                                           const int *__restrict__ seg, int nseg,
@@ -849,7 +947,8 @@ __device__ __forceinline__ void eval_list(const JobDev *__restrict__ J,
                                           const double (&pz)[PPL], double (&acc)[PPL],
                                           double R, bool ws = false,
                                           double4 wsph = make_double4(0.0, 0.0, 0.0, 0.0),
-                                          uint16_t *__restrict__ wl = nullptr, int phase = 0) {
+                                          uint16_t *__restrict__ wl = nullptr, int phase = 0,
+                                          PB pb = PB(), int lengths = 0) {
     const bool do_fs = phase != 1, do_near = phase != 2;
     const bool clamp = MATH == MATH_MIXED && do_near && uniform(seg[kSegInts * nseg]) != 0;
     const double rc2 = J->rc2, min_r2 = J->min_r2;
@@ -871,6 +970,13 @@ __device__ __forceinline__ void eval_list(const JobDev *__restrict__ J,
         const int sb = uniform(g[2]), se = uniform(g[kSegInts + 2]);
         const int nb = uniform(g[3]), ne = uniform(g[kSegInts + 3]);
         if (fe - fb + se - sb + ne - nb == 0) continue;
+        if constexpr (PB::one) {
+            const int w = ws ? __builtin_amdgcn_readlane(lengths, s) : (se - sb) << 16;
+            const int fs = groups_of(fe - fb, kShellGroup) + groups_of(w & 0xffff, kShellGroup) +
+                           groups_of(w >> 16, kShellGroup);
+            if (pb.skip((do_fs ? fs : 0) + (do_near ? groups_of(ne - nb, kNearGroup) : 0)))
+                continue;
+        }
         const TypeParams P = J->types[t];
         if (MATH == MATH_OVERLAP) {
             // src/computegridsheet.h:154: overlap iff r^2 < sigma_ij^2 (every
@@ -925,7 +1031,9 @@ __device__ __forceinline__ void eval_list(const JobDev *__restrict__ J,
             // kFlushPairs pairs per point (blocks of 8 unrolled records),
             // then flushed into the FP64 energy
             auto blocks = [&](int b, int e, auto &&pair_at) {
+                if constexpr (PB::one) pb.clip(b, e, kShellGroup);
                 for (int r = b; r < e; r += kFlushPairs) {
+                    if constexpr (PB::on && !PB::one) pb.run(acc, 1);
                     float a3[PPL], a6[PPL];
 #pragma unroll
                     for (int q = 0; q < PPL; ++q) a3[q] = a6[q] = 0.0f;
@@ -950,17 +1058,25 @@ __device__ __forceinline__ void eval_list(const JobDev *__restrict__ J,
                 });
             if (!do_fs) {
             } else if (ws) {
-                int nwf, nws;
-                wave_shell_lists(J, Ls, capA, capA, sb, se, wsph, wl, nwf, nws);
+                int nwf, nws, first = 0, last = capA - 1;  // (entries of wl)
+                if constexpr (PB::on) {
+                    const int w = __builtin_amdgcn_readlane(lengths, s);
+                    nwf = w & 0xffff;
+                    nws = w >> 16;
+                    first = sb;
+                    last = se - 1;
+                } else {
+                    wave_shell_lists(J, Ls, capA, capA, sb, se, wsph, wl, nwf, nws);
+                }
                 const char *__restrict__ Lb = reinterpret_cast<const char *>(L);
                 auto rec = [&](int e) {
                     return *reinterpret_cast<const double4 *>(Lb + wl[e]);
                 };
                 blocks(0, nwf, [&](int e, float (&s3)[PPL], float (&s6)[PPL]) {
-                    far_pair(rec(e), s3, s6);
+                    far_pair(rec(first + e), s3, s6);
                 });
                 blocks(0, nws, [&](int e, float (&s3)[PPL], float (&s6)[PPL]) {
-                    shell_pair(rec(capA - 1 - e), s3, s6);
+                    shell_pair(rec(last - e), s3, s6);
                 });
             } else {
                 blocks(sb, se, [&](int k, float (&s3)[PPL], float (&s6)[PPL]) {
@@ -974,8 +1090,6 @@ __device__ __forceinline__ void eval_list(const JobDev *__restrict__ J,
             // reciprocal and one Newton step (~1e-14 relative), and FP64 sums
             // of u^3 and u^6 scaled by 4 eps sigma^6 / sigma^12 per segment.
             double b3[PPL], b6[PPL];
-#pragma unroll
-            for (int q = 0; q < PPL; ++q) b3[q] = b6[q] = 0.0;
             // A near record lies within r_FP64 + R of the tile centre, so
             // within r_FP64 + 2R of every point: when that is inside r_c the
             // strict cutoff test (src/computegridsheet.h:79) passes for every
@@ -985,7 +1099,7 @@ __device__ __forceinline__ void eval_list(const JobDev *__restrict__ J,
             // the clamp two points take 27 instead of 30 VALU instructions a record.
             // Grid tiles have NEAR = 2 records in flight (4.9e7 points, 2400 atoms: 6.48 ms
             // with one, 6.37 with two); bins one (a Henry run of 1.7e7: 2.11, 2.15 ms).
-            auto near_pairs = [&](auto clamp, auto test) {
+            auto near_pairs = [&](int nb, int ne, auto clamp, auto test) {
 #pragma unroll NEAR
                 for (int k = nb; k < ne; ++k) {
                     double r2[PPL];
@@ -1005,11 +1119,26 @@ __device__ __forceinline__ void eval_list(const JobDev *__restrict__ J,
             };
             using no = std::integral_constant<bool, false>;
             using yes = std::integral_constant<bool, true>;
-            if (!all_in) near_pairs(yes(), yes());
-            else if (clamp) near_pairs(yes(), no());
-            else near_pairs(no(), no());
+            auto near_run = [&](int nb, int ne) {
 #pragma unroll
-            for (int q = 0; q < PPL; ++q) acc[q] = fma(c6, b6[q], fma(c3, b3[q], acc[q]));
+                for (int q = 0; q < PPL; ++q) b3[q] = b6[q] = 0.0;
+                if (!all_in) near_pairs(nb, ne, yes(), yes());
+                else if (clamp) near_pairs(nb, ne, yes(), no());
+                else near_pairs(nb, ne, no(), no());
+#pragma unroll
+                for (int q = 0; q < PPL; ++q) acc[q] = fma(c6, b6[q], fma(c3, b3[q], acc[q]));
+            };
+            if constexpr (PB::on && !PB::one) {
+                for (int k = nb; k < ne;) {
+                    const int e = k + kNearGroup * pb.run(acc, groups_of(ne - k, kNearGroup));
+                    near_run(k, e < ne ? e : ne);
+                    k = e;
+                }
+            } else {
+                int b = nb, e = ne;
+                if constexpr (PB::one) pb.clip(b, e, kNearGroup);
+                near_run(b, e);
+            }
             continue;
         }
         // FP64 grids: every pair in FP64.  The expanded FP64 r^2 of the near
@@ -1046,54 +1175,96 @@ __device__ __forceinline__ void eval_list(const JobDev *__restrict__ J,
         };
         using no = std::integral_constant<bool, false>;
         using yes = std::integral_constant<bool, true>;
-        // (two records in flight: a 173^3-point grid of 424 atoms takes 745 us with one,
+        auto scale = [&]() {
+#pragma unroll
+            for (int q = 0; q < PPL; ++q) {
+                acc[q] = fma(c6, b6[q], fma(c3, b3[q], acc[q]));
+                b3[q] = b6[q] = 0.0;
+            }
+        };
+        // a run of records of one kind, in parts if the sums are
+        auto run = [&](int n, auto group, auto &&add) {
+            constexpr int G = decltype(group)::value;
+            if constexpr (PB::on && !PB::one) {
+                for (int k = 0; k < n;) {
+                    if (pb.ended()) scale();
+                    const int e = k + G * pb.run(acc, groups_of(n - k, G));
+                    add(k, e < n ? e : n);
+                    k = e;
+                }
+            } else {
+                int b = 0, e = n;
+                if constexpr (PB::one) pb.clip(b, e, G);
+                add(b, e);
+            }
+        };
+        using shells = std::integral_constant<int, kShellGroup>;
+        // (NEAR records in flight: a 173^3-point grid of 424 atoms takes 745 us with one,
         // 662 with two, 663 with four)
-#pragma unroll 2
-        for (int k = fb; k < fe; ++k) fp64_pair(L[k], no(), no());
+        run(fe - fb, shells(), [&](int b, int e) {
+#pragma unroll NEAR
+            for (int k = b; k < e; ++k) fp64_pair(L[fb + k], no(), no());
+        });
         // wave lists of an FP64 tile hold as many entries as an FP32 tile's
         // (the far + shell part of the FP32 list), which keeps four
         // workgroups per CU; a segment with more shell records than that
         // takes the tile-level path
         const int wcap = mixed_far_shell_cap(cap);
-        if (ws && se - sb <= wcap) {
+        if (ws && (PB::on || se - sb <= wcap)) {
             // shell records against the wave's own sphere (as for FP32
             // grids): wave-far ones need no cutoff test, those beyond r_c of
             // every point of the wave contribute exactly 0 and are skipped
-            int nwf, nws;
-            wave_shell_lists(J, Ls, capA, wcap, sb, se, wsph, wl, nwf, nws);
+            int nwf, nws, first = 0, last = wcap - 1;  // (entries of wl)
+            if constexpr (PB::on) {
+                const int w = __builtin_amdgcn_readlane(lengths, s);
+                nwf = w & 0xffff;
+                nws = w >> 16;
+                first = sb;
+                last = se - 1;
+            } else {
+                wave_shell_lists(J, Ls, capA, wcap, sb, se, wsph, wl, nwf, nws);
+            }
             const char *__restrict__ Lb = reinterpret_cast<const char *>(L);
-#pragma unroll 2
-            for (int e = 0; e < nwf; ++e)
-                fp64_pair(*reinterpret_cast<const double4 *>(Lb + wl[e]), no(), no());
-#pragma unroll 2
-            for (int e = 0; e < nws; ++e)
-                fp64_pair(*reinterpret_cast<const double4 *>(Lb + wl[wcap - 1 - e]), no(), yes());
+            run(nwf, shells(), [&](int b, int e) {
+#pragma unroll NEAR
+                for (int k = b; k < e; ++k)
+                    fp64_pair(*reinterpret_cast<const double4 *>(Lb + wl[first + k]), no(), no());
+            });
+            run(nws, shells(), [&](int b, int e) {
+#pragma unroll NEAR
+                for (int k = b; k < e; ++k)
+                    fp64_pair(*reinterpret_cast<const double4 *>(Lb + wl[last - k]), no(), yes());
+            });
         } else {
-            for (int k = sb; k < se; ++k) fp64_pair(Ls[-k], no(), yes());
+            run(se - sb, shells(), [&](int b, int e) {
+                for (int k = b; k < e; ++k) fp64_pair(Ls[-(sb + k)], no(), yes());
+            });
         }
         // Near records (an atom within R of the tile centre, where a grid
         // point may sit on the atom): r^2 from the FP64 differences, as
         // src/computegridsheet.h:71-75 forms it, so that a point on an atom
         // gives exactly 0 and the reference's clamp (the expanded form would
         // leave a rounding residue of either sign there).
-        for (int k = nb; k < ne; ++k) {
-            const double4 A = Ln[k];
+        run(ne - nb, std::integral_constant<int, kNearGroup>(), [&](int b, int e) {
+            for (int k = nb + b; k < nb + e; ++k) {
+                const double4 A = Ln[k];
 #pragma unroll
-            for (int q = 0; q < PPL; ++q) {
-                const double dx = px[q] - A.x, dy = py[q] - A.y, dz = pz[q] - A.z;
-                const double rr = fmax(dx * dx + dy * dy + dz * dz, min_r2);  // :77
-                double y = (double)__builtin_amdgcn_rcpf((float)rr);
-                y = fma(fma(-rr, y, 1.0), y, y);
-                y = fma(fma(-rr, y, 1.0), y, y);
-                double y3 = y * y * y;
-                y3 = rr < rc2 ? y3 : 0.0;  // src/computegridsheet.h:79
-                b3[q] += y3;
-                b6[q] = fma(y3, y3, b6[q]);
+                for (int q = 0; q < PPL; ++q) {
+                    const double dx = px[q] - A.x, dy = py[q] - A.y, dz = pz[q] - A.z;
+                    const double rr = fmax(dx * dx + dy * dy + dz * dz, min_r2);  // :77
+                    double y = (double)__builtin_amdgcn_rcpf((float)rr);
+                    y = fma(fma(-rr, y, 1.0), y, y);
+                    y = fma(fma(-rr, y, 1.0), y, y);
+                    double y3 = y * y * y;
+                    y3 = rr < rc2 ? y3 : 0.0;  // src/computegridsheet.h:79
+                    b3[q] += y3;
+                    b6[q] = fma(y3, y3, b6[q]);
+                }
             }
-        }
-#pragma unroll
-        for (int q = 0; q < PPL; ++q) acc[q] = fma(c6, b6[q], fma(c3, b3[q], acc[q]));
+        });
+        scale();
     }
+    if constexpr (PB::on && !PB::one) pb.flush(acc);
 }
 
 // ---- far field of a block of tiles from nodes -------------------------------
@@ -1187,7 +1358,8 @@ __device__ __forceinline__ void node_energies(const BlockNodes &bn, int il, int 
 
 // Energies of one grid tile (tile coordinates tc), candidates streamed from
 // src / tbeg (the framework's near list, or a region's sub-list of it).
-template <int PPL, int MATH>
+// (PARTS: sums in parts, see there; such jobs have the quadrant layout)
+template <int PPL, int MATH, bool PARTS = false>
 __device__ void grid_tile(const JobDev *__restrict__ J, const int tc[3],
                           const double4 *__restrict__ src, const uint32_t *__restrict__ sidx,
                           const int *__restrict__ tbeg, int cap,
@@ -1274,7 +1446,37 @@ __device__ void grid_tile(const JobDev *__restrict__ J, const int tc[3],
         const int nseg =
             fill_list<MATH, kWG>(J, src, sidx, tbeg, tl, cur_t, cur_pos, cap, s_list, s_seg, s_cnt);
         __syncthreads();
-        if (!idle) {
+        if constexpr (PARTS) {
+            // the wave's shell lists of every segment, their lengths in lane s
+            const int capA = near_region_start<MATH>(cap);
+            int lengths = 0;
+            for (int s = 0; s < nseg && !idle; ++s) {
+                const int sb = uniform(s_seg[kSegInts * s + 2]),
+                          se = uniform(s_seg[kSegInts * (s + 1) + 2]);
+                int nwf = 0, nws = 0;
+                if (se > sb)
+                    wave_shell_lists(J, s_list + capA - 1, capA, se - sb, sb, se, wsph,
+                                     s_wl + sb, nwf, nws);
+                if (lane == s) lengths = nwf | nws << 16;
+            }
+            const int2 groups = count_groups(s_seg, nseg, [&](int s) {
+                return __builtin_amdgcn_readlane(lengths, s);
+            });
+            double e[PPL], sum[PPL];
+#pragma unroll
+            for (int q = 0; q < PPL; ++q) e[q] = sum[q] = 0.0;
+            const PartSums<PPL> pb(sum, groups.x + groups.y, uniform(J->parts));
+            if (idle) {
+            } else if (xl) {
+                eval_list<PPL, MATH, true, 2>(J, s_list, cap, s_seg, nseg, px, py, pz, e, tl.R, ws,
+                                              wsph, s_wl, 0, pb, lengths);
+            } else {
+                eval_list<PPL, MATH, false, 2>(J, s_list, cap, s_seg, nseg, px, py, pz, e, tl.R,
+                                               ws, wsph, s_wl, 0, pb, lengths);
+            }
+#pragma unroll
+            for (int q = 0; q < PPL; ++q) acc[q] += sum[q];
+        } else if (!idle) {
             if (xl)
                 eval_list<PPL, MATH, true, 2>(J, s_list, cap, s_seg, nseg, px, py, pz, acc, tl.R,
                                               ws, wsph, s_wl);
@@ -1444,9 +1646,9 @@ __device__ BlockNodes grid_block(const JobDev *__restrict__ J, const int b0[3], 
         if (tid == 0) s_seg[kSegInts * ns + 1] = take;
         __syncthreads();
         if (xl)
-            eval_list<2, MATH_FP64, true>(J, s_list, cap, s_seg, ns, px, py, pz, acc, bs.R);
+            eval_list<2, MATH_FP64, true, 2>(J, s_list, cap, s_seg, ns, px, py, pz, acc, bs.R);
         else
-            eval_list<2, MATH_FP64, false>(J, s_list, cap, s_seg, ns, px, py, pz, acc, bs.R);
+            eval_list<2, MATH_FP64, false, 2>(J, s_list, cap, s_seg, ns, px, py, pz, acc, bs.R);
         __syncthreads();
         first_t += ns - 1;
         if (tid < left) s_list[tid] = rest;
@@ -1527,12 +1729,17 @@ __device__ BlockNodes grid_block(const JobDev *__restrict__ J, const int b0[3], 
     return nodes;
 }
 
-template <int PPL, int MATH>
-__global__ __launch_bounds__(kWG, MATH == MATH_NODES ? 4 : 1) void k_tiles(const JobDev *__restrict__ jobs, int njobs,
-                                               long long total_items,
-                                               unsigned long long *__restrict__ counter,
-                                               int cap, uint32_t *__restrict__ scratch,
-                                               int scratch_cap) {
+constexpr bool parts_math(int math) { return math == MATH_IN_PARTS || math == MATH_IN_PARTS_FP64; }
+
+template <int PPL, int VARIANT>
+__global__ __launch_bounds__(kWG, VARIANT == MATH_NODES || parts_math(VARIANT) ? 4 : 1)
+void k_tiles(const JobDev *__restrict__ jobs, int njobs, long long total_items,
+             unsigned long long *__restrict__ counter, int cap, uint32_t *__restrict__ scratch,
+             int scratch_cap) {
+    constexpr bool PARTS = parts_math(VARIANT);
+    constexpr int MATH = VARIANT == MATH_IN_PARTS        ? MATH_MIXED
+                         : VARIANT == MATH_IN_PARTS_FP64 ? MATH_FP64
+                                                         : VARIANT;
     extern __shared__ double4 s_list[];
     __shared__ int s_seg[kSegInts * (kMaxSeg + 1)];
     __shared__ int s_cnt[7 * (kWG / 64)];  // fill: 3 counts + 4 stop fields per wave
@@ -1543,7 +1750,8 @@ __global__ __launch_bounds__(kWG, MATH == MATH_NODES ? 4 : 1) void k_tiles(const
         scratch ? scratch + (size_t)blockIdx.x * (size_t)scratch_cap : nullptr;
     // per-wave shell offset lists after the LDS list (FP32 and FP64 grids)
     uint16_t *__restrict__ s_wl = (MATH == MATH_MIXED || MATH == MATH_FP64 || MATH == MATH_NODES)
-        ? reinterpret_cast<uint16_t *>(s_list + cap) + (tid >> 6) * mixed_far_shell_cap(cap)
+        ? reinterpret_cast<uint16_t *>(s_list + cap) +
+              (tid >> 6) * (PARTS ? near_region_start<MATH>(cap) : mixed_far_shell_cap(cap))
         : nullptr;
 
     for (;;) {
@@ -1652,7 +1860,8 @@ __global__ __launch_bounds__(kWG, MATH == MATH_NODES ? 4 : 1) void k_tiles(const
             int tc[3];
             cell_of(ti, tc);
             if (grid) {
-                grid_tile<PPL, MATH>(J, tc, src, sidx, tbeg, cap, s_list, s_seg, s_cnt, s_wl);
+                grid_tile<PPL, MATH, PARTS>(J, tc, src, sidx, tbeg, cap, s_list, s_seg, s_cnt,
+                                            s_wl);
                 continue;
             }
             // ---- one Widom bin: every insertion whose point falls in it ----
@@ -1697,12 +1906,35 @@ __global__ __launch_bounds__(kWG, MATH == MATH_NODES ? 4 : 1) void k_tiles(const
                     return __all(all) != 0;
                 };
                 if (sat && !first && saturated(lb_near + lb_fs + lb_later)) return false;
-                eval_list<P, MATH, false>(J, s_list, cap, s_seg, nseg, px, py, pz, acc, tl.R,
-                                          false, make_double4(0.0, 0.0, 0.0, 0.0), nullptr, 1);
-                if (!(sat && saturated(lb_fs + lb_later)))
-                    eval_list<P, MATH, false>(J, s_list, cap, s_seg, nseg, px, py, pz, acc,
-                                              tl.R, false, make_double4(0.0, 0.0, 0.0, 0.0),
-                                              nullptr, 2);
+                if constexpr (PARTS) {
+                    auto wn = [&](int s) {
+                        return (uniform(s_seg[kSegInts * (s + 1) + 2]) -
+                                uniform(s_seg[kSegInts * s + 2])) << 16;
+                    };
+                    // (e: the current part, zero again after each call)
+                    double e[P];
+#pragma unroll
+                    for (int q = 0; q < P; ++q) e[q] = 0.0;
+                    const int parts = uniform(J->parts);
+                    const int2 groups = count_groups(s_seg, nseg, wn);
+                    eval_list<P, MATH, false>(
+                        J, s_list, cap, s_seg, nseg, px, py, pz, e, tl.R, false,
+                        make_double4(0.0, 0.0, 0.0, 0.0), nullptr, 1,
+                        PartSums<P>(acc, groups.x, parts));
+                    if (!(sat && saturated(lb_fs + lb_later)))
+                        eval_list<P, MATH, false>(
+                            J, s_list, cap, s_seg, nseg, px, py, pz, e, tl.R, false,
+                            make_double4(0.0, 0.0, 0.0, 0.0), nullptr, 2,
+                            PartSums<P>(acc, groups.y, parts));
+                } else {
+                    eval_list<P, MATH, false>(J, s_list, cap, s_seg, nseg, px, py, pz, acc, tl.R,
+                                              false, make_double4(0.0, 0.0, 0.0, 0.0), nullptr,
+                                              1);
+                    if (!(sat && saturated(lb_fs + lb_later)))
+                        eval_list<P, MATH, false>(J, s_list, cap, s_seg, nseg, px, py, pz, acc,
+                                                  tl.R, false, make_double4(0.0, 0.0, 0.0, 0.0),
+                                                  nullptr, 2);
+                }
 #pragma unroll
                 for (int q = 0; q < P; ++q) out[q] = first ? acc[q] : prev[q] + acc[q];
                 return true;
@@ -1858,185 +2090,25 @@ __global__ __launch_bounds__(kWG, MATH == MATH_NODES ? 4 : 1) void k_tiles(const
 // wave on a SIMD to wait for every LDS read and every FP64 result.  Such jobs
 // (JobDev::parts) give each cell four workgroups of eight waves, or of four when
 // the device would not hold them all at once.  A workgroup has the 128 points of
-// one wave of grid_tile or of a bin (two per lane), makes the same lists, and its
-// waves share the records out: group g of 16 far or shell records (the FP32 sums'
-// groups, so every FP32 sum is the same) or of 8 near records goes to wave g mod
-// WAVES, and the waves' FP64 energies are added in order at the end.  For grids up
+// one wave of grid_tile or of a bin (two per lane), makes the same lists, and each
+// of its waves makes one part of a pass's sums (see "sums in parts").  For grids up
 // to twice as many cells as CUs a workgroup of eight waves has a whole cell, two
-// waves for each of its four parts, which share the list: up to four waves on a
+// waves for each of its four quarters, which share the list: up to four waves on a
 // SIMD instead of two, in one round.
 //
-// us a call, one workgroup per cell / eight waves / four waves: FP32 grid of 8
-// cells, 400 atoms 114 / 54 / 65, 64 cells 85 / 46 / 56, 216 cells 80 / 77 / 65,
-// 343 cells 87 / - / 88; Henry run of 1e3 insertions (2 bins), 1500 atoms 716 /
-// 235 / 304, 2e4 (42) 320 / 147 / 184, 1e5 (209) 260 / 231 / 212, 1.5e5 (313) 285 /
-// - / 275, 2e5 (417) 343 / - / 373.  One workgroup per cell / two waves a part: FP32
-// grid of 343 cells, 400 atoms 83 / 74, 512 cells 83 / 77, 729 cells 95 / 101; FP64
-// 95 / 81, 95 / 83, 109 / 109.
-constexpr int kNearGroup = 8;
-
-// This wave's groups of the LDS list, for the points of all of the workgroup.
-// wn: wave-far and wave-shell counts per segment of the shared lists wl (grid
-// tiles; segment's entries at its shell offset), or nullptr.
-template <int MATH, bool XL, int WAVES, int PARTS>
-__device__ __forceinline__ void eval_groups(const JobDev *__restrict__ J,
-                                            const double4 *__restrict__ L, int cap,
-                                            const int *__restrict__ seg, int nseg,
-                                            const double (&px)[2], const double (&py)[2],
-                                            const double (&pz)[2], double (&acc)[2], double R,
-                                            const int *__restrict__ wn,
-                                            const uint16_t *__restrict__ wl) {
-    const int wave = uniform(threadIdx.x >> 6) & (WAVES - 1);  // of the part's waves
-    const double rc2 = J->rc2, min_r2 = J->min_r2;
-    const int capA = near_region_start<MATH>(cap);
-    const double4 *__restrict__ Ls = L + capA - 1, *__restrict__ Ln = L + capA;
-    const char *__restrict__ Lb = reinterpret_cast<const char *>(L);
-    double mx[2], my[2], mz[2], p2[2];
-#pragma unroll
-    for (int q = 0; q < 2; ++q) {
-        mx[q] = -2.0 * px[q];
-        my[q] = -2.0 * py[q];
-        mz[q] = -2.0 * pz[q];
-        p2[q] = px[q] * px[q] + py[q] * py[q] + pz[q] * pz[q];
-    }
-    const bool clamp = MATH == MATH_MIXED && uniform(seg[kSegInts * nseg]) != 0;
-    int u = 0;  // groups before this one
-    for (int s = 0; s < nseg; ++s) {
-        const int *g = seg + kSegInts * s;
-        const int fb = uniform(g[1]), fe = uniform(g[kSegInts + 1]);
-        const int sb = uniform(g[2]), se = uniform(g[kSegInts + 2]);
-        const int nb = uniform(g[3]), ne = uniform(g[kSegInts + 3]);
-        if (fe - fb + se - sb + ne - nb == 0) continue;
-        const TypeParams P = J->types[uniform(g[0])];
-        // groups of `size` records of [0, n) that are this wave's
-        auto mine = [&](int n, auto size, auto &&group) {
-            constexpr int S = decltype(size)::value;
-            for (int r = S * ((wave - u) & (WAVES - 1)); r < n; r += S * WAVES)
-                group(r, r + S < n ? r + S : n);
-            u += (n + S - 1) / S;
-        };
-        using sixteen = std::integral_constant<int, kFlushPairs>;
-        using eight = std::integral_constant<int, kNearGroup>;
-        auto fp32 = [&](auto &&rec, auto test) {
-            return [&, rec](int b, int e) {
-                float a3[2] = {0.0f, 0.0f}, a6[2] = {0.0f, 0.0f};
-                auto pair = [&](int k) {
-                    double r2[2];
-                    pair_r2<2, XL>(rec(k), mx, my, mz, p2, r2);
-#pragma unroll
-                    for (int q = 0; q < 2; ++q) {
-                        const float w = __builtin_amdgcn_rcpf((float)r2[q]);
-                        if (decltype(test)::value) {
-                            float w3 = w * w * w;
-                            w3 = r2[q] < rc2 ? w3 : 0.0f;  // src/computegridsheet.h:79
-                            a3[q] += w3;
-                            a6[q] = __builtin_fmaf(w3, w3, a6[q]);
-                        } else {
-                            const float w2 = w * w, w3 = w2 * w;
-                            a3[q] = __builtin_fmaf(w2, w, a3[q]);
-                            a6[q] = __builtin_fmaf(w3, w3, a6[q]);
-                        }
-                    }
-                };
-                int k = b;
-                for (; k + 4 <= e; k += 4) {
-#pragma unroll
-                    for (int v = 0; v < 4; ++v) pair(k + v);
-                }
-                for (; k < e; ++k) pair(k);
-#pragma unroll
-                for (int q = 0; q < 2; ++q)
-                    acc[q] = fma(P.c6, (double)a6[q], fma(P.c3, (double)a3[q], acc[q]));
-            };
-        };
-        // FP64 pairs: NEWTON steps, the reference's clamp and cutoff test
-        auto fp64 = [&](auto &&r2_of, auto newton, auto clamp, auto test) {
-            return [&, r2_of](int b, int e) {
-                double b3[2] = {0.0, 0.0}, b6[2] = {0.0, 0.0};
-                auto pair = [&](int k) {
-                    double r2[2];
-                    r2_of(k, r2);
-#pragma unroll
-                    for (int q = 0; q < 2; ++q) {
-                        const double rr = decltype(clamp)::value ? fmax(r2[q], min_r2) : r2[q];
-                        double y = (double)__builtin_amdgcn_rcpf((float)rr);
-#pragma unroll
-                        for (int i = 0; i < decltype(newton)::value; ++i)
-                            y = fma(fma(-rr, y, 1.0), y, y);
-                        double y3 = y * y * y;
-                        if (decltype(test)::value) y3 = rr < rc2 ? y3 : 0.0;
-                        b3[q] += y3;
-                        b6[q] = fma(y3, y3, b6[q]);
-                    }
-                };
-                int k = b;
-                for (; k + 4 <= e; k += 4) {
-#pragma unroll
-                    for (int v = 0; v < 4; ++v) pair(k + v);
-                }
-                for (; k < e; ++k) pair(k);
-#pragma unroll
-                for (int q = 0; q < 2; ++q)
-                    acc[q] = fma(P.c6, b6[q], fma(P.c3, b3[q], acc[q]));
-            };
-        };
-        using no = std::integral_constant<bool, false>;
-        using yes = std::integral_constant<bool, true>;
-        using one = std::integral_constant<int, 1>;
-        using two = std::integral_constant<int, 2>;
-        auto far_rec = [&](int k) { return L[fb + k]; };
-        auto shell_rec = [&](int k) { return Ls[-(sb + k)]; };
-        auto wfar_rec = [&](int k) {
-            return *reinterpret_cast<const double4 *>(Lb + wl[sb + k]);
-        };
-        auto wshell_rec = [&](int k) {
-            return *reinterpret_cast<const double4 *>(Lb + wl[se - 1 - k]);
-        };
-        auto near_rec = [&](int k) { return Ln[nb + k]; };
-        const int nwf = wn ? uniform(wn[2 * s]) : 0;
-        const int nws = wn ? uniform(wn[2 * s + 1]) : se - sb;
-        if (MATH == MATH_MIXED) {
-            mine(fe - fb, sixteen(), fp32(far_rec, no()));
-            if (wn) {
-                mine(nwf, sixteen(), fp32(wfar_rec, no()));
-                mine(nws, sixteen(), fp32(wshell_rec, yes()));
-            } else {
-                mine(nws, sixteen(), fp32(shell_rec, yes()));
-            }
-            auto r2_of = [&](int k, double (&r2)[2]) {
-                pair_r2<2, XL>(near_rec(k), mx, my, mz, p2, r2);
-            };
-            if (P.rclose + 2.0 * R + 3.0 * kMargin >= J->rc)  // see eval_list
-                mine(ne - nb, eight(), fp64(r2_of, one(), yes(), yes()));
-            else if (clamp)
-                mine(ne - nb, eight(), fp64(r2_of, one(), yes(), no()));
-            else
-                mine(ne - nb, eight(), fp64(r2_of, one(), no(), no()));
-        } else {
-            auto expanded = [&](auto &&rec) {
-                return [&, rec](int k, double (&r2)[2]) {
-                    pair_r2<2, XL>(rec(k), mx, my, mz, p2, r2);
-                };
-            };
-            mine(fe - fb, eight(), fp64(expanded(far_rec), one(), no(), no()));
-            if (wn) {
-                mine(nwf, eight(), fp64(expanded(wfar_rec), one(), no(), no()));
-                mine(nws, eight(), fp64(expanded(wshell_rec), one(), no(), yes()));
-            } else {
-                mine(nws, eight(), fp64(expanded(shell_rec), one(), no(), yes()));
-            }
-            auto differences = [&](int k, double (&r2)[2]) {
-                const double4 A = near_rec(k);
-#pragma unroll
-                for (int q = 0; q < 2; ++q) {
-                    const double dx = px[q] - A.x, dy = py[q] - A.y, dz = pz[q] - A.z;
-                    r2[q] = dx * dx + dy * dy + dz * dz;
-                }
-            };
-            mine(ne - nb, eight(), fp64(differences, two(), yes(), yes()));
-        }
-    }
-}
+// us a call, one workgroup of four waves per cell / eight waves a quarter / four:
+// FP32 grid of 8 cells, 400 atoms 115 / 50 / 65, 64 cells 88 / 42 / 56, 216 cells
+// 83 / 77 / 61, 343 cells 87 / - / 88; Henry run of 1e3 insertions (2 bins), 1500
+// atoms 720 / 205 / 304, 2e4 (42) 360 / 111 / 184, 1e5 (209) 300 / 231 / 175, 1.5e5
+// (313) 322 / - / 250, 2e5 (417) 343 / - / 373.  Four waves a cell / two waves a
+// quarter: FP32 grid of 343 cells, 400 atoms 83 / 69, 512 cells 83 / 71, 729 cells
+// 95 / 101; FP64 95 / 79, 95 / 80, 109 / 109.
+//
+// In company (a batch whose jobs fill the device, see batch_create) the four
+// workgroups of a cell only repeat its fills: 256 grids of 0.5 A took 8.4 ms, 4.0 ms
+// in k_tiles<., MATH_IN_PARTS>, whose one wave a quarter makes the parts one after
+// the other (3.9 ms without parts); 256 Henry runs of 1e5 insertions 13.0 and 6.3 ms,
+// a step of both 21.5 and 10.3.
 
 template <int MATH, int WAVES, int PARTS>
 __global__ __launch_bounds__(64 * WAVES * PARTS, 4) void k_parts(const JobDev *__restrict__ jobs,
@@ -2057,7 +2129,7 @@ __global__ __launch_bounds__(64 * WAVES * PARTS, 4) void k_parts(const JobDev *_
     const JobDev *__restrict__ J = jobs + jl;
     const long long local = item - J->item_begin + J->local0;
     const int part = PARTS == 4 ? uniform(wave / WAVES) : (int)(local & 3);
-    const int pwave = wave & (WAVES - 1);  // of the part's waves
+    const int pwave = uniform(wave & (WAVES - 1));  // of the part's waves
     const bool grid = MATH == MATH_FP64 || PARTS == 4 || J->kind == JOB_GRID;
     const int *nc = grid ? J->ntiles : J->nbins;
     int tc[3];
@@ -2110,12 +2182,12 @@ __global__ __launch_bounds__(64 * WAVES * PARTS, 4) void k_parts(const JobDev *_
     const bool xl = grid && J->t[3] == 0.0 && J->t[6] == 0.0;
     // (a grid's part is one round; a bin has one for every 512 insertions)
     for (uint64_t c = run_slot(s0, 64 * part); grid || c < s1; c += 512) {
-        double px[2], py[2], pz[2], acc[2];
+        double px[2], py[2], pz[2];
+        double total = 0.0;  // of point pwave of the part's two
         long long at[2];
         bool ok[2];
 #pragma unroll
         for (int q = 0; q < 2; ++q) {
-            acc[q] = 0.0;
             if (grid) {
                 int gi = i0[0] + lane / (h1 * h2) + q * (J->tile[0] / 2);
                 int gj = i0[1] + (part & 1) * h1 + (lane / h2) % h1;
@@ -2164,30 +2236,59 @@ __global__ __launch_bounds__(64 * WAVES * PARTS, 4) void k_parts(const JobDev *_
                 }
                 __syncthreads();
             }
-            if (idle) {
-            } else if (xl) {
-                eval_groups<MATH, true, WAVES, PARTS>(J, s_list, cap, s_seg, nseg, px, py, pz, acc,
-                                                      tl.R, s_wn, s_wl);
-            } else {
-                eval_groups<MATH, false, WAVES, PARTS>(J, s_list, cap, s_seg, nseg, px, py, pz,
-                                                       acc, tl.R, grid ? s_wn : nullptr, s_wl);
+            // this wave's part of the groups (Widom: of the near ones, and of the others)
+            double e[2] = {0.0, 0.0}, far[2] = {0.0, 0.0};
+            const double4 none = make_double4(0.0, 0.0, 0.0, 0.0);
+            if (!grid) {
+                auto wn = [&](int s) {
+                    return (uniform(s_seg[kSegInts * (s + 1) + 2]) -
+                            uniform(s_seg[kSegInts * s + 2])) << 16;
+                };
+                const int2 groups = count_groups(s_seg, nseg, wn);
+                eval_list<2, MATH, false, 4>(J, s_list, cap, s_seg, nseg, px, py, pz, e, tl.R,
+                                             false, none, nullptr, 1,
+                                             OnePart(pwave, groups.x, WAVES));
+                eval_list<2, MATH, false, 4>(J, s_list, cap, s_seg, nseg, px, py, pz, far, tl.R,
+                                             false, none, nullptr, 2,
+                                             OnePart(pwave, groups.y, WAVES));
+            } else if (!idle) {
+                const int lengths =
+                    lane < nseg ? s_wn[2 * lane] | s_wn[2 * lane + 1] << 16 : 0;
+                const int2 groups = count_groups(s_seg, nseg, [&](int s) {
+                    return __builtin_amdgcn_readlane(lengths, s);
+                });
+                const OnePart part(pwave, groups.x + groups.y, WAVES);
+                if (xl)
+                    eval_list<2, MATH, true, 4>(J, s_list, cap, s_seg, nseg, px, py, pz, e, tl.R,
+                                                true, none, s_wl, 0, part, lengths);
+                else
+                    eval_list<2, MATH, false, 4>(J, s_list, cap, s_seg, nseg, px, py, pz, e,
+                                                 tl.R, true, none, s_wl, 0, part, lengths);
             }
             __syncthreads();
-        } while (cur_t < J->ntypes);
-        // the waves' energies, added in order
-        double *red = reinterpret_cast<double *>(s_list);
+            // the parts of the pass, added in order
+            double *red = reinterpret_cast<double *>(s_list);
 #pragma unroll
-        for (int q = 0; q < 2; ++q) red[(2 * wave + q) * 64 + lane] = acc[q];
-        __syncthreads();
+            for (int q = 0; q < 2; ++q) {
+                red[(2 * wave + q) * 64 + lane] = e[q];
+                if (!grid) red[(2 * (wave + WG / 64) + q) * 64 + lane] = far[q];
+            }
+            __syncthreads();
+            if (pwave < 2) {
+                const double *r = red + (2 * (PARTS == 4 ? part * WAVES : 0) + pwave) * 64 + lane;
+                double sum = 0.0;
+                for (int w = 0; w < WAVES; ++w) sum += r[128 * w];
+                for (int w = 0; w < WAVES && !grid; ++w) sum += r[128 * (w + WG / 64)];
+                total += sum;
+            }
+            // (the next fill meets two barriers before it writes the list)
+        } while (cur_t < J->ntypes);
         if (pwave < 2) {
-            double e = 0.0;
-            const int w0 = PARTS == 4 ? part * WAVES : 0;
-            for (int w = w0; w < w0 + WAVES; ++w) e += red[(2 * w + pwave) * 64 + lane];
             const long long o = pwave == 0 ? at[0] : at[1];
             if (pwave == 0 ? ok[0] : ok[1]) {
-                if (!grid) J->e_out[o] = e;
-                else if (J->mode == OUT_F64) ((double *)J->out)[o] = e;
-                else ((float *)J->out)[o] = (float)(e < (double)FLT_MAX ? e : (double)FLT_MAX);
+                if (!grid) J->e_out[o] = total;
+                else if (J->mode == OUT_F64) ((double *)J->out)[o] = total;
+                else ((float *)J->out)[o] = (float)(total < (double)FLT_MAX ? total : (double)FLT_MAX);
             }
         }
         if (grid) return;
@@ -2432,8 +2533,10 @@ hipError_t launch_bin_all(const BinJob *jobs, int njobs, long long total_blocks,
 
 size_t tiles_lds_bytes(int cap, int math) {
     size_t b = (size_t)cap * sizeof(double4);
-    if (math == MATH_MIXED || math == MATH_FP64 || math == MATH_NODES)
+    if (math == MATH_MIXED || math == MATH_FP64 || math == MATH_NODES || math == MATH_IN_PARTS)
         b += (size_t)(kWG / 64) * mixed_far_shell_cap(cap) * sizeof(uint16_t);
+    if (math == MATH_IN_PARTS_FP64)
+        b += (size_t)(kWG / 64) * near_region_start<MATH_FP64>(cap) * sizeof(uint16_t);
     return (b + 15) & ~(size_t)15;
 }
 
@@ -2478,6 +2581,8 @@ hipError_t launch_tiles(int math, int ppl, const JobDev *jobs, int njobs, long l
     ER_TILES(1, MATH_COUNT) ER_TILES(2, MATH_COUNT) ER_TILES(4, MATH_COUNT)
     ER_TILES(1, MATH_OVERLAP) ER_TILES(2, MATH_OVERLAP) ER_TILES(4, MATH_OVERLAP)
     ER_TILES(2, MATH_NODES)
+    if (parts_math(math)) ppl = 2;  // (insertions have the same energies whatever it is)
+    ER_TILES(2, MATH_IN_PARTS) ER_TILES(2, MATH_IN_PARTS_FP64)
 #undef ER_TILES
     return hipErrorInvalidValue;
 }
@@ -2490,6 +2595,8 @@ int tiles_occupancy(int math, int ppl, int cap) {
     ER_OCC(1, MATH_COUNT) ER_OCC(2, MATH_COUNT) ER_OCC(4, MATH_COUNT)
     ER_OCC(1, MATH_OVERLAP) ER_OCC(2, MATH_OVERLAP) ER_OCC(4, MATH_OVERLAP)
     ER_OCC(2, MATH_NODES)
+    if (parts_math(math)) ppl = 2;
+    ER_OCC(2, MATH_IN_PARTS) ER_OCC(2, MATH_IN_PARTS_FP64)
 #undef ER_OCC
     return 1;
 }

@@ -102,8 +102,9 @@ int grid_compute_noalloc(Context *ctx, FrameworkDev *fw, const int n[3], int pre
 
     // regions sized for this array's slices; a tile's list, and so every
     // value, does not depend on the region it is in
-    const JobDev job = make_grid_job(fw, n, precision, d_out, ctx->tuning,
-                                     precision == 1 ? MATH_FP64 : MATH_MIXED, kNoAllocRecords);
+    JobDev job = make_grid_job(fw, n, precision, d_out, ctx->tuning,
+                               precision == 1 ? MATH_FP64 : MATH_MIXED, kNoAllocRecords);
+    share_parts(&job);
     const int math = job_math(job);
     hipStream_t s = ctx->stream;
     if ((e = launch_setup(job, d_job, counter, nullptr, nullptr, s)) != hipSuccess)

@@ -240,7 +240,7 @@ int tiles_workgroups(const Context *ctx, int math, long long items, int scratch_
 int scratch_ensure(Context *ctx, hipStream_t s, uint32_t **buf, int *wgs) {
     int occ = 1;
     for (int m : {(int)MATH_MIXED, (int)MATH_FP64, (int)MATH_COUNT, (int)MATH_OVERLAP,
-                  (int)MATH_NODES})
+                  (int)MATH_NODES, (int)MATH_IN_PARTS, (int)MATH_IN_PARTS_FP64})
         occ = std::max(occ, tiles_occupancy(m, ctx->tuning.ppl, ctx->tuning.cap));
     int need = ctx->n_cu * occ;
     if (*buf && *wgs >= need) return ST_OK;
@@ -672,11 +672,19 @@ void use_parts(JobDev *j, const Tuning &tu) {
     // the same energies whatever the points per lane
     if (grid && (tu.ppl != 2 || j->tile[0] % 2 || j->tile[1] % 2 || j->tile[2] % 2)) return;
     j->parts = cells <= kPartCells8 ? 8 : cells <= kPartCells4 ? 4 : 2;
+}
+
+void share_parts(JobDev *j) {
+    if (!j->parts) return;
+    const int *nc = j->kind == JOB_GRID ? j->ntiles : j->nbins;
+    long long cells = 1;
     for (int d = 0; d < 3; d++) {
         j->region[d] = 1;
         j->nregions[d] = nc[d];
+        cells *= nc[d];
     }
     j->n_items = j->parts == 2 ? cells : 4 * cells;
+    j->shared = 1;
 }
 
 JobDev make_widom_job(const FrameworkDev *fw, uint64_t n_ins, uint64_t seed,
@@ -910,6 +918,7 @@ int grid_compute(Context *ctx, FrameworkDev *fw, const int n[3], int precision, 
     Scoped tmp{ctx, {}};
     const int math = precision == 1 ? MATH_FP64 : MATH_MIXED;
     JobDev job = make_grid_job(fw, n, precision, pinned ? pinned : g->d_data, ctx->tuning, math);
+    share_parts(&job);
     JobDev *d_job = nullptr;
     int st = pool_alloc(ctx, 1, &d_job, &tmp.ptrs);
     if (st) {
@@ -963,6 +972,7 @@ int widom_run(Context *ctx, FrameworkDev *fw, uint64_t n_ins, double temperature
     JobDev job = make_widom_job(fw, n_ins, seed, wb, ctx->tuning, kMinGridItems,
                                 energies_host ? 0.0 : temperature);
     use_parts(&job, ctx->tuning);
+    share_parts(&job);
     hipStream_t s = ctx->stream;
     ST_TRY(widom_enqueue_binning(job, wb, n_ins, seed, 0u, ctx->d_counter, s));
     ST_TRY(run_job(ctx, job_math(job), wb.d_job, job.n_items));
@@ -1075,9 +1085,10 @@ Batch::~Batch() {
 namespace {
 
 // Launches of a batch, in this order.
-constexpr int kBatchMath[kBatchLaunches] = {MATH_NODES,  MATH_MIXED,       MATH_FP64,
-                                              MATH_PARTS2, MATH_PARTS2_FP64, MATH_PARTS4,
-                                              MATH_PARTS4_FP64, MATH_PARTS8, MATH_PARTS8_FP64};
+constexpr int kBatchMath[kBatchLaunches] = {
+    MATH_NODES,         MATH_MIXED,  MATH_FP64,        MATH_IN_PARTS,
+    MATH_IN_PARTS_FP64, MATH_PARTS2, MATH_PARTS2_FP64, MATH_PARTS4,
+    MATH_PARTS4_FP64,   MATH_PARTS8, MATH_PARTS8_FP64};
 
 // Expected in-cutoff pairs per point: the ordering key of the LPT schedule.
 double job_cost_per_item(const FrameworkDev *fw, const JobDev &j, const Tuning &tu) {
@@ -1139,6 +1150,19 @@ int batch_create(Context *ctx, const Task *tasks, int n, bool use_graph, Batch *
         return st;
     };
     std::vector<std::pair<double, JobDev>> found;
+    double parts_waves = 0.0, longest = 0.0;
+    int part_kinds = 0;
+    auto add = [&](const FrameworkDev *fw, const JobDev &j) {
+        if (j.parts) {
+            const int *nc = j.kind == JOB_GRID ? j.ntiles : j.nbins;
+            const double list = fw->n_atoms / std::max(fw->volume, 1e-9) *
+                                std::pow(fw->rc + j.cell_R, 3.0);
+            parts_waves += (double)nc[0] * nc[1] * nc[2] * j.parts * list;
+            longest = std::max(longest, list);
+            part_kinds |= j.parts;
+        }
+        found.push_back({job_cost_per_item(fw, j, ctx->tuning), j});
+    };
     uint64_t ins_total = 0;
     for (int t = 0; t < n; t++) {
         const Task &tk = tasks[t];
@@ -1167,7 +1191,7 @@ int batch_create(Context *ctx, const Task *tasks, int n, bool use_graph, Batch *
             b->grids[t] = g;
             const int math = tk.precision == 1 ? MATH_FP64 : MATH_MIXED;
             JobDev j = make_grid_job(tk.fw, tk.grid_n, tk.precision, g->d_data, ctx->tuning, math);
-            found.push_back({job_cost_per_item(tk.fw, j, ctx->tuning), j});
+            add(tk.fw, j);
         }
         if (tk.n_ins > 0) {
             if (!(tk.temperature > 0.0)) {
@@ -1189,9 +1213,19 @@ int batch_create(Context *ctx, const Task *tasks, int n, bool use_graph, Batch *
                                       std::max<long long>(1, kMinGridItems / std::max(n, 1)),
                                       tk.temperature);
             use_parts(&j, ctx->tuning);
-            found.push_back({job_cost_per_item(tk.fw, j, ctx->tuning), j});
+            add(tk.fw, j);
         }
     }
+    // Jobs in parts share them out if that leaves the device idle no less than one job
+    // alone does: waves of a quarter of a cell's points, each weighed by its list
+    // against the longest list, which is what the launch takes if they are not shared
+    // out; every variant is one more launch.  us a run, shared out / not (weighed waves,
+    // variants): 256 Henry runs of 1e3 insertions (1780, 1) 743 / 1190, 16 of 1e4
+    // (785, 1) 190 / 435, two 0.5 A grids (750, 1) 47 / 79; four of them (1920, 3) 133 /
+    // 109, 16 (4350, 3) 620 / 343, 256 (70 000, 3) 8400 / 4040.
+    const int variants = !!(part_kinds & 8) + !!(part_kinds & 4) + !!(part_kinds & 2);
+    if (parts_waves * variants <= kPartWaves * longest)
+        for (auto &pj : found) share_parts(&pj.second);
     b->bin_chunk_len = bin_chunk(ins_total, b->bin_max_keys);
     for (BinJob &bj : b->bin_jobs) {
         bj.block0 = b->bin_blocks_total;

@@ -219,9 +219,13 @@ void choose_region(const FrameworkDev *fw, const double cell_frac[3], const int 
 JobDev make_widom_job(const FrameworkDev *fw, uint64_t n_ins, uint64_t seed,
                       const WidomBuffers &wb, const Tuning &tu, long long min_items,
                       double temperature = 0.0);
-// Makes a grid or Widom job of few cells a job of parts (see k_parts): the
-// choice depends on the cells and the knobs alone, so a job is the same on every path.
+// Has the energies of a grid or Widom job of few cells summed in parts (see
+// eval_range).  The choice depends on the cells and the knobs alone, so a job has the
+// same values on every path.
 void use_parts(JobDev *j, const Tuning &tu);
+// Shares the parts of such a job out to waves (see k_parts), for jobs that have the
+// device to themselves; the values are the same.
+void share_parts(JobDev *j);
 // Allocates the Widom buffers of a job (owned pointers appended to `owned`).
 int widom_prepare(Context *ctx, FrameworkDev *fw, uint64_t n_ins, WidomBuffers *wb,
                   std::vector<void *> *owned);
@@ -261,7 +265,7 @@ struct Task {
     uint64_t seed = 0;
 };
 
-constexpr int kBatchLaunches = 9;  // tiled-kernel variants of a batch, one launch each
+constexpr int kBatchLaunches = 11;  // tiled-kernel variants of a batch, one launch each
 
 class Batch {
   public:

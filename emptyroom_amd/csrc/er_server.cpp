@@ -336,6 +336,7 @@ bool Server::admit_one(Req *r, FwEntry *hit) {
         const int math = s.precision == 1 ? MATH_FP64 : MATH_MIXED;
         r->grid_job = make_grid_job(r->fw, s.grid_n, s.precision, r->grid->d_data, ctx_->tuning,
                                     math);
+        share_parts(&r->grid_job);
         r->items_total += r->grid_job.n_items;
     }
     if (st == ST_OK && s.n_ins) {
@@ -344,6 +345,7 @@ bool Server::admit_one(Req *r, FwEntry *hit) {
             r->widom_job = make_widom_job(r->fw, s.n_ins, s.seed, r->wb, ctx_->tuning,
                                           kMinGridItems, s.temperature);
             use_parts(&r->widom_job, ctx_->tuning);
+            share_parts(&r->widom_job);
             r->items_total += r->widom_job.n_items;
             st = widom_enqueue_binning(r->widom_job, r->wb, s.n_ins, s.seed, 0u,
                                        ctx_->d_counter, ctx_->stream);
