@@ -378,7 +378,8 @@ int widom_grid_run(Context *ctx, GridDev *g, uint64_t n_ins, double temperature,
     hipStream_t s = ctx->stream;
     // (without the memory for them the run does without face records)
     const size_t fb = tri_faces_bytes(g->n, n_ins);
-    float4 *faces = fb ? (float4 *)sc.get<char>(fb) : nullptr;
+    float4 *faces = fb ? (float4 *)ctx->pool.alloc_optional(fb) : nullptr;
+    if (faces) sc.ptrs.push_back(faces);
     HIP_TRY(launch_widom_grid((const float *)g->d_data, faces, g->n, seed, 1u, n_ins, temperature,
                               e, partials, s));
     HIP_TRY(launch_widom_final(partials, kTriBlocks, ctx->h_sums, s));

@@ -85,25 +85,34 @@ size_t DevicePool::round_size(size_t b) {
     return (b + mb - 1) / mb * mb;
 }
 
+void *DevicePool::take(size_t sz) {
+    auto it = cache_.find(sz);
+    if (it == cache_.end() || it->second.empty()) return nullptr;
+    void *p = it->second.back();
+    it->second.pop_back();
+    live_[p] = sz;
+    in_use_ += sz;
+    return p;
+}
+
+void *DevicePool::make(size_t sz) {
+    void *p = nullptr;
+    if (hipMalloc(&p, sz) != hipSuccess) {
+        (void)hipGetLastError();
+        return nullptr;
+    }
+    live_[p] = sz;
+    in_use_ += sz;
+    reserved_ += sz;
+    return p;
+}
+
 void *DevicePool::alloc(size_t bytes) {
     std::lock_guard<std::mutex> lk(mu_);
     const size_t sz = round_size(bytes);
-    auto it = cache_.find(sz);
-    if (it != cache_.end() && !it->second.empty()) {
-        void *p = it->second.back();
-        it->second.pop_back();
-        live_[p] = sz;
-        in_use_ += sz;
-        return p;
-    }
+    if (void *p = take(sz)) return p;
     if (ctx_->hbm_cap && reserved_ + sz > ctx_->hbm_cap) {
-        // give cached blocks back before refusing
-        for (auto &kv : cache_)
-            for (void *p : kv.second) {
-                (void)hipFree(p);
-                reserved_ -= kv.first;
-            }
-        cache_.clear();
+        trim();
         if (reserved_ + sz > ctx_->hbm_cap) {
             std::ostringstream os;
             os << "HBM cap exceeded: need " << sz << " B with " << reserved_ << " of "
@@ -112,18 +121,41 @@ void *DevicePool::alloc(size_t bytes) {
             return nullptr;
         }
     }
-    void *p = nullptr;
-    if (hipMalloc(&p, sz) != hipSuccess) {
-        (void)hipGetLastError();
+    void *p = make(sz);
+    if (!p && !cache_.empty()) {
+        trim();
+        p = make(sz);
+    }
+    if (!p) {
         std::ostringstream os;
         os << "hipMalloc of " << sz << " B failed";
         set_error(os.str());
-        return nullptr;
     }
-    live_[p] = sz;
-    in_use_ += sz;
-    reserved_ += sz;
     return p;
+}
+
+void *DevicePool::alloc_optional(size_t bytes) {
+    std::lock_guard<std::mutex> lk(mu_);
+    const size_t sz = round_size(bytes);
+    auto it = cache_.find(optional_size_);
+    if (optional_ && it != cache_.end()) {
+        auto at = std::find(it->second.begin(), it->second.end(), optional_);
+        if (at != it->second.end()) {  // not in use
+            it->second.erase(at);
+            if (optional_size_ >= sz) {
+                live_[optional_] = optional_size_;
+                in_use_ += optional_size_;
+                return optional_;
+            }
+            (void)hipFree(optional_);
+            reserved_ -= optional_size_;
+        }
+    }
+    optional_ = nullptr;
+    if (ctx_->hbm_cap && reserved_ + sz > ctx_->hbm_cap) return nullptr;
+    optional_ = make(sz);
+    optional_size_ = sz;
+    return optional_;
 }
 
 void DevicePool::free(void *p) {
@@ -137,7 +169,6 @@ void DevicePool::free(void *p) {
 }
 
 void DevicePool::trim() {
-    std::lock_guard<std::mutex> lk(mu_);
     for (auto &kv : cache_)
         for (void *p : kv.second) {
             (void)hipFree(p);

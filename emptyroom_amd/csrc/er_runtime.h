@@ -70,19 +70,27 @@ class DevicePool {
   public:
     explicit DevicePool(Context *ctx) : ctx_(ctx) {}
     ~DevicePool();
-    // Returns nullptr and sets the error if the cap would be exceeded.
+    // Returns nullptr and sets the error if the cap would be exceeded.  Cached blocks are
+    // given back to the device before an allocation is refused.
     void *alloc(size_t bytes);
+    // For memory that a call can do without: nullptr, with no error set and nothing given
+    // back, if it is not there.  The pool keeps one such block, of the largest size so far.
+    void *alloc_optional(size_t bytes);
     void free(void *p);
     size_t in_use() const { return in_use_; }
     size_t reserved() const { return reserved_; }
-    void trim();
 
   private:
     static size_t round_size(size_t b);
+    void *take(size_t sz);  // a cached block, or nullptr
+    void *make(size_t sz);  // a block from the device, or nullptr
+    void trim();
     Context *ctx_;
     std::map<size_t, std::vector<void *>> cache_;
     std::map<void *, size_t> live_;
     size_t in_use_ = 0, reserved_ = 0;
+    void *optional_ = nullptr;  // the optional block, ...
+    size_t optional_size_ = 0;  // ... of this size
     std::mutex mu_;
 };
 
