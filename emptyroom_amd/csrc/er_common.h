@@ -155,7 +155,9 @@ constexpr int kBinChunkMax = 16384;  // insertions per binning block, at most
 constexpr int kBinGroups = 1024;  // groups of a Widom job that is binned in two steps
 constexpr int kBinDirectMax = 4096;  // bins up to which a job is binned in one step
 constexpr int kBinGroupMax = 15360;  // bins a group may hold (the second step's LDS counts)
-constexpr int kBinLdsKeys = 7168;    // keys a binning block histograms in LDS (28 KiB)
+constexpr int kBinLdsKeys = 7168;    // keys a binning block histograms in LDS (28 KiB), and so
+                                     // most groups of a job; bins accordingly:
+constexpr long long kBinsMax = (long long)kBinLdsKeys * kBinGroupMax;
 constexpr int kRegionRecords = 8192;  // entries of one workgroup's region sub-list (near-list
                                       // indices, 32 KiB)
 constexpr int kBlockList = 3072;  // of these, entries of a block's list (see grid_block)

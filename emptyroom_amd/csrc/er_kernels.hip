@@ -232,28 +232,23 @@ __global__ __launch_bounds__(kWG) void k_bin_zero(const BinJob *__restrict__ job
 }
 
 __global__ __launch_bounds__(kWG) void k_bin_count(const BinJob *__restrict__ jobs, int njobs,
-                                                   int chunk, int lds_keys) {
+                                                   int chunk) {
     extern __shared__ uint32_t s_hist[];
     const int j = bin_job_of(jobs, njobs, blockIdx.x);
     const BinJob &J = jobs[j];
     const uint64_t i0 = (uint64_t)(blockIdx.x - J.block0) * (uint64_t)chunk;
     const uint64_t i1 = i0 + (uint64_t)chunk < J.n ? i0 + (uint64_t)chunk : J.n;
     const uint32_t group = (uint32_t)J.group;
-    const bool lds = J.ngroups <= lds_keys;
     uint32_t *__restrict__ keys = group > 1 ? J.sorted : reinterpret_cast<uint32_t *>(J.tmp);
-    if (lds) {
-        for (int b = threadIdx.x; b < J.ngroups; b += kWG) s_hist[b] = 0u;
-        __syncthreads();
-    }
+    for (int b = threadIdx.x; b < J.ngroups; b += kWG) s_hist[b] = 0u;
+    __syncthreads();
     for (uint64_t i = i0 + threadIdx.x; i < i1; i += kWG) {
         double f[3];
         widom_point(J.seed, J.stream, i, f);
         const uint32_t bin = widom_bin(f, J.nb);
-        const uint32_t key = group > 1 ? bin / group : bin;
         keys[i] = bin;
-        atomicAdd(lds ? &s_hist[key] : &J.count[key], 1u);
+        atomicAdd(&s_hist[group > 1 ? bin / group : bin], 1u);
     }
-    if (!lds) return;
     __syncthreads();
     for (int b = threadIdx.x; b < J.ngroups; b += kWG)
         if (s_hist[b]) atomicAdd(&J.count[b], s_hist[b]);
@@ -270,7 +265,7 @@ __global__ __launch_bounds__(kWG) void k_bin_scan(const BinJob *__restrict__ job
 // instead of 64 separate lines.
 template <int PER>
 __global__ __launch_bounds__(kBinWG) void k_bin_scatter(const BinJob *__restrict__ jobs,
-                                                        int njobs, int lds_keys) {
+                                                        int njobs) {
     extern __shared__ uint32_t s_hist[];
     __shared__ uint32_t s_part[kBinWG / 64];
     constexpr int chunk = PER * kBinWG;
@@ -288,18 +283,6 @@ __global__ __launch_bounds__(kBinWG) void k_bin_scatter(const BinJob *__restrict
     for (int q = 0; q < PER; ++q) {
         const int l = q * kBinWG + tid;
         bin[q] = keys[l < cnt ? l : 0];
-    }
-    if (nk > lds_keys) {
-#pragma unroll
-        for (int q = 0; q < PER; ++q) {
-            const int l = q * kBinWG + tid;
-            if (l >= cnt) continue;
-            const uint32_t key = group > 1 ? bin[q] / group : bin[q];
-            const uint32_t pos = atomicAdd(&J.cursor[key], 1u);
-            if (group > 1) J.tmp[pos] = make_uint2(bin[q] - key * group, (uint32_t)(i0 + l));
-            else J.sorted[pos] = (uint32_t)(i0 + l);
-        }
-        return;
     }
     // s_hist[nk]: counts, then first slots in the block's order; s_dst[nk]:
     // first slot in the job's order; s_key, s_loc[chunk]: the sorted insertions
@@ -2502,15 +2485,13 @@ hipError_t launch_bin_all(const BinJob *jobs, int njobs, long long total_blocks,
                           bool cleared, hipStream_t s) {
     if (njobs <= 0 || total_blocks <= 0) return hipSuccess;
     if (chunk < kBinWG || chunk > kBinChunkMax || (chunk & (chunk - 1)) ||
-        total_blocks > (1LL << 31) - 1 || max_keys <= 0 || max_group < 1 ||
+        total_blocks > (1LL << 31) - 1 || max_keys <= 0 || max_keys > kBinLdsKeys || max_group < 1 ||
         max_group > kBinGroupMax || total_groups < 0 || total_groups > (1LL << 31) - 1)
         return hipErrorInvalidValue;
-    // a job whose keys do not fit the histogram uses one global atomic per insertion
-    const int lds_keys = (int)(max_keys < kBinLdsKeys ? max_keys : kBinLdsKeys);
-    const size_t lds_bytes = sizeof(uint32_t) * (size_t)lds_keys;
+    const size_t lds_bytes = sizeof(uint32_t) * (size_t)max_keys;
     if (!cleared) hipLaunchKernelGGL(k_bin_zero, dim3(njobs), dim3(kWG), 0, s, jobs);
     hipLaunchKernelGGL(k_bin_count, dim3((unsigned)total_blocks), dim3(kWG), lds_bytes, s, jobs,
-                       njobs, chunk, lds_keys);
+                       njobs, chunk);
     hipLaunchKernelGGL(k_bin_scan, dim3(njobs), dim3(kWG), 0, s, jobs);
     const size_t scatter_lds = 2 * lds_bytes + 6 * (size_t)chunk;
 #define ER_SCATTER(P)                                                                          \
@@ -2521,7 +2502,7 @@ hipError_t launch_bin_all(const BinJob *jobs, int njobs, long long total_blocks,
                                 8 * kBinLdsKeys + 6 * P * kBinWG) == hipSuccess;               \
         if (!lds_ok) return hipErrorInvalidValue;                                              \
         hipLaunchKernelGGL(k_bin_scatter<P>, dim3((unsigned)total_blocks), dim3(kBinWG),       \
-                           scatter_lds, s, jobs, njobs, lds_keys);                             \
+                           scatter_lds, s, jobs, njobs);                                       \
     }
     ER_SCATTER(1) ER_SCATTER(2) ER_SCATTER(4) ER_SCATTER(8) ER_SCATTER(16)
 #undef ER_SCATTER

@@ -484,11 +484,12 @@ void choose_grid_tile(const FrameworkDev *fw, const int n[3], const Tuning &tu, 
 }
 
 // Bins of near-cubic shape (per perpendicular width) whose mean occupancy is
-// at most widom_per_bin: the tile kernel takes a bin's insertions 256 x
-// (points per lane, at most 2) at a time, so a mean just below a multiple of
-// that keeps the last chunk full while bins above the mean stay rare.  Refines the rounded counts: adds bins
-// along the axis with the widest bins until the mean fits, then removes any
-// bin whose removal keeps it fitting.
+// at most widom_per_bin (unless that is more bins than the binning takes): the
+// tile kernel takes a bin's insertions 256 x (points per lane, at most 2) at a
+// time, so a mean just below a multiple of that keeps the last chunk full while
+// bins above the mean stay rare.  Refines the rounded counts: adds bins along the
+// axis with the widest bins until the mean fits, then removes any bin whose
+// removal keeps it fitting.
 void choose_widom_bins(const FrameworkDev *fw, uint64_t n_ins, const Tuning &tu, int nb[3]) {
     double w[3];
     for (int d = 0; d < 3; d++) w[d] = perp_width(fw->inv_t, d);
@@ -502,7 +503,7 @@ void choose_widom_bins(const FrameworkDev *fw, uint64_t n_ins, const Tuning &tu,
         int d = -1;
         for (int e = 0; e < 3; e++)
             if (nb[e] < (1 << 10) && (d < 0 || w[e] / nb[e] > w[d] / nb[d])) d = e;
-        if (d < 0) break;
+        if (d < 0 || (long long)(nb[d] + 1) * nb[(d + 1) % 3] * nb[(d + 2) % 3] > kBinsMax) break;
         nb[d]++;
     }
     for (bool changed = true; changed;) {
