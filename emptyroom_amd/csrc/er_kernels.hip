@@ -21,8 +21,8 @@
 // against its own, smaller point box.  A Widom bin of at most one chunk of
 // insertions keeps their points and partial energies in registers across
 // its LDS passes.  Fine FP32 grids take the far field of blocks of tiles from
-// interpolation nodes (grid_block), and jobs of a few hundred cells share the
-// points of a wave between several (k_parts).
+// interpolation nodes (grid_block).  Jobs of a few hundred cells sum an energy in
+// parts, which several waves make at once where the device is idle (k_parts).
 #include "er_kernels.h"
 
 #include <float.h>
@@ -416,8 +416,9 @@ __global__ void k_fill_u64(unsigned long long *p, unsigned long long v, long lon
 
 // The descriptors of a job that runs alone, by value: one launch writes them and
 // clears the counters, in place of a copy per descriptor and a fill per counter.
-// With the sums written to pinned memory a Henry run is 6 launches and no copy (8
-// and 3 before): 1e5 insertions, 200 atoms 128 -> 97 us.
+// With the sums written to pinned memory a Henry run is 7 launches (8 if its bins are
+// grouped) and no copy, two launches and three copies less: 1e5 insertions, 200 atoms
+// 128 -> 97 us.
 struct Setup {
     JobDev job;
     BinJob bin;
@@ -852,7 +853,8 @@ struct PartSums {
     double (&sum)[P];
     int groups, parts;
     int u = 0, v = 0, next = 0;  // next group, next part, its first group
-    __device__ __forceinline__ PartSums(double (&s)[P], int g, int p) : sum(s), groups(g), parts(p) {}
+    __device__ __forceinline__ PartSums(double (&s)[P], int g, int p)
+        : sum(s), groups(g), parts(p) {}
     __device__ __forceinline__ bool ended() const { return uniform(u) == uniform(next); }
     // up to n groups of one part begin here
     __device__ __forceinline__ int run(double (&e)[P], int n) {
@@ -1484,7 +1486,8 @@ __device__ void grid_tile(const JobDev *__restrict__ J, const int tc[3],
         if (MATH == MATH_COUNT) {
             ((uint32_t *)J->out)[oidx[q]] = (uint32_t)acc[q];
         } else if (MATH == MATH_OVERLAP) {
-            ((double *)J->out)[oidx[q]] = acc[q] > 0.0 ? 0.0 : 1.0;  // src/computegridsheet.h:159-162
+            // src/computegridsheet.h:159-162
+            ((double *)J->out)[oidx[q]] = acc[q] > 0.0 ? 0.0 : 1.0;
         } else if (J->mode == OUT_F64) {
             ((double *)J->out)[oidx[q]] = acc[q];
         } else {
@@ -1834,234 +1837,235 @@ void k_tiles(const JobDev *__restrict__ jobs, int njobs, long long total_items,
                             nodes.first[1] = 8 * o1;
                             nodes.first[2] = 8 * o2;
                             grid_tile<PPL, MATH_MIXED>(reread(J), tc, src, bidx, bbeg,
-                                                       cap - kNodeRecords, s_list, s_seg, s_cnt, s_wl, nodes);
+                                                       cap - kNodeRecords, s_list, s_seg, s_cnt,
+                                                       s_wl, nodes);
                         }
                     }
             continue;
         } else {
-        for (int ti = 0; ti < nt; ++ti) {
-            int tc[3];
-            cell_of(ti, tc);
-            if (grid) {
-                grid_tile<PPL, MATH, PARTS>(J, tc, src, sidx, tbeg, cap, s_list, s_seg, s_cnt,
-                                            s_wl);
-                continue;
-            }
-            // ---- one Widom bin: every insertion whose point falls in it ----
-            // (at most 2 per lane: bins hold a few hundred insertions).  A
-            // chunk's slots are c + q*256 + tid; a wave none of whose lanes
-            // holds a second slot evaluates one point per lane, and a wave
-            // with no slot at all skips the chunk (the energies do not depend
-            // on the points per lane).  Each pass adds its near records, then
-            // its far and shell records, to the insertion's energy.
-            //
-            // Saturation (J->sat_e > 0, jobs whose energies only feed the
-            // Boltzmann sums): no pair energy is below -eps_ij, and none of a
-            // far or shell record (beyond r_FP64 of every point) below
-            // -fs_floor eps_ij, so once an insertion's partial energy plus
-            // those floors for every record not yet evaluated (-eps_ij of its
-            // type for records not yet classified) reaches sat_e = 800 T, its exact
-            // energy is at least 800 T as well, exp(-E/T) is exactly 0 in
-            // FP64 for both, and neither sum changes.  A wave whose valid insertions are all
-            // saturated stops evaluating them; the stored partial energy
-            // (>= 800 T) then stands in for the exact one.
-            constexpr int PW = PPL > 2 ? 2 : PPL;
-            // One pass of this wave's P points (px.., valid where ok) over the
-            // LDS list: the near records, then, unless every valid point is
-            // saturated by then, the far and shell records.  out = prev + the
-            // pass's terms (the terms alone in the first pass).  Returns false,
-            // out untouched, if the points were saturated before the pass:
-            // their stored energies stand.
-            auto one_pass = [&](auto pw, const auto &px, const auto &py, const auto &pz,
-                                const auto &ok, const auto &prev, auto &out, const Tile &tl,
-                                int nseg, bool first, double lb_near, double lb_fs,
-                                double lb_later) {
-                constexpr int P = decltype(pw)::value;
-                double acc[P];
+            for (int ti = 0; ti < nt; ++ti) {
+                int tc[3];
+                cell_of(ti, tc);
+                if (grid) {
+                    grid_tile<PPL, MATH, PARTS>(J, tc, src, sidx, tbeg, cap, s_list, s_seg, s_cnt,
+                                                s_wl);
+                    continue;
+                }
+                // ---- one Widom bin: every insertion whose point falls in it ----
+                // (at most 2 per lane: bins hold a few hundred insertions).  A
+                // chunk's slots are c + q*256 + tid; a wave none of whose lanes
+                // holds a second slot evaluates one point per lane, and a wave
+                // with no slot at all skips the chunk (the energies do not depend
+                // on the points per lane).  Each pass adds its near records, then
+                // its far and shell records, to the insertion's energy.
+                //
+                // Saturation (J->sat_e > 0, jobs whose energies only feed the
+                // Boltzmann sums): no pair energy is below -eps_ij, and none of a
+                // far or shell record (beyond r_FP64 of every point) below
+                // -fs_floor eps_ij, so once an insertion's partial energy plus
+                // those floors for every record not yet evaluated (-eps_ij of its
+                // type for records not yet classified) reaches sat_e = 800 T, its exact
+                // energy is at least 800 T as well, exp(-E/T) is exactly 0 in
+                // FP64 for both, and neither sum changes.  A wave whose valid insertions are all
+                // saturated stops evaluating them; the stored partial energy
+                // (>= 800 T) then stands in for the exact one.
+                constexpr int PW = PPL > 2 ? 2 : PPL;
+                // One pass of this wave's P points (px.., valid where ok) over the
+                // LDS list: the near records, then, unless every valid point is
+                // saturated by then, the far and shell records.  out = prev + the
+                // pass's terms (the terms alone in the first pass).  Returns false,
+                // out untouched, if the points were saturated before the pass:
+                // their stored energies stand.
+                auto one_pass = [&](auto pw, const auto &px, const auto &py, const auto &pz,
+                                    const auto &ok, const auto &prev, auto &out, const Tile &tl,
+                                    int nseg, bool first, double lb_near, double lb_fs,
+                                    double lb_later) {
+                    constexpr int P = decltype(pw)::value;
+                    double acc[P];
 #pragma unroll
-                for (int q = 0; q < P; ++q) acc[q] = 0.0;
-                const bool sat = J->sat_e > 0.0;
-                auto saturated = [&](double lb) {
-                    bool all = true;
+                    for (int q = 0; q < P; ++q) acc[q] = 0.0;
+                    const bool sat = J->sat_e > 0.0;
+                    auto saturated = [&](double lb) {
+                        bool all = true;
 #pragma unroll
-                    for (int q = 0; q < P; ++q)
-                        if (ok[q]) all = all && prev[q] + acc[q] + lb >= J->sat_e;
-                    return __all(all) != 0;
-                };
-                if (sat && !first && saturated(lb_near + lb_fs + lb_later)) return false;
-                if constexpr (PARTS) {
-                    auto wn = [&](int s) {
-                        return (uniform(s_seg[kSegInts * (s + 1) + 2]) -
-                                uniform(s_seg[kSegInts * s + 2])) << 16;
+                        for (int q = 0; q < P; ++q)
+                            if (ok[q]) all = all && prev[q] + acc[q] + lb >= J->sat_e;
+                        return __all(all) != 0;
                     };
-                    // (e: the current part, zero again after each call)
-                    double e[P];
+                    if (sat && !first && saturated(lb_near + lb_fs + lb_later)) return false;
+                    if constexpr (PARTS) {
+                        auto wn = [&](int s) {
+                            return (uniform(s_seg[kSegInts * (s + 1) + 2]) -
+                                    uniform(s_seg[kSegInts * s + 2])) << 16;
+                        };
+                        // (e: the current part, zero again after each call)
+                        double e[P];
 #pragma unroll
-                    for (int q = 0; q < P; ++q) e[q] = 0.0;
-                    const int parts = uniform(J->parts);
-                    const int2 groups = count_groups(s_seg, nseg, wn);
-                    eval_list<P, MATH, false>(
-                        J, s_list, cap, s_seg, nseg, px, py, pz, e, tl.R, false,
-                        make_double4(0.0, 0.0, 0.0, 0.0), nullptr, 1,
-                        PartSums<P>(acc, groups.x, parts));
-                    if (!(sat && saturated(lb_fs + lb_later)))
+                        for (int q = 0; q < P; ++q) e[q] = 0.0;
+                        const int parts = uniform(J->parts);
+                        const int2 groups = count_groups(s_seg, nseg, wn);
                         eval_list<P, MATH, false>(
                             J, s_list, cap, s_seg, nseg, px, py, pz, e, tl.R, false,
-                            make_double4(0.0, 0.0, 0.0, 0.0), nullptr, 2,
-                            PartSums<P>(acc, groups.y, parts));
-                } else {
-                    eval_list<P, MATH, false>(J, s_list, cap, s_seg, nseg, px, py, pz, acc, tl.R,
-                                              false, make_double4(0.0, 0.0, 0.0, 0.0), nullptr,
-                                              1);
-                    if (!(sat && saturated(lb_fs + lb_later)))
+                            make_double4(0.0, 0.0, 0.0, 0.0), nullptr, 1,
+                            PartSums<P>(acc, groups.x, parts));
+                        if (!(sat && saturated(lb_fs + lb_later)))
+                            eval_list<P, MATH, false>(
+                                J, s_list, cap, s_seg, nseg, px, py, pz, e, tl.R, false,
+                                make_double4(0.0, 0.0, 0.0, 0.0), nullptr, 2,
+                                PartSums<P>(acc, groups.y, parts));
+                    } else {
                         eval_list<P, MATH, false>(J, s_list, cap, s_seg, nseg, px, py, pz, acc,
                                                   tl.R, false, make_double4(0.0, 0.0, 0.0, 0.0),
-                                                  nullptr, 2);
+                                                  nullptr, 1);
+                        if (!(sat && saturated(lb_fs + lb_later)))
+                            eval_list<P, MATH, false>(
+                                J, s_list, cap, s_seg, nseg, px, py, pz, acc, tl.R, false,
+                                make_double4(0.0, 0.0, 0.0, 0.0), nullptr, 2);
+                    }
+#pragma unroll
+                    for (int q = 0; q < P; ++q) out[q] = first ? acc[q] : prev[q] + acc[q];
+                    return true;
+                };
+                // A chunk of up to P * 256 of the bin's insertions, slots
+                // c + q * 256 + tid: points generated and energies loaded and
+                // stored for this pass.
+                auto chunk = [&](auto pw, uint64_t c, uint64_t end, const Tile &tl, int nseg,
+                                 bool first, double lb_near, double lb_fs, double lb_later) {
+                    constexpr int P = decltype(pw)::value;
+                    double px[P], py[P], pz[P], prev[P], out[P];
+                    uint32_t ins[P];
+                    bool ok[P];
+#pragma unroll
+                    for (int q = 0; q < P; ++q) {
+                        const uint64_t p = c + (uint64_t)(q * kWG + tid);
+                        ok[q] = p < end;
+                        ins[q] = J->sorted[ok[q] ? p : c];
+                        double f[3];
+                        widom_point(J->seed, J->stream, ins[q], f);
+                        frac_to_cart(J->t, f[0], f[1], f[2], px[q], py[q], pz[q]);
+                        px[q] -= tl.cx;
+                        py[q] -= tl.cy;
+                        pz[q] -= tl.cz;
+                        prev[q] = first ? 0.0 : J->e_out[ins[q]];
+                    }
+                    if (!one_pass(pw, px, py, pz, ok, prev, out, tl, nseg, first, lb_near, lb_fs,
+                                  lb_later))
+                        return;
+#pragma unroll
+                    for (int q = 0; q < P; ++q)
+                        if (ok[q]) J->e_out[ins[q]] = out[q];
+                };
+                // A bin whose insertions fit one chunk (at most PW * 256, most
+                // bins) keeps each lane's points and partial energies in
+                // registers across the passes and writes the energies once; the
+                // passes add the same terms in the same order as the chunked
+                // form, which stores and reloads them after every pass.
+                auto resident = [&](auto pw, const double (&X)[PW], const double (&Y)[PW],
+                                    const double (&Z)[PW], const bool (&OK)[PW], double (&T)[PW],
+                                    const Tile &tl, int nseg, bool first, double lb_near,
+                                    double lb_fs, double lb_later) {
+                    constexpr int P = decltype(pw)::value;
+                    double px[P], py[P], pz[P], prev[P], out[P];
+                    bool ok[P];
+#pragma unroll
+                    for (int q = 0; q < P; ++q) {
+                        px[q] = X[q];
+                        py[q] = Y[q];
+                        pz[q] = Z[q];
+                        ok[q] = OK[q];
+                        prev[q] = first ? 0.0 : T[q];
+                    }
+                    if (!one_pass(pw, px, py, pz, ok, prev, out, tl, nseg, first, lb_near, lb_fs,
+                                  lb_later))
+                        return;
+#pragma unroll
+                    for (int q = 0; q < P; ++q) T[q] = out[q];
+                };
+                const int b = (tc[0] * J->nbins[1] + tc[1]) * J->nbins[2] + tc[2];
+                const uint32_t s0 = J->bin_start[b], s1 = J->bin_start[b + 1];
+                if (s0 == s1) continue;
+                const Tile tl = cell_sphere(J, tc);
+                // one chunk: this wave's points per lane (wave-uniform; 0 for a
+                // wave with no slot); several chunks: -1.  Only the FP32-grid /
+                // Widom pair math keeps bins resident: Widom jobs never run with
+                // the other variants, whose registers the resident state would
+                // only crowd (FP64 grids would drop to three waves per SIMD).
+                const uint64_t wv0 = s0 + (uint64_t)(tid & ~63);
+                const int mode = (MATH != MATH_MIXED || s1 - s0 > (uint32_t)(PW * kWG)) ? -1
+                                 : wv0 >= s1                     ? 0
+                                 : (PW > 1 && wv0 + kWG >= s1)   ? 1
+                                                                 : PW;
+                double rx[PW], ry[PW], rz[PW], rt[PW];
+                uint32_t rins[PW];
+                bool rok[PW];
+#pragma unroll
+                for (int q = 0; q < PW; ++q) {
+                    rx[q] = ry[q] = rz[q] = rt[q] = 0.0;
+                    rins[q] = 0;
+                    rok[q] = false;
+                    if (q < mode) {
+                        const uint64_t p = s0 + (uint64_t)(q * kWG + tid);
+                        rok[q] = p < s1;
+                        rins[q] = J->sorted[rok[q] ? p : s0];
+                        double f[3];
+                        widom_point(J->seed, J->stream, rins[q], f);
+                        frac_to_cart(J->t, f[0], f[1], f[2], rx[q], ry[q], rz[q]);
+                        rx[q] -= tl.cx;
+                        ry[q] -= tl.cy;
+                        rz[q] -= tl.cz;
+                    }
                 }
+                int cur_t = 0, cur_pos = uniform(tbeg[0]);
+                bool first = true;
+                do {
+                    const int nseg = fill_list<MATH, kWG>(J, src, sidx, tbeg, tl, cur_t, cur_pos,
+                                                          cap, s_list, s_seg, s_cnt);
+                    __syncthreads();
+                    // -eps_ij for every record of this pass (near; far and shell)
+                    // and every source record after it
+                    double lb_near = 0.0, lb_fs = 0.0, lb_later = 0.0;
+                    if (J->sat_e > 0.0) {
+                        for (int sg = 0; sg < nseg; ++sg) {
+                            const int *g = s_seg + kSegInts * sg, *e = g + kSegInts;
+                            const double eps = 0.25 * J->types[uniform(g[0])].eps4;
+                            lb_fs -= eps * J->fs_floor *
+                                     (double)(uniform(e[1]) - uniform(g[1]) + uniform(e[2]) -
+                                              uniform(g[2]));
+                            lb_near -= eps * (double)(uniform(e[3]) - uniform(g[3]));
+                        }
+                        // source records after this pass, each at -eps of its type:
+                        // the rest of the current type, then every later type
+                        if (cur_t < J->ntypes) {
+                            lb_later = -0.25 * J->types[cur_t].eps4 *
+                                       (double)(uniform(tbeg[cur_t + 1]) - cur_pos);
+                            for (int u = cur_t + 1; u < J->ntypes; ++u)
+                                lb_later -= 0.25 * J->types[u].eps4 *
+                                            (double)(uniform(tbeg[u + 1]) - uniform(tbeg[u]));
+                        }
+                    }
+                    if (mode == PW)
+                        resident(std::integral_constant<int, PW>(), rx, ry, rz, rok, rt, tl, nseg,
+                                 first, lb_near, lb_fs, lb_later);
+                    else if (PW > 1 && mode == 1)
+                        resident(std::integral_constant<int, 1>(), rx, ry, rz, rok, rt, tl, nseg,
+                                 first, lb_near, lb_fs, lb_later);
+                    for (uint64_t c = s0; mode < 0 && c < s1; c += (uint64_t)(PW * kWG)) {
+                        const uint64_t w0 = c + (uint64_t)(tid & ~63);  // wave-uniform
+                        if (w0 >= s1) continue;
+                        if (PW > 1 && w0 + kWG >= s1)
+                            chunk(std::integral_constant<int, 1>(), c, s1, tl, nseg, first, lb_near,
+                                  lb_fs, lb_later);
+                        else
+                            chunk(std::integral_constant<int, PW>(), c, s1, tl, nseg, first,
+                                  lb_near, lb_fs, lb_later);
+                    }
+                    first = false;
+                    __syncthreads();
+                } while (cur_t < J->ntypes);
 #pragma unroll
-                for (int q = 0; q < P; ++q) out[q] = first ? acc[q] : prev[q] + acc[q];
-                return true;
-            };
-            // A chunk of up to P * 256 of the bin's insertions, slots
-            // c + q * 256 + tid: points generated and energies loaded and
-            // stored for this pass.
-            auto chunk = [&](auto pw, uint64_t c, uint64_t end, const Tile &tl, int nseg,
-                             bool first, double lb_near, double lb_fs, double lb_later) {
-                constexpr int P = decltype(pw)::value;
-                double px[P], py[P], pz[P], prev[P], out[P];
-                uint32_t ins[P];
-                bool ok[P];
-#pragma unroll
-                for (int q = 0; q < P; ++q) {
-                    const uint64_t p = c + (uint64_t)(q * kWG + tid);
-                    ok[q] = p < end;
-                    ins[q] = J->sorted[ok[q] ? p : c];
-                    double f[3];
-                    widom_point(J->seed, J->stream, ins[q], f);
-                    frac_to_cart(J->t, f[0], f[1], f[2], px[q], py[q], pz[q]);
-                    px[q] -= tl.cx;
-                    py[q] -= tl.cy;
-                    pz[q] -= tl.cz;
-                    prev[q] = first ? 0.0 : J->e_out[ins[q]];
-                }
-                if (!one_pass(pw, px, py, pz, ok, prev, out, tl, nseg, first, lb_near, lb_fs,
-                              lb_later))
-                    return;
-#pragma unroll
-                for (int q = 0; q < P; ++q)
-                    if (ok[q]) J->e_out[ins[q]] = out[q];
-            };
-            // A bin whose insertions fit one chunk (at most PW * 256, most
-            // bins) keeps each lane's points and partial energies in
-            // registers across the passes and writes the energies once; the
-            // passes add the same terms in the same order as the chunked
-            // form, which stores and reloads them after every pass.
-            auto resident = [&](auto pw, const double (&X)[PW], const double (&Y)[PW],
-                                const double (&Z)[PW], const bool (&OK)[PW], double (&T)[PW],
-                                const Tile &tl, int nseg, bool first, double lb_near,
-                                double lb_fs, double lb_later) {
-                constexpr int P = decltype(pw)::value;
-                double px[P], py[P], pz[P], prev[P], out[P];
-                bool ok[P];
-#pragma unroll
-                for (int q = 0; q < P; ++q) {
-                    px[q] = X[q];
-                    py[q] = Y[q];
-                    pz[q] = Z[q];
-                    ok[q] = OK[q];
-                    prev[q] = first ? 0.0 : T[q];
-                }
-                if (!one_pass(pw, px, py, pz, ok, prev, out, tl, nseg, first, lb_near, lb_fs,
-                              lb_later))
-                    return;
-#pragma unroll
-                for (int q = 0; q < P; ++q) T[q] = out[q];
-            };
-            const int b = (tc[0] * J->nbins[1] + tc[1]) * J->nbins[2] + tc[2];
-            const uint32_t s0 = J->bin_start[b], s1 = J->bin_start[b + 1];
-            if (s0 == s1) continue;
-            const Tile tl = cell_sphere(J, tc);
-            // one chunk: this wave's points per lane (wave-uniform; 0 for a
-            // wave with no slot); several chunks: -1.  Only the FP32-grid /
-            // Widom pair math keeps bins resident: Widom jobs never run with
-            // the other variants, whose registers the resident state would
-            // only crowd (FP64 grids would drop to three waves per SIMD).
-            const uint64_t wv0 = s0 + (uint64_t)(tid & ~63);
-            const int mode = (MATH != MATH_MIXED || s1 - s0 > (uint32_t)(PW * kWG)) ? -1
-                             : wv0 >= s1                     ? 0
-                             : (PW > 1 && wv0 + kWG >= s1)   ? 1
-                                                             : PW;
-            double rx[PW], ry[PW], rz[PW], rt[PW];
-            uint32_t rins[PW];
-            bool rok[PW];
-#pragma unroll
-            for (int q = 0; q < PW; ++q) {
-                rx[q] = ry[q] = rz[q] = rt[q] = 0.0;
-                rins[q] = 0;
-                rok[q] = false;
-                if (q < mode) {
-                    const uint64_t p = s0 + (uint64_t)(q * kWG + tid);
-                    rok[q] = p < s1;
-                    rins[q] = J->sorted[rok[q] ? p : s0];
-                    double f[3];
-                    widom_point(J->seed, J->stream, rins[q], f);
-                    frac_to_cart(J->t, f[0], f[1], f[2], rx[q], ry[q], rz[q]);
-                    rx[q] -= tl.cx;
-                    ry[q] -= tl.cy;
-                    rz[q] -= tl.cz;
-                }
+                for (int q = 0; q < PW; ++q)
+                    if (q < mode && rok[q]) J->e_out[rins[q]] = rt[q];
             }
-            int cur_t = 0, cur_pos = uniform(tbeg[0]);
-            bool first = true;
-            do {
-                const int nseg = fill_list<MATH, kWG>(J, src, sidx, tbeg, tl, cur_t, cur_pos, cap, s_list,
-                                                 s_seg, s_cnt);
-                __syncthreads();
-                // -eps_ij for every record of this pass (near; far and shell)
-                // and every source record after it
-                double lb_near = 0.0, lb_fs = 0.0, lb_later = 0.0;
-                if (J->sat_e > 0.0) {
-                    for (int sg = 0; sg < nseg; ++sg) {
-                        const int *g = s_seg + kSegInts * sg, *e = g + kSegInts;
-                        const double eps = 0.25 * J->types[uniform(g[0])].eps4;
-                        lb_fs -= eps * J->fs_floor *
-                                 (double)(uniform(e[1]) - uniform(g[1]) + uniform(e[2]) -
-                                          uniform(g[2]));
-                        lb_near -= eps * (double)(uniform(e[3]) - uniform(g[3]));
-                    }
-                    // source records after this pass, each at -eps of its type:
-                    // the rest of the current type, then every later type
-                    if (cur_t < J->ntypes) {
-                        lb_later = -0.25 * J->types[cur_t].eps4 *
-                                   (double)(uniform(tbeg[cur_t + 1]) - cur_pos);
-                        for (int u = cur_t + 1; u < J->ntypes; ++u)
-                            lb_later -= 0.25 * J->types[u].eps4 *
-                                        (double)(uniform(tbeg[u + 1]) - uniform(tbeg[u]));
-                    }
-                }
-                if (mode == PW)
-                    resident(std::integral_constant<int, PW>(), rx, ry, rz, rok, rt, tl, nseg,
-                             first, lb_near, lb_fs, lb_later);
-                else if (PW > 1 && mode == 1)
-                    resident(std::integral_constant<int, 1>(), rx, ry, rz, rok, rt, tl, nseg,
-                             first, lb_near, lb_fs, lb_later);
-                for (uint64_t c = s0; mode < 0 && c < s1; c += (uint64_t)(PW * kWG)) {
-                    const uint64_t w0 = c + (uint64_t)(tid & ~63);  // wave-uniform
-                    if (w0 >= s1) continue;
-                    if (PW > 1 && w0 + kWG >= s1)
-                        chunk(std::integral_constant<int, 1>(), c, s1, tl, nseg, first, lb_near,
-                              lb_fs, lb_later);
-                    else
-                        chunk(std::integral_constant<int, PW>(), c, s1, tl, nseg, first, lb_near,
-                              lb_fs, lb_later);
-                }
-                first = false;
-                __syncthreads();
-            } while (cur_t < J->ntypes);
-#pragma unroll
-            for (int q = 0; q < PW; ++q)
-                if (q < mode && rok[q]) J->e_out[rins[q]] = rt[q];
-        }
         }
     }
 }
@@ -2271,7 +2275,9 @@ __global__ __launch_bounds__(64 * WAVES * PARTS, 4) void k_parts(const JobDev *_
             if (pwave == 0 ? ok[0] : ok[1]) {
                 if (!grid) J->e_out[o] = total;
                 else if (J->mode == OUT_F64) ((double *)J->out)[o] = total;
-                else ((float *)J->out)[o] = (float)(total < (double)FLT_MAX ? total : (double)FLT_MAX);
+                else
+                    ((float *)J->out)[o] =
+                        (float)(total < (double)FLT_MAX ? total : (double)FLT_MAX);
             }
         }
         if (grid) return;
@@ -2467,7 +2473,8 @@ int bin_blocks(uint64_t n, int chunk) { return (int)((n + (uint64_t)chunk - 1) /
 // flushes its whole histogram, which a chunk of 2 insertions per key pays for.
 int bin_chunk(uint64_t total_insertions, long long max_keys) {
     int chunk = kBinWG;
-    while (chunk < kBinChunkMax && ((uint64_t)chunk * 1024 < total_insertions || chunk < 2 * max_keys))
+    while (chunk < kBinChunkMax &&
+           ((uint64_t)chunk * 1024 < total_insertions || chunk < 2 * max_keys))
         chunk <<= 1;
     return chunk;
 }
@@ -2485,7 +2492,8 @@ hipError_t launch_bin_all(const BinJob *jobs, int njobs, long long total_blocks,
                           bool cleared, hipStream_t s) {
     if (njobs <= 0 || total_blocks <= 0) return hipSuccess;
     if (chunk < kBinWG || chunk > kBinChunkMax || (chunk & (chunk - 1)) ||
-        total_blocks > (1LL << 31) - 1 || max_keys <= 0 || max_keys > kBinLdsKeys || max_group < 1 ||
+        total_blocks > (1LL << 31) - 1 || max_keys <= 0 || max_keys > kBinLdsKeys ||
+        max_group < 1 ||
         max_group > kBinGroupMax || total_groups < 0 || total_groups > (1LL << 31) - 1)
         return hipErrorInvalidValue;
     const size_t lds_bytes = sizeof(uint32_t) * (size_t)max_keys;

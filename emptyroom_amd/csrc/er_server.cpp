@@ -461,8 +461,9 @@ void Server::run() {
                     if (part) {
                         e = launch_widom_partials(r->wb.e, (long long)r->spec.n_ins,
                                                   r->spec.temperature, part, s);
-                        if (e == hipSuccess) e = launch_widom_final(part, reduce_blocks((long long)r->spec.n_ins),
-                                               r->h_sums, s);
+                        if (e == hipSuccess)
+                            e = launch_widom_final(part, reduce_blocks((long long)r->spec.n_ins),
+                                                   r->h_sums, s);
                         if (e == hipSuccess) e = hipEventRecord(r->reduced, s);
                     }
                     if (e != hipSuccess) {

@@ -10,7 +10,7 @@
 // 156, 16 MiB 970 / 630, 64 MiB 6640 / 2240, 256 MiB 25700 / 7260.  Uploads above
 // 1 MiB reach 30 GB/s by the runtime's own path, which they keep.
 //
-// The contexts of a device share one Transfer (the pinned memory, 18 MiB at
+// The contexts of a device share one Transfer (the pinned memory, 19 MiB at
 // most, and the threads are made by the first copy that uses them and given back
 // with the last context).  One copy at a time uses it; a copy that finds it in
 // use takes the runtime's path.  The ring is taken when the stream has ended what is
