@@ -663,15 +663,26 @@ hipError_t launch_cc_block(const CCGrid *grids, int ng, long long total_blocks, 
     return hipGetLastError();
 }
 
-// Records pay for their pass when insertions outnumber the voxels, and not where
-// the grid fits the L2 of an XCD but its records (four times as large) do not.
-// us without / with records (their pass included), 1e7 insertions: 0.8 MB grid
-// 166 / 95, 4.0 MB 165 / 160, 7.9 MB 324 / 188, 16 MB 502 / 222, 42 MB 660 / 258;
-// 1e6 insertions: 0.8 MB 23 / 22, 7.9 MB 37 / 35, 16 MB 55 / 47, 42 MB 71 / 69.
+// Insertions from which the records pay for their pass (and not at all where the grid
+// fits the L2 of an XCD but its records, four times as large, do not).  us without /
+// with records, their pass included, either side of the line:
+//   0.1e6 voxels  1e6 insertions 33 / 33, 1.5e6 40 / 38, 1e7 164 / 100
+//   0.26e6        1e6 33 / 38, 2e6 48 / 45, 1e7 172 / 104
+//   1.0e6         1e7 165 / 160
+//   1.33e6        2e6 59 / 61, 3e6 80 / 77, 1e7 223 / 189
+//   1.52e6        1.5e6 52 / 56, 3e6 86 / 80
+//   1.76e6        1e6 46 / 48, 2e6 74 / 64
+//   2.0e6         1e6 50 / 48, 2e6 83 / 65, 4e6 148 / 100
+//   1.06e7        5.3e6 366 / 172;  1.25e8  6.2e7 4695 / 2252
 size_t tri_faces_bytes(const int n[3], uint64_t nins) {
-    const uint64_t nv = (uint64_t)n[0] * n[1] * n[2];
+    const uint64_t nv = (uint64_t)n[0] * n[1] * n[2], million = 1000000;
     const bool fits = nv <= (1u << 18), large = nv >= 1300000 && nv <= (1u << 27);
-    if (!(fits || large) || nins < 1000000 || nins < nv / 2) return 0;
+    const uint64_t from = fits            ? million + 4 * nv
+                          : nv < 1750000  ? 2 * nv
+                          : nv < 2000000  ? nv
+                          : nv / 2 < million ? million
+                                             : nv / 2;
+    if (!(fits || large) || nins < from) return 0;
     return sizeof(float4) * (size_t)(n[1] - 1) * (n[2] - 1) * n[0];
 }
 
