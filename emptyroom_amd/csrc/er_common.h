@@ -160,7 +160,7 @@ constexpr int kBinLdsKeys = 7168;    // keys a binning block histograms in LDS (
 constexpr long long kBinsMax = (long long)kBinLdsKeys * kBinGroupMax;
 constexpr int kRegionRecords = 8192;  // entries of one workgroup's region sub-list (near-list
                                       // indices, 32 KiB)
-constexpr int kBlockList = 3072;  // of these, entries of a block's list (see grid_block)
+constexpr int kBlockList = 6144;  // of these, entries of a block's list (see grid_block)
 // Margin (Angstrom) applied to every list classification so that FP64 rounding
 // of radii and distances can never misclassify a pair.
 constexpr double kMargin = 1e-6;
