@@ -629,10 +629,12 @@ bool use_nodes(const FrameworkDev *fw, const int n[3], const int tile[3], const 
     lo += R;
     const double hi = fw->rc - R;
     const double pi = 3.14159265358979323846;
-    const double far = hi > lo ? 4.0 / 3.0 * pi * (hi * hi * hi - lo * lo * lo) * fw->n_atoms /
-                                     std::max(fw->volume, 1e-9)
-                               : 0.0;
-    return blocks >= kNodeMinBlocks && far >= kNodeMinFar;
+    const double dens = 4.0 / 3.0 * pi * fw->n_atoms / std::max(fw->volume, 1e-9);
+    const double far = hi > lo ? dens * (hi * hi * hi - lo * lo * lo) : 0.0;
+    // ... and a list of the others that fits its room (0.6 atoms/A^3 at 0.14 A, 7000
+    // others: 16.5 ms without, 20.7 with blocks that turn nodes down one by one)
+    const double rest = dens * std::pow(fw->rc + R, 3.0) - far;
+    return blocks >= kNodeMinBlocks && far >= kNodeMinFar && rest <= 0.9 * kBlockList;
 }
 
 }  // namespace
