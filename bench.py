@@ -6,8 +6,8 @@ cell lengths U[8,40] A, angles U[60,120] deg, grid spacing in {0.1,0.2,0.5} A
 (FP32 grids), 1e6 Widom insertions each at 298 K, guests CH4/Xe/Kr, r_c 12.5 A.
 
 A step is one pass of the hot path over the whole batch: every grid and every
-Widom run, launched as one batch (binning kernels, one persistent tiled-kernel
-launch, reductions).  Inputs are resident in HBM before the timed region.
+Widom run, launched as one batch (binning kernels, a persistent tiled-kernel launch
+for each of its variants, reductions).  Inputs are resident in HBM before the timed region.
 After the timed steps, the default run also measures:
 - the plain path (one framework per launch, synchronous, grids left
   resident as the batch leaves them) on the same work: batched/plain, against
@@ -28,7 +28,12 @@ After the timed steps, the default run also measures:
   rejections, framework uploads avoided by residency).
 
 value = pair-evals/s in the reference's enumeration (P*N*I for grids plus
-n_ins*N*I for Widom, the same count for every path).
+n_ins*N*I for Widom, the same count for every path), so a rate of the
+reference's work, not of pairs evaluated here: interpolated far fields and
+saturated insertions count in full.  roofline.achieved likewise is the direct
+method's work per second; roofline.valu_issue is the share of the device's
+VALU issue slots that the launches use (instructions from the committed
+counters).
 """
 import argparse
 import json
@@ -45,6 +50,7 @@ sys.path.insert(0, ROOT)
 PEAK_FP32_TFLOPS = 157.3  # MI355X FP32 vector peak (packed FP32)
 PEAK_FP32_UNPACKED_TFLOPS = 78.6  # without packed FP32, as this build compiles
 PEAK_FP64_TFLOPS = 78.6  # MI355X FP64 vector peak
+VALU_ISSUE_PER_S = 256 * 2.4e9  # wave instructions: one a clock and CU (four SIMDs, four clocks)
 TARGET_BATCHED_OVER_PLAIN = 5.0
 DEFAULT_TUNING_FILE = os.path.join(ROOT, "emptyroom_amd", "tuning", "mi355x_config3.json")
 WORKLOAD_TEXT = {
@@ -442,10 +448,10 @@ def bench_copy():
 TRAFFIC_FILE = os.path.join(ROOT, "profiles", "k_tiles_traffic_config3_256fw.txt")
 
 
-def measured_traffic(tuning, n_frameworks):
-    """HBM bytes per launch of the batched k_tiles dispatch from the committed
-    rocprofv3 FETCH_SIZE / WRITE_SIZE runs (scaled by the copy calibration),
-    if they were taken on this workload and tuning; else None."""
+def measured_counters(tuning, n_frameworks):
+    """(HBM bytes, VALU wave instructions) of the grid-only launches from the
+    committed rocprofv3 runs (bytes scaled by the copy calibration), if they
+    were taken on this workload and tuning; else (None, None)."""
     try:
         kv = {}
         with open(TRAFFIC_FILE) as fh:
@@ -456,11 +462,12 @@ def measured_traffic(tuning, n_frameworks):
         knobs = {k: v for k, v in tuning.items() if k != "source"}
         filed = {k: v for k, v in json.loads(kv["tuning"]).items() if k != "source"}
         if int(kv["frameworks"]) != n_frameworks or filed != knobs:
-            return None
-        return (float(kv["fetch_kib"]) * float(kv["fetch_scale"]) +
-                float(kv["write_kib"]) * float(kv["write_scale"])) * 1024.0
+            return None, None
+        return ((float(kv["fetch_kib"]) * float(kv["fetch_scale"]) +
+                 float(kv["write_kib"]) * float(kv["write_scale"])) * 1024.0,
+                float(kv["valu_insts"]))
     except (OSError, KeyError, ValueError):
-        return None
+        return None, None
 
 
 def batch_kernel_ms(api, ctx, tasks, runs):
@@ -792,6 +799,9 @@ def main():
 
     value = (grid_pe + widom_pe) / t_batched
     ratio = (plain_s / t_batched) if plain_s else None
+    traffic = valu_insts = None
+    if args.workload == "config3" and gprec == api.ER_FP32:
+        traffic, valu_insts = measured_counters(tuning, len(fws))
     out = {
         "metric": "LJ pair-evals/s + Widom inserts/s, batched vs plain, at K_H rel err <=1e-4",
         "value": value,
@@ -833,21 +843,25 @@ def main():
                      "frac": achieved / PEAK_FP32_TFLOPS,
                      "attainable_peak": PEAK_FP32_UNPACKED_TFLOPS,
                      "frac_attainable": achieved / PEAK_FP32_UNPACKED_TFLOPS,
-                     "traffic": measured_traffic(tuning, len(fws))
-                     if args.workload == "config3" and gprec == api.ER_FP32 else None,
-                     "kernel": f"k_tiles<{tuning['ppl']},MIXED>, its variant with nodes and "
-                               f"k_parts on the step's {len(fws)} grids alone (a launch each)"
+                     "valu_issue": valu_insts / (VALU_ISSUE_PER_S * grid_ms / 1e3)
+                     if valu_insts else None,
+                     "traffic": traffic,
+                     "kernel": f"k_tiles<{tuning['ppl']},MIXED> and its variants with nodes and "
+                               f"for small grids, on the step's {len(fws)} grids alone (a launch "
+                               "each)"
                                if gprec == api.ER_FP32 else
-                               f"k_tiles<{tuning['ppl']},FP64> and k_parts on the step's grids "
-                               "alone",
+                               f"k_tiles<{tuning['ppl']},FP64> and its variant for small grids, "
+                               "on the step's grids alone",
                      "kernel_ms": grid_ms,
                      "flop_per_pair": FLOP_PER_PAIR,
                      "incut_pairs": incut_grid,
-                     "note": "16 FLOP x every in-cutoff pair of the step's grids / the grid-only "
-                             "launches: the direct method's work per second (the far pairs of "
-                             "fine grids are evaluated at an eighth of the points and "
-                             "interpolated); peak 157.3 is the packed-FP32 rate, which this "
-                             "build does not use (attainable_peak 78.6)"},
+                     "note": "achieved and frac: 16 FLOP x every in-cutoff pair of the step's grids "
+                             "/ the grid-only launches, the direct method's work per second, not "
+                             "issued FLOPs (the far pairs of fine grids are evaluated at an "
+                             "eighth of the points and interpolated); valu_issue: VALU wave "
+                             "instructions of the committed counter run / issue slots (256 CUs x "
+                             "2.4 GHz) of this run; peak 157.3 is the packed-FP32 rate, which "
+                             "this build does not use (attainable_peak 78.6)"},
         "widom_alone": {"kernel_ms": widom_ms, "insertions_per_s": n_ins / (widom_ms / 1e3),
                         "incut_pairs": incut_widom,
                         "note": "insertions stop once their energy is certain to reach 800 T "

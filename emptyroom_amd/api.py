@@ -417,7 +417,7 @@ def henry_result(sum_b: float, sum_eb: float, n_total: float, temperature: float
 
 
 class Batch:
-    """Many (framework, grid, Widom) tasks in one persistent launch / hipGraph."""
+    """Many (framework, grid, Widom) tasks in a launch per kernel variant / hipGraph."""
 
     def __init__(self, ctx: Context, tasks: Sequence[dict], use_graph: bool = True):
         arr = (Task * max(len(tasks), 1))()

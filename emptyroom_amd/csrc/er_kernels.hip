@@ -1561,8 +1561,8 @@ __device__ bool build_region_list(const JobDev *__restrict__ J, double cx, doubl
 // directly, as without nodes.  Direct tiles are bound by VALU issue (98% of the
 // cycles), and at 0.1 A half of what they issue is for such pairs: a grid of
 // 1.48e7 points and 3000 atoms (0.21 atoms/A^3) issued 5.0e9 wave instructions
-// in 10.3 ms and with nodes 3.5e9 in 7.2 ms (6.9 ms now); one of 4.9e7 points and
-// 2400 atoms (0.05 atoms/A^3) took 10.6, then 7.8 ms (6.7 now).
+// in 10.3 ms and with nodes 3.5e9 in 7.2 ms (6.6 ms now); one of 4.9e7 points and
+// 2400 atoms (0.05 atoms/A^3) took 10.6, then 7.8 ms (6.4 now).
 //
 // Accuracy: an atom at D from the middle of a segment of half-length h through
 // the box has a Chebyshev interpolation error on it of at most
@@ -1574,7 +1574,7 @@ __device__ bool build_region_list(const JobDev *__restrict__ J, double cx, doubl
 // less than the FP32 arithmetic of the same pairs rounds off.  The nodes' pairs are
 // evaluated in FP64 like those of an FP64 grid: interpolated FP32 sums were up to 8%
 // further off (rms) than direct tiles, FP64 ones are 8 to 40% nearer
-// (|E| < 1000 K, 0.07 to 0.12 A), for 2 to 3% of the grid's time.
+// (|E| < 1000 K, 0.07 to 0.12 A), for 3 to 5% of the grid's time.
 //
 // Returns no nodes if the block's list does not fit kBlockList entries, which
 // depends on the block alone.

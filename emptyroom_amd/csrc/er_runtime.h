@@ -262,7 +262,7 @@ int grid_energies(Context *ctx, GridDev *g, const double *frac_host, uint64_t n,
 // from < 0 = no link); returns the number of pockets, -1 on bad links.
 int classify_pockets(int nseg, const int *links, long long nlinks, std::vector<uint8_t> *pocket);
 
-// Batched path: many (framework, grid, Widom) tasks in one persistent launch,
+// Batched path: many (framework, grid, Widom) tasks in a launch per kernel variant,
 // captured in a hipGraph on first run and replayed.
 struct Task {
     FrameworkDev *fw = nullptr;

@@ -193,7 +193,7 @@ void er_henry_result(double sum_b, double sum_eb, double n_total, double tempera
 
 /* ---- batched path ----------------------------------------------------------
  * No reference counterpart (the reference runs one framework per process).
- * Many (framework, grid, Widom) tasks run as one persistent launch; with
+ * Many (framework, grid, Widom) tasks run as a launch per kernel variant; with
  * use_graph the whole batch is captured in a hipGraph on the first run and
  * replayed afterwards.  Results are identical to the plain path. */
 typedef struct er_task {
